@@ -67,6 +67,11 @@ struct idgx_batch
     int qbegin[2][idgx::kMaxClasses][idgx::kQueues + 1] = {};
     int single_qbegin[2][idgx::kQueues + 1] = {};
     int *d_counters = nullptr;
+    // Classes that take the separable kernels: their tables, and in device memory the
+    // subgrids heaviest first, then per direction the marks of those left to the per-pair kernels.
+    bool separable[idgx::kMaxClasses] = {};
+    idgx::SeparableTables tables[idgx::kMaxClasses] = {};
+    int *d_order[idgx::kMaxClasses] = {};
     // Degridder pixels prepared once per subgrid and pass (per class): split words, FP16 scales, slot n table.
     uint4 *d_prepared[idgx::kMaxClasses] = {};
     int *d_prepared_scale[idgx::kMaxClasses] = {};
@@ -163,6 +168,28 @@ struct Item
     uint2 v;
     double cost;
 };
+
+// Subgrids by visibility count, most first, equal ones in plan order (a counting sort over 2^16 ranges of counts, each
+// sorted only where it holds more than one count).
+std::vector<int> heaviest_first(const std::vector<int64_t> &V)
+{
+    const int64_t most = *std::max_element(V.begin(), V.end());
+    constexpr int64_t kRanges = 1 << 16;
+    const int64_t width = most / kRanges + 1;
+    std::vector<int> start(static_cast<size_t>(most / width) + 2, 0), order(V.size());
+    const auto range = [&](int64_t v) { return static_cast<size_t>((most - v) / width); };
+    for (const int64_t v : V)
+        ++start[range(v) + 1];
+    for (size_t r = 1; r < start.size(); ++r)
+        start[r] += start[r - 1];
+    std::vector<int> at(start);
+    for (size_t s = 0; s < V.size(); ++s)
+        order[at[range(V[s])]++] = static_cast<int>(s);
+    for (size_t r = 0; width > 1 && r + 1 < start.size(); ++r)
+        std::stable_sort(order.begin() + start[r], order.begin() + start[r + 1],
+                         [&](int x, int y) { return V[x] > V[y]; });
+    return order;
+}
 
 // Work items of class k with tile shape `shape`, heaviest first.
 std::vector<Item> build_items(const idgx_batch *b, bool gridder, int k, int shape)
@@ -373,6 +400,27 @@ int make_queue_args(const idgx_batch *b, const idgx_batch_data *d, bool gridder,
     return IDGX_OK;
 }
 
+// Counters of one direction: the queues', then each class's "any leftover" flag (cleared together before a run).
+constexpr int kDirCounters = idgx::kMaxClasses * idgx::kQueues + idgx::kMaxClasses;
+
+// Class k's subgrids through the separable kernel; q.cls[k] then names the ones it leaves to the per-pair launch.
+hipError_t run_separable(idgx_batch *b, QueueArgs &q, int k, bool gridder, hipStream_t st)
+{
+    const int dir = gridder ? 0 : 1;
+    KernelArgs &a = q.cls[k];
+    if (!gridder || !b->separable[k] || a.p.nr_subgrids == 0)
+        return hipSuccess;
+    idgx::SeparableArgs sp{};
+    sp.tables = b->tables[k];
+    sp.order = b->d_order[k];
+    sp.leftover = b->d_order[k] + (1 + dir) * static_cast<size_t>(a.p.nr_subgrids);
+    sp.leftover_any = b->d_counters + dir * kDirCounters + idgx::kMaxClasses * idgx::kQueues + k;
+    const hipError_t e = idgx::launch_grid_separable(a, sp, b->precision, st);
+    a.leftover = sp.leftover;
+    a.leftover_any = sp.leftover_any;
+    return e;
+}
+
 // One persistent launch per class (each with its own tile shape), or only class `only` when it is >= 0; in
 // single-launch mode (and `only` < 0) one launch over the merged queue.
 int run(idgx_batch *b, const idgx_batch_data *d, bool gridder, hipStream_t st, int only = -1)
@@ -382,14 +430,18 @@ int run(idgx_batch *b, const idgx_batch_data *d, bool gridder, hipStream_t st, i
     int rc = make_queue_args(b, d, gridder, q);
     if (rc != IDGX_OK)
         return rc;
-    constexpr int kDirCounters = idgx::kMaxClasses * idgx::kQueues;
     hipError_t e = idgx::launch_reset_counters(b->d_counters + dir * kDirCounters, kDirCounters, st);
     b->last_launches[dir] = 0;
     if (only < 0 && single_mode(b, dir))
     {
-        for (int k = 0; k < b->nr_classes && e == hipSuccess && !gridder && !plain(b); ++k)
-            if (b->nr_items[dir][k] > 0)
+        for (int k = 0; k < b->nr_classes && e == hipSuccess && !plain(b); ++k)
+        {
+            if (b->nr_items[dir][k] == 0)
+                continue;
+            e = run_separable(b, q, k, gridder, st);
+            if (e == hipSuccess && !gridder)
                 e = idgx::launch_degrid_prepare(q.cls[k], b->precision, st);
+        }
         if (e != hipSuccess || b->single_items[dir] == 0)
             return to_status(e);
         q.items = b->d_items[dir] + b->single_offset[dir];
@@ -406,15 +458,21 @@ int run(idgx_batch *b, const idgx_batch_data *d, bool gridder, hipStream_t st, i
     {
         if ((only >= 0 && k != only) || b->nr_items[dir][k] == 0)
             continue;
-        if (!gridder && !plain(b))
-            e = idgx::launch_degrid_prepare(q.cls[k], b->precision, st);
+        QueueArgs qk = q;
+        for (int j = 0; j < b->nr_classes; ++j)
+            if (j != k)
+                qk.cls[j].p.nr_subgrids = 0; // this launch's work is class k's
+        if (!plain(b))
+            e = run_separable(b, qk, k, gridder, st);
+        if (e == hipSuccess && !gridder && !plain(b))
+            e = idgx::launch_degrid_prepare(qk.cls[k], b->precision, st);
         if (e != hipSuccess)
             break;
-        q.items = b->d_items[dir] + b->offset[dir][k];
-        std::memcpy(q.queue_begin, b->qbegin[dir][k], sizeof(q.queue_begin));
-        q.nr_queues = idgx::kQueues;
-        q.counter = b->d_counters + dir * kDirCounters + k * idgx::kQueues;
-        e = launch_queue(b, q, gridder, b->shape[dir][k], b->workgroups[dir][k], st);
+        qk.items = b->d_items[dir] + b->offset[dir][k];
+        std::memcpy(qk.queue_begin, b->qbegin[dir][k], sizeof(qk.queue_begin));
+        qk.nr_queues = idgx::kQueues;
+        qk.counter = b->d_counters + dir * kDirCounters + k * idgx::kQueues;
+        e = launch_queue(b, qk, gridder, b->shape[dir][k], b->workgroups[dir][k], st);
         b->last_launches[dir] += e == hipSuccess;
     }
     return to_status(e);
@@ -484,7 +542,22 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
         e = hipMalloc(&b->d_items[dir], std::max<size_t>(1, 2 * total) * sizeof(uint2));
     }
     if (e == hipSuccess)
-        e = hipMalloc(&b->d_counters, 2 * idgx::kMaxClasses * idgx::kQueues * sizeof(int));
+        e = hipMalloc(&b->d_counters, 2 * kDirCounters * sizeof(int));
+    for (int k = 0; k < nr_classes && e == hipSuccess; ++k)
+    {
+        const idgx_plan &p = b->plans[k];
+        idgx::PlanDev geometry{};
+        geometry.S = p.subgrid_size;
+        geometry.image_size = p.image_size;
+        b->separable[k] = p.nr_subgrids > 0 && idgx::separable_tables(geometry, b->precision, b->tables[k]);
+        if (!b->separable[k])
+            continue;
+        const std::vector<int> order = heaviest_first(b->vis_count[k]);
+        // The order, then each direction's leftover marks.
+        e = hipMalloc(&b->d_order[k], 3 * order.size() * sizeof(int));
+        if (e == hipSuccess)
+            e = hipMemcpy(b->d_order[k], order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice);
+    }
     for (int k = 0; k < nr_classes && e == hipSuccess && !plain(b); ++k)
     {
         const int S = b->plans[k].subgrid_size;
@@ -846,6 +919,8 @@ extern "C" void idgx_batch_destroy(idgx_batch *b)
         (void)hipFree(b->d_counters);
     for (int k = 0; k < idgx::kMaxClasses; ++k)
     {
+        if (b->d_order[k])
+            (void)hipFree(b->d_order[k]);
         if (b->d_prepared[k])
             (void)hipFree(b->d_prepared[k]);
         if (b->d_prepared_scale[k])

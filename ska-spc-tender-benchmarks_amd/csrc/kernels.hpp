@@ -34,6 +34,10 @@ struct KernelArgs
     const uint4 *prepared;
     const int *prepared_scale;
     const float4 *slot_coord;
+    // Batches whose subgrids take the separable kernels first: per subgrid, 1 where they left it to the per-pair
+    // kernels, and whether they left any (null: every subgrid is the per-pair kernels').
+    const int *leftover;
+    const int *leftover_any;
 };
 
 // Persistent-kernel work over up to kMaxClasses subgrid classes (one subgrid size each): the items are
@@ -90,6 +94,21 @@ __device__ __forceinline__ bool next_queue_item(const QueueArgs &q, int &cls, in
     return true;
 }
 
+// Whether any class of a per-pair launch has subgrids for it (uniform over the launch).
+__device__ __forceinline__ bool queue_has_work(const QueueArgs &q)
+{
+    for (int k = 0; k < kMaxClasses; ++k)
+        if (q.cls[k].p.nr_subgrids > 0 && (!q.cls[k].leftover_any || *q.cls[k].leftover_any))
+            return true;
+    return false;
+}
+
+// Whether the separable kernels have done subgrid s (uniform over the workgroup).
+__device__ __forceinline__ bool subgrid_done(const KernelArgs &a, int s)
+{
+    return a.leftover && !a.leftover[s];
+}
+
 // Gridder queue "shape" of a single launch over several classes in which each item takes its class's tiles per
 // wave (QueueArgs::tiles: 2, 3, 4, 6 or 8), with the default LDS batch and phases on the VALU.
 constexpr int kShapeTilesPerClass = IDGX_SHAPE_TILES_PER_CLASS;
@@ -130,6 +149,25 @@ __host__ __device__ inline int degrid_row_stride(int S)
 {
     return (S + 3) & ~3;
 }
+
+// Separable forms of the split mixed kernels (fp16x3, bf16x3).  Column x's additive part of n, and its factor of n's
+// remainder relative to the corner's, by its distance from the centre; eps = 2 pi x the remainder at the corner.
+constexpr int kSeparableMax = 64; // largest subgrid size
+struct SeparableTables
+{
+    float a[kSeparableMax / 2], g[kSeparableMax / 2];
+    float eps, a_max;
+};
+struct SeparableArgs
+{
+    SeparableTables tables;
+    const int *order;  // workgroup -> subgrid (null: plan order)
+    int *leftover;     // per subgrid: 1 where the per-pair kernels have to run (null: they run inside the launch)
+    int *leftover_any; // set to 1 with the first of them
+};
+// Whether the plan's subgrids take the separable kernels, and their tables.
+bool separable_tables(const PlanDev &p, int precision, SeparableTables &t);
+hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, hipStream_t st);
 
 hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream);
 hipError_t launch_degrid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream);

@@ -86,9 +86,13 @@ template <int DT, bool SPLIT, int PT, int VB, bool PM>
 __global__ __launch_bounds__(kThreads, (gridder_min_blocks<PT, VB>())) void gridder_mfma_queue(QueueArgs q)
 {
     __shared__ GridderShared<PT, VB> sm;
+    if (!queue_has_work(q))
+        return;
     int cls, s, blk;
     while (next_queue_item(q, cls, s, blk))
     {
+        if (subgrid_done(q.cls[cls], s))
+            continue;
         gridder_item<DT, SPLIT, PT, VB, PM>(q.cls[cls], s, blk, sm);
         __syncthreads();
     }
@@ -101,9 +105,13 @@ template <int DT, bool SPLIT>
 __global__ __launch_bounds__(kThreads, (gridder_min_blocks<8, kDefaultVB>())) void gridder_mfma_queue_tiles(QueueArgs q)
 {
     __shared__ GridderShared<8, kDefaultVB> sm;
+    if (!queue_has_work(q))
+        return;
     int cls, s, blk;
     while (next_queue_item(q, cls, s, blk))
     {
+        if (subgrid_done(q.cls[cls], s))
+            continue;
         switch (q.tiles[cls]) // workgroup-uniform
         {
         case 2:
@@ -432,6 +440,9 @@ hipError_t launch_queue(const QueueArgs &q, int precision, bool gridder, int sha
 
 hipError_t launch_grid_mixed(const KernelArgs &a, int precision, bool pm, hipStream_t st)
 {
+    SeparableArgs sp{};
+    if (!pm && separable_tables(a.p, precision, sp.tables))
+        return launch_grid_separable(a, sp, precision, st);
     switch (precision)
     {
     case IDGX_MIXED_BF16X3:

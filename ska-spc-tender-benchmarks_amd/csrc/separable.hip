@@ -1,0 +1,728 @@
+// Separable mixed-precision gridder for gfx950: phasors per (row, visibility) and per (column,
+// visibility) instead of per (pixel, visibility), contracted on v_mfma_f32_16x16x32_{f16,bf16}.
+//
+// Phase.  With half-integer pixel coordinates xh = x + 1/2 - S/2 (l = xh delta, delta = image_size / S) the phase of a
+// visibility at a pixel is, in revolutions,
+//     qu xh + qv yh + dw n(l, m),    qu = du delta, qv = dv delta  (du, dv, dw relative to the subgrid's centre).
+// The w-term is taken apart in two steps.  Per subgrid, w0 = the middle of the range of w over its visibilities:
+// e^{2 pi i w0 n} is one exact rotation per pixel, applied to the gridder's result.
+// For the rest, d = dw - w0, n splits into an additive part and a remainder that is a product to about 1e-6 of itself:
+//     n(l, m) = a(l) + a(m) + c g(l) g(m),   a(l) = n(l, l0) - n(l0, l0) / 2,  l0 = l_max / sqrt(2),
+// where c = n's remainder at the corner and g, |g| <= 1, its profile along the edge (n = (l^2 + m^2) / 2 + (l^2 + m^2)^2
+// / 8 + ..., so the remainder is (l^2 - l0^2)(m^2 - l0^2) / 4 to first order: 3.5e-7 at a field of 0.1 rad).  So
+//     e^{2 pi i phase} = X(x) Y(y) (1 + i eps g(x) g(y)),   eps = 2 pi c d,
+//     X = e^{2 pi i (qu xh + d a(x))},  Y = e^{2 pi i (qv yh + d a(y))}
+// up to eps^2 / 2.  Subgrids with |eps| <= kEpsNone run without the product term; up to kEpsMost with it; the others
+// (fields far wider than 0.1 rad, or w far from constant over a subgrid) take the per-pair items.
+//
+// Contraction, on v_mfma_f32_32x32x16: pixel[y][x, corr] = sum_v Y[y][v] (V[v][corr] X[v][x]), one real GEMM
+// with the rows (y, re/im), the columns (x, corr) and k = (v, re/im): the rows hold Y's two real embeddings, the B operand
+// the product V X, which a lane forms in FP32 for one (x, corr) and four visibilities and splits into hi/lo halves: per
+// (pixel, visibility) pair 1/S of that work.  Three MFMAs per tile (hi hi, lo hi, hi lo; BF16 also lo lo) and one for the
+// product term, whose factor i eps g(y) goes into a second set of rows and g(x) into the columns, as single halves (eps
+// <= 1e-3 scales their rounding).  A wave owns all rows of NT column tiles (8 columns x 4 correlations each) and its own
+// chunks of visibilities; no operand passes through LDS, and the waves only meet when their sums are added.
+//
+// What bounds it: the matrix cores, at the power limit.  A pair costs 128 flop there (4 products of 32).  On 128 stations,
+// 64 channels, 76,865 subgrids of 32^2 (136.3 G pairs) a pass is 17.4 PFLOP, 14.7 ms at the rate a large FP16 product
+// reaches on the card (1186 TFLOP/s, clocks at 1.7 to 2.0 GHz).  Measured: 41.2 -> 15.8 ms; the per-pair kernel, 8.25 VALU instructions per pair (two of them transcendental), was VALU-issue bound at
+// 97 %; this one issues 2.2.  The interleaving of MFMA and VALU instructions (scheduling groups, wave priorities)
+// and the tile (16 x 16 x 32: more cycles at a higher clock) moved the time by less than 3 %.
+#include "mixed_device.hpp"
+
+#include <algorithm>
+#include <cmath>
+#include <cstddef>
+
+namespace idgx
+{
+namespace
+{
+constexpr float kEpsNone = 3e-7F; // below the FP32 rounding of the phases
+constexpr float kEpsMost = 1e-3F; // eps^2 / 2 <= 5e-7 at one corner pixel for the visibility farthest in w
+constexpr float kTurnsMost = 4.F; // |d a|: keeps the phases' FP32 rounding at the level of qu xh
+constexpr float kTermScale = 1024.F; // moves the product term's factors into FP16's normal range
+// Plans take these kernels where a spread of w of S / image_size wavelengths (the subgrid's own extent in u and v)
+// stays within four times kEpsMost: fields up to about 0.17 rad at S = 32, 0.13 at S = 64.  In wider ones the per-pair
+// items would often run inside these kernels, at fewer waves per SIMD than in their own.
+constexpr double kSeparableField = 4e-3;
+constexpr int kFewSubgrids = 256;  // the CUs: a workgroup per subgrid would leave some of them idle
+constexpr int kChunk = 64;        // visibilities a wave stages at a time, one per lane
+constexpr int kValStride = 80;    // staged values of one correlation (64, padded: fewer LDS bank conflicts)
+
+// One wave's staged visibilities.
+struct alignas(16) GridStage
+{
+    float qu[kChunk], qv[kChunk], de[kChunk];
+    float2 val[4][kValStride];
+};
+// LDS of a workgroup: a column's (a, g) at its index, and one of the phases' working sets.
+template <int TAB, int COLS, int SPLITS> struct alignas(16) GridLds
+{
+    float2 tab[TAB];
+    union
+    {
+        GridStage stage[kWaves];
+        float2 sum[SPLITS][16 * COLS * 4]; // the splits' partial sums of 16 rows
+        GridderShared<kDefaultPT, kDefaultVB> direct;
+    };
+};
+struct WRange
+{
+    double centre; // middle of k w / 2 pi over the subgrid's rows and channels
+    float half;    // half its width
+};
+
+// Range of w (wavelengths) over a subgrid's rows and channel window; every thread of the workgroup gets the same.
+// (LDS-only barriers: the first visibilities' loads stay in flight across them.)
+template <int WAVES>
+__device__ __forceinline__ WRange w_range(const KernelArgs &a, long long row0, int T, int c0, int nc, float *slots)
+{
+    float wlo = __builtin_inff(), whi = -__builtin_inff(), klo = __builtin_inff(), khi = -__builtin_inff();
+    for (int t = threadIdx.x; t < T; t += 64 * WAVES)
+    {
+        const float w = a.uvw[3 * (row0 + t) + 2];
+        wlo = fminf(wlo, w);
+        whi = fmaxf(whi, w);
+    }
+    for (int c = threadIdx.x; c < nc; c += 64 * WAVES)
+    {
+        const float k = a.wavenumbers[c0 + c];
+        klo = fminf(klo, k);
+        khi = fmaxf(khi, k);
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1)
+    {
+        wlo = fminf(wlo, __shfl_xor(wlo, d));
+        whi = fmaxf(whi, __shfl_xor(whi, d));
+        klo = fminf(klo, __shfl_xor(klo, d));
+        khi = fmaxf(khi, __shfl_xor(khi, d));
+    }
+    if ((threadIdx.x & 63) == 0)
+    {
+        float *s = slots + 4 * (threadIdx.x >> 6);
+        s[0] = wlo, s[1] = whi, s[2] = klo, s[3] = khi;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+    {
+        wlo = fminf(wlo, slots[4 * w]);
+        whi = fmaxf(whi, slots[4 * w + 1]);
+        klo = fminf(klo, slots[4 * w + 2]);
+        khi = fmaxf(khi, slots[4 * w + 3]);
+    }
+    lds_barrier();
+    const double p0 = static_cast<double>(wlo) * klo, p1 = static_cast<double>(wlo) * khi;
+    const double p2 = static_cast<double>(whi) * klo, p3 = static_cast<double>(whi) * khi;
+    const double lo = fmin(fmin(p0, p1), fmin(p2, p3)) * kInv2Pi, hi = fmax(fmax(p0, p1), fmax(p2, p3)) * kInv2Pi;
+    return {0.5 * (lo + hi), static_cast<float>(0.5 * (hi - lo))};
+}
+
+// Reduced phase coordinates of one visibility, signed by sgn: slopes per pixel in [-1/2, 1/2], w relative to the
+// subgrid's middle, and the parity of the whole turns taken off the slopes (half-integer coordinates turn each of
+// them into half a turn: a factor -1).
+struct Slopes
+{
+    float qu, qv, de;
+    bool odd;
+};
+
+__device__ __forceinline__ Slopes reduce_slopes(float u, float v, float w, float k, const CentreOffsets &o, double wc,
+                                                double delta, float sgn)
+{
+    const double kk = static_cast<double>(k) * kInv2Pi;
+    const double qu = __builtin_fma(kk, static_cast<double>(u), -o.u) * delta;
+    const double qv = __builtin_fma(kk, static_cast<double>(v), -o.v) * delta;
+    const double ru = __builtin_rint(qu), rv = __builtin_rint(qv);
+    const double turns = 0.5 * (ru + rv);
+    Slopes s;
+    s.qu = sgn * static_cast<float>(qu - ru);
+    s.qv = sgn * static_cast<float>(qv - rv);
+    s.de = sgn * static_cast<float>(__builtin_fma(kk, static_cast<double>(w), -wc));
+    s.odd = turns != __builtin_rint(turns);
+    return s;
+}
+
+// n(l, m) = 1 - sqrt(1 - r^2) by its series: within 1e-11 of itself for r^2 <= 0.02 (fields up to 0.2 rad).
+__device__ __forceinline__ double pixel_n_series(double l, double m)
+{
+    const double r2 = __builtin_fma(l, l, m * m);
+    double p = 33.0 / 2048.0;
+    p = __builtin_fma(p, r2, 21.0 / 1024.0);
+    p = __builtin_fma(p, r2, 7.0 / 256.0);
+    p = __builtin_fma(p, r2, 5.0 / 128.0);
+    p = __builtin_fma(p, r2, 1.0 / 16.0);
+    p = __builtin_fma(p, r2, 1.0 / 8.0);
+    p = __builtin_fma(p, r2, 1.0 / 2.0);
+    return p * r2;
+}
+
+// e^{2 pi i w n} of pixel (x, y).
+__device__ __forceinline__ cfloat pixel_rotation(int x, int y, int S, double delta, double w)
+{
+    const double n = pixel_n_series((x + 0.5 - 0.5 * S) * delta, (y + 0.5 - 0.5 * S) * delta);
+    double t = w * n;
+    t -= __builtin_rint(t);
+    const float f = static_cast<float>(t);
+    return {__builtin_amdgcn_cosf(f), __builtin_amdgcn_sinf(f)};
+}
+
+// (vr + i vi) (cs + i sn) with the phasor of lane J of the quad: four FMA-class instructions that read the phasor
+// through DPP (the compiler would copy it first).  The leading s_nop covers the two wait states between a VALU write
+// and a DPP read of the same register.
+template <int J> __device__ __forceinline__ cfloat quad_product(float cs, float sn, float vr, float vi)
+{
+    cfloat r;
+    if constexpr (J == 0)
+        asm("s_nop 1\n\t"
+            "v_mul_f32_dpp %0, %2, %4 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %1, %2, %5 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %0, -%3, %5 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %3, %4 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf"
+            : "=&v"(r.re), "=&v"(r.im)
+            : "v"(cs), "v"(sn), "v"(vr), "v"(vi));
+    else if constexpr (J == 1)
+        asm("s_nop 1\n\t"
+            "v_mul_f32_dpp %0, %2, %4 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %1, %2, %5 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %0, -%3, %5 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %3, %4 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf"
+            : "=&v"(r.re), "=&v"(r.im)
+            : "v"(cs), "v"(sn), "v"(vr), "v"(vi));
+    else if constexpr (J == 2)
+        asm("s_nop 1\n\t"
+            "v_mul_f32_dpp %0, %2, %4 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %1, %2, %5 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %0, -%3, %5 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %3, %4 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf"
+            : "=&v"(r.re), "=&v"(r.im)
+            : "v"(cs), "v"(sn), "v"(vr), "v"(vi));
+    else
+        asm("s_nop 1\n\t"
+            "v_mul_f32_dpp %0, %2, %4 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %1, %2, %5 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %0, -%3, %5 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %3, %4 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf"
+            : "=&v"(r.re), "=&v"(r.im)
+            : "v"(cs), "v"(sn), "v"(vr), "v"(vi));
+    return r;
+}
+
+// Element-wise products of packed halves: a * b for FP16 (v_pk_mul_f16).
+__device__ __forceinline__ uint32_t mul_f16x2(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, a) * __builtin_bit_cast(f16x2, b));
+}
+
+// The two rows of a phasor c + i s (packed pairs along k): re = (c, -s), im = (s, c), hi and lo halves.
+template <int DT>
+__device__ __forceinline__ void split_rows(float c, float s, uint32_t &re_hi, uint32_t &re_lo, uint32_t &im_hi,
+                                           uint32_t &im_lo)
+{
+    re_hi = pack2<DT>(c, -s);
+    im_hi = pack2<DT>(s, c);
+    float rc, rs;
+    if constexpr (DT == kFP16)
+    {
+        rs = sub_f16_lo(s, im_hi);
+        rc = sub_f16_hi(c, im_hi);
+    }
+    else
+    {
+        float h0, h1;
+        unpack2<DT>(im_hi, h0, h1);
+        rs = s - h0;
+        rc = c - h1;
+    }
+    re_lo = pack2<DT>(rc, -rs);
+    im_lo = pack2<DT>(rs, rc);
+}
+
+// The rows of i f (c + i s) in single halves, from the split rows (FP16) or the phasor (BF16): re = -f (s, c),
+// im = f (c, -s).
+template <int DT>
+__device__ __forceinline__ void term_rows(float c, float s, float f, uint32_t re_hi, uint32_t im_hi, uint32_t &re,
+                                          uint32_t &im)
+{
+    if constexpr (DT == kFP16)
+    {
+        const f16x2 ff = __builtin_bit_cast(f16x2, pack2<DT>(f, f));
+        re = __builtin_bit_cast(uint32_t, -ff * __builtin_bit_cast(f16x2, im_hi));
+        im = __builtin_bit_cast(uint32_t, ff * __builtin_bit_cast(f16x2, re_hi));
+    }
+    else
+    {
+        re = pack2<DT>(-f * s, -f * c);
+        im = pack2<DT>(f * c, -f * s);
+    }
+}
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// D[32][32] += A[32][16] B[16][32]: lane l holds A[l % 32][8 (l / 32) + 0..7], B[8 (l / 32) + 0..7][l % 32] and
+// D[8 (i / 4) + 4 (l / 32) + i % 4][l % 32] in element i.  Twice the tile of the 16 x 16 form per instruction: with two
+// waves per SIMD and 6 to 8 VALU instructions beside each, 15 to 19 ns per instruction against 2 x (11 to 15) ns.
+template <int DT> __device__ __forceinline__ f32x16 mfma32(const uint32_t *a, const uint32_t *b, f32x16 c)
+{
+    const u32x4 av = {a[0], a[1], a[2], a[3]}, bv = {b[0], b[1], b[2], b[3]};
+    if constexpr (DT == kFP16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, av), __builtin_bit_cast(f16x8, bv), c, 0,
+                                                      0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv), c,
+                                                       0, 0, 0);
+}
+
+// Swaps a's odd 16-lane rows with b's even ones.
+__device__ __forceinline__ void swap_rows16(uint32_t &a, uint32_t &b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+// The order of a wave's own LDS writes and reads (no other wave touches its staging).
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ---- gridder ----------------------------------------------------------------------------------------------------
+
+// Rows of the gridder's GEMM in tiles of 32: pairs of tiles hold re and im of 32 subgrid rows; with an odd number of
+// 16-row blocks the last tile holds both of 16.
+template <int YT> struct RowCoords
+{
+    static constexpr int kPairs = YT / 2, kBlocks = kPairs + YT % 2;
+    float yh[kBlocks], ya[kBlocks], yg[kBlocks]; // this lane's row of each block: coordinate, a, term factor
+};
+
+// 8 staged visibilities onto the wave's pixels: all rows, NT tiles of 8 columns x 4 correlations.
+template <int DT, int YT, int NT, bool TERM>
+__device__ __forceinline__ void grid_step(const GridStage &st, const float2 *tab, int base, int x0, float half_s,
+                                          const RowCoords<YT> &rc, f32x16 (&acc)[NT][YT])
+{
+    const int lane = threadIdx.x & 63, corr = lane & 3;
+    const int v = base + 4 * (lane >> 5);
+    uint32_t ah[YT][4], al[YT][4], at[YT][4];
+    if constexpr (YT >= 2)
+    {
+        const f32x4 qv = *reinterpret_cast<const f32x4 *>(&st.qv[v]);
+        const f32x4 de = *reinterpret_cast<const f32x4 *>(&st.de[v]);
+#pragma unroll
+        for (int t = 0; t < YT / 2; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const float ph = __builtin_fmaf(qv[j], rc.yh[t], de[j] * rc.ya[t]);
+                const float sn = __builtin_amdgcn_sinf(ph), cs = __builtin_amdgcn_cosf(ph);
+                split_rows<DT>(cs, sn, ah[2 * t][j], al[2 * t][j], ah[2 * t + 1][j], al[2 * t + 1][j]);
+                if constexpr (TERM)
+                    term_rows<DT>(cs, sn, de[j] * rc.yg[t], ah[2 * t][j], ah[2 * t + 1][j], at[2 * t][j],
+                                  at[2 * t + 1][j]);
+            }
+    }
+    if constexpr (YT % 2 == 1)
+    {
+        // Lanes l and l + 16 share a row: each forms the phasors of two of the four visibilities, then they swap, so
+        // that the first holds all four real rows and the second all four imaginary ones.
+        const int w = v + 2 * ((lane >> 4) & 1);
+        const float2 qv = *reinterpret_cast<const float2 *>(&st.qv[w]);
+        const float2 de = *reinterpret_cast<const float2 *>(&st.de[w]);
+        constexpr int t = YT - 1, k = YT / 2;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+        {
+            const float d = j ? de.y : de.x;
+            const float ph = __builtin_fmaf(j ? qv.y : qv.x, rc.yh[k], d * rc.ya[k]);
+            const float sn = __builtin_amdgcn_sinf(ph), cs = __builtin_amdgcn_cosf(ph);
+            split_rows<DT>(cs, sn, ah[t][j], al[t][j], ah[t][j + 2], al[t][j + 2]);
+            if constexpr (TERM)
+            {
+                term_rows<DT>(cs, sn, d * rc.yg[k], ah[t][j], ah[t][j + 2], at[t][j], at[t][j + 2]);
+                swap_rows16(at[t][j], at[t][j + 2]);
+            }
+            swap_rows16(ah[t][j], ah[t][j + 2]);
+            swap_rows16(al[t][j], al[t][j + 2]);
+        }
+    }
+    // This lane's column phasor is that of visibility v + corr; the quad shares its four.
+    const float qux = st.qu[v + corr], dex = st.de[v + corr];
+    const f32x4 v01 = *reinterpret_cast<const f32x4 *>(&st.val[corr][v]);
+    const f32x4 v23 = *reinterpret_cast<const f32x4 *>(&st.val[corr][v + 2]);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+    {
+        const int x = x0 + 8 * nt + ((lane & 31) >> 2);
+        const float2 tb = tab[x];
+        const float ph = __builtin_fmaf(qux, static_cast<float>(x) - half_s, dex * tb.x);
+        const float sn = __builtin_amdgcn_sinf(ph), cs = __builtin_amdgcn_cosf(ph);
+        const cfloat vx[4] = {quad_product<0>(cs, sn, v01[0], v01[1]), quad_product<1>(cs, sn, v01[2], v01[3]),
+                              quad_product<2>(cs, sn, v23[0], v23[1]), quad_product<3>(cs, sn, v23[2], v23[3])};
+        uint32_t bh[4], bl[4], bt[4];
+        const uint32_t gg = pack2<DT>(tb.y, tb.y);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            split2<DT>(vx[j].re, vx[j].im, bh[j], bl[j]);
+            if constexpr (TERM)
+                bt[j] = DT == kFP16 ? mul_f16x2(bh[j], gg) : pack2<DT>(vx[j].re * tb.y, vx[j].im * tb.y);
+        }
+#pragma unroll
+        for (int t = 0; t < YT; ++t)
+            acc[nt][t] = mfma32<DT>(ah[t], bh, acc[nt][t]);
+#pragma unroll
+        for (int t = 0; t < YT; ++t)
+            acc[nt][t] = mfma32<DT>(al[t], bh, acc[nt][t]);
+#pragma unroll
+        for (int t = 0; t < YT; ++t)
+            acc[nt][t] = mfma32<DT>(ah[t], bl, acc[nt][t]);
+        if constexpr (DT == kBF16) // its lo x lo is 2^-18 of the product: above the other errors
+        {
+#pragma unroll
+            for (int t = 0; t < YT; ++t)
+                acc[nt][t] = mfma32<DT>(al[t], bl, acc[nt][t]);
+        }
+        if constexpr (TERM)
+        {
+#pragma unroll
+            for (int t = 0; t < YT; ++t)
+                acc[nt][t] = mfma32<DT>(at[t], bt, acc[nt][t]);
+        }
+    }
+}
+
+struct RawVisibility
+{
+    float4 x0, x1;
+    float u, v, w, k;
+    bool valid;
+};
+
+__device__ __forceinline__ RawVisibility load_visibility(const KernelArgs &a, const Selection &sel, int v, int V,
+                                                         int T, int nc, long long row0, int c0)
+{
+    RawVisibility r;
+    r.x0 = r.x1 = make_float4(0.F, 0.F, 0.F, 0.F);
+    r.u = r.v = r.w = r.k = 0.F;
+    r.valid = false;
+    if (v < V)
+    {
+        int t, c;
+        sel.at(v, t, c);
+        if (entry_ok(t, c, T, nc))
+        {
+            const long long row = row0 + t;
+            const float4 *vis = reinterpret_cast<const float4 *>(a.visibilities) + (row * a.p.nr_channels + c0 + c) * 2;
+            r.x0 = vis[0];
+            r.x1 = vis[1];
+            r.u = a.uvw[3 * row];
+            r.v = a.uvw[3 * row + 1];
+            r.w = a.uvw[3 * row + 2];
+            r.k = a.wavenumbers[c0 + c];
+            r.valid = true;
+        }
+    }
+    return r;
+}
+
+// One wave's chunks of V visibilities: chunk `first` (whose visibilities are in raw), then every step-th.  n
+// visibilities per chunk, a multiple of 8, at most kChunk.
+template <int DT, int YT, int NT, bool TERM>
+__device__ __forceinline__ int grid_sum(const KernelArgs &a, const SeparableArgs &sp, const Selection &sel, int V, int T,
+                                        int nc, long long row0, int c0, const CentreOffsets &off, double wc,
+                                        int first, int step, int n, RawVisibility raw, int x0, GridStage &st,
+                                        const float2 *tab, f32x16 (&acc)[NT][YT])
+{
+    const int lane = threadIdx.x & 63;
+    const double delta = static_cast<double>(a.p.image_size) / a.p.S;
+    const float half_s = 0.5F * static_cast<float>(a.p.S) - 0.5F;
+    RowCoords<YT> rc;
+#pragma unroll
+    for (int t = 0; t < RowCoords<YT>::kBlocks; ++t)
+    {
+        const int y = 32 * t + (t < YT / 2 ? lane & 31 : lane & 15);
+        rc.yh[t] = static_cast<float>(y) - half_s;
+        rc.ya[t] = tab[y].x;
+        rc.yg[t] = tab[y].y * (sp.tables.eps * kTermScale * kTermScale); // tab holds g / kTermScale
+    }
+    int scale_exp = -126; // FP16: power-of-two scale of the staged visibilities
+    for (int v0 = first * n; v0 < V; v0 += step * n)
+    {
+        cfloat val[4] = {{raw.x0.x, raw.x0.y}, {raw.x0.z, raw.x0.w}, {raw.x1.x, raw.x1.y}, {raw.x1.z, raw.x1.w}};
+        Slopes s = {0.F, 0.F, 0.F, false};
+        if (raw.valid)
+            s = reduce_slopes(raw.u, raw.v, raw.w, raw.k, off, wc, delta, -1.F);
+        float f = s.odd ? -1.F : 1.F;
+        if constexpr (DT == kFP16)
+        {
+            float m = 0.F;
+#pragma unroll
+            for (int pol = 0; pol < 4; ++pol)
+                m = fmaxf(m, fmaxf(fabsf(val[pol].re), fabsf(val[pol].im)));
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1)
+                m = fmaxf(m, __shfl_xor(m, d));
+            const int e_new = max(scale_exp, __builtin_amdgcn_readfirstlane(scale_exponent(m)));
+            if (e_new > scale_exp)
+            {
+                const float r = ldexpf(1.F, scale_exp - e_new);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int t = 0; t < YT; ++t)
+                        acc[nt][t] *= r;
+                scale_exp = e_new;
+            }
+            f *= ldexpf(1.F, -scale_exp);
+        }
+        wave_lds_fence();
+        st.qu[lane] = s.qu;
+        st.qv[lane] = s.qv;
+        st.de[lane] = s.de;
+#pragma unroll
+        for (int pol = 0; pol < 4; ++pol)
+            st.val[pol][lane] = make_float2(val[pol].re * f, val[pol].im * f);
+        wave_lds_fence();
+        // The next chunk's visibilities, in flight during the sums.
+        raw = load_visibility(a, sel, lane < n ? v0 + step * n + lane : V, V, T, nc, row0, c0);
+        const int nsteps = min(n, V - v0 + 7) >> 3;
+        for (int k = 0; k < nsteps; ++k)
+            grid_step<DT, YT, NT, TERM>(st, tab, 8 * k, x0, half_s, rc, acc);
+    }
+    return scale_exp;
+}
+
+// Columns (x, a(x) and g(x)) of the subgrid in LDS; g is scaled for the product term's columns.
+__device__ __forceinline__ void fill_table(float2 *tab, const SeparableArgs &sp, int S)
+{
+    const int x = threadIdx.x;
+    if (x < kSeparableMax)
+    {
+        const int j = x >= S / 2 ? min(x - S / 2, kSeparableMax / 2 - 1) : S / 2 - 1 - x;
+        tab[x] = make_float2(sp.tables.a[j], sp.tables.g[j] * (1.F / kTermScale));
+    }
+}
+
+// Workgroup (part, subgrid) grids columns [part, part + 1) x 8 NT NX of a subgrid: its waves take NX column ranges and
+// kWaves / NX interleaved chunks of visibilities; the partial sums meet in LDS 16 rows at a time, in a fixed order.
+template <int DT, int YT, int NT, int NX>
+__global__ __launch_bounds__(kThreads, YT * NT <= 2 ? 4 : YT * NT <= 3 ? 3 : 2)
+    void grid_separable(KernelArgs a, SeparableArgs sp)
+{
+    constexpr int kCols = NX * NT * 8, kSplits = kWaves / NX;
+    __shared__ GridLds<kSeparableMax, kCols, kSplits> sm;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int part = blockIdx.x / a.p.nr_subgrids, b = blockIdx.x - part * a.p.nr_subgrids;
+    const int s = sp.order ? sp.order[b] : b;
+    const int S = a.p.S, P = S * S;
+    const idgx_metadata m = a.metadata[s];
+    int c0, nc;
+    channel_window(a, s, c0, nc);
+    const long long row0 = first_row(a.metadata, m);
+    const bool ok = subgrid_in_bounds(a.p, m, row0, c0, nc);
+    Selection sel;
+    const int T = m.nr_timesteps, V = ok ? selection_of(a, s, T, nc, sel) : 0;
+    // Chunks short enough for every split to have one.
+    const int split = wave / NX, n = min(kChunk, ((V + kSplits - 1) / kSplits + 7) & ~7);
+    RawVisibility raw = load_visibility(a, sel, lane < n ? split * n + lane : V, V, T, nc, row0, c0);
+    WRange wr = {0.0, 0.F};
+    if (V > 0)
+        wr = w_range<kWaves>(a, row0, T, c0, nc, reinterpret_cast<float *>(sm.tab));
+    const float eps = wr.half * sp.tables.eps;
+    const bool fits = eps <= kEpsMost && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
+    if (sp.leftover && tid == 0 && part == 0)
+    {
+        sp.leftover[s] = fits ? 0 : 1;
+        if (!fits)
+            *sp.leftover_any = 1;
+    }
+    if (!fits)
+    {
+        if (!sp.leftover && part == 0)
+        {
+            const int items = (grid_units(S, kDefaultPT).units + kWaves - 1) / kWaves;
+            for (int i = 0; i < items; ++i)
+            {
+                gridder_item<DT, true, kDefaultPT, kDefaultVB, false>(a, s, i, sm.direct);
+                __syncthreads();
+            }
+        }
+        return; // uniform
+    }
+    fill_table(sm.tab, sp, S);
+    lds_barrier();
+    const CentreOffsets off = centre_offsets(a.p, m);
+    const double delta = static_cast<double>(a.p.image_size) / S;
+    f32x16 acc[NT][YT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int t = 0; t < YT; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                acc[nt][t][i] = 0.F;
+    const int xb = part * kCols, x0 = xb + (wave % NX) * NT * 8;
+    int scale_exp;
+    if (eps <= kEpsNone)
+        scale_exp = grid_sum<DT, YT, NT, false>(a, sp, sel, V, T, nc, row0, c0, off, wr.centre, split, kSplits, n, raw,
+                                                x0, sm.stage[wave], sm.tab, acc);
+    else
+        scale_exp = grid_sum<DT, YT, NT, true>(a, sp, sel, V, T, nc, row0, c0, off, wr.centre, split, kSplits, n, raw,
+                                               x0, sm.stage[wave], sm.tab, acc);
+    const float unscale = DT == kFP16 ? ldexpf(1.F, scale_exp) : 1.F;
+    float2 *out = reinterpret_cast<float2 *>(a.subgrids_out) + static_cast<size_t>(s) * kCorr * P;
+    const float4 *aterms = reinterpret_cast<const float4 *>(a.aterms);
+    const size_t abase = ok ? static_cast<size_t>(m.aterm_index) * a.p.nr_stations : 0;
+    const double w0 = V > 0 ? off.w - wr.centre : 0.0; // minus the gridder's sign
+    const int h = lane >> 5, xi = (lane & 31) >> 2, corr = lane & 3;
+    const int cols = min(kCols, S - xb);
+#pragma unroll
+    for (int t = 0; t < YT; ++t) // 16 rows of the subgrid at a time
+    {
+        if (16 * t >= S)
+            break; // uniform
+        constexpr int kPairs = YT / 2;
+        const bool paired = t < 2 * kPairs;
+        // This thread's pixels' A-terms, in flight while the sums meet in LDS.
+        constexpr int kPer = (16 * kCols + kThreads - 1) / kThreads;
+        cfloat a1[kPer][4], a2[kPer][4];
+        float taper[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+        {
+            const int q = tid + i * kThreads, row = q / cols, x = xb + q - row * cols, y = 16 * t + row;
+            if (row < 16 && y < S && ok)
+            {
+                const int p = y * S + x;
+                load_jones(aterms, (abase + m.station1) * P + p, a1[i]);
+                load_jones(aterms, (abase + m.station2) * P + p, a2[i]);
+                taper[i] = a.spheroidal[p];
+            }
+        }
+        lds_barrier(); // the staging, or the previous rows, are done with
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+        {
+            const int x = x0 - xb + 8 * nt + xi;
+            if (x >= cols)
+                continue;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+            {
+                // Row 8 (i / 4) + 4 h + i % 4 of the block.
+                const float re = paired ? acc[nt][t / 2 * 2][t % 2 * 8 + i] : acc[nt][YT - 1][i];
+                const float im = paired ? acc[nt][t / 2 * 2 + (YT > 1)][t % 2 * 8 + i] : acc[nt][YT - 1][8 + i];
+                sm.sum[split][((i / 4 * 8 + 4 * h + i % 4) * cols + x) * 4 + corr] =
+                    make_float2(re * unscale, im * unscale);
+            }
+        }
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+        {
+            const int q = tid + i * kThreads, row = q / cols, x = xb + q - row * cols, y = 16 * t + row;
+            if (row >= 16 || y >= S)
+                continue;
+            const int p = y * S + x;
+            cfloat px[4] = {{0.F, 0.F}, {0.F, 0.F}, {0.F, 0.F}, {0.F, 0.F}};
+            if (ok)
+            {
+                const cfloat r = pixel_rotation(x, y, S, delta, w0);
+#pragma unroll
+                for (int pol = 0; pol < 4; ++pol)
+                {
+                    float2 v = sm.sum[0][q * 4 + pol];
+#pragma unroll
+                    for (int k = 1; k < kSplits; ++k)
+                    {
+                        const float2 u = sm.sum[k][q * 4 + pol];
+                        v = make_float2(v.x + u.x, v.y + u.y);
+                    }
+                    px[pol] = cmul({v.x, v.y}, r);
+                }
+                apply_a1h_p_a2(px, a1[i], a2[i]);
+#pragma unroll
+                for (int pol = 0; pol < 4; ++pol)
+                    px[pol] = {px[pol].re * taper[i], px[pol].im * taper[i]};
+            }
+#pragma unroll
+            for (int pol = 0; pol < 4; ++pol)
+                out[pol * P + p] = make_float2(px[pol].re, px[pol].im);
+        }
+    }
+}
+
+// ---- launchers --------------------------------------------------------------------------------------------------
+
+template <int DT, int YT, int NT, int NX>
+hipError_t launch_grid(const KernelArgs &a, const SeparableArgs &sp, hipStream_t st)
+{
+    const long long parts = (a.p.S + 8 * NT * NX - 1) / (8 * NT * NX), blocks = parts * a.p.nr_subgrids;
+    if (blocks > 0x7fffffffLL)
+        return hipErrorInvalidConfiguration;
+    grid_separable<DT, YT, NT, NX><<<static_cast<unsigned>(blocks), kThreads, 0, st>>>(a, sp);
+    return hipGetLastError();
+}
+
+// Row tiles and column tiles per wave and column ranges for subgrid size S.  One wave holds all columns up to S = 32
+// (128 accumulators); larger subgrids spread them over two or four waves.  A plan that would leave CUs without work
+// takes a workgroup per 8 columns, which forms the row phasors once per 8 columns.
+template <int DT> hipError_t grid_size(const KernelArgs &a, const SeparableArgs &sp, hipStream_t st)
+{
+    const int S = a.p.S;
+    const bool few = a.p.nr_subgrids <= kFewSubgrids;
+    if (S <= 16)
+        return few ? launch_grid<DT, 1, 1, 1>(a, sp, st) : launch_grid<DT, 1, 2, 1>(a, sp, st);
+    if (S <= 32 && few)
+        return launch_grid<DT, 2, 1, 1>(a, sp, st);
+    if (S <= 24)
+        return launch_grid<DT, 2, 3, 1>(a, sp, st);
+    if (S <= 32)
+        return launch_grid<DT, 2, 4, 1>(a, sp, st);
+    if (S <= 48)
+        return few ? launch_grid<DT, 3, 1, 1>(a, sp, st) : launch_grid<DT, 3, 3, 2>(a, sp, st);
+    return few ? launch_grid<DT, 4, 1, 1>(a, sp, st) : launch_grid<DT, 4, 2, 4>(a, sp, st);
+}
+
+double host_n(double l, double m)
+{
+    const double r2 = l * l + m * m;
+    return r2 / (1.0 + std::sqrt(1.0 - r2));
+}
+} // namespace
+
+bool separable_tables(const PlanDev &p, int precision, SeparableTables &t)
+{
+    const int S = p.S;
+    const double image = p.image_size;
+    if ((precision != IDGX_MIXED_FP16X3 && precision != IDGX_MIXED_BF16X3) || S > kSeparableMax || !(image <= 0.2))
+        return false;
+    const int half = S / 2;
+    const double delta = image / S, l_max = (half - 0.5) * delta, l0 = l_max * std::sqrt(0.5);
+    const double a0 = 0.5 * host_n(l0, l0);
+    const auto add = [&](double l) { return host_n(l, l0) - a0; };
+    const double a_edge = add(l_max), c = host_n(l_max, l_max) - 2.0 * a_edge;
+    t = SeparableTables{};
+    double a_max = 0.0;
+    for (int j = 0; j < half; ++j)
+    {
+        const double l = (j + 0.5) * delta, al = add(l);
+        t.a[j] = static_cast<float>(al);
+        t.g[j] = c > 0.0 ? static_cast<float>((host_n(l, l_max) - al - a_edge) / c) : 0.F;
+        a_max = std::max(a_max, std::fabs(al));
+    }
+    t.a_max = static_cast<float>(a_max);
+    t.eps = static_cast<float>(2.0 * M_PI * c);
+    return t.eps * (S / image) <= kSeparableField;
+}
+
+hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, hipStream_t st)
+{
+    return precision == IDGX_MIXED_FP16X3 ? grid_size<kFP16>(a, sp, st) : grid_size<kBF16>(a, sp, st);
+}
+} // namespace idgx
