@@ -67,10 +67,11 @@ struct idgx_batch
     int qbegin[2][idgx::kMaxClasses][idgx::kQueues + 1] = {};
     int single_qbegin[2][idgx::kQueues + 1] = {};
     int *d_counters = nullptr;
-    // Classes that take the separable kernels: their tables, and in device memory the
+    // Classes that take the separable kernels: their tables, most visibilities of one subgrid, and in device memory the
     // subgrids heaviest first, then per direction the marks of those left to the per-pair kernels.
     bool separable[idgx::kMaxClasses] = {};
     idgx::SeparableTables tables[idgx::kMaxClasses] = {};
+    long long most_vis[idgx::kMaxClasses] = {};
     int *d_order[idgx::kMaxClasses] = {};
     // Degridder pixels prepared once per subgrid and pass (per class): split words, FP16 scales, slot n table.
     uint4 *d_prepared[idgx::kMaxClasses] = {};
@@ -408,14 +409,16 @@ hipError_t run_separable(idgx_batch *b, QueueArgs &q, int k, bool gridder, hipSt
 {
     const int dir = gridder ? 0 : 1;
     KernelArgs &a = q.cls[k];
-    if (!gridder || !b->separable[k] || a.p.nr_subgrids == 0)
+    if (!b->separable[k] || a.p.nr_subgrids == 0)
         return hipSuccess;
     idgx::SeparableArgs sp{};
     sp.tables = b->tables[k];
     sp.order = b->d_order[k];
     sp.leftover = b->d_order[k] + (1 + dir) * static_cast<size_t>(a.p.nr_subgrids);
     sp.leftover_any = b->d_counters + dir * kDirCounters + idgx::kMaxClasses * idgx::kQueues + k;
-    const hipError_t e = idgx::launch_grid_separable(a, sp, b->precision, st);
+    sp.per = idgx::separable_chunk(b->most_vis[k], a.p.nr_subgrids);
+    const hipError_t e = gridder ? idgx::launch_grid_separable(a, sp, b->precision, st)
+                                 : idgx::launch_degrid_separable(a, sp, b->precision, b->most_vis[k], st);
     a.leftover = sp.leftover;
     a.leftover_any = sp.leftover_any;
     return e;
@@ -553,6 +556,7 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
         if (!b->separable[k])
             continue;
         const std::vector<int> order = heaviest_first(b->vis_count[k]);
+        b->most_vis[k] = b->vis_count[k][order[0]];
         // The order, then each direction's leftover marks.
         e = hipMalloc(&b->d_order[k], 3 * order.size() * sizeof(int));
         if (e == hipSuccess)

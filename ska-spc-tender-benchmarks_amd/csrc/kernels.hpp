@@ -164,10 +164,15 @@ struct SeparableArgs
     const int *order;  // workgroup -> subgrid (null: plan order)
     int *leftover;     // per subgrid: 1 where the per-pair kernels have to run (null: they run inside the launch)
     int *leftover_any; // set to 1 with the first of them
+    long long per;     // degridder: visibilities per workgroup, a multiple of 256
 };
 // Whether the plan's subgrids take the separable kernels, and their tables.
 bool separable_tables(const PlanDev &p, int precision, SeparableTables &t);
+// Degridder visibilities per workgroup (SeparableArgs::per) for n subgrids of at most max_vis visibilities.
+long long separable_chunk(long long max_vis, int n);
 hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, hipStream_t st);
+hipError_t launch_degrid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, long long max_vis,
+                                   hipStream_t st);
 
 hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream);
 hipError_t launch_degrid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream);

@@ -138,9 +138,12 @@ template <int DT, bool SPLIT, int VT, int PB, bool PM>
 __global__ __launch_bounds__(kThreads, (degridder_min_blocks<VT, PB>())) void degridder_mfma_queue(QueueArgs q)
 {
     __shared__ DegridderShared<VT, PB> sm;
+    if (!queue_has_work(q))
+        return;
     int cls, s, blk;
     while (next_queue_item(q, cls, s, blk))
-        degridder_item<DT, SPLIT, VT, PB, PM, true>(q.cls[cls], s, blk, sm);
+        if (!subgrid_done(q.cls[cls], s))
+            degridder_item<DT, SPLIT, VT, PB, PM, true>(q.cls[cls], s, blk, sm);
 }
 
 __global__ void reset_counters_kernel(int *counters, int n)
@@ -159,6 +162,8 @@ template <int DT, bool SPLIT, int CACHED>
 __global__ __launch_bounds__(kThreads) void degrid_prepare_kernel(KernelArgs a)
 {
     __shared__ unsigned maxbits;
+    if (a.leftover_any && !*a.leftover_any)
+        return; // uniform: the separable kernel has done every subgrid
     const int s = xcd_contiguous(blockIdx.x, gridDim.x), tid = threadIdx.x;
     const int S = a.p.S, P = S * S, Sp = degrid_row_stride(S), nslots = S * Sp;
     float4 *slot_coord = const_cast<float4 *>(a.slot_coord);
@@ -172,6 +177,8 @@ __global__ __launch_bounds__(kThreads) void degrid_prepare_kernel(KernelArgs a)
             slot_coord[q] = make_float4(pixel_offset(sx, S), pixel_offset(sy, S), n, 0.F);
         }
     }
+    if (subgrid_done(a, s))
+        return; // uniform
     const idgx_metadata m = a.metadata[s];
     int c0, nc;
     channel_window(a, s, c0, nc);
@@ -460,6 +467,13 @@ hipError_t launch_grid_mixed(const KernelArgs &a, int precision, bool pm, hipStr
 
 hipError_t launch_degrid_mixed(const KernelArgs &a, int precision, bool pm, hipStream_t st)
 {
+    SeparableArgs sp{};
+    if (!pm && separable_tables(a.p, precision, sp.tables))
+    {
+        const long long vmax = static_cast<long long>(a.p.max_nr_timesteps) * a.p.nr_channels;
+        sp.per = separable_chunk(vmax, a.p.nr_subgrids);
+        return launch_degrid_separable(a, sp, precision, vmax, st);
+    }
     switch (precision)
     {
     case IDGX_MIXED_BF16X3:

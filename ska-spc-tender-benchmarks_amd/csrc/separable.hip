@@ -1,11 +1,11 @@
-// Separable mixed-precision gridder for gfx950: phasors per (row, visibility) and per (column,
+// Separable mixed-precision gridder and degridder for gfx950: phasors per (row, visibility) and per (column,
 // visibility) instead of per (pixel, visibility), contracted on v_mfma_f32_16x16x32_{f16,bf16}.
 //
 // Phase.  With half-integer pixel coordinates xh = x + 1/2 - S/2 (l = xh delta, delta = image_size / S) the phase of a
 // visibility at a pixel is, in revolutions,
 //     qu xh + qv yh + dw n(l, m),    qu = du delta, qv = dv delta  (du, dv, dw relative to the subgrid's centre).
 // The w-term is taken apart in two steps.  Per subgrid, w0 = the middle of the range of w over its visibilities:
-// e^{2 pi i w0 n} is one exact rotation per pixel, applied to the gridder's result.
+// e^{2 pi i w0 n} is one exact rotation per pixel, applied to the gridder's result and to the degridder's pixels.
 // For the rest, d = dw - w0, n splits into an additive part and a remainder that is a product to about 1e-6 of itself:
 //     n(l, m) = a(l) + a(m) + c g(l) g(m),   a(l) = n(l, l0) - n(l0, l0) / 2,  l0 = l_max / sqrt(2),
 // where c = n's remainder at the corner and g, |g| <= 1, its profile along the edge (n = (l^2 + m^2) / 2 + (l^2 + m^2)^2
@@ -15,18 +15,21 @@
 // up to eps^2 / 2.  Subgrids with |eps| <= kEpsNone run without the product term; up to kEpsMost with it; the others
 // (fields far wider than 0.1 rad, or w far from constant over a subgrid) take the per-pair items.
 //
-// Contraction, on v_mfma_f32_32x32x16: pixel[y][x, corr] = sum_v Y[y][v] (V[v][corr] X[v][x]), one real GEMM
+// Contraction, on v_mfma_f32_32x32x16.  Gridder: pixel[y][x, corr] = sum_v Y[y][v] (V[v][corr] X[v][x]), one real GEMM
 // with the rows (y, re/im), the columns (x, corr) and k = (v, re/im): the rows hold Y's two real embeddings, the B operand
 // the product V X, which a lane forms in FP32 for one (x, corr) and four visibilities and splits into hi/lo halves: per
 // (pixel, visibility) pair 1/S of that work.  Three MFMAs per tile (hi hi, lo hi, hi lo; BF16 also lo lo) and one for the
 // product term, whose factor i eps g(y) goes into a second set of rows and g(x) into the columns, as single halves (eps
 // <= 1e-3 scales their rounding).  A wave owns all rows of NT column tiles (8 columns x 4 correlations each) and its own
 // chunks of visibilities; no operand passes through LDS, and the waves only meet when their sums are added.
+// Degridder: H[x, corr][v] = sum_y P[y][x, corr] Y[y][v], the pixels split once per workgroup and read from LDS in the A
+// operand's order, then vis[v][corr] = sum_x X[x][v] H[x, corr][v] on the VALU: 16 FMAs per (column, visibility).
 //
 // What bounds it: the matrix cores, at the power limit.  A pair costs 128 flop there (4 products of 32).  On 128 stations,
 // 64 channels, 76,865 subgrids of 32^2 (136.3 G pairs) a pass is 17.4 PFLOP, 14.7 ms at the rate a large FP16 product
-// reaches on the card (1186 TFLOP/s, clocks at 1.7 to 2.0 GHz).  Measured: 41.2 -> 15.8 ms; the per-pair kernel, 8.25 VALU instructions per pair (two of them transcendental), was VALU-issue bound at
-// 97 %; this one issues 2.2.  The interleaving of MFMA and VALU instructions (scheduling groups, wave priorities)
+// reaches on the card (1186 TFLOP/s, clocks at 1.7 to 2.0 GHz).  Measured: gridder 41.2 -> 15.8 ms, degridder 41.3 ->
+// 15.2 ms; the per-pair kernels, 8.25 VALU instructions per pair (two of them transcendental), were VALU-issue bound at
+// 97 %; these issue 2.2 and 1.7.  The interleaving of MFMA and VALU instructions (scheduling groups, wave priorities)
 // and the tile (16 x 16 x 32: more cycles at a higher clock) moved the time by less than 3 %.
 #include "mixed_device.hpp"
 
@@ -56,6 +59,12 @@ struct alignas(16) GridStage
     float qu[kChunk], qv[kChunk], de[kChunk];
     float2 val[4][kValStride];
 };
+struct alignas(16) DegridStage
+{
+    float qu[kChunk], qv[kChunk], de[kChunk], scale[kChunk];
+    long long out[kChunk];
+};
+
 // LDS of a workgroup: a column's (a, g) at its index, and one of the phases' working sets.
 template <int TAB, int COLS, int SPLITS> struct alignas(16) GridLds
 {
@@ -67,6 +76,23 @@ template <int TAB, int COLS, int SPLITS> struct alignas(16) GridLds
         GridderShared<kDefaultPT, kDefaultVB> direct;
     };
 };
+template <int WAVES> struct alignas(16) DegridLds
+{
+    float2 tab[kSeparableMax];
+    unsigned maxbits;
+    DegridStage stage[WAVES];
+    uint4 pixels[1]; // as many as the subgrid needs
+};
+
+// Bytes of LDS a degridder workgroup takes: the pixels in the A operand's order (hi and lo words of 4 correlations), and
+// never less than the per-pair item's staging.
+template <int WAVES> size_t degrid_lds_bytes(int S, int rows)
+{
+    const size_t cols = static_cast<size_t>((S + 7) / 8) * 8;
+    return std::max(offsetof(DegridLds<WAVES>, pixels) + rows * cols * 4 * 2 * sizeof(uint32_t),
+                    sizeof(DegridderShared<kDefaultVT, kDefaultPB>));
+}
+
 struct WRange
 {
     double centre; // middle of k w / 2 pi over the subgrid's rows and channels
@@ -657,6 +683,307 @@ __global__ __launch_bounds__(kThreads, YT * NT <= 2 ? 4 : YT * NT <= 3 ? 3 : 2)
     }
 }
 
+// ---- degridder --------------------------------------------------------------------------------------------------
+
+// Row blocks of the degridder: its k runs over 8 rows per MFMA, at most 4 of those (32 rows) with their phasors in
+// registers at once.  KS of them per pass and YB passes cover the subgrid's rows.
+//
+// 32 staged visibilities from the subgrid's pixels: element p of `sum` is re / im (p % 2) of correlation p / 2 of
+// visibility base + lane % 32, over this lane half's columns (x % 2 = lane / 32).
+template <int DT, int KS, int YB, bool TERM>
+__device__ __forceinline__ void degrid_tile(const DegridStage &st, const float2 *tab, const uint4 *pixels, int mts,
+                                            int base, float half_s, float eps, float (&sum)[8])
+{
+    const int lane = threadIdx.x & 63, h = lane >> 5, v = base + (lane & 31);
+    const float qu = st.qu[v], qv = st.qv[v], de = st.de[v];
+    const float term = de * eps;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        sum[i] = 0.F;
+#pragma unroll
+    for (int yb = 0; yb < YB; ++yb)
+    {
+        uint32_t reh[KS][4], rel[KS][4], imh[KS][4], iml[KS][4], ret[KS][4], imt[KS][4];
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+        {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const int y = 8 * (yb * KS + k) + 4 * h + j;
+                const float2 tb = tab[y];
+                const float p = __builtin_fmaf(qv, static_cast<float>(y) - half_s, de * tb.x);
+                const float sn = __builtin_amdgcn_sinf(p), cs = __builtin_amdgcn_cosf(p);
+                split_rows<DT>(cs, sn, reh[k][j], rel[k][j], imh[k][j], iml[k][j]);
+                if constexpr (TERM)
+                    term_rows<DT>(cs, sn, term * tb.y, reh[k][j], imh[k][j], ret[k][j], imt[k][j]);
+            }
+        }
+        for (int mt = 0; mt < mts; ++mt)
+        {
+            f32x16 hr, hi;
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                hr[i] = hi[i] = 0.F;
+            const float gx = tab[8 * mt + ((lane & 31) >> 2)].y;
+            const uint32_t gg = pack2<DT>(gx, gx);
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+            {
+                const uint4 *px = pixels + (((yb * KS + k) * 2 + h) * mts + mt) * 64 + (lane & 31);
+                const uint4 wh = px[0], wl = px[32];
+                const uint32_t ph[4] = {wh.x, wh.y, wh.z, wh.w}, pl[4] = {wl.x, wl.y, wl.z, wl.w};
+                hr = mfma32<DT>(ph, reh[k], hr);
+                hi = mfma32<DT>(ph, imh[k], hi);
+                hr = mfma32<DT>(pl, reh[k], hr);
+                hi = mfma32<DT>(pl, imh[k], hi);
+                hr = mfma32<DT>(ph, rel[k], hr);
+                hi = mfma32<DT>(ph, iml[k], hi);
+                if constexpr (DT == kBF16)
+                {
+                    hr = mfma32<DT>(pl, rel[k], hr);
+                    hi = mfma32<DT>(pl, iml[k], hi);
+                }
+                if constexpr (TERM)
+                {
+                    uint32_t pt[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                    {
+                        if constexpr (DT == kFP16)
+                        {
+                            pt[j] = mul_f16x2(ph[j], gg);
+                        }
+                        else
+                        {
+                            float re, im;
+                            unpack2<DT>(ph[j], re, im);
+                            pt[j] = pack2<DT>(re * gx, im * gx);
+                        }
+                    }
+                    hr = mfma32<DT>(pt, ret[k], hr);
+                    hi = mfma32<DT>(pt, imt[k], hi);
+                }
+            }
+            // Element 4 c + pol is column 8 mt + 2 c + h, correlation pol.
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+            {
+                const int x = 8 * mt + 2 * c + h;
+                const float p = __builtin_fmaf(qu, static_cast<float>(x) - half_s, de * tab[x].x);
+                const float sn = __builtin_amdgcn_sinf(p), cs = __builtin_amdgcn_cosf(p);
+#pragma unroll
+                for (int pol = 0; pol < 4; ++pol)
+                {
+                    const float re = hr[4 * c + pol], im = hi[4 * c + pol];
+                    sum[2 * pol] = __builtin_fmaf(cs, re, sum[2 * pol]);
+                    sum[2 * pol] = __builtin_fmaf(-sn, im, sum[2 * pol]);
+                    sum[2 * pol + 1] = __builtin_fmaf(cs, im, sum[2 * pol + 1]);
+                    sum[2 * pol + 1] = __builtin_fmaf(sn, re, sum[2 * pol + 1]);
+                }
+            }
+        }
+    }
+}
+
+struct RawCoords
+{
+    float u, v, w, k;
+    long long out; // -1: no visibility
+};
+
+__device__ __forceinline__ RawCoords load_coords(const KernelArgs &a, const Selection &sel, int v, int v_end, int T,
+                                                 int nc, long long row0, int c0)
+{
+    RawCoords r = {0.F, 0.F, 0.F, 0.F, -1};
+    if (v < v_end)
+    {
+        int t, c;
+        sel.at(v, t, c);
+        if (entry_ok(t, c, T, nc))
+        {
+            const long long row = row0 + t;
+            r.u = a.uvw[3 * row];
+            r.v = a.uvw[3 * row + 1];
+            r.w = a.uvw[3 * row + 2];
+            r.k = a.wavenumbers[c0 + c];
+            r.out = (row * a.p.nr_channels + c0 + c) * 2;
+        }
+    }
+    return r;
+}
+
+// Visibilities [v_begin, v_end) of one subgrid, in chunks interleaved over the waves.
+template <int DT, int KS, int YB, bool TERM>
+__device__ __forceinline__ void degrid_range(const KernelArgs &a, const SeparableArgs &sp, const Selection &sel,
+                                             int v_begin, int v_end, int T, int nc, long long row0, int c0,
+                                             const CentreOffsets &off, double wc, float unscale, const uint4 *pixels,
+                                             int mts, DegridStage &st, const float2 *tab)
+{
+    const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6, lane = threadIdx.x & 63;
+    const double delta = static_cast<double>(a.p.image_size) / a.p.S;
+    const float half_s = 0.5F * static_cast<float>(a.p.S) - 0.5F;
+    float4 *vout = reinterpret_cast<float4 *>(a.visibilities_out);
+    // Chunks of one or two tiles: one where that gives every wave work.
+    const int n = v_end - v_begin <= waves * 32 ? 32 : kChunk;
+    RawCoords raw = load_coords(a, sel, lane < n ? v_begin + wave * n + lane : v_end, v_end, T, nc, row0, c0);
+    for (int v0 = v_begin + wave * n; v0 < v_end; v0 += waves * n)
+    {
+        Slopes s = {0.F, 0.F, 0.F, false};
+        if (raw.out >= 0)
+            s = reduce_slopes(raw.u, raw.v, raw.w, raw.k, off, wc, delta, 1.F);
+        wave_lds_fence();
+        st.qu[lane] = s.qu;
+        st.qv[lane] = s.qv;
+        st.de[lane] = s.de;
+        st.scale[lane] = s.odd ? -unscale : unscale;
+        st.out[lane] = raw.out;
+        wave_lds_fence();
+        // The next chunk's coordinates, in flight during the tiles.
+        raw = load_coords(a, sel, lane < n ? v0 + waves * n + lane : v_end, v_end, T, nc, row0, c0);
+        const int ntiles = min(n, v_end - v0 + 31) >> 5;
+        for (int k = 0; k < ntiles; ++k)
+        {
+            float sum[8];
+            degrid_tile<DT, KS, YB, TERM>(st, tab, pixels, mts, 32 * k, half_s,
+                                          sp.tables.eps * kTermScale * kTermScale, sum);
+            // Both lane halves' columns: the first half keeps correlations 0 and 1, the second 2 and 3.
+            float x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum[i]), __float_as_uint(sum[i + 4]),
+                                                                false, false);
+                x[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+            }
+            const int q = 32 * k + (lane & 31);
+            const long long at = st.out[q];
+            const float f = st.scale[q];
+            if (at >= 0)
+                vout[at + (lane >> 5)] = make_float4(x[0] * f, x[1] * f, x[2] * f, x[3] * f);
+        }
+    }
+}
+
+// Workgroup (chunk, subgrid): degrids visibilities [chunk * per, (chunk + 1) * per) of a subgrid (per a multiple of
+// 256).  The subgrid's pixels (taper, A-terms and the rotation to the middle of its w range applied, FP16: scaled by a
+// power of two) are split once into LDS in the A operand's order; the waves take visibilities and never meet again.
+// WAVES: 4 (two workgroups per CU), or 8 where the pixels take more than half of LDS.
+template <int DT, int KS, int YB, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid_separable(KernelArgs a, SeparableArgs sp)
+{
+    constexpr int kCount = 64 * WAVES;
+    extern __shared__ __align__(16) unsigned char lds[];
+    auto &sm = *reinterpret_cast<DegridLds<WAVES> *>(lds);
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const int chunk = blockIdx.x / a.p.nr_subgrids, b = blockIdx.x - chunk * a.p.nr_subgrids;
+    const int s = sp.order ? sp.order[b] : b;
+    const int S = a.p.S, P = S * S;
+    const idgx_metadata m = a.metadata[s];
+    int c0, nc;
+    channel_window(a, s, c0, nc);
+    const long long row0 = first_row(a.metadata, m);
+    if (!subgrid_in_bounds(a.p, m, row0, c0, nc) || nc == 0)
+    {
+        if (sp.leftover && tid == 0)
+            sp.leftover[s] = 0;
+        return; // uniform: nothing of this subgrid is written
+    }
+    Selection sel;
+    const int T = m.nr_timesteps, V = selection_of(a, s, T, nc, sel);
+    const long long v_first = static_cast<long long>(chunk) * sp.per;
+    if (v_first >= V)
+    {
+        if (sp.leftover && tid == 0 && chunk == 0)
+            sp.leftover[s] = 0;
+        return; // uniform
+    }
+    const int v_begin = static_cast<int>(v_first);
+    const int v_end = static_cast<int>(v_first + sp.per < V ? v_first + sp.per : V);
+    const WRange wr = w_range<WAVES>(a, row0, T, c0, nc, reinterpret_cast<float *>(sm.tab));
+    const float eps = wr.half * sp.tables.eps;
+    const bool fits = eps <= kEpsMost && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
+    if (sp.leftover && tid == 0 && chunk == 0)
+    {
+        sp.leftover[s] = fits ? 0 : 1;
+        if (!fits)
+            *sp.leftover_any = 1;
+    }
+    if (!fits)
+    {
+        if (sp.leftover || tid >= kThreads) // waves that have ended do not take part in the others' barriers
+            return;
+        constexpr int per = kWaves * kDefaultVT * 16;
+        auto &direct = *reinterpret_cast<DegridderShared<kDefaultVT, kDefaultPB> *>(lds);
+        for (int v = v_begin; v < v_end; v += per)
+            degridder_item<DT, true, kDefaultVT, kDefaultPB, false, false>(a, s, v / per, direct);
+        return; // uniform
+    }
+    fill_table(sm.tab, sp, S);
+    const CentreOffsets off = centre_offsets(a.p, m);
+    const double delta = static_cast<double>(a.p.image_size) / S;
+    const double w0 = wr.centre - off.w;
+    const float2 *sub = reinterpret_cast<const float2 *>(a.subgrids) + static_cast<size_t>(s) * kCorr * P;
+
+    // Pixels q, q + kCount, ... of the padded KS YB 8 x mts 8 (zero past the subgrid).
+    constexpr int kRows = 8 * KS * YB, kPer = (kRows * kRows + kCount - 1) / kCount;
+    const int mts = (S + 7) / 8, cols = 8 * mts;
+    uint32_t *words = reinterpret_cast<uint32_t *>(sm.pixels);
+    cfloat px[kPer][4];
+    float vmax = 0.F;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+    {
+        const int q = tid + i * kCount, y = q / cols, x = q - y * cols;
+#pragma unroll
+        for (int pol = 0; pol < 4; ++pol)
+            px[i][pol] = {0.F, 0.F};
+        if (y < S && x < S)
+        {
+            degrid_pixel(a, m, sub, y * S + x, px[i]);
+            const cfloat r = pixel_rotation(x, y, S, delta, w0);
+#pragma unroll
+            for (int pol = 0; pol < 4; ++pol)
+            {
+                px[i][pol] = cmul(px[i][pol], r);
+                vmax = fmaxf(vmax, fmaxf(fabsf(px[i][pol].re), fabsf(px[i][pol].im)));
+            }
+        }
+    }
+    float unscale = 1.F, inv = 1.F;
+    if constexpr (DT == kFP16)
+    {
+        const int e = scale_exponent(block_max(vmax, sm.maxbits));
+        unscale = ldexpf(1.F, e);
+        inv = ldexpf(1.F, -e);
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+    {
+        const int q = tid + i * kCount, y = q / cols, x = q - y * cols;
+        if (y >= kRows)
+            continue;
+        // Word y % 4 of lane (y / 4 % 2, x % 8, correlation) of tile (y / 8, x / 8); the low halves 32 lanes on.
+        uint32_t *w = words + ((((y >> 3) * 2 + ((y >> 2) & 1)) * mts + (x >> 3)) * 64 + (x & 7) * 4) * 4 + (y & 3);
+#pragma unroll
+        for (int pol = 0; pol < 4; ++pol)
+        {
+            uint32_t hi, lo;
+            split2<DT>(px[i][pol].re * inv, px[i][pol].im * inv, hi, lo);
+            w[pol * 4] = hi;
+            w[128 + pol * 4] = lo;
+        }
+    }
+    __syncthreads();
+    DegridStage &st = sm.stage[wave];
+    if (eps <= kEpsNone)
+        degrid_range<DT, KS, YB, false>(a, sp, sel, v_begin, v_end, T, nc, row0, c0, off, wr.centre, unscale, sm.pixels,
+                                        mts, st, sm.tab);
+    else
+        degrid_range<DT, KS, YB, true>(a, sp, sel, v_begin, v_end, T, nc, row0, c0, off, wr.centre, unscale, sm.pixels,
+                                       mts, st, sm.tab);
+}
+
 // ---- launchers --------------------------------------------------------------------------------------------------
 
 template <int DT, int YT, int NT, int NX>
@@ -687,6 +1014,36 @@ template <int DT> hipError_t grid_size(const KernelArgs &a, const SeparableArgs 
     if (S <= 48)
         return few ? launch_grid<DT, 3, 1, 1>(a, sp, st) : launch_grid<DT, 3, 3, 2>(a, sp, st);
     return few ? launch_grid<DT, 4, 1, 1>(a, sp, st) : launch_grid<DT, 4, 2, 4>(a, sp, st);
+}
+
+template <int DT, int KS, int YB, int WAVES>
+hipError_t launch_degrid(const KernelArgs &a, const SeparableArgs &sp, long long blocks, hipStream_t st)
+{
+    const size_t lds = degrid_lds_bytes<WAVES>(a.p.S, 8 * KS * YB);
+    if (lds > 64 * 1024)
+    {
+        const void *fn = reinterpret_cast<const void *>(&degrid_separable<DT, KS, YB, WAVES>);
+        const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        if (e != hipSuccess)
+            return e;
+    }
+    degrid_separable<DT, KS, YB, WAVES><<<static_cast<unsigned>(blocks), 64 * WAVES, lds, st>>>(a, sp);
+    return hipGetLastError();
+}
+
+// 8-row steps held at once, and passes, for subgrid size S.
+template <int DT> hipError_t degrid_size(const KernelArgs &a, const SeparableArgs &sp, long long blocks, hipStream_t st)
+{
+    const int S = a.p.S;
+    if (S <= 16)
+        return launch_degrid<DT, 2, 1, 4>(a, sp, blocks, st);
+    if (S <= 24)
+        return launch_degrid<DT, 3, 1, 4>(a, sp, blocks, st);
+    if (S <= 32)
+        return launch_degrid<DT, 4, 1, 4>(a, sp, blocks, st);
+    if (S <= 48)
+        return launch_degrid<DT, 3, 2, 4>(a, sp, blocks, st);
+    return launch_degrid<DT, 4, 2, 8>(a, sp, blocks, st);
 }
 
 double host_n(double l, double m)
@@ -721,8 +1078,30 @@ bool separable_tables(const PlanDev &p, int precision, SeparableTables &t)
     return t.eps * (S / image) <= kSeparableField;
 }
 
+// A whole subgrid per workgroup (its pixels are prepared once) unless that leaves CUs without work: then as many
+// chunks as make 4 workgroups per CU.
+long long separable_chunk(long long max_vis, int n)
+{
+    constexpr long long kWorkgroups = 1024, kStep = kWaves * kChunk;
+    const long long most = std::max(1LL, (max_vis + kStep - 1) / kStep);
+    const long long chunks = std::min(most, std::max(1LL, kWorkgroups / std::max(1, n)));
+    return (most + chunks - 1) / chunks * kStep;
+}
+
 hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, hipStream_t st)
 {
     return precision == IDGX_MIXED_FP16X3 ? grid_size<kFP16>(a, sp, st) : grid_size<kBF16>(a, sp, st);
+}
+
+hipError_t launch_degrid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, long long max_vis,
+                                   hipStream_t st)
+{
+    const long long blocks = (max_vis + sp.per - 1) / sp.per * a.p.nr_subgrids;
+    if (blocks <= 0)
+        return hipSuccess;
+    if (blocks > 0x7fffffffLL)
+        return hipErrorInvalidConfiguration;
+    return precision == IDGX_MIXED_FP16X3 ? degrid_size<kFP16>(a, sp, blocks, st)
+                                          : degrid_size<kBF16>(a, sp, blocks, st);
 }
 } // namespace idgx

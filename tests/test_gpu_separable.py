@@ -124,13 +124,13 @@ EDGES = (1, 2, 7, 8, 9, 15, 29, 40)
 @pytest.mark.parametrize("form", ["fp16x3", "bf16x3"])
 @pytest.mark.parametrize("S", [8, 10, 16, 18, 24, 26, 32, 34, 40, 48, 50, 64])
 def test_every_tile_with_few_subgrids_vs_fp64(S, form):
-    """Without and with the product term, one-shot and batch (the same bits of the gridder)."""
+    """Without and with the product term, one-shot and batch (the same bits)."""
     w = make(S, EDGES, [0.0, 1e-4, 5e-4, 1e-6, 0.0, 2e-4, 8e-4, 3e-4], w_step=40.0)
     sub = model(w)
     got, vis = run_oneshot(w, form, sub)
     check(w, form, sub, got, vis)
-    bgot, _ = run_batch(w, form, sub)
-    assert np.array_equal(got, bgot)
+    bgot, bvis = run_batch(w, form, sub)
+    assert np.array_equal(got, bgot) and np.array_equal(vis, bvis)
 
 
 @pytest.mark.parametrize("S", [12, 24, 32, 40, 64])
