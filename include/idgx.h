@@ -484,10 +484,11 @@ int idgx_batch_last_launches(const idgx_batch *batch, int *gridder_launches, int
 int idgx_batch_items(const idgx_batch *batch, int *gridder_items, int *degridder_items, int *gridder_workgroups,
                      int *degridder_workgroups);
 
-/* Work per thread of the plain FP32 one-shot kernels for a plan (idgx_grid / idgx_degrid with IDGX_PLAIN_FP32):
- * gridder pixels per thread (4, or 3 where that leaves fewer lanes idle: S = 24, 48) and degridder channels per
- * thread (4 without channel windows when the channel count is a multiple of 4, else 2).  They name the kernel
- * instantiation a profile reports (gridder_plain<pixels, 1>, degridder_plain<channels, 1>).  No GPU needed. */
+/* Work per thread of the plain FP32 forms for a plan that fills the chip: pixels per thread of a batch's gridder items
+ * (4, or 3 where that fits the subgrid better: S = 24, 48; the one-shot gridder takes one) and channels per thread of
+ * the one-shot degridder (4 without channel windows when the channel count is a multiple of 4, else 2), which name the
+ * kernel instantiation a profile reports (degridder_plain<channels, 1>).  Smaller plans run one pixel, channel or
+ * visibility per thread in every form.  No GPU needed. */
 int idgx_plain_kernel_shape(const idgx_plan *plan, int has_channel_windows, int *gridder_pixels_per_thread,
                             int *degridder_channels_per_thread);
 

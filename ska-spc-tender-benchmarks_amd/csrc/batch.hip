@@ -48,6 +48,7 @@ struct idgx_batch
     idgx_plan plans[idgx::kMaxClasses];
     std::vector<int64_t> vis_count[idgx::kMaxClasses]; // V_s per subgrid
     int precision = IDGX_MIXED_BF16X3;
+    bool fine[2] = {}; // plain FP32, per direction: too few items to fill the chip, so one pixel or visibility per thread
     // Per direction (0 gridder, 1 degridder) and class: tile shape, resident workgroups, queue slice.
     int shape[2][idgx::kMaxClasses] = {};
     int workgroups[2][idgx::kMaxClasses] = {};
@@ -126,31 +127,48 @@ int default_shape(const idgx_batch *b, bool gridder, int S)
     return plain(b) ? idgx::plain_default_shape(gridder, S) : idgx::mixed_default_shape(gridder, S);
 }
 
+// Plain FP32: pixels (gridder) or visibilities (degridder) per thread of a shape's items.
+int plain_work(const idgx_batch *b, bool gridder, int shape)
+{
+    if (b->fine[gridder ? 0 : 1])
+        return 1;
+    return gridder ? idgx::plain_shape(shape).pixels : idgx::plain_shape(shape).entries;
+}
+
 int grid_items_per_subgrid(const idgx_batch *b, int shape, int S)
 {
-    return plain(b) ? idgx::plain_grid_items_per_subgrid(shape, S) : idgx::grid_items_per_subgrid(shape, S);
+    return plain(b) ? idgx::plain_grid_items_per_subgrid(plain_work(b, true, shape), S)
+                    : idgx::grid_items_per_subgrid(shape, S);
 }
 
 long long grid_item_pixels(const idgx_batch *b, int shape, int S, int item)
 {
-    return plain(b) ? idgx::plain_grid_item_pixels(shape, S, item) : idgx::grid_item_pixels(shape, S, item);
+    return plain(b) ? idgx::plain_grid_item_pixels(plain_work(b, true, shape), S, item)
+                    : idgx::grid_item_pixels(shape, S, item);
 }
 
 long long degrid_visibilities_per_item(const idgx_batch *b, int shape)
 {
-    return plain(b) ? idgx::plain_degrid_visibilities_per_item(shape) : idgx::degrid_visibilities_per_item(shape);
+    return plain(b) ? idgx::plain_degrid_visibilities_per_item(plain_work(b, false, shape))
+                    : idgx::degrid_visibilities_per_item(shape);
 }
 
 // Per-item tiles of a gridder single launch with each class's own shape: tiles per wave (mixed) or pixels per
 // thread (plain) of the class's gridder shape.
 int class_tiles(const idgx_batch *b, int shape)
 {
-    return plain(b) ? idgx::plain_shape(shape).pixels : idgx::mixed_shape(shape).tiles;
+    return plain(b) ? plain_work(b, true, shape) : idgx::mixed_shape(shape).tiles;
+}
+
+// What a plain launch of `shape` (or of every class's own) asks the kernels for.
+int plain_launch(const idgx_batch *b, bool gridder, int shape)
+{
+    return shape == idgx::kShapeTilesPerClass ? shape : plain_work(b, gridder, shape);
 }
 
 int workgroups_for(const idgx_batch *b, bool gridder, int shape)
 {
-    return plain(b) ? idgx::plain_queue_workgroups(accurate_sincos(b), gridder, shape)
+    return plain(b) ? idgx::plain_queue_workgroups(accurate_sincos(b), gridder, plain_launch(b, gridder, shape))
                     : idgx::queue_workgroups(b->precision, gridder, shape);
 }
 
@@ -158,8 +176,11 @@ hipError_t launch_queue(const idgx_batch *b, const QueueArgs &q, bool gridder, i
                         hipStream_t st)
 {
     if (plain(b))
-        return gridder ? idgx::launch_grid_plain_queue(q, accurate_sincos(b), shape, workgroups, st)
-                       : idgx::launch_degrid_plain_queue(q, accurate_sincos(b), shape, workgroups, st);
+    {
+        const int work = plain_launch(b, gridder, shape);
+        return gridder ? idgx::launch_grid_plain_queue(q, accurate_sincos(b), work, workgroups, st)
+                       : idgx::launch_degrid_plain_queue(q, accurate_sincos(b), work, workgroups, st);
+    }
     return gridder ? idgx::launch_grid_mixed_queue(q, b->precision, shape, workgroups, st)
                    : idgx::launch_degrid_mixed_queue(q, b->precision, shape, workgroups, st);
 }
@@ -273,24 +294,25 @@ void layout_queues(const std::vector<Item> &items, std::vector<uint2> &flat, int
     begin[idgx::kQueues] = static_cast<int>(flat.size());
 }
 
-// Queue slice of class k: room for its items under any shape (the counts build_items gives).
+// Items of class k under `shape`: as many as build_items gives.
+size_t item_count(const idgx_batch *b, bool gridder, int k, int shape)
+{
+    if (gridder)
+        return static_cast<size_t>(b->plans[k].nr_subgrids) *
+               static_cast<size_t>(grid_items_per_subgrid(b, shape, b->plans[k].subgrid_size));
+    const long long per = degrid_visibilities_per_item(b, shape);
+    size_t n = 0;
+    for (const int64_t V : b->vis_count[k])
+        n += static_cast<size_t>((V + per - 1) / per);
+    return n;
+}
+
+// Queue slice of class k: room for its items under any shape.
 size_t max_items(const idgx_batch *b, bool gridder, int k)
 {
     size_t m = 0;
     for (int sh = 0; sh < shape_count(b); ++sh)
-    {
-        size_t n = 0;
-        if (gridder)
-            n = static_cast<size_t>(b->plans[k].nr_subgrids) *
-                static_cast<size_t>(grid_items_per_subgrid(b, sh, b->plans[k].subgrid_size));
-        else
-        {
-            const long long per = degrid_visibilities_per_item(b, sh);
-            for (const int64_t V : b->vis_count[k])
-                n += static_cast<size_t>((V + per - 1) / per);
-        }
-        m = std::max(m, n);
-    }
+        m = std::max(m, item_count(b, gridder, k, sh));
     return m;
 }
 
@@ -529,6 +551,14 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
             }
             b->vis_count[k][s] = v;
         }
+    }
+    for (int dir = 0; dir < 2 && plain(b); ++dir)
+    {
+        long long items = 0;
+        for (int k = 0; k < nr_classes; ++k)
+            items += static_cast<long long>(
+                item_count(b, dir == 0, k, default_shape(b, dir == 0, b->plans[k].subgrid_size)));
+        b->fine[dir] = idgx::plain_fine_items(dir == 0, items);
     }
     hipError_t e = hipSuccess;
     for (int dir = 0; dir < 2 && e == hipSuccess; ++dir)

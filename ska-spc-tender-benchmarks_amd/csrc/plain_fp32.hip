@@ -4,8 +4,7 @@
 // gridding/src/degridding_benchmark.cpp:157-166): the whole file is compiled with contraction off, so
 // `a * b + c` rounds twice; the complex multiply-accumulates are written as explicit fused multiply-adds.
 //
-// Gridder: one workgroup of 256 threads owns 1024 or 768 pixels of one subgrid (4 or 3 per thread, 4 correlations
-//   each, held in VGPRs).  Visibilities and uvw of the subgrid stream through LDS in batches of 256 visibilities;
+// Gridder: one workgroup of 256 threads owns 256 pixels of one subgrid (one per thread, its 4 correlations held in VGPRs).  Visibilities and uvw of the subgrid stream through LDS in batches of 256 visibilities;
 //   every lane reads the same LDS address per visibility (broadcast, conflict-free).  Taper and A-term are
 //   applied in the epilogue, which overwrites the subgrid.
 // Degridder: one workgroup owns 256 (timestep, channel-chunk) items of one subgrid, each thread one timestep x
@@ -64,11 +63,65 @@ __device__ __forceinline__ void channel_window(const KernelArgs &a, int s, int &
     }
 }
 
-// Five workgroups per CU (five waves per SIMD) with the hardware sin/cos.  The kernel needs 89 VGPRs with or
-// without the bound, yet the bounded build measured 3 % faster on the SKA-Low-like workload (the compiler
-// schedules for the tighter budget).
-template <int NPIX, int SC>
-__global__ __launch_bounds__(kThreads, SC == kSincosHw ? 5 : 1) void gridder_plain(KernelArgs a)
+// One pixel of a thread: its coordinates, the phase of the subgrid's offset, and its sums.
+struct PlainPixel
+{
+    float l, m, n, offset;
+    float acc[8];
+};
+
+__device__ __forceinline__ PlainPixel plain_pixel(const KernelArgs &a, const Offsets &off, int p)
+{
+    const int S = a.p.S, x = p % S, y = p / S;
+    PlainPixel px;
+    px.l = pixel_lm(x, S, a.p.image_size);
+    px.m = pixel_lm(y, S, a.p.image_size);
+    px.n = pixel_n(px.l, px.m);
+    px.offset = (off.u * px.l + off.v * px.m) + off.w * px.n;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        px.acc[k] = 0.F;
+    return px;
+}
+
+// P <- taper * A1^H P A2 of pixel p, overwriting the subgrid's (zeros for a subgrid rejected by its bounds).
+__device__ __forceinline__ void store_plain_pixel(const KernelArgs &a, const idgx_metadata &m, int s, int p, bool ok,
+                                                  const float *acc)
+{
+    const int P = a.p.S * a.p.S;
+    float2 *out = reinterpret_cast<float2 *>(a.subgrids_out) + static_cast<size_t>(s) * kCorr * P;
+    cfloat px[4] = {{acc[0], acc[1]}, {acc[2], acc[3]}, {acc[4], acc[5]}, {acc[6], acc[7]}};
+    if (ok)
+    {
+        const float4 *aterms = reinterpret_cast<const float4 *>(a.aterms);
+        const size_t base = static_cast<size_t>(m.aterm_index) * a.p.nr_stations;
+        cfloat a1[4], a2[4];
+        load_jones(aterms, (base + m.station1) * P + p, a1);
+        load_jones(aterms, (base + m.station2) * P + p, a2);
+        apply_a1h_p_a2(px, a1, a2);
+        const float taper = a.spheroidal[p];
+#pragma unroll
+        for (int pol = 0; pol < 4; ++pol)
+            out[pol * P + p] = make_float2(px[pol].re * taper, px[pol].im * taper);
+    }
+    else
+    {
+#pragma unroll
+        for (int pol = 0; pol < 4; ++pol)
+            out[pol * P + p] = make_float2(0.F, 0.F);
+    }
+}
+
+// Visibilities whose phasors a gridder of one pixel per thread forms side by side: its independent work in flight (the
+// terms are still added in order), and the registers of one pixel leave room for eight waves per SIMD.
+constexpr int kGridUnroll = 4;
+
+// A workgroup grids 256 pixels of a subgrid; waves past the last pixel only stage.  VALU issue bound.  Against 4 (S = 32)
+// or 3 (S = 24, 48) pixels per thread side by side at five waves per SIMD, 780 baselines x 256 timesteps x 64 channels:
+// S = 32 7956 -> 7278 us, S = 48 16333 -> 15777 us, S = 24 (where a third of the lanes' third pixels were idle) 5541 ->
+// 4300 us; 45 subgrids of 32^2 with 2048 visibilities each, which leave CUs idle either way, 478 -> 143 us.
+template <int SC>
+__global__ __launch_bounds__(kThreads, SC == kSincosHw ? 8 : 1) void gridder_plain(KernelArgs a)
 {
     __shared__ float4 s_vis[2 * kGridBatchVis];
     __shared__ float4 s_uvw[kGridBatchVis];
@@ -76,113 +129,57 @@ __global__ __launch_bounds__(kThreads, SC == kSincosHw ? 5 : 1) void gridder_pla
 
     const int s = blockIdx.x;
     const int tid = threadIdx.x;
-    const int S = a.p.S;
-    const int P = S * S;
+    const int P = a.p.S * a.p.S;
     const idgx_metadata m = a.metadata[s];
     int c0, nc;
     channel_window(a, s, c0, nc);
     const long long row0 = first_row(a.metadata, m);
     const bool ok = subgrid_in_bounds(a.p, m, row0, c0, nc);
     const long long C = a.p.nr_channels;
-    const int pbase = blockIdx.y * (kThreads * NPIX);
-
-    const Offsets off = gridder_offsets(m, S, a.p.G, a.p.image_size, a.p.w_step);
-    float l[NPIX], mm[NPIX], n[NPIX], poff[NPIX];
-    float acc[NPIX][8];
-#pragma unroll
-    for (int i = 0; i < NPIX; ++i)
+    const Offsets off = gridder_offsets(m, a.p.S, a.p.G, a.p.image_size, a.p.w_step);
+    const float4 *vis = reinterpret_cast<const float4 *>(a.visibilities);
+    const int pbase = blockIdx.y * kThreads, p = pbase + tid;
+    const bool wave_live = pbase + (tid & ~63) < P; // wave-uniform
+    PlainPixel px = plain_pixel(a, off, min(p, P - 1));
+    for (int cb = 0; ok && cb < nc; cb += kGridChunk)
     {
-        const int p = min(pbase + i * kThreads + tid, P - 1);
-        const int x = p % S, y = p / S;
-        l[i] = pixel_lm(x, S, a.p.image_size);
-        mm[i] = pixel_lm(y, S, a.p.image_size);
-        n[i] = pixel_n(l[i], mm[i]);
-        poff[i] = (off.u * l[i] + off.v * mm[i]) + off.w * n[i];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            acc[i][k] = 0.F;
-    }
-
-    if (ok)
-    {
-        const float4 *vis = reinterpret_cast<const float4 *>(a.visibilities);
-        for (int cb = 0; cb < nc; cb += kGridChunk)
+        const int cc = min(kGridChunk, nc - cb);
+        const int tb_max = kGridBatchVis / cc;
+        for (int t0 = 0; t0 < m.nr_timesteps; t0 += tb_max)
         {
-            const int cc = min(kGridChunk, nc - cb);
-            const int tb_max = kGridBatchVis / cc;
-            for (int t0 = 0; t0 < m.nr_timesteps; t0 += tb_max)
+            const int tb = min(tb_max, m.nr_timesteps - t0);
+            __syncthreads(); // previous stage fully consumed
+            if (tid < cc)
+                s_wn[tid] = a.wavenumbers[c0 + cb + tid];
+            for (int q = tid; q < tb; q += kThreads)
             {
-                const int tb = min(tb_max, m.nr_timesteps - t0);
-                __syncthreads(); // previous stage fully consumed
-                if (tid < cc)
-                    s_wn[tid] = a.wavenumbers[c0 + cb + tid];
-                for (int q = tid; q < tb; q += kThreads)
+                const float *uv = a.uvw + 3 * (row0 + t0 + q);
+                s_uvw[q] = make_float4(uv[0], uv[1], uv[2], 0.F);
+            }
+            for (int q = tid; q < 2 * tb * cc; q += kThreads)
+            {
+                const int item = q >> 1;
+                const int t = item / cc, c = item - t * cc;
+                s_vis[q] = vis[((row0 + t0 + t) * C + c0 + cb + c) * 2 + (q & 1)];
+            }
+            __syncthreads();
+            for (int t = 0; wave_live && t < tb; ++t)
+            {
+                const float4 uv = s_uvw[t];
+                const float pidx = (uv.x * px.l + uv.y * px.m) + uv.z * px.n;
+#pragma unroll kGridUnroll
+                for (int c = 0; c < cc; ++c)
                 {
-                    const float *uv = a.uvw + 3 * (row0 + t0 + q);
-                    s_uvw[q] = make_float4(uv[0], uv[1], uv[2], 0.F);
-                }
-                for (int q = tid; q < 2 * tb * cc; q += kThreads)
-                {
-                    const int item = q >> 1;
-                    const int t = item / cc, c = item - t * cc;
-                    s_vis[q] = vis[((row0 + t0 + t) * C + c0 + cb + c) * 2 + (q & 1)];
-                }
-                __syncthreads();
-                for (int t = 0; t < tb; ++t)
-                {
-                    const float4 uv = s_uvw[t];
-                    float pidx[NPIX];
-#pragma unroll
-                    for (int i = 0; i < NPIX; ++i)
-                        pidx[i] = (uv.x * l[i] + uv.y * mm[i]) + uv.z * n[i];
-                    for (int c = 0; c < cc; ++c)
-                    {
-                        const float k = s_wn[c];
-                        const float4 va = s_vis[2 * (t * cc + c)];
-                        const float4 vb = s_vis[2 * (t * cc + c) + 1];
-#pragma unroll
-                        for (int i = 0; i < NPIX; ++i)
-                        {
-                            const float phase = poff[i] - pidx[i] * k;
-                            float sn, cs;
-                            sincos_rad<SC>(phase, sn, cs);
-                            cmac4(acc[i], va, vb, cs, sn);
-                        }
-                    }
+                    const float phase = px.offset - pidx * s_wn[c];
+                    float sn, cs;
+                    sincos_rad<SC>(phase, sn, cs);
+                    cmac4(px.acc, s_vis[2 * (t * cc + c)], s_vis[2 * (t * cc + c) + 1], cs, sn);
                 }
             }
         }
     }
-
-    // Epilogue: P <- taper * A1^H P A2, overwrite the subgrid (zeros for a subgrid rejected above).
-    float2 *out = reinterpret_cast<float2 *>(a.subgrids_out) + static_cast<size_t>(s) * kCorr * P;
-    const float4 *aterms = reinterpret_cast<const float4 *>(a.aterms);
-#pragma unroll
-    for (int i = 0; i < NPIX; ++i)
-    {
-        const int p = pbase + i * kThreads + tid;
-        if (p >= P)
-            continue;
-        cfloat px[4] = {{acc[i][0], acc[i][1]}, {acc[i][2], acc[i][3]}, {acc[i][4], acc[i][5]}, {acc[i][6], acc[i][7]}};
-        if (ok)
-        {
-            const size_t base = static_cast<size_t>(m.aterm_index) * a.p.nr_stations;
-            cfloat a1[4], a2[4];
-            load_jones(aterms, (base + m.station1) * P + p, a1);
-            load_jones(aterms, (base + m.station2) * P + p, a2);
-            apply_a1h_p_a2(px, a1, a2);
-            const float taper = a.spheroidal[p];
-#pragma unroll
-            for (int pol = 0; pol < 4; ++pol)
-                out[pol * P + p] = make_float2(px[pol].re * taper, px[pol].im * taper);
-        }
-        else
-        {
-#pragma unroll
-            for (int pol = 0; pol < 4; ++pol)
-                out[pol * P + p] = make_float2(0.F, 0.F);
-        }
-    }
+    if (p < P)
+        store_plain_pixel(a, m, s, p, ok, px.acc);
 }
 
 // Workgroups per CU with the hardware sin/cos: two channels per thread fit six (the most the 24 KB of LDS allows)
@@ -196,6 +193,7 @@ template <int NCH, int SC>
 __global__ __launch_bounds__(kThreads, (degrid_plain_min_blocks<NCH, SC>())) void degridder_plain(KernelArgs a,
                                                                                                   int per)
 {
+    constexpr int kUnroll = NCH <= 2 ? 4 : 1; // pixels whose phasors are in flight together (added in order)
     // Per staged pixel: (l, m, n, phase offset), then the four correlations, side by side (one address register
     // serves the pixel loop's three reads).
     __shared__ float4 s_px[3 * kDegridPixBatch];
@@ -285,6 +283,7 @@ __global__ __launch_bounds__(kThreads, (degrid_plain_min_blocks<NCH, SC>())) voi
         __syncthreads();
         if (active)
         {
+#pragma unroll kUnroll
             for (int q = 0; q < np; ++q)
             {
                 const float4 g = s_px[3 * q];
@@ -376,15 +375,57 @@ __device__ __forceinline__ bool plain_entry(const uint32_t *index, int v, int nr
     return true;
 }
 
-// Gridder item: pixels [pblk * 256 * NPIX, ...) of subgrid s.  Entries are staged 256 at a time; the entries of a
-// stage that share a timestep form a run (a workgroup scan over "timestep differs from the previous entry"), and
-// each run forms the per-pixel index term (u l + v m) + w n once, as the dense kernel does per timestep.
+// The staged runs of visibilities onto N pixels of every thread.
+template <int N, int UNROLL, int SC>
+__device__ __forceinline__ void grid_runs(const PlainGridShared &sm, int nruns, PlainPixel *px)
+{
+    for (int r = 0; r < nruns; ++r)
+    {
+        const float4 uv = sm.run_uvw[r];
+        const int e0 = __builtin_amdgcn_readfirstlane(sm.run_start[r]);
+        const int e1 = __builtin_amdgcn_readfirstlane(sm.run_start[r + 1]);
+        float pidx[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            pidx[i] = (uv.x * px[i].l + uv.y * px[i].m) + uv.z * px[i].n;
+        const auto entry = [&](int e) {
+            const float4 va = sm.ent[3 * e];
+            const float4 vb = sm.ent[3 * e + 1];
+            const float k = sm.ent[3 * e + 2].x;
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+            {
+                const float phase = px[i].offset - pidx[i] * k;
+                float sn, cs;
+                sincos_rad<SC>(phase, sn, cs);
+                cmac4(px[i].acc, va, vb, cs, sn);
+            }
+        };
+        if constexpr (UNROLL > 1)
+        {
+#pragma unroll UNROLL
+            for (int e = e0; e < e1; ++e)
+                entry(e);
+        }
+        else
+        {
+            for (int e = e0; e < e1; ++e)
+                entry(e);
+        }
+    }
+}
+
+// Gridder item: pixels [pblk * 256 * NPIX, ...) of subgrid s.  A wave with fewer than NPIX pixels per thread takes them one
+// by one, two visibilities at a time (four spill, and S = 32 runs 2 % slower): S = 24, where three waves of four have two,
+// 4982 -> 3964 us (780 baselines x 256 timesteps x 64 channels).
+// Entries are staged 256 at a time; the entries of a stage that share a timestep form a run (a workgroup scan over
+// "timestep differs from the previous entry"), and each run forms the per-pixel index term (u l + v m) + w n once, as
+// the dense kernel does per timestep.
 template <int NPIX, int SC>
 __device__ __forceinline__ void gridder_plain_item(const KernelArgs &a, int s, int pblk, PlainGridShared &sm)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int S = a.p.S;
-    const int P = S * S;
+    const int P = a.p.S * a.p.S;
     const idgx_metadata m = a.metadata[s];
     int c0, nc;
     channel_window(a, s, c0, nc);
@@ -393,23 +434,16 @@ __device__ __forceinline__ void gridder_plain_item(const KernelArgs &a, int s, i
     const long long C = a.p.nr_channels;
     const int T = m.nr_timesteps;
     const int pbase = pblk * (kThreads * NPIX);
-
-    const Offsets off = gridder_offsets(m, S, a.p.G, a.p.image_size, a.p.w_step);
-    float l[NPIX], mm[NPIX], n[NPIX], poff[NPIX];
-    float acc[NPIX][8];
+    const Offsets off = gridder_offsets(m, a.p.S, a.p.G, a.p.image_size, a.p.w_step);
+    PlainPixel px[NPIX];
+    int live = 0; // pixels per thread of this wave (the last may end inside it)
 #pragma unroll
     for (int i = 0; i < NPIX; ++i)
     {
-        const int p = min(pbase + i * kThreads + tid, P - 1);
-        const int x = p % S, y = p / S;
-        l[i] = pixel_lm(x, S, a.p.image_size);
-        mm[i] = pixel_lm(y, S, a.p.image_size);
-        n[i] = pixel_n(l[i], mm[i]);
-        poff[i] = (off.u * l[i] + off.v * mm[i]) + off.w * n[i];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            acc[i][k] = 0.F;
+        px[i] = plain_pixel(a, off, min(pbase + i * kThreads + tid, P - 1));
+        live += pbase + i * kThreads + wave * 64 < P;
     }
+    live = __builtin_amdgcn_readfirstlane(live);
 
     const uint32_t *index = nullptr;
     const int V = ok && T > 0 && nc > 0 ? plain_selection(a, s, T, nc, index) : 0;
@@ -469,60 +503,24 @@ __device__ __forceinline__ void gridder_plain_item(const KernelArgs &a, int s, i
             sm.run_start[nruns] = nb;
         __syncthreads();
         nruns = __builtin_amdgcn_readfirstlane(nruns);
-        for (int r = 0; r < nruns; ++r)
+        if (live == NPIX)
         {
-            const float4 uv = sm.run_uvw[r];
-            const int e0 = __builtin_amdgcn_readfirstlane(sm.run_start[r]);
-            const int e1 = __builtin_amdgcn_readfirstlane(sm.run_start[r + 1]);
-            float pidx[NPIX];
-#pragma unroll
-            for (int i = 0; i < NPIX; ++i)
-                pidx[i] = (uv.x * l[i] + uv.y * mm[i]) + uv.z * n[i];
-            for (int e = e0; e < e1; ++e)
-            {
-                const float4 va = sm.ent[3 * e];
-                const float4 vb = sm.ent[3 * e + 1];
-                const float k = sm.ent[3 * e + 2].x;
-#pragma unroll
-                for (int i = 0; i < NPIX; ++i)
-                {
-                    const float phase = poff[i] - pidx[i] * k;
-                    float sn, cs;
-                    sincos_rad<SC>(phase, sn, cs);
-                    cmac4(acc[i], va, vb, cs, sn);
-                }
-            }
-        }
-    }
-
-    // Epilogue: P <- taper * A1^H P A2, overwrite the item's pixels (zeros for a subgrid rejected above).
-    float2 *out = reinterpret_cast<float2 *>(a.subgrids_out) + static_cast<size_t>(s) * kCorr * P;
-    const float4 *aterms = reinterpret_cast<const float4 *>(a.aterms);
-#pragma unroll
-    for (int i = 0; i < NPIX; ++i)
-    {
-        const int p = pbase + i * kThreads + tid;
-        if (p >= P)
-            continue;
-        cfloat px[4] = {{acc[i][0], acc[i][1]}, {acc[i][2], acc[i][3]}, {acc[i][4], acc[i][5]}, {acc[i][6], acc[i][7]}};
-        if (ok)
-        {
-            const size_t base = static_cast<size_t>(m.aterm_index) * a.p.nr_stations;
-            cfloat a1[4], a2[4];
-            load_jones(aterms, (base + m.station1) * P + p, a1);
-            load_jones(aterms, (base + m.station2) * P + p, a2);
-            apply_a1h_p_a2(px, a1, a2);
-            const float taper = a.spheroidal[p];
-#pragma unroll
-            for (int pol = 0; pol < 4; ++pol)
-                out[pol * P + p] = make_float2(px[pol].re * taper, px[pol].im * taper);
+            grid_runs<NPIX, NPIX == 1 ? kGridUnroll : 1, SC>(sm, nruns, px);
         }
         else
         {
 #pragma unroll
-            for (int pol = 0; pol < 4; ++pol)
-                out[pol * P + p] = make_float2(0.F, 0.F);
+            for (int i = 0; i < NPIX - 1; ++i)
+                if (i < live)
+                    grid_runs<1, 2, SC>(sm, nruns, px + i);
         }
+    }
+#pragma unroll
+    for (int i = 0; i < NPIX; ++i)
+    {
+        const int p = pbase + i * kThreads + tid;
+        if (p < P)
+            store_plain_pixel(a, m, s, p, ok, px[i].acc);
     }
 }
 
@@ -679,7 +677,7 @@ __device__ __forceinline__ void degridder_plain_item(const KernelArgs &a, int s,
 }
 
 template <int NPIX, int SC>
-__global__ __launch_bounds__(kThreads, SC == kSincosHw ? 5 : 1) void gridder_plain_queue(QueueArgs q)
+__global__ __launch_bounds__(kThreads, SC == kSincosHw ? (NPIX == 1 ? 8 : 5) : 1) void gridder_plain_queue(QueueArgs q)
 {
     __shared__ PlainGridShared sm;
     int cls, s, blk;
@@ -697,6 +695,9 @@ __global__ __launch_bounds__(kThreads, SC == kSincosHw ? 5 : 1) void gridder_pla
     {
         switch (q.tiles[cls]) // workgroup-uniform
         {
+        case 1:
+            gridder_plain_item<1, SC>(q.cls[cls], s, blk, sm);
+            break;
         case 2:
             gridder_plain_item<2, SC>(q.cls[cls], s, blk, sm);
             break;
@@ -732,49 +733,52 @@ __global__ __launch_bounds__(kThreads, (degrid_plain_queue_min_blocks<NCH, SC>()
 constexpr PlainShape kPlainShapes[] = {{4, 2}, {3, 4}, {2, 1}};
 constexpr int kNumPlainShapes = sizeof(kPlainShapes) / sizeof(kPlainShapes[0]);
 
-template <int SC> void *plain_grid_queue_fn(int shape)
+template <int SC> void *plain_grid_queue_fn(int pixels)
 {
-    if (shape == kShapeTilesPerClass)
-        return reinterpret_cast<void *>(&gridder_plain_queue_tiles<SC>);
-    if (shape < 0 || shape >= kNumPlainShapes)
-        return nullptr;
-    switch (kPlainShapes[shape].pixels)
+    switch (pixels)
     {
+    case kShapeTilesPerClass:
+        return reinterpret_cast<void *>(&gridder_plain_queue_tiles<SC>);
+    case 1:
+        return reinterpret_cast<void *>(&gridder_plain_queue<1, SC>);
     case 2:
         return reinterpret_cast<void *>(&gridder_plain_queue<2, SC>);
     case 3:
         return reinterpret_cast<void *>(&gridder_plain_queue<3, SC>);
-    default:
+    case 4:
         return reinterpret_cast<void *>(&gridder_plain_queue<4, SC>);
+    default:
+        return nullptr;
     }
 }
 
-template <int SC> void *plain_degrid_queue_fn(int shape)
+template <int SC> void *plain_degrid_queue_fn(int entries)
 {
-    if (shape < 0 || shape >= kNumPlainShapes)
-        return nullptr;
-    switch (kPlainShapes[shape].entries)
+    switch (entries)
     {
     case 1:
         return reinterpret_cast<void *>(&degridder_plain_queue<1, SC>);
     case 2:
         return reinterpret_cast<void *>(&degridder_plain_queue<2, SC>);
-    default:
+    case 4:
         return reinterpret_cast<void *>(&degridder_plain_queue<4, SC>);
+    default:
+        return nullptr;
     }
 }
 
-void *plain_queue_fn(bool accurate_sincos, bool gridder, int shape)
+// `work`: gridder pixels per thread (or kShapeTilesPerClass), degridder visibilities per thread.
+void *plain_queue_fn(bool accurate_sincos, bool gridder, int work)
 {
     if (gridder)
-        return accurate_sincos ? plain_grid_queue_fn<kSincosOcml>(shape) : plain_grid_queue_fn<kSincosHw>(shape);
-    return accurate_sincos ? plain_degrid_queue_fn<kSincosOcml>(shape) : plain_degrid_queue_fn<kSincosHw>(shape);
+        return accurate_sincos ? plain_grid_queue_fn<kSincosOcml>(work) : plain_grid_queue_fn<kSincosHw>(work);
+    return accurate_sincos ? plain_degrid_queue_fn<kSincosOcml>(work) : plain_degrid_queue_fn<kSincosHw>(work);
 }
 
-hipError_t launch_plain_queue(const QueueArgs &q, bool accurate_sincos, bool gridder, int shape, int workgroups,
+hipError_t launch_plain_queue(const QueueArgs &q, bool accurate_sincos, bool gridder, int work, int workgroups,
                               hipStream_t st)
 {
-    void *fn = plain_queue_fn(accurate_sincos, gridder, shape);
+    void *fn = plain_queue_fn(accurate_sincos, gridder, work);
     if (!fn || workgroups <= 0)
         return hipErrorInvalidValue;
     QueueArgs arg = q;
@@ -783,26 +787,21 @@ hipError_t launch_plain_queue(const QueueArgs &q, bool accurate_sincos, bool gri
 }
 } // namespace
 
-template <int NPIX> hipError_t launch_grid_plain_pixels(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
+hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
-    const int P = a.p.S * a.p.S;
-    const dim3 grid(a.p.nr_subgrids, (P + kThreads * NPIX - 1) / (kThreads * NPIX));
+    const dim3 grid(a.p.nr_subgrids, (a.p.S * a.p.S + kThreads - 1) / kThreads);
     if (accurate_sincos)
-        gridder_plain<NPIX, kSincosOcml><<<grid, kThreads, 0, stream>>>(a);
+        gridder_plain<kSincosOcml><<<grid, kThreads, 0, stream>>>(a);
     else
-        gridder_plain<NPIX, kSincosHw><<<grid, kThreads, 0, stream>>>(a);
+        gridder_plain<kSincosHw><<<grid, kThreads, 0, stream>>>(a);
     return hipGetLastError();
 }
 
-// Pixels per gridder thread: 4 (1024 per workgroup) unless 3 (768) leaves fewer lanes idle, as for S = 24 (576
-// pixels: 75 % of the lanes busy with 3, 56 % with 4) and S = 48 (2304: 100 % with 3, 75 % with 4).  Lanes past
-// the last pixel still run the visibility loop, so idle lanes cost time; the per-pixel cost is the same for both.
-hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
-{
-    if (plain_grid_pixels_for(a.p.S) == 3)
-        return launch_grid_plain_pixels<3>(a, accurate_sincos, stream);
-    return launch_grid_plain_pixels<4>(a, accurate_sincos, stream);
-}
+// Items of the default shapes, or one-shot degridder workgroups, that fill the chip.  Smaller plans run one pixel or
+// visibility per thread.  Batches of 45 subgrids of 32^2 with 2048 visibilities each: gridder 586 -> 360 us, degridder
+// 291 -> 246 us; 276 of them 753 -> 577 us, where the degridder gains at S = 32 and 48 (436 -> 411 us) and loses at S = 24
+// (262 -> 286 us), so its line lies below (1104 items).
+constexpr long long kGridFill = 2048, kDegridItems = 1024, kDegridFill = 1280;
 
 template <int NCH> hipError_t launch_degrid_plain_chunks(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
@@ -824,14 +823,20 @@ template <int NCH> hipError_t launch_degrid_plain_chunks(const KernelArgs &a, bo
 // takes all channels (no windows) and their count is a multiple of 4, two otherwise.  Measured: the reference
 // generator's workload (16 channels, no windows) 17.1 ms with four, 18.3 ms with two; the SKA-Low-like workload
 // (windows of 13.5 channels on average: 90 % of the lanes busy with four, 96.7 % with two) 82.3 and 79.6 ms.
+// Plans too small to fill the chip take one: 45 subgrids of 32^2 with 2048 visibilities each 202 -> 143 us, 276 of them
+// 428 -> 385 us (496: 628 -> 640 us).
 hipError_t launch_degrid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
+    const long long pairs = static_cast<long long>(a.p.max_nr_timesteps) * ((a.p.nr_channels + 1) / 2);
+    if ((pairs + kThreads - 1) / kThreads * a.p.nr_subgrids < kDegridFill)
+        return launch_degrid_plain_chunks<1>(a, accurate_sincos, stream);
     if (plain_degrid_channels_for(a.channels != nullptr, a.p.nr_channels) == 4)
         return launch_degrid_plain_chunks<4>(a, accurate_sincos, stream);
     return launch_degrid_plain_chunks<2>(a, accurate_sincos, stream);
 }
 
-// Pixels per gridder thread for subgrid size S: 4 unless 3 leaves fewer lanes idle (see launch_grid_plain).
+// Pixels per thread of a batch's gridder items for subgrid size S: 4 (1024 per item) unless 3 (768) fits the subgrid
+// better, as for S = 24 (576 pixels) and S = 48 (2304).
 int plain_grid_pixels_for(int S)
 {
     const long long P = static_cast<long long>(S) * S;
@@ -866,39 +871,44 @@ int plain_default_shape(bool gridder, int S)
     return 0;
 }
 
-int plain_grid_items_per_subgrid(int shape, int S)
+bool plain_fine_items(bool gridder, long long items)
 {
-    const long long per = static_cast<long long>(kThreads) * kPlainShapes[shape].pixels;
+    return items < (gridder ? kGridFill : kDegridItems);
+}
+
+int plain_grid_items_per_subgrid(int pixels, int S)
+{
+    const long long per = static_cast<long long>(kThreads) * pixels;
     return static_cast<int>((static_cast<long long>(S) * S + per - 1) / per);
 }
 
-long long plain_grid_item_pixels(int shape, int S, int item)
+long long plain_grid_item_pixels(int pixels, int S, int item)
 {
-    const long long per = static_cast<long long>(kThreads) * kPlainShapes[shape].pixels;
+    const long long per = static_cast<long long>(kThreads) * pixels;
     const long long P = static_cast<long long>(S) * S;
     return std::max(0LL, std::min(per, P - item * per));
 }
 
-int plain_degrid_visibilities_per_item(int shape)
+int plain_degrid_visibilities_per_item(int entries)
 {
-    return kThreads * kPlainShapes[shape].entries;
+    return kThreads * entries;
 }
 
-hipError_t launch_grid_plain_queue(const QueueArgs &q, bool accurate_sincos, int shape, int workgroups,
+hipError_t launch_grid_plain_queue(const QueueArgs &q, bool accurate_sincos, int work, int workgroups,
                                    hipStream_t st)
 {
-    return launch_plain_queue(q, accurate_sincos, true, shape, workgroups, st);
+    return launch_plain_queue(q, accurate_sincos, true, work, workgroups, st);
 }
 
-hipError_t launch_degrid_plain_queue(const QueueArgs &q, bool accurate_sincos, int shape, int workgroups,
+hipError_t launch_degrid_plain_queue(const QueueArgs &q, bool accurate_sincos, int work, int workgroups,
                                      hipStream_t st)
 {
-    return launch_plain_queue(q, accurate_sincos, false, shape, workgroups, st);
+    return launch_plain_queue(q, accurate_sincos, false, work, workgroups, st);
 }
 
-int plain_queue_workgroups(bool accurate_sincos, bool gridder, int shape)
+int plain_queue_workgroups(bool accurate_sincos, bool gridder, int work)
 {
-    void *fn = plain_queue_fn(accurate_sincos, gridder, shape);
+    void *fn = plain_queue_fn(accurate_sincos, gridder, work);
     if (!fn)
         return 0;
     int dev = 0, cus = 0, per_cu = 0;

@@ -480,7 +480,8 @@ def plan_segments_device(uvw, frequencies, station1, station2, seg_bl, seg_t0, s
 
 
 def plain_kernel_shape(plan, has_channel_windows):
-    """(gridder pixels per thread, degridder channels per thread) of the plain FP32 one-shot kernels for `plan`."""
+    """(pixels per thread of a batch's gridder items, channels per thread of the one-shot degridder) of the plain FP32
+    forms for a plan of this shape that fills the chip."""
     px, nch = ctypes.c_int(), ctypes.c_int()
     _check(lib().idgx_plain_kernel_shape(ctypes.byref(plan), int(bool(has_channel_windows)), ctypes.byref(px),
                                          ctypes.byref(nch)), "idgx_plain_kernel_shape")
