@@ -320,7 +320,8 @@ int idgx_wstack_from_image(const idgx_plan *plan, const void *d_image, int z_min
  * For the three-pass sizes (G = 1024 ... 16384) the screens and the sum over layers run inside the row pass: each
  * image row is transformed for every layer while n(l, m) stays in registers, so neither the layers' image-domain
  * planes nor a separate w-screen pass touch HBM.  The screens there take v_sin / v_cos of the FP64-reduced fraction
- * of a turn (about 1e-7 absolute), not FP64 sincospi.  idgx_grid_to_image keeps a scratch of
+ * of a turn (about 1e-7 absolute), not FP64 sincospi.  One layer at w_step 0 has no screen to apply and takes the
+ * passes of idgx_grid_fft_box, reading from one array and writing to the other.  idgx_grid_to_image otherwise keeps a scratch of
  * nr_layers x G x (box width rounded out to 64-column tiles) cells per device, allocated on first use and grown
  * (after a device synchronisation, which also makes a growing call unsuitable for hipGraph capture) when a call
  * needs more; calls that overlap on one device share it, so issue them from one host thread on one stream.  Other

@@ -71,6 +71,23 @@ __device__ __forceinline__ double image_n(int X, int Y, int G, double image_size
     return r2 >= 1.0 ? 1.0 : r2 / (1.0 + sqrt(1.0 - r2));
 }
 
+// image_n by its series, within 1e-11 of itself for r^2 <= 0.02 (fields up to 0.2 rad): 10 FP64 operations instead of a
+// square root and a division.
+constexpr double kSeriesField = 0.2;
+__device__ __forceinline__ double image_n_series(int X, int Y, int G, double image_size)
+{
+    const double l = (X - 0.5 * G) * (image_size / G), m = (Y - 0.5 * G) * (image_size / G);
+    const double r2 = __builtin_fma(l, l, m * m);
+    double p = 33.0 / 2048.0;
+    p = __builtin_fma(p, r2, 21.0 / 1024.0);
+    p = __builtin_fma(p, r2, 7.0 / 256.0);
+    p = __builtin_fma(p, r2, 5.0 / 128.0);
+    p = __builtin_fma(p, r2, 1.0 / 16.0);
+    p = __builtin_fma(p, r2, 1.0 / 8.0);
+    p = __builtin_fma(p, r2, 1.0 / 2.0);
+    return p * r2;
+}
+
 // exp(sign 2 pi i w n) with w = (z + 0.5) w_step, reduced to a fraction of a turn in FP64.
 __device__ __forceinline__ cfloat wscreen(double n, int z, double w_step, double sign)
 {
@@ -495,9 +512,18 @@ template <int L, int SG> __global__ __launch_bounds__(L / 16, (L >= 2048 ? 4 : 2
         asm volatile("" : "+v"(j0));
         // The thread's points j0 + t kQ (t < 16), in and out: n once per row; (-1)^k = (-1)^j0 (kQ is even).
         double nn[16];
+        if (W.image_size <= kSeriesField)
+        {
 #pragma unroll
-        for (int t = 0; t < 16; ++t)
-            nn[t] = image_n(j0 + t * kQ, y, L, W.image_size);
+            for (int t = 0; t < 16; ++t)
+                nn[t] = image_n_series(j0 + t * kQ, y, L, W.image_size);
+        }
+        else
+        {
+#pragma unroll
+            for (int t = 0; t < 16; ++t)
+                nn[t] = image_n(j0 + t * kQ, y, L, W.image_size);
+        }
         const bool odd = (j0 & 1) != 0;
         auto screen = [&](double wz, int t) {
             // An opaque copy: the screen is formed where it is used, not ahead of the transform (which would hold 16
@@ -1032,26 +1058,12 @@ hipError_t static_scratch(float2 *&out)
 // group 0.57 ms per direction, two planes 0.64 ms).
 constexpr long long kScratchBytes = 64LL << 20;
 
-// Copies rows [y0, y0 + ny) x columns [c0, c0 + nc) of every plane from src to dst (planes of G x G).
-__global__ __launch_bounds__(kThreads) void copy_box_kernel(const float2 *src, float2 *dst, int G, int y0, int ny,
-                                                            int c0, int nc, long long total)
-{
-    const long long i = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i >= total)
-        return;
-    const long long r = i / nc; // plane * ny + row
-    const int c = c0 + static_cast<int>(i - r * nc);
-    const long long pl = r / ny;
-    const size_t e = (static_cast<size_t>(pl) * G + y0 + (r - pl * ny)) * G + c;
-    dst[e] = src[e];
-}
-
 // Restriction of a transform to a box of cells [x0, x1) x [y0, y1) of every plane.  kSparseInput: the input is
 // zero outside the box, so the column passes take only the column tiles that meet [x0, x1) and the row pass reads
 // only those columns (zeros elsewhere); the whole output is produced.  kRowsOut: only the box's cells (within the
-// column tiles around it) of the output are produced: the row pass runs first, in place and dense, then the column
-// passes take only the box's column tiles and column pass 2 stores only its rows into the scratch, from which they
-// are copied back (one dense pass instead of two; the rounding differs from the column-first order).
+// column tiles around it) of the output are produced: the row pass runs first, dense, then the column passes take only
+// the box's column tiles and column pass 2 stores only its rows (one dense pass instead of two; the rounding differs
+// from the column-first order).
 enum BoxMode
 {
     kFullTransform = 0,
@@ -1129,27 +1141,30 @@ hipError_t stockham_fft2d(const float2 *src, float2 *dst, int gx, int gy, long l
     {
         const int t0 = box.x0 / kColTile, t1 = (box.x1 + kColTile - 1) / kColTile;
         const int ny = std::max(0, box.y1 - box.y0);
-        if (src != dst)
-            return hipErrorInvalidValue; // the grid transforms run in place
+        if (src != dst && box.rows_done)
+            return hipErrorInvalidValue;
         if (t1 <= t0 || ny == 0)
             return hipSuccess; // nothing to produce
         for (long long p = 0; p < planes && e == hipSuccess; p += group)
         {
             A.nplanes = static_cast<int>(std::min(group, planes - p));
             float2 *g = dst + static_cast<size_t>(p) * plane;
-            // 1. Rows, in place and dense, with the input signs.
+            // 1. Rows, dense, with the input signs.
             if (!box.rows_done)
             {
                 FftArgs R = A;
-                R.scratch = g;
+                R.scratch = const_cast<float2 *>(src) + static_cast<size_t>(p) * plane; // the row pass's input
                 R.grid = g;
                 R.rows_first = 1;
                 e = launch_row_pass<SG>(R, st);
             }
-            // 2. Columns of the box's column tiles; column pass 2 stores the box's rows into the scratch.
+            // 2. Columns of the box's column tiles: column pass 1 into the scratch, column pass 2 from there the box's
+            // rows into the grid (in place, with the box copied back from the scratch, took 46 us more per plane at
+            // G = 4096, 62 us for a box of 4400^2 cells at G = 8192).
             FftArgs C = A;
             C.src = g;
-            C.grid = g;
+            C.grid = A.scratch;
+            C.scratch = g;
             C.rows_first = 1;
             C.ct0 = t0;
             C.nct = t1 - t0;
@@ -1160,15 +1175,6 @@ hipError_t stockham_fft2d(const float2 *src, float2 *dst, int gx, int gy, long l
                 e = launch_col_pass<kPassCol1, SG>(C, C.N1, static_cast<int>(col_sets * C.N2), st);
             if (e == hipSuccess)
                 e = launch_col_pass<kPassCol2, SG>(C, C.N2, static_cast<int>(col_sets * C.N1), st);
-            // 3. The box back into the grid.
-            const int nc = (t1 - t0) * kColTile;
-            const long long total = static_cast<long long>(C.nplanes) * ny * nc;
-            if (e == hipSuccess)
-            {
-                copy_box_kernel<<<static_cast<unsigned>((total + kThreads - 1) / kThreads), kThreads, 0, st>>>(
-                    C.scratch, g, gx, box.y0, ny, t0 * kColTile, nc, total);
-                e = hipGetLastError();
-            }
         }
         return e;
     }
@@ -1292,14 +1298,15 @@ hipError_t launch_grid_fft(void *grid, int G, long long nr_layers, bool forward,
             if (forward)
             {
                 // In plane-sized reads + writes, the boxed transform to uv costs 1 (dense rows) + fx (column pass 1)
-                // + fx (1 + fy) / 2 (column pass 2) + fx fy (copy back), fx and fy being the shares of the grid's
-                // columns (whole tiles) and rows that the box takes; the full transform costs 3 and produces every
-                // cell.  A box that covers most of the grid takes the full transform (measured at G = 4096 with a
-                // box of 4095 x 4005 cells: 0.69 ms boxed, 0.55 ms full).
+                // + fx (1 + fy) / 2 (column pass 2), fx and fy being the shares of the grid's columns (whole tiles)
+                // and rows that the box takes; the full transform costs 3 and produces every cell.  Measured, four
+                // planes, boxes of 0.7 / 0.9 / all of each side: 405 / 478 / 504 us against 538 us in full at
+                // G = 4096, 7957 / 9638 / 10423 against 10308 at G = 16384.  So the full transform is left where the
+                // box would save less than 2 % of the traffic.
                 const int t0 = b.x0 / kColTile, t1 = (b.x1 + kColTile - 1) / kColTile;
                 const double fx = static_cast<double>(t1 - t0) * kColTile / G;
                 const double fy = static_cast<double>(b.y1 - b.y0) / G;
-                if (1.5 * fx * (1.0 + fy) >= 2.0)
+                if (fx * (1.5 + 0.5 * fy) >= 1.95)
                     b.mode = kFullTransform;
             }
         }
@@ -1582,6 +1589,20 @@ hipError_t launch_grid_wstack(void *grid, void *image, int G, int z_min, int nr_
     }
     // The box's whole column tiles, as the boxed transform takes them.
     const int t0 = box[0] / kColTile, t1 = std::max(t0, (box[1] + kColTile - 1) / kColTile);
+    // One layer at w = 0: every screen is 1, so the plain row pass serves, without n and the screens (G = 4096: 87 -> 46 us
+    // a plane).  From the image a box of few columns still takes the w-stacked one, which writes only those.
+    if (nr_layers == 1 && w_step == 0.F && (to_image || 4 * (t1 - t0) * kColTile >= 3 * G))
+    {
+        FftBox b;
+        b.mode = to_image ? kSparseInput : kRowsOut;
+        b.x0 = box[0];
+        b.x1 = box[1];
+        b.y0 = box[2];
+        b.y1 = box[3];
+        float2 *g = static_cast<float2 *>(grid), *img = static_cast<float2 *>(image);
+        return to_image ? stockham_fft2d<-1>(g, img, G, G, planes, true, st, b)
+                        : stockham_fft2d<1>(img, g, G, G, planes, true, st, b);
+    }
     WsArgs W{};
     W.nr_layers = nr_layers;
     W.z_min = z_min;
