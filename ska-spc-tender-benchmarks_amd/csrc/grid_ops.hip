@@ -8,12 +8,17 @@
 // Conflict-free adder.  The grid is cut into tiles of T >= S cells; a subgrid belongs to the tile holding its
 // corner and can only touch that tile's 2T x 2T region (the tile and its right/lower neighbours).  Tiles are
 // coloured by the parity of their tile coordinates: two different tiles of one colour are at least two tiles
-// apart in x or y, so their regions are disjoint.  One launch per colour.  A workgroup takes one correlation of
-// one row block (at most 1024 cells) of one quadrant of a tile's region, walks the tile's subgrids in plan order
-// accumulating the covered cells in registers, and then adds each accumulated cell to the grid once.  Every
-// cell therefore sees a fixed summation order (deterministic, no atomics), and a tile crowded with subgrids is
-// spread over 16 x (row blocks) workgroups instead of one.  The tile lists are built on the host from the plan
-// (idgx_adder_plan_build).
+// apart in x or y, so their regions are disjoint.  One launch per colour.  A thread owns the four cells of the region
+// that agree modulo T, of which a subgrid covers exactly one when T = S (at most one otherwise): it walks the tile's
+// subgrids in plan order, reads its cell of each and adds it to one of four sums, and at the end adds each sum to the
+// grid once.  Every cell therefore sees a fixed summation order (deterministic, no atomics).  The tile lists are built
+// on the host from the plan (idgx_adder_plan_build).
+//
+// What bounds them: HBM.  76,865 subgrids of 32^2 (2.52 GB) and a 4096^2 grid: the adder reads each subgrid row whole,
+// once, past the caches (nontemporal), 3.7 GB with the grid in 0.76 ms (4.9 TB/s, as a large copy); with a thread per
+// cell of the region, three of four idle for each subgrid and lines fetched by several workgroups, it took 1.15 ms, and
+// 0.93 ms with cached reads.  The splitter writes 2.52 GB past the caches, which keeps the grid's cells there: 0.63 ms,
+// against 0.88 ms with cached stores, a division per cell and neighbouring subgrids on different XCDs.
 #include "idgx_device.hpp"
 #include "kernels.hpp"
 
@@ -22,20 +27,73 @@ namespace idgx
 namespace
 {
 constexpr int kThreads = 256;
+constexpr int kAdderUnroll = 8; // subgrids whose loads the adder keeps in flight together (4: 202 us, 16: 202, 8: 189)
+constexpr int kAdderPols = 2;   // correlations per workgroup (4: 8 % slower where a tile holds hundreds of subgrids)
+constexpr int kLoadOnce = 2;    // cache policy of a buffer load: nontemporal
+constexpr int kRun = 64;        // consecutive subgrids that the splitter keeps on one XCD
 
-constexpr int kAdderCells = 4;  // grid cells per thread of the adder
-constexpr int kAdderUnroll = 4; // subgrids whose loads the adder keeps in flight together
-
+typedef float f32x4 __attribute__((ext_vector_type(4), aligned(8)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ int floordiv_dev(int a, int b)
 {
     return a >= 0 ? a / b : -((-a + b - 1) / b);
 }
 
-// Rows of a tile quadrant one adder workgroup covers (at most kThreads * kAdderCells cells).
-__host__ __device__ inline int adder_rows(int T)
+// Workgroups per tile of the adder: one residue (x mod T, y mod T) and kAdderPols correlations per thread.
+__host__ __device__ inline int adder_blocks(int T)
 {
-    const int r = (kThreads * kAdderCells) / T;
-    return r < T ? r : T;
+    return (T * T + kThreads - 1) / kThreads * (kCorr / kAdderPols);
+}
+
+// A thread's residue of one tile.
+struct AdderCells
+{
+    const float2 *subgrids;
+    int S, T, p0, rx, ry;
+    bool live;
+};
+
+// The next U subgrids of a tile's list (n left) onto the thread's cells, their loads in flight together.  Offset -1 is
+// past the buffer's end: such a lane reads nothing (and the value is not used).
+template <int U>
+__device__ __forceinline__ void adder_step(const AdderCells &c, const int4 *list, int n, float2 (&acc)[4][kAdderPols],
+                                           bool (&touched)[4])
+{
+    const int P = c.S * c.S;
+    u32x2 val[U][kAdderPols];
+    bool on[U], right[U], below[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+    {
+        const int4 m = list[min(u, n - 1)];
+        const int s = __builtin_amdgcn_readfirstlane(m.x);
+        const int ox = __builtin_amdgcn_readfirstlane(m.y), oy = __builtin_amdgcn_readfirstlane(m.z);
+        const bool in_tile = u < n && ox >= 0 && ox < c.T && oy >= 0 && oy < c.T; // uniform
+        right[u] = c.rx < ox;
+        below[u] = c.ry < oy;
+        const int dx = c.rx - ox + (right[u] ? c.T : 0), dy = c.ry - oy + (below[u] ? c.T : 0);
+        on[u] = c.live && in_tile && dx < c.S && dy < c.S;
+        const int off = on[u] ? (dy * c.S + dx) * 8 : -1;
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float2 *>(c.subgrids) + static_cast<size_t>(s) * kCorr * P, 0, kCorr * P * 8, 0x00020000);
+#pragma unroll
+        for (int p = 0; p < kAdderPols; ++p)
+            val[u][p] = __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, (c.p0 + p) * P * 8, kLoadOnce);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (on[u] && right[u] == (q & 1) && below[u] == (q >> 1))
+            {
+                touched[q] = true;
+#pragma unroll
+                for (int p = 0; p < kAdderPols; ++p)
+                {
+                    acc[q][p].x += __uint_as_float(val[u][p].x);
+                    acc[q][p].y += __uint_as_float(val[u][p].y);
+                }
+            }
 }
 
 __global__ __launch_bounds__(kThreads) void adder_kernel(const idgx_metadata *md, const int32_t *order,
@@ -43,114 +101,107 @@ __global__ __launch_bounds__(kThreads) void adder_kernel(const idgx_metadata *md
                                                          int T, int G, int z_min, int nr_layers,
                                                          const float2 *subgrids, float2 *grid)
 {
-    const int R = adder_rows(T), nrb = (T + R - 1) / R;
-    const int per_tile = 16 * nrb;
-    // Workgroup b -> (tile, sub-block): workgroups reach the 8 XCDs in turn (b % 8), so XCD x takes tiles x, x + 8,
-    // x + 16, ... of the colour (heaviest first), each with all its sub-blocks.  The rows of a subgrid that straddle
-    // the boundary between two quadrants are then read by workgroups of one XCD, so each cache line they share is
-    // fetched into one L2 once.  The grid is padded to a multiple of 8 tiles; the padding exits.
+    __shared__ int4 list[kThreads];
+    const int per_tile = adder_blocks(T);
+    // Workgroup b -> (tile, residues): workgroups reach the 8 XCDs in turn (b % 8), so XCD x takes tiles x, x + 8,
+    // x + 16, ... of the colour (heaviest first), each with all its residues.  The grid is padded to a multiple of 8
+    // tiles; the padding exits.
     const int b = static_cast<int>(blockIdx.x), k = b >> 3;
     const int tl = (k / per_tile) * 8 + (b & 7);
     if (tl >= ntiles)
         return; // uniform
     const int tile = tile_begin + tl;
-    const int sub_b = k % per_tile;
-    const int pol = sub_b / (4 * nrb), quad = (sub_b / nrb) & 3, rb = sub_b % nrb;
     const int first = tile_start[tile], last = tile_start[tile + 1];
     const idgx_metadata m0 = md[order[first]];
     // All subgrids of a tile share one w-layer (the plan keys tiles by layer); single-layer plans ignore z.
     const int layer = nr_layers > 1 ? m0.z - z_min : 0;
     if (layer < 0 || layer >= nr_layers)
         return; // uniform; the layered plan builder rejects such subgrids
-    // Cells [by, by + nrows) x [bx, bx + T) of the grid.  The tile origin is taken from the tile index as the plan
-    // keys it (clamped to -1 .. G/T + 1), so every subgrid of the tile agrees on it.
+    // The tile's origin, from its index as the plan keys it (clamped to -1 .. G / T + 1: subgrids beyond those tiles
+    // meet no cell of the grid).
     const int ntiles_axis = floordiv_dev(G, T) + 3;
-    const int tx = min(max(floordiv_dev(m0.x, T) + 1, 0), ntiles_axis - 1) - 1;
-    const int ty = min(max(floordiv_dev(m0.y, T) + 1, 0), ntiles_axis - 1) - 1;
-    const int bx = tx * T + (quad & 1) * T;
-    const int by = ty * T + (quad >> 1) * T + rb * R;
-    const int nrows = min(R, T - rb * R);
-    const int ncells = nrows * T;
-    const int P = S * S;
-    float2 acc[kAdderCells];
-    bool touched[kAdderCells];
-    int cx[kAdderCells], cy[kAdderCells];
+    const int bx = (min(max(floordiv_dev(m0.x, T) + 1, 0), ntiles_axis - 1) - 1) * T;
+    const int by = (min(max(floordiv_dev(m0.y, T) + 1, 0), ntiles_axis - 1) - 1) * T;
+    const int tid = threadIdx.x, sub_b = k % per_tile, p0 = sub_b % (kCorr / kAdderPols) * kAdderPols;
+    const int e = sub_b / (kCorr / kAdderPols) * kThreads + tid;
+    const int ry = e / T, rx = e - ry * T;
+    float2 acc[4][kAdderPols];
+    bool touched[4] = {false, false, false, false};
 #pragma unroll
-    for (int k = 0; k < kAdderCells; ++k)
-    {
-        const int c = threadIdx.x + k * kThreads;
-        cy[k] = by + c / T;
-        cx[k] = bx + c % T;
-        acc[k] = make_float2(0.F, 0.F);
-        touched[k] = false;
-        if (c >= ncells)
-            cy[k] = -0x40000000; // never covered
-    }
-    // kAdderUnroll subgrids per step: their loads are all in flight together, then added in plan order.
-    for (int i0 = first; i0 < last; i0 += kAdderUnroll)
-    {
-        float2 val[kAdderUnroll][kAdderCells];
-        bool hit[kAdderUnroll][kAdderCells];
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int u = 0; u < kAdderUnroll; ++u)
+        for (int p = 0; p < kAdderPols; ++p)
+            acc[q][p] = make_float2(0.F, 0.F);
+    const AdderCells c = {subgrids, S, T, p0, rx, ry, ry < T};
+    for (int i0 = first; i0 < last; i0 += kThreads)
+    {
+        const int n = min(last - i0, kThreads);
+        __syncthreads(); // the previous list is done with
+        if (tid < n)
         {
-            const int i = i0 + u;
-            int s = 0, x0 = 0, y0 = 0;
-            bool any = i < last;
-            if (any)
-            {
-                s = order[i];
-                x0 = md[s].x;
-                y0 = md[s].y;
-                any = !(x0 + S <= bx || x0 >= bx + T || y0 + S <= by || y0 >= by + nrows); // uniform
-            }
-            const float2 *sub = subgrids + (static_cast<size_t>(s) * kCorr + pol) * P;
-#pragma unroll
-            for (int k = 0; k < kAdderCells; ++k)
-            {
-                const int dx = cx[k] - x0, dy = cy[k] - y0;
-                hit[u][k] = any && dx >= 0 && dx < S && dy >= 0 && dy < S;
-                val[u][k] = hit[u][k] ? sub[dy * S + dx] : make_float2(0.F, 0.F);
-            }
+            const int s = order[i0 + tid];
+            list[tid] = make_int4(s, md[s].x - bx, md[s].y - by, 0);
         }
-#pragma unroll
-        for (int u = 0; u < kAdderUnroll; ++u)
-#pragma unroll
-            for (int k = 0; k < kAdderCells; ++k)
-                if (hit[u][k])
-                {
-                    acc[k].x += val[u][k].x;
-                    acc[k].y += val[u][k].y;
-                    touched[k] = true;
-                }
+        __syncthreads();
+        int u0 = 0;
+        for (; n - u0 > kAdderUnroll / 2; u0 += kAdderUnroll)
+            adder_step<kAdderUnroll>(c, list + u0, n - u0, acc, touched);
+        if (n - u0 > kAdderUnroll / 4)
+            adder_step<kAdderUnroll / 2>(c, list + u0, n - u0, acc, touched);
+        else if (n > u0)
+            adder_step<kAdderUnroll / 4>(c, list + u0, n - u0, acc, touched);
     }
     const size_t GG = static_cast<size_t>(G) * G;
-    float2 *plane = grid + (static_cast<size_t>(layer) * kCorr + pol) * GG;
+    grid += (static_cast<size_t>(layer) * kCorr + p0) * GG;
 #pragma unroll
-    for (int k = 0; k < kAdderCells; ++k)
+    for (int q = 0; q < 4; ++q)
     {
-        if (touched[k] && cx[k] >= 0 && cx[k] < G && cy[k] >= 0 && cy[k] < G)
-        {
-            float2 *g = plane + static_cast<size_t>(cy[k]) * G + cx[k];
-            const float2 o = *g;
-            *g = make_float2(o.x + acc[k].x, o.y + acc[k].y);
-        }
+        const int cx = bx + rx + (q & 1) * T, cy = by + ry + (q >> 1) * T;
+        if (!touched[q] || cx < 0 || cx >= G || cy < 0 || cy >= G)
+            continue;
+        float2 *g = grid + static_cast<size_t>(cy) * G + cx;
+        float2 o[kAdderPols];
+#pragma unroll
+        for (int p = 0; p < kAdderPols; ++p)
+            o[p] = g[p * GG];
+#pragma unroll
+        for (int p = 0; p < kAdderPols; ++p)
+            g[p * GG] = make_float2(o[p].x + acc[q][p].x, o[p].y + acc[q][p].y);
     }
 }
 
 __global__ __launch_bounds__(kThreads) void splitter_kernel(const idgx_metadata *md, int S, int G, int z_min,
                                                             int nr_layers, const float2 *grid, float2 *subgrids)
 {
-    // Subgrids in launch order, spread over the XCDs: an XCD-contiguous order (neighbours in uv on one XCD) read
-    // 1.52 GB instead of 3.13 GB for 76,865 subgrids of 32^2 on a 4096^2 grid, but took 0.98 ms instead of 0.84 ms.
-    const long long s = blockIdx.x;
+    // Workgroups reach the 8 XCDs in turn: runs of kRun subgrids, near each other in uv, on one XCD read most of the
+    // grid from its L2 (76,865 subgrids of 32^2: 740 us in launch order, 742 in runs of 4, 662 of 16, 639 of 64 and of
+    // 256; XCD-contiguous 719, but 10 % slower than launch order for 13,747 of 64^2).
+    const int whole = static_cast<int>(gridDim.x) / (8 * kRun) * (8 * kRun), b = static_cast<int>(blockIdx.x);
+    const long long s = b < whole ? (b / (8 * kRun) * 8 + (b & 7)) * kRun + (b >> 3) % kRun : b;
     const int x0 = md[s].x, y0 = md[s].y;
-    const int P = S * S;
+    const int P = S * S, H = S / 2;
     const size_t GG = static_cast<size_t>(G) * G;
     const int layer = nr_layers > 1 ? md[s].z - z_min : 0;
     const bool on = layer >= 0 && layer < nr_layers; // uniform: a subgrid of no layer reads zeros
     grid += static_cast<size_t>(on ? layer : 0) * kCorr * GG;
     float2 *sub = subgrids + static_cast<size_t>(s) * kCorr * P;
+    if (on && x0 >= 0 && y0 >= 0 && x0 <= G - S && y0 <= G - S) // uniform: every cell is in the grid
+    {
+        const float2 *g = grid + static_cast<size_t>(y0) * G + x0;
+#pragma unroll 2
+        for (int i = threadIdx.x; i < P / 2; i += kThreads)
+        {
+            const int y = i / H, x = 2 * (i - y * H);
+            f32x4 v[kCorr]; // two cells (S is even), 8-byte aligned in the grid
+#pragma unroll
+            for (int p = 0; p < kCorr; ++p)
+                v[p] = *reinterpret_cast<const f32x4 *>(g + p * GG + static_cast<size_t>(y) * G + x);
+#pragma unroll
+            for (int p = 0; p < kCorr; ++p)
+                __builtin_nontemporal_store(v[p], reinterpret_cast<f32x4 *>(sub + p * P + 2 * i));
+        }
+        return;
+    }
     for (int q = threadIdx.x; q < kCorr * P; q += kThreads)
     {
         const int pol = q / P, rem = q - pol * P;
@@ -168,10 +219,9 @@ hipError_t launch_adder(const idgx_metadata *md, const int32_t *order, const int
                         const int32_t *color_begin, int S, int T, int G, int z_min, int nr_layers,
                         const void *subgrids, void *grid, hipStream_t st)
 {
-    if (T < S || T <= 0)
+    if (T < S || T <= 0 || T > 32768)
         return hipErrorInvalidValue;
-    const int R = adder_rows(T);
-    const long long per_tile = 16LL * ((T + R - 1) / R);
+    const long long per_tile = adder_blocks(T);
     for (int c = 0; c < 4; ++c)
     {
         const long long n = color_begin[c + 1] - color_begin[c];
