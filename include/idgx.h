@@ -277,7 +277,7 @@ int idgx_grid_clear_box(const idgx_plan *plan, void *d_grid, int nr_layers, cons
  * precision = IDGX_FFT_FP64.  d_in == d_out transforms in place.  This library's kernels run:
  *   - FP32 64 x 64 and 128 x 128: one pass with the plane in registers;
  *   - other nx, ny powers of two in 16 .. 512, FP32 or FP64: LDS tiles (one pass when both sides are <= 128 and the
- *     plane fits 132 KB of LDS, i.e. up to 128 x 64 in FP64; else a row pass and a column pass, 64 MB of planes at
+ *     plane fits 132 KB of LDS, i.e. up to 128 x 64 in FP64; else a row pass and a column pass, 256 MB of planes at
  *     a time);
  *   - other power-of-two shapes with nx up to 16384 (FP32) / 8192 (FP64) and ny up to 16384 (FP64 every such
  *     shape; FP32 those with a side below 1024): rows in one LDS pass, columns longer than 512 in two four-step

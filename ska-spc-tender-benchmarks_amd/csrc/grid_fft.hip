@@ -222,6 +222,29 @@ template <int R, int SG> __device__ __forceinline__ void dft(float2 *v)
     }
 }
 
+// A point loaded or stored past the caches (nontemporal) or through them.
+template <bool ONCE> __device__ __forceinline__ float2 load_point(const float2 *p)
+{
+    if constexpr (ONCE)
+    {
+        typedef float pair __attribute__((ext_vector_type(2)));
+        const pair r = __builtin_nontemporal_load(reinterpret_cast<const pair *>(p));
+        return make_float2(r[0], r[1]);
+    }
+    else
+        return *p;
+}
+template <bool ONCE> __device__ __forceinline__ void store_point(float2 *p, float2 v)
+{
+    if constexpr (ONCE)
+    {
+        typedef float pair __attribute__((ext_vector_type(2)));
+        __builtin_nontemporal_store(pair{v.x, v.y}, reinterpret_cast<pair *>(p));
+    }
+    else
+        *p = v;
+}
+
 enum FftPass
 {
     kPassCol1 = 0,
@@ -248,6 +271,8 @@ struct FftArgs
     // for whole planes, (gy nc, nc, first column) for a box of nc columns stored compactly.
     int spitch, sx0;
     long long splane;
+    bool large;    // a plane exceeds what the caches hold from one pass to the next
+    bool src_once; // column pass 1's input is another array, and not worth a place in the memory-side cache
 };
 
 constexpr int ilog2(int n)
@@ -601,7 +626,8 @@ template <int L, int SG> __global__ __launch_bounds__(L / 16, (L >= 2048 ? 4 : 2
 // gridDim.x, ...  The next tile is loaded into registers while the current one is transformed.  L = 16 kRl:
 // a radix-16 stage from global memory, one LDS exchange, a radix-kRl stage to global memory.
 // ROWS (column pass 1 of a box): input rows outside [iy0, iy1) are zero and not read.
-template <int PASS, int L, int SG, bool ROWS = false>
+// ONCE: pass 1 loads, and pass 2 loads and stores, past the caches (launch_cols says when).
+template <int PASS, int L, int SG, bool ROWS, bool ONCE>
 __global__ __launch_bounds__(kColTile * L / 16) void fft_col_kernel(FftArgs A, int nr_tiles)
 {
     constexpr int kLog = ilog2(L);
@@ -630,7 +656,7 @@ __global__ __launch_bounds__(kColTile * L / 16) void fft_col_kernel(FftArgs A, i
     auto load = [&](int tile, int i) {
         const int q = (tile / A.nct) & ((1 << log_q) - 1);
         return static_cast<unsigned>(A.N2 * i + q - A.iy0) < static_cast<unsigned>(A.iy1 - A.iy0)
-                   ? in[element(tile, i)]
+                   ? load_point<ONCE>(in + element(tile, i))
                    : make_float2(0.F, 0.F);
     };
 
@@ -641,7 +667,7 @@ __global__ __launch_bounds__(kColTile * L / 16) void fft_col_kernel(FftArgs A, i
         const int j = threadIdx.x / kColTile;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            nxt[r] = ROWS ? load(tile, j + r * kQ) : in[element(tile, j + r * kQ)];
+            nxt[r] = ROWS ? load(tile, j + r * kQ) : load_point<ONCE>(in + element(tile, j + r * kQ));
     }
     for (; tile < nr_tiles; tile += gridDim.x)
     {
@@ -662,7 +688,7 @@ __global__ __launch_bounds__(kColTile * L / 16) void fft_col_kernel(FftArgs A, i
         {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                nxt[r] = ROWS ? load(tn, j0 + r * kQ) : in[element(tn, j0 + r * kQ)];
+                nxt[r] = ROWS ? load(tn, j0 + r * kQ) : load_point<ONCE>(in + element(tn, j0 + r * kQ));
         }
         dft<16, SG>(v);
         // Output r of butterfly j0 is element 16 j0 + r; the radix-kRl stage takes elements j0 + b kQ + r (L / kRl).
@@ -708,8 +734,8 @@ __global__ __launch_bounds__(kColTile * L / 16) void fft_col_kernel(FftArgs A, i
                     // Only the rows the row pass reads ([ry0, ry0 + nry), all rows when dense).
                     const int row = q + A.N1 * k;
                     if (static_cast<unsigned>(row - A.ry0) < static_cast<unsigned>(A.nry))
-                        A.scratch[sbase + static_cast<size_t>(row) * A.spitch + x] =
-                            (A.centred && (row & 1)) ? make_float2(-u[r].x, -u[r].y) : u[r];
+                        store_point<ONCE>(A.scratch + sbase + static_cast<size_t>(row) * A.spitch + x,
+                                          (A.centred && (row & 1)) ? make_float2(-u[r].x, -u[r].y) : u[r]);
                 }
             }
         }
@@ -885,27 +911,37 @@ hipError_t resident_blocks(const void *fn, int threads, int work, int &blocks)
     return e;
 }
 
-template <int PASS, int L, int SG, bool ROWS>
+template <int PASS, int L, int SG, bool ROWS, bool ONCE>
 hipError_t launch_cols_kernel(const FftArgs &A, int nr_tiles, hipStream_t st)
 {
     constexpr int threads = kColTile * L / 16;
     int blocks = 0;
-    const hipError_t e = resident_blocks(reinterpret_cast<const void *>(&fft_col_kernel<PASS, L, SG, ROWS>), threads,
+    const hipError_t e = resident_blocks(reinterpret_cast<const void *>(&fft_col_kernel<PASS, L, SG, ROWS, ONCE>), threads,
                                          nr_tiles, blocks);
     if (e != hipSuccess)
         return e;
-    fft_col_kernel<PASS, L, SG, ROWS><<<blocks, threads, 0, st>>>(A, nr_tiles);
+    fft_col_kernel<PASS, L, SG, ROWS, ONCE><<<blocks, threads, 0, st>>>(A, nr_tiles);
     return hipGetLastError();
 }
 
+// Past the caches where they cannot hold what the pass reads until it is used again: planes above 128 MB (G = 8192:
+// pass 1 / pass 2 to the image and back 78 / 114 and 112 / 78 us -> 66 / 104 and 87 / 77 for a box of half the columns;
+// smaller planes in place lose, 554 -> 612 us at G = 4096), and pass 1 from another array than it writes where the two
+// exceed the memory-side cache (G = 4096: 57 -> 50 us a plane; four planes at G = 1024 would lose 5 %).
 template <int PASS, int L, int SG> hipError_t launch_cols(const FftArgs &A, int nr_tiles, hipStream_t st)
 {
     if constexpr (PASS == kPassCol1)
     {
+        const bool once = A.large || A.src_once;
         if (A.iy0 > 0 || A.iy1 < A.gy)
-            return launch_cols_kernel<PASS, L, SG, true>(A, nr_tiles, st);
+            return once ? launch_cols_kernel<PASS, L, SG, true, true>(A, nr_tiles, st)
+                        : launch_cols_kernel<PASS, L, SG, true, false>(A, nr_tiles, st);
+        return once ? launch_cols_kernel<PASS, L, SG, false, true>(A, nr_tiles, st)
+                    : launch_cols_kernel<PASS, L, SG, false, false>(A, nr_tiles, st);
     }
-    return launch_cols_kernel<PASS, L, SG, false>(A, nr_tiles, st);
+    else
+        return A.large ? launch_cols_kernel<PASS, L, SG, false, true>(A, nr_tiles, st)
+                       : launch_cols_kernel<PASS, L, SG, false, false>(A, nr_tiles, st);
 }
 
 template <int PASS, int SG> hipError_t launch_col_pass(const FftArgs &A, int L, int nr_tiles, hipStream_t st)
@@ -1057,6 +1093,7 @@ hipError_t static_scratch(float2 *&out)
 // is still in the 256 MB Infinity Cache when the row pass reads it (measured at G = 4096: one 128 MB plane per
 // group 0.57 ms per direction, two planes 0.64 ms).
 constexpr long long kScratchBytes = 64LL << 20;
+constexpr long long kCacheBytes = 256LL << 20; // the memory-side cache
 
 // Restriction of a transform to a box of cells [x0, x1) x [y0, y1) of every plane.  kSparseInput: the input is
 // zero outside the box, so the column passes take only the column tiles that meet [x0, x1) and the row pass reads
@@ -1102,6 +1139,8 @@ FftArgs fft_args(int gx, int gy, bool centred)
     A.sx0 = 0;
     A.iy0 = 0;
     A.iy1 = gy;
+    A.large = static_cast<long long>(sizeof(float2)) * gx * gy > kCacheBytes / 2;
+    A.src_once = false;
     return A;
 }
 
@@ -1136,6 +1175,7 @@ hipError_t stockham_fft2d(const float2 *src, float2 *dst, int gx, int gy, long l
         A.iy0 = box.y0;
         A.iy1 = std::max(box.y0, box.y1);
     }
+    A.src_once = src != dst && planes * plane_bytes > kCacheBytes;
     A.rows_first = 0;
     if (box.mode == kRowsOut)
     {
@@ -1165,6 +1205,7 @@ hipError_t stockham_fft2d(const float2 *src, float2 *dst, int gx, int gy, long l
             C.src = g;
             C.grid = A.scratch;
             C.scratch = g;
+            C.src_once = 2 * group * plane_bytes >= kCacheBytes; // the rows: read once, with the scratch beside them
             C.rows_first = 1;
             C.ct0 = t0;
             C.nct = t1 - t0;

@@ -9,7 +9,7 @@
 // - Otherwise, with ny <= 512: rows (max(1, 4096 / nx) whole rows per tile, contiguous loads; nx up to 16384 in
 //   FP32, 8192 in FP64, whose padded row fills 128 KB; FP32 rows of 256 and 512 points in registers,
 //   rows_regs_kernel below), then columns in place (a tile of ny rows x C columns,
-//   C = max(4096 / ny, 128 bytes / point), so that every row segment is a whole 128-byte line); 64 MB of planes at
+//   C = max(4096 / ny, 128 bytes / point), so that every row segment is a whole 128-byte line); 256 MB of planes at
 //   a time, so that the column pass reads the row pass's output from the memory-side cache.
 // - With ny > 512: columns of ny = N1 N2 points in two four-step passes over tiles of C columns (A, in place: the
 //   N1-point DFTs over rows n1 N2 + n2, times W_ny^(n2 k1); B: the N2-point DFTs over rows k1 N2 + n2, into a
@@ -29,6 +29,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 
 namespace idgx
@@ -49,6 +50,41 @@ template <> struct Vec<double>
 {
     using type = double2;
 };
+
+// A point loaded or stored past the caches (nontemporal) or through them.
+template <bool ONCE, class V> __device__ __forceinline__ V load_point(const V *p)
+{
+    if constexpr (ONCE)
+    {
+        typedef decltype(V::x) pair __attribute__((ext_vector_type(2)));
+        const pair r = __builtin_nontemporal_load(reinterpret_cast<const pair *>(p));
+        V v;
+        v.x = r[0];
+        v.y = r[1];
+        return v;
+    }
+    else
+        return *p;
+}
+template <bool ONCE, class V> __device__ __forceinline__ void store_point(V *p, V v)
+{
+    if constexpr (ONCE)
+    {
+        typedef decltype(V::x) pair __attribute__((ext_vector_type(2)));
+        __builtin_nontemporal_store(pair{v.x, v.y}, reinterpret_cast<pair *>(p));
+    }
+    else
+        *p = v;
+}
+
+// body(std::bool_constant<once>): one of two copies of a tile's loads or stores, by a launch-wide flag.
+template <class Body> __device__ __forceinline__ void with_policy(bool once, Body &&body)
+{
+    if (once)
+        body(std::true_type{});
+    else
+        body(std::false_type{});
+}
 
 // cos(2 pi q / 16) and sin(2 pi q / 16) for any integer q, from cos(pi / 8), cos(pi / 4) and cos(3 pi / 8).
 constexpr double kCosEighthPi[5] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173, 0.0};
@@ -301,7 +337,7 @@ template <int NX, int NY> constexpr int plane_threads()
 template <int NX, int NY, int SG, class T>
 __global__ __launch_bounds__((plane_threads<NX, NY>())) void small_fft_planes_kernel(const typename Vec<T>::type *in,
                                                                                    typename Vec<T>::type *out,
-                                                                                   long long planes)
+                                                                                   long long planes, bool once)
 {
     using V = typename Vec<T>::type;
     constexpr int P = planes_per_tile<NX, NY>(), THREADS = plane_threads<NX, NY>();
@@ -316,15 +352,19 @@ __global__ __launch_bounds__((plane_threads<NX, NY>())) void small_fft_planes_ke
         const long long p0 = tile * P;
         const int np = static_cast<int>(planes - p0 < P ? planes - p0 : P);
         const V *src = in + p0 * PLANE;
-        for (int i = threadIdx.x; i < np * PLANE; i += THREADS)
-            lds[(i / NX) * PITCH + i % NX] = src[i];
+        with_policy(once, [&](auto o) {
+            for (int i = threadIdx.x; i < np * PLANE; i += THREADS)
+                lds[(i / NX) * PITCH + i % NX] = load_point<o.value>(src + i);
+        });
         lds_barrier();
         fft_lines<NX, P * NY, THREADS, SG>(lds, tw, [](int line, int e) { return line * PITCH + e; });
         fft_lines<NY, P * NX, THREADS, SG>(
             lds, tw + NX, [](int line, int e) { return ((line / NX) * NY + e) * PITCH + line % NX; });
         V *dst = out + p0 * PLANE;
-        for (int i = threadIdx.x; i < np * PLANE; i += THREADS)
-            dst[i] = lds[(i / NX) * PITCH + i % NX];
+        with_policy(once, [&](auto o) {
+            for (int i = threadIdx.x; i < np * PLANE; i += THREADS)
+                store_point<o.value>(dst + i, lds[(i / NX) * PITCH + i % NX]);
+        });
         lds_barrier();
     }
 }
@@ -340,6 +380,8 @@ __global__ __launch_bounds__((plane_threads<NX, NY>())) void small_fft_planes_ke
 // points (lanes j of 32-lane halves of a wave land in distinct banks both ways); the transpose pitch N + 32 / R
 // makes its column reads conflict-free.  At N = 128 the 64-VGPR limit leaves 24 bytes per lane in scratch; a form
 // that recomputed the line indices in each phase spilled less and measured slower (71.0 against 64.7 ns per plane).
+// Loads and stores go through the caches: several of them share each line (16384 planes of 64 x 64: 213 us, past the
+// caches 289).
 template <int N> constexpr int plane_regs_waves_per_simd()
 {
     return N * N / 16 / 64 / 4 * 2; // two workgroups of N^2 / 16 threads per CU
@@ -433,7 +475,7 @@ __global__ __launch_bounds__(N * N / 16, plane_regs_waves_per_simd<N>()) void pl
 //            X[kk + 16 q + 256 j1] = Z_0[q] + (-1)^j1 W_32^q Z_1[q], a butterfly between neighbouring lanes (a DPP
 //            lane swap).
 // LDS holds one float per point (real parts, then imaginary parts) with one pad slot per 16 points.
-template <int N, int SG>
+template <int N, int SG, bool ONCE>
 __global__ __launch_bounds__(256) void rows_regs_kernel(const float2 *in, float2 *out, long long rows)
 {
     constexpr int THREADS = 256, R = N / 16, ROWS = THREADS / R, LP = N + N / 16;
@@ -461,7 +503,7 @@ __global__ __launch_bounds__(256) void rows_regs_kernel(const float2 *in, float2
         float2 v[16];
 #pragma unroll
         for (int m = 0; m < 16; ++m)
-            v[m] = live ? src[j + R * m] : make_float2(0.F, 0.F);
+            v[m] = live ? load_point<ONCE>(src + j + R * m) : make_float2(0.F, 0.F);
         dft<16, SG>(v);
 #pragma unroll
         for (int k = 1; k < 16; ++k)
@@ -539,7 +581,7 @@ template <int NX> constexpr int row_threads()
 
 template <int NX, int SG, class T>
 __global__ __launch_bounds__((row_threads<NX>())) void small_fft_rows_kernel(const typename Vec<T>::type *in,
-                                                                           typename Vec<T>::type *out, long long rows)
+                                                                           typename Vec<T>::type *out, long long rows, bool once)
 {
     using V = typename Vec<T>::type;
     constexpr int ROWS = rows_per_tile<NX>(), THREADS = row_threads<NX>(), PITCH = NX + 1;
@@ -552,8 +594,10 @@ __global__ __launch_bounds__((row_threads<NX>())) void small_fft_rows_kernel(con
         const long long r0 = tile * ROWS;
         const int nr = static_cast<int>(rows - r0 < ROWS ? rows - r0 : ROWS);
         const V *src = in + r0 * NX;
-        for (int i = threadIdx.x; i < nr * NX; i += THREADS)
-            lds[(i / NX) * PITCH + i % NX] = src[i];
+        with_policy(once, [&](auto o) {
+            for (int i = threadIdx.x; i < nr * NX; i += THREADS)
+                lds[(i / NX) * PITCH + i % NX] = load_point<o.value>(src + i);
+        });
         lds_barrier();
         fft_lines<NX, ROWS, THREADS, SG>(lds, tw, [](int line, int e) { return line * PITCH + e; });
         V *dst = out + r0 * NX;
@@ -570,7 +614,7 @@ template <int NY, class T> constexpr int column_tile()
 }
 
 // Column pass, in place: tiles of NY rows x C columns of one plane (C consecutive points of every row).
-template <int NY, int SG, class T>
+template <int NY, int SG, class T, bool ONCE>
 __global__ __launch_bounds__((NY * column_tile<NY, T>() / kPointsPerThread)) void small_fft_columns_kernel(
     typename Vec<T>::type *data, int nx, long long tiles)
 {
@@ -586,11 +630,11 @@ __global__ __launch_bounds__((NY * column_tile<NY, T>() / kPointsPerThread)) voi
         const int c0 = static_cast<int>(tile - plane * per_plane) * C;
         V *p = data + plane * static_cast<long long>(nx) * NY + c0;
         for (int i = threadIdx.x; i < NY * C; i += THREADS)
-            lds[i] = p[static_cast<long long>(i / C) * nx + i % C];
+            lds[i] = load_point<ONCE>(p + static_cast<long long>(i / C) * nx + i % C);
         lds_barrier();
         fft_lines<NY, C, THREADS, SG>(lds, tw, [](int line, int e) { return e * C + line; });
         for (int i = threadIdx.x; i < NY * C; i += THREADS)
-            p[static_cast<long long>(i / C) * nx + i % C] = lds[i];
+            store_point<ONCE>(p + static_cast<long long>(i / C) * nx + i % C, lds[i]);
         lds_barrier();
     }
 }
@@ -662,11 +706,16 @@ unsigned grid_for(long long tiles)
     return static_cast<unsigned>(tiles < kMaxGrid ? tiles : kMaxGrid);
 }
 
-template <int N, int SG> hipError_t rows_regs_pass(const void *in, void *out, long long rows, hipStream_t st)
+template <int N, int SG> hipError_t rows_regs_pass(const void *in, void *out, long long rows, bool once, hipStream_t st)
 {
     constexpr int ROWS = 256 / (N / 16);
-    rows_regs_kernel<N, SG><<<grid_for((rows + ROWS - 1) / ROWS), 256, 0, st>>>(static_cast<const float2 *>(in),
-                                                                                static_cast<float2 *>(out), rows);
+    const unsigned blocks = grid_for((rows + ROWS - 1) / ROWS);
+    const float2 *src = static_cast<const float2 *>(in);
+    float2 *dst = static_cast<float2 *>(out);
+    if (once)
+        rows_regs_kernel<N, SG, true><<<blocks, 256, 0, st>>>(src, dst, rows);
+    else
+        rows_regs_kernel<N, SG, false><<<blocks, 256, 0, st>>>(src, dst, rows);
     return hipGetLastError();
 }
 
@@ -678,69 +727,74 @@ template <int N, int SG> hipError_t plane_regs_pass(const void *in, void *out, l
 }
 
 template <int NX, int NY, int SG, class T>
-hipError_t planes_pass(const void *in, void *out, long long batch, hipStream_t st)
+hipError_t planes_pass(const void *in, void *out, long long batch, bool once, hipStream_t st)
 {
     using V = typename Vec<T>::type;
     constexpr int P = planes_per_tile<NX, NY>();
     small_fft_planes_kernel<NX, NY, SG, T><<<grid_for((batch + P - 1) / P), plane_threads<NX, NY>(), 0, st>>>(
-        static_cast<const V *>(in), static_cast<V *>(out), batch);
+        static_cast<const V *>(in), static_cast<V *>(out), batch, once);
     return hipGetLastError();
 }
 
-template <int NX, int SG, class T> hipError_t rows_pass(const void *in, void *out, long long rows, hipStream_t st)
+template <int NX, int SG, class T> hipError_t rows_pass(const void *in, void *out, long long rows, bool once, hipStream_t st)
 {
     using V = typename Vec<T>::type;
     constexpr int ROWS = rows_per_tile<NX>();
     small_fft_rows_kernel<NX, SG, T><<<grid_for((rows + ROWS - 1) / ROWS), row_threads<NX>(), 0, st>>>(
-        static_cast<const V *>(in), static_cast<V *>(out), rows);
+        static_cast<const V *>(in), static_cast<V *>(out), rows, once);
     return hipGetLastError();
 }
 
-template <int NY, int SG, class T> hipError_t columns_pass(void *data, int nx, long long batch, hipStream_t st)
+template <int NY, int SG, class T> hipError_t columns_pass(void *data, int nx, long long batch, bool once, hipStream_t st)
 {
     using V = typename Vec<T>::type;
     constexpr int C = column_tile<NY, T>();
     if (nx % C != 0)
         return hipErrorInvalidValue;
     const long long tiles = batch * (nx / C);
-    small_fft_columns_kernel<NY, SG, T><<<grid_for(tiles), NY * C / kPointsPerThread, 0, st>>>(static_cast<V *>(data),
-                                                                                             nx, tiles);
+    const unsigned blocks = grid_for(tiles);
+    if (once)
+        small_fft_columns_kernel<NY, SG, T, true><<<blocks, NY * C / kPointsPerThread, 0, st>>>(static_cast<V *>(data),
+                                                                                               nx, tiles);
+    else
+        small_fft_columns_kernel<NY, SG, T, false><<<blocks, NY * C / kPointsPerThread, 0, st>>>(static_cast<V *>(data),
+                                                                                                nx, tiles);
     return hipGetLastError();
 }
 
-template <int SG, class T> hipError_t rows_any(int nx, const void *in, void *out, long long rows, hipStream_t st)
+template <int SG, class T> hipError_t rows_any(int nx, const void *in, void *out, long long rows, bool once, hipStream_t st)
 {
     switch (nx)
     {
     case 16:
-        return rows_pass<16, SG, T>(in, out, rows, st);
+        return rows_pass<16, SG, T>(in, out, rows, once, st);
     case 32:
-        return rows_pass<32, SG, T>(in, out, rows, st);
+        return rows_pass<32, SG, T>(in, out, rows, once, st);
     case 64:
-        return rows_pass<64, SG, T>(in, out, rows, st);
+        return rows_pass<64, SG, T>(in, out, rows, once, st);
     case 128:
-        return rows_pass<128, SG, T>(in, out, rows, st);
+        return rows_pass<128, SG, T>(in, out, rows, once, st);
     case 256:
         if constexpr (sizeof(T) == sizeof(float))
-            return rows_regs_pass<256, SG>(in, out, rows, st);
+            return rows_regs_pass<256, SG>(in, out, rows, once, st);
         else
-            return rows_pass<256, SG, T>(in, out, rows, st);
+            return rows_pass<256, SG, T>(in, out, rows, once, st);
     case 512:
         if constexpr (sizeof(T) == sizeof(float))
-            return rows_regs_pass<512, SG>(in, out, rows, st);
+            return rows_regs_pass<512, SG>(in, out, rows, once, st);
         else
-            return rows_pass<512, SG, T>(in, out, rows, st);
+            return rows_pass<512, SG, T>(in, out, rows, once, st);
     case 1024:
-        return rows_pass<1024, SG, T>(in, out, rows, st);
+        return rows_pass<1024, SG, T>(in, out, rows, once, st);
     case 2048:
-        return rows_pass<2048, SG, T>(in, out, rows, st);
+        return rows_pass<2048, SG, T>(in, out, rows, once, st);
     case 4096:
-        return rows_pass<4096, SG, T>(in, out, rows, st);
+        return rows_pass<4096, SG, T>(in, out, rows, once, st);
     case 8192:
-        return rows_pass<8192, SG, T>(in, out, rows, st);
+        return rows_pass<8192, SG, T>(in, out, rows, once, st);
     case 16384:
         if constexpr (sizeof(T) == 4) // a padded FP64 row of 16384 points does not fit LDS
-            return rows_pass<16384, SG, T>(in, out, rows, st);
+            return rows_pass<16384, SG, T>(in, out, rows, once, st);
         else
             return hipErrorInvalidValue;
     default:
@@ -748,22 +802,22 @@ template <int SG, class T> hipError_t rows_any(int nx, const void *in, void *out
     }
 }
 
-template <int SG, class T> hipError_t columns_any(int ny, void *data, int nx, long long batch, hipStream_t st)
+template <int SG, class T> hipError_t columns_any(int ny, void *data, int nx, long long batch, bool once, hipStream_t st)
 {
     switch (ny)
     {
     case 16:
-        return columns_pass<16, SG, T>(data, nx, batch, st);
+        return columns_pass<16, SG, T>(data, nx, batch, once, st);
     case 32:
-        return columns_pass<32, SG, T>(data, nx, batch, st);
+        return columns_pass<32, SG, T>(data, nx, batch, once, st);
     case 64:
-        return columns_pass<64, SG, T>(data, nx, batch, st);
+        return columns_pass<64, SG, T>(data, nx, batch, once, st);
     case 128:
-        return columns_pass<128, SG, T>(data, nx, batch, st);
+        return columns_pass<128, SG, T>(data, nx, batch, once, st);
     case 256:
-        return columns_pass<256, SG, T>(data, nx, batch, st);
+        return columns_pass<256, SG, T>(data, nx, batch, once, st);
     case 512:
-        return columns_pass<512, SG, T>(data, nx, batch, st);
+        return columns_pass<512, SG, T>(data, nx, batch, once, st);
     default:
         return hipErrorInvalidValue;
     }
@@ -830,13 +884,13 @@ template <int NX, int NY, class T> constexpr bool one_pass()
 }
 
 template <int SG, class T, int NX, int NY>
-bool try_planes(int nx, int ny, const void *in, void *out, long long b, hipStream_t st, hipError_t &e)
+bool try_planes(int nx, int ny, const void *in, void *out, long long b, bool once, hipStream_t st, hipError_t &e)
 {
     if constexpr (one_pass<NX, NY, T>())
     {
         if (nx == NX && ny == NY)
         {
-            e = planes_pass<NX, NY, SG, T>(in, out, b, st);
+            e = planes_pass<NX, NY, SG, T>(in, out, b, once, st);
             return true;
         }
     }
@@ -844,18 +898,18 @@ bool try_planes(int nx, int ny, const void *in, void *out, long long b, hipStrea
 }
 
 template <int SG, class T, int NX, int... LY>
-bool try_row(int nx, int ny, const void *in, void *out, long long b, hipStream_t st, hipError_t &e,
+bool try_row(int nx, int ny, const void *in, void *out, long long b, bool once, hipStream_t st, hipError_t &e,
              std::integer_sequence<int, LY...>)
 {
-    return (try_planes<SG, T, NX, (16 << LY)>(nx, ny, in, out, b, st, e) || ...);
+    return (try_planes<SG, T, NX, (16 << LY)>(nx, ny, in, out, b, once, st, e) || ...);
 }
 
 // Sides 16, 32, 64, 128 (16 << 0 .. 16 << 3) in both directions.
 template <int SG, class T, int... LX>
-bool planes_any(int nx, int ny, const void *in, void *out, long long b, hipStream_t st, hipError_t &e,
+bool planes_any(int nx, int ny, const void *in, void *out, long long b, bool once, hipStream_t st, hipError_t &e,
                 std::integer_sequence<int, LX...>)
 {
-    return (try_row<SG, T, (16 << LX)>(nx, ny, in, out, b, st, e, std::make_integer_sequence<int, 4>()) || ...);
+    return (try_row<SG, T, (16 << LX)>(nx, ny, in, out, b, once, st, e, std::make_integer_sequence<int, 4>()) || ...);
 }
 
 bool pow2_in(int n, int lo, int hi)
@@ -865,12 +919,23 @@ bool pow2_in(int n, int lo, int hi)
 
 // Planes per launch group of the four-step path: the scratch holds one group (64 MB, or one plane when larger).
 constexpr long long kGroupBytes = 64LL << 20;
+// Planes per launch group of the two-pass path: the row pass's output of a group, which the column pass finds in the
+// 256 MB memory-side cache as long as nothing else passes through it (256 planes of 512 x 512 FP32, 512 MB: groups of
+// 64 MB 514 us, and past the caches with groups of 128 / 192 / 256 / 512 MB 461 / 450 / 436 / 432 us).
+constexpr long long kCacheBytes = 256LL << 20;
+// Batches above this read their input and write their final output past the caches (nontemporal), which could not keep
+// them for the next kernel anyway.  Half of the cache's size: 100 planes of 256 x 256 FP32 (52 MB) took 47.6 us through
+// the caches and 49.2 past them, 64 of 512 x 512 (134 MB) 126 and 120, with the groups above.
+constexpr long long kOnceBytes = 128LL << 20;
 
 template <int SG, class T>
 hipError_t lds_fft(const void *in, void *out, int nx, int ny, long long batch, hipStream_t st)
 {
     using V = typename Vec<T>::type;
     hipError_t e = hipSuccess;
+    const long long plane = static_cast<long long>(nx) * ny;
+    const long long plane_bytes = plane * static_cast<long long>(sizeof(V));
+    const bool once = batch > kOnceBytes / plane_bytes;
     if constexpr (sizeof(T) == sizeof(float))
     {
         if (nx == ny && nx == 64)
@@ -878,27 +943,26 @@ hipError_t lds_fft(const void *in, void *out, int nx, int ny, long long batch, h
         if (nx == ny && nx == 128)
             return plane_regs_pass<128, SG>(in, out, batch, st);
     }
-    if (planes_any<SG, T>(nx, ny, in, out, batch, st, e, std::make_integer_sequence<int, 4>()))
+    if (planes_any<SG, T>(nx, ny, in, out, batch, once, st, e, std::make_integer_sequence<int, 4>()))
         return e;
-    const long long plane = static_cast<long long>(nx) * ny;
-    const long long plane_bytes = plane * static_cast<long long>(sizeof(V));
-    const long long group = std::max(1LL, std::min(batch, kGroupBytes / plane_bytes));
     if (ny <= 512)
     {
         // Rows in -> out, then the columns in place, a group of planes at a time: the column pass finds the row
         // pass's output of its group in the memory-side cache instead of HBM.
+        const long long group = std::max(1LL, std::min(batch, kCacheBytes / plane_bytes));
         const V *src = static_cast<const V *>(in);
         V *dst = static_cast<V *>(out);
         for (long long p = 0; p < batch && e == hipSuccess; p += group)
         {
             const long long n = std::min(group, batch - p);
-            e = rows_any<SG, T>(nx, src + p * plane, dst + p * plane, n * ny, st);
+            e = rows_any<SG, T>(nx, src + p * plane, dst + p * plane, n * ny, once, st);
             if (e == hipSuccess)
-                e = columns_any<SG, T>(ny, dst + p * plane, nx, n, st);
+                e = columns_any<SG, T>(ny, dst + p * plane, nx, n, once, st);
         }
         return e;
     }
     // Four-step columns (in -> out, out -> scratch), then the rows scratch -> out, a group of planes at a time.
+    const long long group = std::max(1LL, std::min(batch, kGroupBytes / plane_bytes));
     float2 *scratch = nullptr;
     e = fft_plane_scratch(group * plane * static_cast<long long>(sizeof(V) / sizeof(float2)), scratch, 2);
     const V *src = static_cast<const V *>(in);
@@ -908,7 +972,7 @@ hipError_t lds_fft(const void *in, void *out, int nx, int ny, long long batch, h
         const long long n = std::min(group, batch - p);
         e = long_columns<SG, T>(ny, src + p * plane, dst + p * plane, scratch, nx, n, st);
         if (e == hipSuccess)
-            e = rows_any<SG, T>(nx, scratch, dst + p * plane, n * ny, st);
+            e = rows_any<SG, T>(nx, scratch, dst + p * plane, n * ny, false, st);
     }
     return e;
 }
