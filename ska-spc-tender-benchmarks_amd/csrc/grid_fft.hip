@@ -40,6 +40,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 
 #include "idgx_device.hpp"
 #include "kernels.hpp"
@@ -334,9 +335,13 @@ template <int L, int SG> __device__ __forceinline__ void row_twiddle_tables(floa
 // (L + L / 16 floats) after each, then a radix-kRl stage when L is not a power of 16.  Output element k, the idx-th
 // (0 .. 15, a compile-time index after unrolling) of this thread's, goes to emit(idx, k, value).  The first exchange
 // waits for every thread's reads of buf from the previous call.
-template <int L, int SG, class Emit>
-__device__ __forceinline__ void row_transform(float2 (&v)[16], int j0, float (&buf)[L + L / 16],
-                                              const float2 (&t_hi)[L / 64], const float2 (&t_lo)[64], Emit &&emit)
+// buf holds floats (the exchanges send real parts, then imaginary parts: half the LDS) or complex values (half the
+// barriers).  stage_tw(Ns, j, r, tw) gives the twiddles W_{16 Ns}^(j r) of the radix-16 stage at Ns, tw being the
+// two-level table; nullptr: that table.
+template <int L, int SG, class Stage, class Emit, class Slot>
+__device__ __forceinline__ void row_transform(float2 (&v)[16], int j0, Slot (&buf)[L + L / 16],
+                                              const float2 (&t_hi)[L / 64], const float2 (&t_lo)[64], Stage stage_tw,
+                                              Emit &&emit)
 {
     constexpr int kLog = ilog2(L);
     constexpr int kStages16 = kLog / 4;
@@ -360,7 +365,12 @@ __device__ __forceinline__ void row_transform(float2 (&v)[16], int j0, float (&b
             const int m = (j0 & (Ns - 1)) * (L / (16 * Ns));
 #pragma unroll
             for (int r = 1; r < 16; ++r)
-                v[r] = f2mul(v[r], tw(m * r));
+            {
+                if constexpr (std::is_same_v<Stage, std::nullptr_t>)
+                    v[r] = f2mul(v[r], tw(m * r));
+                else
+                    v[r] = f2mul(v[r], stage_tw(Ns, j0 & (Ns - 1), r, tw));
+            }
         }
         dft<16, SG>(v);
         if (st == kStages16 - 1 && kRl == 1)
@@ -379,23 +389,36 @@ __device__ __forceinline__ void row_transform(float2 (&v)[16], int j0, float (&b
             const int rb = j0 + (j0 >> 4);
             const bool next16 = st + 1 < kStages16;
             auto rslot = [&](int t) { return next16 ? rb + t * kQs : rb + (t / kRl) * kQs + (t % kRl) * kRs; };
-            float re[16];
             lds_barrier(); // the previous exchange's reads are done
+            if constexpr (std::is_same_v<Slot, float2>)
+            {
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                buf[wb + r * ws] = v[r].x;
-            lds_barrier();
+                for (int r = 0; r < 16; ++r)
+                    buf[wb + r * ws] = v[r];
+                lds_barrier();
 #pragma unroll
-            for (int t = 0; t < 16; ++t)
-                re[t] = buf[rslot(t)];
-            lds_barrier();
+                for (int t = 0; t < 16; ++t)
+                    v[t] = buf[rslot(t)];
+            }
+            else
+            {
+                float re[16];
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                buf[wb + r * ws] = v[r].y;
-            lds_barrier();
+                for (int r = 0; r < 16; ++r)
+                    buf[wb + r * ws] = v[r].x;
+                lds_barrier();
 #pragma unroll
-            for (int t = 0; t < 16; ++t)
-                v[t] = make_float2(re[t], buf[rslot(t)]);
+                for (int t = 0; t < 16; ++t)
+                    re[t] = buf[rslot(t)];
+                lds_barrier();
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    buf[wb + r * ws] = v[r].y;
+                lds_barrier();
+#pragma unroll
+                for (int t = 0; t < 16; ++t)
+                    v[t] = make_float2(re[t], buf[rslot(t)]);
+            }
         }
         Ns *= 16;
     }
@@ -465,7 +488,7 @@ __global__ __launch_bounds__(L / 16, (fft_row_waves_per_simd<L, R3>())) void fft
 #pragma unroll
         for (int r = 0; r < 16; ++r)
             v[r] = load(gr, in_row, j0 + r * kQ);
-        row_transform<L, SG>(v, j0, buf, t_hi, t_lo, emit);
+        row_transform<L, SG>(v, j0, buf, t_hi, t_lo, nullptr, emit);
     };
     for (int i = blockIdx.x; i < rows; i += gridDim.x)
     {
@@ -524,13 +547,27 @@ struct WsArgs
     double image_size, w_step;
 };
 
+// What bounds it: VALU issue, at the four waves per SIMD that its registers leave (n, the sums and the row: 96 VGPRs).
+// They hold two workgroups per CU at L = 8192, so LDS has room for complex exchanges and for the second stage's
+// twiddles in a table of their own: 8192 rows, 6 layers, half the columns in use: 1140 -> 1048 us to the image, 1129
+// -> 985 from it (33 KB more of LDS for the third stage's twiddles as well, with exchanges in floats: 1068 and 1054).
 template <int L, int SG> __global__ __launch_bounds__(L / 16, (L >= 2048 ? 4 : 2)) void wstack_row_kernel(WsArgs W)
 {
     constexpr int kQ = L / 16;
-    __shared__ float buf[L + L / 16];
+    __shared__ float2 buf[L + L / 16];
     __shared__ float2 t_hi[L / 64], t_lo[64];
+    __shared__ float2 t_256[15 * 15 + 1]; // W_256^q, q = j r of the second stage
     row_twiddle_tables<L, SG>(t_hi, t_lo);
+    for (int i = threadIdx.x; i <= 15 * 15; i += L / 16)
+    {
+        double sn, cs;
+        sincospi(2.0 * i / 256, &sn, &cs);
+        t_256[i] = make_float2(static_cast<float>(cs), static_cast<float>(SG * sn));
+    }
     __syncthreads();
+    const auto stage_tw = [&](int Ns, int j, int r, auto &&two_level) {
+        return Ns == 16 ? t_256[j * r] : two_level(j * (L / (16 * Ns)) * r);
+    };
     for (int y = blockIdx.x; y < L; y += gridDim.x)
     {
         int j0 = threadIdx.x; // opaque per row, as in the row pass
@@ -579,7 +616,7 @@ template <int L, int SG> __global__ __launch_bounds__(L / 16, (L >= 2048 ? 4 : 2
                     const int col = jz + r * kQ;
                     v[r] = col >= W.cx0 && col < W.cx1 ? in_row[col - W.cx0] : make_float2(0.F, 0.F);
                 }
-                row_transform<L, SG>(v, jz, buf, t_hi, t_lo, [&](int idx, int, float2 val) {
+                row_transform<L, SG>(v, jz, buf, t_hi, t_lo, stage_tw, [&](int idx, int, float2 val) {
                     const int t = row_out_t<L>(idx);
                     const float2 w = screen(wz, t);
                     acc[t].x = __builtin_fmaf(val.x, w.x, __builtin_fmaf(-val.y, w.y, acc[t].x));
@@ -612,7 +649,7 @@ template <int L, int SG> __global__ __launch_bounds__(L / 16, (L >= 2048 ? 4 : 2
                 float2 *out_row = W.rows_out + z * W.layer_stride + static_cast<long long>(y) * W.pitch;
                 int jz = j0;
                 asm volatile("" : "+v"(jz));
-                row_transform<L, SG>(v, jz, buf, t_hi, t_lo, [&](int, int k, float2 val) {
+                row_transform<L, SG>(v, jz, buf, t_hi, t_lo, stage_tw, [&](int, int k, float2 val) {
                     if (k >= W.cx0 && k < W.cx1)
                         out_row[k] = odd ? make_float2(-val.x, -val.y) : val;
                 });
