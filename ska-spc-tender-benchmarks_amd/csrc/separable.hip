@@ -1,5 +1,5 @@
 // Separable mixed-precision gridder and degridder for gfx950: phasors per (row, visibility) and per (column,
-// visibility) instead of per (pixel, visibility), contracted on v_mfma_f32_16x16x32_{f16,bf16}.
+// visibility) instead of per (pixel, visibility), contracted on v_mfma_f32_32x32x16_{f16,bf16}.
 //
 // Phase.  With half-integer pixel coordinates xh = x + 1/2 - S/2 (l = xh delta, delta = image_size / S) the phase of a
 // visibility at a pixel is, in revolutions,
@@ -66,20 +66,21 @@ struct alignas(16) DegridStage
 };
 
 // LDS of a workgroup: a column's (a, g) at its index, and one of the phases' working sets.
-template <int TAB, int COLS, int SPLITS> struct alignas(16) GridLds
+template <int COLS, int SPLITS, int ROWS, int WAVES> struct alignas(16) GridLds
 {
-    float2 tab[TAB];
+    float2 tab[kSeparableMax];
+    float slots[WAVES][5];
     union
     {
-        GridStage stage[kWaves];
-        float2 sum[SPLITS][16 * COLS * 4]; // the splits' partial sums of 16 rows
+        GridStage stage[WAVES];
+        float2 sum[SPLITS][ROWS * COLS * 4]; // the splits' partial sums of a pass of rows
         GridderShared<kDefaultPT, kDefaultVB> direct;
     };
 };
 template <int WAVES> struct alignas(16) DegridLds
 {
     float2 tab[kSeparableMax];
-    unsigned maxbits;
+    float slots[WAVES][5];
     DegridStage stage[WAVES];
     uint4 pixels[1]; // as many as the subgrid needs
 };
@@ -99,10 +100,11 @@ struct WRange
     float half;    // half its width
 };
 
-// Range of w (wavelengths) over a subgrid's rows and channel window; every thread of the workgroup gets the same.
-// (LDS-only barriers: the first visibilities' loads stay in flight across them.)
-template <int WAVES>
-__device__ __forceinline__ WRange w_range(const KernelArgs &a, long long row0, int T, int c0, int nc, float *slots)
+// Range of w (wavelengths) over a subgrid's rows and channel window, and the largest vmax: every thread of the workgroup
+// gets the same.  One LDS-only barrier, which also covers what the caller has written (loads stay in flight across it).
+template <int WAVES, bool MAX>
+__device__ __forceinline__ WRange w_range(const KernelArgs &a, long long row0, int T, int c0, int nc,
+                                          float (&slots)[WAVES][5], float &vmax)
 {
     float wlo = __builtin_inff(), whi = -__builtin_inff(), klo = __builtin_inff(), khi = -__builtin_inff();
     for (int t = threadIdx.x; t < T; t += 64 * WAVES)
@@ -124,27 +126,44 @@ __device__ __forceinline__ WRange w_range(const KernelArgs &a, long long row0, i
         whi = fmaxf(whi, __shfl_xor(whi, d));
         klo = fminf(klo, __shfl_xor(klo, d));
         khi = fmaxf(khi, __shfl_xor(khi, d));
+        if constexpr (MAX)
+            vmax = fmaxf(vmax, __shfl_xor(vmax, d));
     }
     if ((threadIdx.x & 63) == 0)
     {
-        float *s = slots + 4 * (threadIdx.x >> 6);
-        s[0] = wlo, s[1] = whi, s[2] = klo, s[3] = khi;
+        float *s = slots[threadIdx.x >> 6];
+        s[0] = wlo, s[1] = whi, s[2] = klo, s[3] = khi, s[4] = vmax;
     }
     lds_barrier();
 #pragma unroll
     for (int w = 0; w < WAVES; ++w)
     {
-        wlo = fminf(wlo, slots[4 * w]);
-        whi = fmaxf(whi, slots[4 * w + 1]);
-        klo = fminf(klo, slots[4 * w + 2]);
-        khi = fmaxf(khi, slots[4 * w + 3]);
+        wlo = fminf(wlo, slots[w][0]);
+        whi = fmaxf(whi, slots[w][1]);
+        klo = fminf(klo, slots[w][2]);
+        khi = fmaxf(khi, slots[w][3]);
+        if constexpr (MAX)
+            vmax = fmaxf(vmax, slots[w][4]);
     }
-    lds_barrier();
     const double p0 = static_cast<double>(wlo) * klo, p1 = static_cast<double>(wlo) * khi;
     const double p2 = static_cast<double>(whi) * klo, p3 = static_cast<double>(whi) * khi;
     const double lo = fmin(fmin(p0, p1), fmin(p2, p3)) * kInv2Pi, hi = fmax(fmax(p0, p1), fmax(p2, p3)) * kInv2Pi;
     return {0.5 * (lo + hi), static_cast<float>(0.5 * (hi - lo))};
 }
+
+// q / cols for q < 4096 and cols <= 64 (q (cols - 1) < 2^20): two instructions instead of a division.
+struct SmallDivisor
+{
+    unsigned magic;
+    __device__ __forceinline__ explicit SmallDivisor(int cols)
+        : magic(((1U << 20) + static_cast<unsigned>(cols) - 1U) / static_cast<unsigned>(cols))
+    {
+    }
+    __device__ __forceinline__ int quotient(int q) const
+    {
+        return static_cast<int>(__umul24(static_cast<unsigned>(q), magic) >> 20);
+    }
+};
 
 // Reduced phase coordinates of one visibility, signed by sgn: slopes per pixel in [-1/2, 1/2], w relative to the
 // subgrid's middle, and the parity of the whole turns taken off the slopes (half-integer coordinates turn each of
@@ -534,14 +553,21 @@ __device__ __forceinline__ void fill_table(float2 *tab, const SeparableArgs &sp,
     }
 }
 
-// Workgroup (part, subgrid) grids columns [part, part + 1) x 8 NT NX of a subgrid: its waves take NX column ranges and
-// kWaves / NX interleaved chunks of visibilities; the partial sums meet in LDS 16 rows at a time, in a fixed order.
-template <int DT, int YT, int NT, int NX>
-__global__ __launch_bounds__(kThreads, YT * NT <= 2 ? 4 : YT * NT <= 3 ? 3 : 2)
-    void grid_separable(KernelArgs a, SeparableArgs sp)
+// Waves per SIMD that the gridder's registers are held to.  YT = 2, NT = 3 (S = 24) spills 42 of them in its prologue
+// and epilogue at three, and is 1 to 4 % faster than at two.
+template <int YT, int NT> constexpr int grid_waves()
 {
-    constexpr int kCols = NX * NT * 8, kSplits = kWaves / NX;
-    __shared__ GridLds<kSeparableMax, kCols, kSplits> sm;
+    return YT * NT <= 2 ? 4 : YT * NT <= 3 || (YT == 2 && NT == 3) ? 3 : 2;
+}
+
+// Workgroup (part, subgrid) grids columns [part, part + 1) x 8 NT NX of a subgrid: its waves take NX column ranges and
+// WAVES / NX interleaved chunks of visibilities; the partial sums meet in LDS 16 or 32 rows at a time, in a fixed order.
+template <int DT, int YT, int NT, int NX, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, (grid_waves<YT, NT>())) void grid_separable(KernelArgs a, SeparableArgs sp)
+{
+    constexpr int kCols = NX * NT * 8, kSplits = WAVES / NX, kCount = 64 * WAVES;
+    constexpr int kPass = NT == 1 ? 32 : 16; // rows of the subgrid whose sums meet at a time
+    __shared__ GridLds<kCols, kSplits, kPass, WAVES> sm;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int part = blockIdx.x / a.p.nr_subgrids, b = blockIdx.x - part * a.p.nr_subgrids;
     const int s = sp.order ? sp.order[b] : b;
@@ -556,9 +582,11 @@ __global__ __launch_bounds__(kThreads, YT * NT <= 2 ? 4 : YT * NT <= 3 ? 3 : 2)
     // Chunks short enough for every split to have one.
     const int split = wave / NX, n = min(kChunk, ((V + kSplits - 1) / kSplits + 7) & ~7);
     RawVisibility raw = load_visibility(a, sel, lane < n ? split * n + lane : V, V, T, nc, row0, c0);
+    fill_table(sm.tab, sp, S);
     WRange wr = {0.0, 0.F};
-    if (V > 0)
-        wr = w_range<kWaves>(a, row0, T, c0, nc, reinterpret_cast<float *>(sm.tab));
+    float none = 0.F;
+    if (V > 0) // (without visibilities nothing reads the table)
+        wr = w_range<WAVES, false>(a, row0, T, c0, nc, sm.slots, none);
     const float eps = wr.half * sp.tables.eps;
     const bool fits = eps <= kEpsMost && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
     if (sp.leftover && tid == 0 && part == 0)
@@ -569,7 +597,7 @@ __global__ __launch_bounds__(kThreads, YT * NT <= 2 ? 4 : YT * NT <= 3 ? 3 : 2)
     }
     if (!fits)
     {
-        if (!sp.leftover && part == 0)
+        if (!sp.leftover && part == 0 && tid < kThreads) // waves that have ended do not take part in the others' barriers
         {
             const int items = (grid_units(S, kDefaultPT).units + kWaves - 1) / kWaves;
             for (int i = 0; i < items; ++i)
@@ -580,8 +608,6 @@ __global__ __launch_bounds__(kThreads, YT * NT <= 2 ? 4 : YT * NT <= 3 ? 3 : 2)
         }
         return; // uniform
     }
-    fill_table(sm.tab, sp, S);
-    lds_barrier();
     const CentreOffsets off = centre_offsets(a.p, m);
     const double delta = static_cast<double>(a.p.image_size) / S;
     f32x16 acc[NT][YT];
@@ -607,22 +633,22 @@ __global__ __launch_bounds__(kThreads, YT * NT <= 2 ? 4 : YT * NT <= 3 ? 3 : 2)
     const double w0 = V > 0 ? off.w - wr.centre : 0.0; // minus the gridder's sign
     const int h = lane >> 5, xi = (lane & 31) >> 2, corr = lane & 3;
     const int cols = min(kCols, S - xb);
+    const SmallDivisor by_cols(cols);
 #pragma unroll
-    for (int t = 0; t < YT; ++t) // 16 rows of the subgrid at a time
+    for (int t0 = 0; t0 < YT; t0 += kPass / 16) // kPass rows of the subgrid at a time
     {
-        if (16 * t >= S)
+        const int y0 = 16 * t0;
+        if (y0 >= S)
             break; // uniform
-        constexpr int kPairs = YT / 2;
-        const bool paired = t < 2 * kPairs;
         // This thread's pixels' A-terms, in flight while the sums meet in LDS.
-        constexpr int kPer = (16 * kCols + kThreads - 1) / kThreads;
+        constexpr int kPer = (kPass * kCols + kCount - 1) / kCount;
         cfloat a1[kPer][4], a2[kPer][4];
         float taper[kPer];
 #pragma unroll
         for (int i = 0; i < kPer; ++i)
         {
-            const int q = tid + i * kThreads, row = q / cols, x = xb + q - row * cols, y = 16 * t + row;
-            if (row < 16 && y < S && ok)
+            const int q = tid + i * kCount, row = by_cols.quotient(q), x = xb + q - row * cols, y = y0 + row;
+            if (row < kPass && y < S && ok)
             {
                 const int p = y * S + x;
                 load_jones(aterms, (abase + m.station1) * P + p, a1[i]);
@@ -632,27 +658,33 @@ __global__ __launch_bounds__(kThreads, YT * NT <= 2 ? 4 : YT * NT <= 3 ? 3 : 2)
         }
         lds_barrier(); // the staging, or the previous rows, are done with
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+        for (int t = t0; t < t0 + kPass / 16 && t < YT; ++t) // 16 rows each
         {
-            const int x = x0 - xb + 8 * nt + xi;
-            if (x >= cols)
-                continue;
+            constexpr int kPairs = YT / 2;
+            const bool paired = t < 2 * kPairs;
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
+            for (int nt = 0; nt < NT; ++nt)
             {
-                // Row 8 (i / 4) + 4 h + i % 4 of the block.
-                const float re = paired ? acc[nt][t / 2 * 2][t % 2 * 8 + i] : acc[nt][YT - 1][i];
-                const float im = paired ? acc[nt][t / 2 * 2 + (YT > 1)][t % 2 * 8 + i] : acc[nt][YT - 1][8 + i];
-                sm.sum[split][((i / 4 * 8 + 4 * h + i % 4) * cols + x) * 4 + corr] =
-                    make_float2(re * unscale, im * unscale);
+                const int x = x0 - xb + 8 * nt + xi;
+                if (x >= cols)
+                    continue;
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                {
+                    // Row 8 (i / 4) + 4 h + i % 4 of the block.
+                    const float re = paired ? acc[nt][t / 2 * 2][t % 2 * 8 + i] : acc[nt][YT - 1][i];
+                    const float im = paired ? acc[nt][t / 2 * 2 + (YT > 1)][t % 2 * 8 + i] : acc[nt][YT - 1][8 + i];
+                    sm.sum[split][((16 * t - y0 + i / 4 * 8 + 4 * h + i % 4) * cols + x) * 4 + corr] =
+                        make_float2(re * unscale, im * unscale);
+                }
             }
         }
         lds_barrier();
 #pragma unroll
         for (int i = 0; i < kPer; ++i)
         {
-            const int q = tid + i * kThreads, row = q / cols, x = xb + q - row * cols, y = 16 * t + row;
-            if (row >= 16 || y >= S)
+            const int q = tid + i * kCount, row = by_cols.quotient(q), x = xb + q - row * cols, y = y0 + row;
+            if (row >= kPass || y >= S)
                 continue;
             const int p = y * S + x;
             cfloat px[4] = {{0.F, 0.F}, {0.F, 0.F}, {0.F, 0.F}, {0.F, 0.F}};
@@ -900,7 +932,40 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
     }
     const int v_begin = static_cast<int>(v_first);
     const int v_end = static_cast<int>(v_first + sp.per < V ? v_first + sp.per : V);
-    const WRange wr = w_range<WAVES>(a, row0, T, c0, nc, reinterpret_cast<float *>(sm.tab));
+    // The table, then the pixels q, q + kCount, ... of the padded KS YB 8 x mts 8 (zero past the subgrid) with taper and
+    // A-terms applied.  FP16: their largest value, for the scale, meets with the range of w, so their loads do not wait
+    // for it (21,768 subgrids of 24^2 with 129 visibilities: 531 -> 478 us, and one barrier instead of six; 45 of 32^2
+    // 22.3 -> 20.4).  BF16 needs no scale and is 4 % faster with the range first.
+    fill_table(sm.tab, sp, S);
+    WRange wr;
+    if constexpr (DT == kBF16)
+    {
+        float none = 0.F;
+        wr = w_range<WAVES, false>(a, row0, T, c0, nc, sm.slots, none);
+    }
+    constexpr int kRows = 8 * KS * YB, kPer = (kRows * kRows + kCount - 1) / kCount;
+    const int mts = (S + 7) / 8, cols = 8 * mts;
+    const SmallDivisor by_cols(cols);
+    const float2 *sub = reinterpret_cast<const float2 *>(a.subgrids) + static_cast<size_t>(s) * kCorr * P;
+    cfloat px[kPer][4];
+    float vmax = 0.F;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+    {
+        const int q = tid + i * kCount, y = by_cols.quotient(q), x = q - y * cols;
+#pragma unroll
+        for (int pol = 0; pol < 4; ++pol)
+            px[i][pol] = {0.F, 0.F};
+        if (y < S && x < S)
+        {
+            degrid_pixel(a, m, sub, y * S + x, px[i]);
+#pragma unroll
+            for (int pol = 0; pol < 4; ++pol)
+                vmax = fmaxf(vmax, fmaxf(fabsf(px[i][pol].re), fabsf(px[i][pol].im)));
+        }
+    }
+    if constexpr (DT == kFP16)
+        wr = w_range<WAVES, true>(a, row0, T, c0, nc, sm.slots, vmax);
     const float eps = wr.half * sp.tables.eps;
     const bool fits = eps <= kEpsMost && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
     if (sp.leftover && tid == 0 && chunk == 0)
@@ -919,50 +984,30 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
             degridder_item<DT, true, kDefaultVT, kDefaultPB, false, false>(a, s, v / per, direct);
         return; // uniform
     }
-    fill_table(sm.tab, sp, S);
     const CentreOffsets off = centre_offsets(a.p, m);
     const double delta = static_cast<double>(a.p.image_size) / S;
     const double w0 = wr.centre - off.w;
-    const float2 *sub = reinterpret_cast<const float2 *>(a.subgrids) + static_cast<size_t>(s) * kCorr * P;
-
-    // Pixels q, q + kCount, ... of the padded KS YB 8 x mts 8 (zero past the subgrid).
-    constexpr int kRows = 8 * KS * YB, kPer = (kRows * kRows + kCount - 1) / kCount;
-    const int mts = (S + 7) / 8, cols = 8 * mts;
     uint32_t *words = reinterpret_cast<uint32_t *>(sm.pixels);
-    cfloat px[kPer][4];
-    float vmax = 0.F;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i)
-    {
-        const int q = tid + i * kCount, y = q / cols, x = q - y * cols;
-#pragma unroll
-        for (int pol = 0; pol < 4; ++pol)
-            px[i][pol] = {0.F, 0.F};
-        if (y < S && x < S)
-        {
-            degrid_pixel(a, m, sub, y * S + x, px[i]);
-            const cfloat r = pixel_rotation(x, y, S, delta, w0);
-#pragma unroll
-            for (int pol = 0; pol < 4; ++pol)
-            {
-                px[i][pol] = cmul(px[i][pol], r);
-                vmax = fmaxf(vmax, fmaxf(fabsf(px[i][pol].re), fabsf(px[i][pol].im)));
-            }
-        }
-    }
     float unscale = 1.F, inv = 1.F;
     if constexpr (DT == kFP16)
     {
-        const int e = scale_exponent(block_max(vmax, sm.maxbits));
+        const int e = scale_exponent(fminf(vmax * 1.4142136F, 3.4028235e38F)); // room for the rotation
         unscale = ldexpf(1.F, e);
         inv = ldexpf(1.F, -e);
     }
 #pragma unroll
     for (int i = 0; i < kPer; ++i)
     {
-        const int q = tid + i * kCount, y = q / cols, x = q - y * cols;
+        const int q = tid + i * kCount, y = by_cols.quotient(q), x = q - y * cols;
         if (y >= kRows)
             continue;
+        if (y < S && x < S)
+        {
+            const cfloat r = pixel_rotation(x, y, S, delta, w0);
+#pragma unroll
+            for (int pol = 0; pol < 4; ++pol)
+                px[i][pol] = cmul(px[i][pol], r);
+        }
         // Word y % 4 of lane (y / 4 % 2, x % 8, correlation) of tile (y / 8, x / 8); the low halves 32 lanes on.
         uint32_t *w = words + ((((y >> 3) * 2 + ((y >> 2) & 1)) * mts + (x >> 3)) * 64 + (x & 7) * 4) * 4 + (y & 3);
 #pragma unroll
@@ -986,25 +1031,32 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
 
 // ---- launchers --------------------------------------------------------------------------------------------------
 
-template <int DT, int YT, int NT, int NX>
+template <int DT, int YT, int NT, int NX, int WAVES = kWaves>
 hipError_t launch_grid(const KernelArgs &a, const SeparableArgs &sp, hipStream_t st)
 {
     const long long parts = (a.p.S + 8 * NT * NX - 1) / (8 * NT * NX), blocks = parts * a.p.nr_subgrids;
     if (blocks > 0x7fffffffLL)
         return hipErrorInvalidConfiguration;
-    grid_separable<DT, YT, NT, NX><<<static_cast<unsigned>(blocks), kThreads, 0, st>>>(a, sp);
+    grid_separable<DT, YT, NT, NX, WAVES><<<static_cast<unsigned>(blocks), 64 * WAVES, 0, st>>>(a, sp);
     return hipGetLastError();
 }
 
 // Row tiles and column tiles per wave and column ranges for subgrid size S.  One wave holds all columns up to S = 32
 // (128 accumulators); larger subgrids spread them over two or four waves.  A plan that would leave CUs without work
-// takes a workgroup per 8 columns, which forms the row phasors once per 8 columns.
+// takes a workgroup per 8 columns, which forms the row phasors once per 8 columns; where even those leave CUs idle, one
+// of 8 waves (45 subgrids of 32^2 with 2048 visibilities: 30.4 -> 25.8 us; of 16^2: 24.2 -> 19.5), which would cost
+// larger plans up to a quarter (231 subgrids of 32^2 with 256: 16.9 -> 20.9) and subgrids above 32^2 a tenth.
 template <int DT> hipError_t grid_size(const KernelArgs &a, const SeparableArgs &sp, hipStream_t st)
 {
     const int S = a.p.S;
     const bool few = a.p.nr_subgrids <= kFewSubgrids;
+    const bool fewer = static_cast<long long>(a.p.nr_subgrids) * ((S + 7) / 8) <= kFewSubgrids;
     if (S <= 16)
-        return few ? launch_grid<DT, 1, 1, 1>(a, sp, st) : launch_grid<DT, 1, 2, 1>(a, sp, st);
+        return fewer ? launch_grid<DT, 1, 1, 1, 8>(a, sp, st)
+               : few ? launch_grid<DT, 1, 1, 1>(a, sp, st)
+                     : launch_grid<DT, 1, 2, 1>(a, sp, st);
+    if (S <= 32 && fewer)
+        return launch_grid<DT, 2, 1, 1, 8>(a, sp, st);
     if (S <= 32 && few)
         return launch_grid<DT, 2, 1, 1>(a, sp, st);
     if (S <= 24)

@@ -160,3 +160,13 @@ def test_subgrids_outside_the_product_term_take_the_per_pair_kernels(S, form):
     for _ in range(2):
         again = run_batch(w, form, sub)
         assert np.array_equal(first[0], again[0]) and np.array_equal(first[1], again[1])
+
+
+@pytest.mark.parametrize("S", [14, 24, 32])
+def test_plans_between_eight_wave_workgroups_and_full_chips_vs_fp64(S):
+    """150 subgrids: a workgroup of four waves per 8 columns, where 8 subgrids take eight waves and 270 all columns."""
+    rng = np.random.default_rng(100 + S)
+    w = make(S, [int(t) for t in rng.integers(1, 30, 150)], list(rng.uniform(0.0, 8e-4, 150)), seed=S)
+    sub = model(w)
+    got, vis = run_oneshot(w, "fp16x3", sub)
+    check(w, "fp16x3", sub, got, vis)
