@@ -4,14 +4,18 @@
 // gridding/src/degridding_benchmark.cpp:157-166): the whole file is compiled with contraction off, so
 // `a * b + c` rounds twice; the complex multiply-accumulates are written as explicit fused multiply-adds.
 //
-// Gridder: one workgroup of 256 threads owns 256 pixels of one subgrid (one per thread, its 4 correlations held in VGPRs).  Visibilities and uvw of the subgrid stream through LDS in batches of 256 visibilities;
-//   every lane reads the same LDS address per visibility (broadcast, conflict-free).  Taper and A-term are
-//   applied in the epilogue, which overwrites the subgrid.
+// Gridder: one workgroup of 256 threads owns 256 pixels of one subgrid (one per thread, its 4 correlations held in
+//   VGPRs).  Visibilities and uvw of the subgrid stream through LDS in batches of 256 visibilities; every lane reads the
+//   same LDS address per visibility (broadcast, conflict-free).  Taper and A-term are applied in the epilogue, which
+//   overwrites the subgrid.
 // Degridder: one workgroup owns 256 (timestep, channel-chunk) items of one subgrid, each thread one timestep x
 //   up to 2 or 4 channels.  Tapered, A-term-corrected pixels plus (l, m, n, phase offset) are staged through LDS in
 //   batches of 512 pixels; each thread sums its visibilities over all pixels in registers, so no cross-lane
 //   reduction is needed.
+// Tile forms, for plans whose waves of 64 pixels or visibilities leave SIMDs idle: a wave sums for 16 of them, on the
+//   matrix cores, with the same bits.
 #include <algorithm>
+#include <type_traits>
 
 #include "idgx_device.hpp"
 #include "kernels.hpp"
@@ -26,26 +30,96 @@ constexpr int kThreads = 256;
 constexpr int kGridBatchVis = 256; // visibilities per LDS stage
 constexpr int kGridChunk = 64;     // channels per chunk (bounds the per-stage uvw count at 256 timesteps)
 constexpr int kDegridPixBatch = 512;
+constexpr int kTilePixBatch = 256; // pixels per LDS stage of the tile form, one per thread
 
-// Visibility x phasor accumulated into acc[0..7] = {XX.re, XX.im, XY.re, ..., YY.im}.
+// Visibility x phasor accumulated into acc[0..7] = {XX.re, XX.im, XY.re, ..., YY.im}, the cosine's terms first.
 __device__ __forceinline__ void cmac4(float *acc, float4 va, float4 vb, float cs, float sn)
 {
     acc[0] = __builtin_fmaf(va.x, cs, acc[0]);
-    acc[0] = __builtin_fmaf(-va.y, sn, acc[0]);
-    acc[1] = __builtin_fmaf(va.x, sn, acc[1]);
     acc[1] = __builtin_fmaf(va.y, cs, acc[1]);
     acc[2] = __builtin_fmaf(va.z, cs, acc[2]);
-    acc[2] = __builtin_fmaf(-va.w, sn, acc[2]);
-    acc[3] = __builtin_fmaf(va.z, sn, acc[3]);
     acc[3] = __builtin_fmaf(va.w, cs, acc[3]);
     acc[4] = __builtin_fmaf(vb.x, cs, acc[4]);
-    acc[4] = __builtin_fmaf(-vb.y, sn, acc[4]);
-    acc[5] = __builtin_fmaf(vb.x, sn, acc[5]);
     acc[5] = __builtin_fmaf(vb.y, cs, acc[5]);
     acc[6] = __builtin_fmaf(vb.z, cs, acc[6]);
+    acc[7] = __builtin_fmaf(vb.w, cs, acc[7]);
+    acc[0] = __builtin_fmaf(-va.y, sn, acc[0]);
+    acc[1] = __builtin_fmaf(va.x, sn, acc[1]);
+    acc[2] = __builtin_fmaf(-va.w, sn, acc[2]);
+    acc[3] = __builtin_fmaf(va.z, sn, acc[3]);
+    acc[4] = __builtin_fmaf(-vb.y, sn, acc[4]);
+    acc[5] = __builtin_fmaf(vb.x, sn, acc[5]);
     acc[6] = __builtin_fmaf(-vb.w, sn, acc[6]);
     acc[7] = __builtin_fmaf(vb.z, sn, acc[7]);
-    acc[7] = __builtin_fmaf(vb.w, cs, acc[7]);
+}
+
+// The same sums of one value on N pixels (visibilities) side by side, acc(i) the i-th one's.  Runs of instructions that
+// read the same component first are faster than N calls of cmac4: 24.25 VALU instructions per pair either way, but the
+// gridder's items of 1024 pixels took 5600 us against 5360 (6409 subgrids of 32^2; with (sin, cos) terms 6340).
+template <int N, class Acc>
+__device__ __forceinline__ void cmac4_group(Acc acc, float4 va, float4 vb, const float (&cs)[N], const float (&sn)[N])
+{
+    const float x[4] = {va.x, va.z, vb.x, vb.z}, y[4] = {va.y, va.w, vb.y, vb.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            acc(i)[2 * j] = __builtin_fmaf(x[j], cs[i], acc(i)[2 * j]);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            acc(i)[2 * j + 1] = __builtin_fmaf(y[j], cs[i], acc(i)[2 * j + 1]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            acc(i)[2 * j + 1] = __builtin_fmaf(x[j], sn[i], acc(i)[2 * j + 1]);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            acc(i)[2 * j] = __builtin_fmaf(-y[j], sn[i], acc(i)[2 * j]);
+    }
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Sums of value x phasor on v_mfma_f32_16x16x4_f32: D[16 rows][8 columns in use] += A[16][4] B[4][8], rows = the 16
+// pixels (visibilities) whose sums these are, columns = (re, im) x 4 correlations, k = (cos, sin) of two of the
+// visibilities (pixels) that are summed.  Lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and, in element i of the sums,
+// D[4 (l / 16) + i][l % 16].  The instruction adds its four products one after the other, each as a fused multiply-add
+// with one rounding, so a sum has the bits of cmac4's in the order of the values, whatever their grouping.
+//
+// Factors of one value in LDS, 16 floats: its columns for the cosine, then for the sine.
+__device__ __forceinline__ void store_factors(float4 *f, float4 va, float4 vb)
+{
+    f[0] = va;
+    f[1] = vb;
+    f[2] = make_float4(-va.y, va.x, -va.w, va.z);
+    f[3] = make_float4(-vb.y, vb.x, -vb.w, vb.z);
+}
+
+// Which of a step's four values lane group l / 16 forms the phasors of: after the swap of step_products the groups hold
+// (cos, sin) of values 0 and 1, and of values 2 and 3.
+__device__ __forceinline__ int step_value()
+{
+    const int g = (threadIdx.x & 63) >> 4;
+    return ((g & 1) << 1) | (g >> 1);
+}
+
+// This lane's factors of the step's values 0 and 1, and 2 and 3; f: the factors of value 0.
+__device__ __forceinline__ float2 step_factors(const float *f)
+{
+    const int at = ((threadIdx.x & 63) >> 4) * 8 + (threadIdx.x & 7);
+    return make_float2(f[at], f[at + 32]);
+}
+
+// Four values onto one tile; cs, sn: the phasor of this lane's row and value.  Every lane of the wave takes part.
+__device__ __forceinline__ void step_products(f32x4 &sums, float2 f, float cs, float sn)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(cs), __float_as_uint(sn), false, false);
+    sums = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(r[0]), f.x, sums, 0, 0, 0);
+    sums = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(r[1]), f.y, sums, 0, 0, 0);
 }
 
 __device__ __forceinline__ void channel_window(const KernelArgs &a, int s, int &c0, int &nc)
@@ -180,6 +254,109 @@ __global__ __launch_bounds__(kThreads, SC == kSincosHw ? 8 : 1) void gridder_pla
     }
     if (p < P)
         store_plain_pixel(a, m, s, p, ok, px.acc);
+}
+
+// Plans that leave SIMDs without a wave of 64 pixels: a wave per 16 pixels, on the matrix cores (a workgroup 64 pixels).
+// Bound by latency there (a step of four visibilities is a chain of about ten VALU instructions and two MFMAs), so two
+// steps go side by side and the next stage's loads are in flight during the sums.  45 subgrids of 32^2 with 2048
+// visibilities each: 156 -> 105 us; on plans that fill the chip the 16-column tile, half of it unused, is slower than the VALU
+// (6409 subgrids 6281 -> 9707 us).
+template <int SC> __global__ __launch_bounds__(kThreads, 8) void gridder_plain_tiles(KernelArgs a)
+{
+    constexpr int kPixels = 64;
+    __shared__ float4 s_fac[4 * kGridBatchVis];
+    __shared__ float s_uvw[3 * kGridBatchVis];
+    __shared__ float s_wn[kGridChunk];
+
+    const int s = blockIdx.x;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int P = a.p.S * a.p.S;
+    const idgx_metadata m = a.metadata[s];
+    int c0, nc;
+    channel_window(a, s, c0, nc);
+    const long long row0 = first_row(a.metadata, m);
+    const bool ok = subgrid_in_bounds(a.p, m, row0, c0, nc);
+    const long long C = a.p.nr_channels;
+    const Offsets off = gridder_offsets(m, a.p.S, a.p.G, a.p.image_size, a.p.w_step);
+    const float4 *vis = reinterpret_cast<const float4 *>(a.visibilities);
+    const int pbase = blockIdx.y * kPixels, pwave = pbase + wave * 16;
+    const bool wave_live = pwave < P; // wave-uniform
+    const PlainPixel px = plain_pixel(a, off, min(pwave + (lane & 15), P - 1));
+    f32x4 sums = {0.F, 0.F, 0.F, 0.F};
+    const int mine = step_value();
+    for (int cb = 0; ok && cb < nc; cb += kGridChunk)
+    {
+        const int cc = min(kGridChunk, nc - cb), steps = (cc + 3) >> 2, padded = 4 * steps;
+        const int tb_max = kGridBatchVis / padded;
+        // This thread's visibility of a stage; channels past the last are zeros, which add nothing.
+        const int te = tid / padded, ce = tid - te * padded;
+        const float4 zero = make_float4(0.F, 0.F, 0.F, 0.F);
+        float4 va = zero, vb = zero;
+        const auto load = [&](int t0) {
+            if (te < min(tb_max, m.nr_timesteps - t0) && ce < cc)
+            {
+                const size_t o = static_cast<size_t>((row0 + t0 + te) * C + c0 + cb + ce) * 2;
+                va = vis[o];
+                vb = vis[o + 1];
+            }
+            else
+                va = vb = zero;
+        };
+        load(0);
+        for (int t0 = 0; t0 < m.nr_timesteps; t0 += tb_max)
+        {
+            const int tb = min(tb_max, m.nr_timesteps - t0);
+            __syncthreads(); // previous stage fully consumed
+            if (tid < padded)
+                s_wn[tid] = tid < cc ? a.wavenumbers[c0 + cb + tid] : 0.F;
+            for (int q = tid; q < 3 * tb; q += kThreads)
+                s_uvw[q] = a.uvw[3 * (row0 + t0) + q];
+            store_factors(s_fac + 4 * tid, va, vb);
+            __syncthreads();
+            if (t0 + tb_max < m.nr_timesteps)
+                load(t0 + tb_max);
+            for (int t = 0; wave_live && t < tb; ++t)
+            {
+                const float pidx = (s_uvw[3 * t] * px.l + s_uvw[3 * t + 1] * px.m) + s_uvw[3 * t + 2] * px.n;
+                const float *fac = reinterpret_cast<const float *>(s_fac + 4 * padded * t);
+                const auto step = [&](auto count, int k) {
+                    constexpr int N = count.value;
+                    float2 f[N];
+                    float sn[N], cs[N];
+#pragma unroll
+                    for (int i = 0; i < N; ++i)
+                    {
+                        f[i] = step_factors(fac + 64 * (k + i));
+                        sincos_rad<SC>(px.offset - pidx * s_wn[4 * (k + i) + mine], sn[i], cs[i]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < N; ++i)
+                        step_products(sums, f[i], cs[i], sn[i]);
+                };
+                int k = 0;
+                for (; k + 2 <= steps; k += 2)
+                    step(std::integral_constant<int, 2>{}, k);
+                for (; k < steps; ++k)
+                    step(std::integral_constant<int, 1>{}, k);
+            }
+        }
+    }
+    // The sums, per pixel, through LDS (the staging is done with).
+    __syncthreads();
+    float *out = reinterpret_cast<float *>(s_fac);
+    if ((lane & 15) < 8)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            out[(wave * 16 + 4 * (lane >> 4) + j) * 8 + (lane & 7)] = sums[j];
+    __syncthreads();
+    if (tid < kPixels && pbase + tid < P)
+    {
+        float acc[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            acc[j] = out[tid * 8 + j];
+        store_plain_pixel(a, m, s, pbase + tid, ok, acc);
+    }
 }
 
 // Workgroups per CU with the hardware sin/cos: two channels per thread fit six (the most the 24 KB of LDS allows)
@@ -318,6 +495,143 @@ __global__ __launch_bounds__(kThreads, (degrid_plain_min_blocks<NCH, SC>())) voi
     }
 }
 
+// As gridder_plain_tiles, for plans that leave SIMDs with fewer than two waves of 64 visibilities: a wave per 16 items
+// (timestep, NCH channels), one tile per channel.  45 subgrids of 32^2 with 2048 visibilities each: 143 -> 94 us (6409
+// subgrids 6470 -> 9157 us).
+template <int NCH, int SC> __global__ __launch_bounds__(kThreads, 6) void degridder_plain_tiles(KernelArgs a, int per)
+{
+    constexpr int kItems = kThreads / 4;
+    __shared__ float4 s_px[kTilePixBatch];       // (l, m, n, phase offset)
+    __shared__ float4 s_fac[4 * kTilePixBatch];  // the corrected pixel's factors
+
+    // Workgroup b = vblock * n + s: a subgrid's workgroups are spread over the XCDs (balances uneven subgrids).
+    const int vblock = blockIdx.x / a.p.nr_subgrids;
+    const int s = blockIdx.x - vblock * a.p.nr_subgrids;
+    if (vblock >= per)
+        return; // uniform
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int S = a.p.S;
+    const int P = S * S;
+    const idgx_metadata m = a.metadata[s];
+    int c0, nc;
+    channel_window(a, s, c0, nc);
+    const long long row0 = first_row(a.metadata, m);
+    if (!subgrid_in_bounds(a.p, m, row0, c0, nc) || nc == 0)
+        return; // uniform: nothing of this subgrid is written
+    const int nchunks = (nc + NCH - 1) / NCH;
+    if (static_cast<long long>(vblock) * kItems >= static_cast<long long>(m.nr_timesteps) * nchunks)
+        return; // uniform: no item of this block exists
+
+    const int item = vblock * kItems + 16 * wave + (lane & 15);
+    const int t = item / nchunks;
+    const int cj = (item - t * nchunks) * NCH;
+    const bool active = t < m.nr_timesteps;
+    const bool wave_live = __ballot(active) != 0ULL; // wave-uniform; idle rows of a live wave sum phasors of k = 0
+    const long long C = a.p.nr_channels;
+
+    float u = 0.F, v = 0.F, w = 0.F;
+    float k[NCH];
+    f32x4 sums[NCH];
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+    {
+        k[j] = 0.F;
+        sums[j] = f32x4{0.F, 0.F, 0.F, 0.F};
+    }
+    if (active)
+    {
+        const float *uv = a.uvw + 3 * (row0 + t);
+        u = uv[0];
+        v = uv[1];
+        w = uv[2];
+#pragma unroll
+        for (int j = 0; j < NCH; ++j)
+            if (cj + j < nc)
+                k[j] = a.wavenumbers[c0 + cj + j];
+    }
+
+    const Offsets off = degridder_offsets(m, S, a.p.G, a.p.image_size, a.p.w_step);
+    const float2 *sub = reinterpret_cast<const float2 *>(a.subgrids) + static_cast<size_t>(s) * kCorr * P;
+    const float4 *aterms = reinterpret_cast<const float4 *>(a.aterms);
+    const size_t abase = static_cast<size_t>(m.aterm_index) * a.p.nr_stations;
+    const int mine = step_value();
+
+    for (int pb = 0; pb < P; pb += kTilePixBatch)
+    {
+        const int np = min(kTilePixBatch, P - pb); // a multiple of 4: S is even
+        __syncthreads();
+        for (int q = tid; q < np; q += kThreads)
+        {
+            const int p = pb + q;
+            const int x = p % S, y = p / S;
+            const float taper = a.spheroidal[p];
+            cfloat px[4];
+#pragma unroll
+            for (int pol = 0; pol < 4; ++pol)
+            {
+                const float2 g = sub[pol * P + p];
+                px[pol] = {taper * g.x, taper * g.y};
+            }
+            cfloat a1[4], a2[4];
+            load_jones(aterms, (abase + m.station1) * P + p, a1);
+            load_jones(aterms, (abase + m.station2) * P + p, a2);
+            if (a.p.convention == IDGX_ATERM_REFERENCE)
+                apply_a1h_p_a2(px, a1, a2);
+            else
+                apply_a1_p_a2h(px, a1, a2);
+            store_factors(s_fac + 4 * q, make_float4(px[0].re, px[0].im, px[1].re, px[1].im),
+                          make_float4(px[2].re, px[2].im, px[3].re, px[3].im));
+            const float l = pixel_lm(x, S, a.p.image_size);
+            const float mm = pixel_lm(y, S, a.p.image_size);
+            const float n = pixel_n(l, mm);
+            s_px[q] = make_float4(l, mm, n, (off.u * l + off.v * mm) + off.w * n);
+        }
+        __syncthreads();
+        if (!wave_live)
+            continue;
+        const auto step = [&](auto count, int q) {
+            constexpr int N = count.value;
+            float2 f[N];
+            float sn[N][NCH], cs[N][NCH];
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+            {
+                const float4 g = s_px[q + 4 * i + mine];
+                f[i] = step_factors(reinterpret_cast<const float *>(s_fac + 4 * (q + 4 * i)));
+                const float pidx = (u * g.x + v * g.y) + w * g.z;
+#pragma unroll
+                for (int j = 0; j < NCH; ++j)
+                    sincos_rad<SC>(pidx * k[j] - g.w, sn[i][j], cs[i][j]);
+            }
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+#pragma unroll
+                for (int j = 0; j < NCH; ++j)
+                    step_products(sums[j], f[i], cs[i][j], sn[i][j]);
+        };
+        int q = 0;
+        for (; q + 8 <= np; q += 8)
+            step(std::integral_constant<int, 2>{}, q);
+        for (; q < np; q += 4)
+            step(std::integral_constant<int, 1>{}, q);
+    }
+    // Row 4 (lane / 16) + i of a tile is the visibility of that lane of the wave.
+    float *out = reinterpret_cast<float *>(a.visibilities_out);
+    const long long first = active ? (row0 + t) * C + c0 + cj : -1;
+    const int count = active ? min(NCH, nc - cj) : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        const int row = 4 * (lane >> 4) + i;
+        const long long o = __shfl(first, row);
+        const int n = __shfl(count, row);
+#pragma unroll
+        for (int j = 0; j < NCH; ++j)
+            if (j < n && (lane & 15) < 8)
+                out[(o + j) * 8 + (lane & 7)] = sums[j][i];
+    }
+}
+
 // ---- persistent work-queue forms (batches) ---------------------------------------------------------------------
 //
 // The same arithmetic as the kernels above, item by item from a device queue, over each subgrid's selected
@@ -392,14 +706,11 @@ __device__ __forceinline__ void grid_runs(const PlainGridShared &sm, int nruns, 
             const float4 va = sm.ent[3 * e];
             const float4 vb = sm.ent[3 * e + 1];
             const float k = sm.ent[3 * e + 2].x;
+            float sn[N], cs[N];
 #pragma unroll
             for (int i = 0; i < N; ++i)
-            {
-                const float phase = px[i].offset - pidx[i] * k;
-                float sn, cs;
-                sincos_rad<SC>(phase, sn, cs);
-                cmac4(px[i].acc, va, vb, cs, sn);
-            }
+                sincos_rad<SC>(px[i].offset - pidx[i] * k, sn[i], cs[i]);
+            cmac4_group<N>([&](int i) { return px[i].acc; }, va, vb, cs, sn);
         };
         if constexpr (UNROLL > 1)
         {
@@ -633,14 +944,11 @@ __device__ __forceinline__ void degridder_plain_item(const KernelArgs &a, int s,
                 const float4 pa = sm.px[3 * q + 1];
                 const float4 pbv = sm.px[3 * q + 2];
                 const float pidx = (us * g.x + vs * g.y) + ws * g.z;
+                float sn[NCH], cs[NCH];
 #pragma unroll
                 for (int j = 0; j < NCH; ++j)
-                {
-                    const float phase = pidx * k[j] - g.w;
-                    float sn, cs;
-                    sincos_rad<SC>(phase, sn, cs);
-                    cmac4(acc[j], pa, pbv, cs, sn);
-                }
+                    sincos_rad<SC>(pidx * k[j] - g.w, sn[j], cs[j]);
+                cmac4_group<NCH>([&](int j) { return acc[j]; }, pa, pbv, cs, sn);
             }
         }
         else
@@ -650,15 +958,14 @@ __device__ __forceinline__ void degridder_plain_item(const KernelArgs &a, int s,
                 const float4 g = sm.px[3 * q];
                 const float4 pa = sm.px[3 * q + 1];
                 const float4 pbv = sm.px[3 * q + 2];
+                float sn[NCH], cs[NCH];
 #pragma unroll
                 for (int j = 0; j < NCH; ++j)
                 {
                     const float pidx = (u[j] * g.x + v[j] * g.y) + w[j] * g.z;
-                    const float phase = pidx * k[j] - g.w;
-                    float sn, cs;
-                    sincos_rad<SC>(phase, sn, cs);
-                    cmac4(acc[j], pa, pbv, cs, sn);
+                    sincos_rad<SC>(pidx * k[j] - g.w, sn[j], cs[j]);
                 }
+                cmac4_group<NCH>([&](int j) { return acc[j]; }, pa, pbv, cs, sn);
             }
         }
     }
@@ -787,8 +1094,24 @@ hipError_t launch_plain_queue(const QueueArgs &q, bool accurate_sincos, bool gri
 }
 } // namespace
 
+// Waves of 64 pixels (visibilities) up to which a one-shot plan takes the tile forms: one per SIMD for the gridder, whose
+// time does not fall below one wave's (45 subgrids of 32^2, 720 waves: 156 -> 105 us; 66, 1056 waves: 185 -> 159; 91, 1456
+// waves: 189 -> 187; 120 of 24^2, 1080 waves: 67 -> 69), two for the degridder (1440 waves: 143 -> 94 us; 120 subgrids of
+// 48^2, 1920 waves: 306 -> 268; 91 of 32^2, 2912 waves: 168 -> 179).
+constexpr long long kTileGridWaves = 1024, kTileDegridWaves = 2048;
+
 hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
+    const long long S = a.p.S, waves = a.p.nr_subgrids * ((S * S + 63) / 64);
+    if (waves <= kTileGridWaves)
+    {
+        const dim3 grid(a.p.nr_subgrids, static_cast<unsigned>((S * S + 63) / 64));
+        if (accurate_sincos)
+            gridder_plain_tiles<kSincosOcml><<<grid, kThreads, 0, stream>>>(a);
+        else
+            gridder_plain_tiles<kSincosHw><<<grid, kThreads, 0, stream>>>(a);
+        return hipGetLastError();
+    }
     const dim3 grid(a.p.nr_subgrids, (a.p.S * a.p.S + kThreads - 1) / kThreads);
     if (accurate_sincos)
         gridder_plain<kSincosOcml><<<grid, kThreads, 0, stream>>>(a);
@@ -828,6 +1151,16 @@ template <int NCH> hipError_t launch_degrid_plain_chunks(const KernelArgs &a, bo
 hipError_t launch_degrid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
     const long long pairs = static_cast<long long>(a.p.max_nr_timesteps) * ((a.p.nr_channels + 1) / 2);
+    if ((2 * pairs + 63) / 64 * a.p.nr_subgrids <= kTileDegridWaves)
+    {
+        const long long per = std::max(1LL, (pairs + kThreads / 4 - 1) / (kThreads / 4));
+        const unsigned blocks = static_cast<unsigned>(per * a.p.nr_subgrids);
+        if (accurate_sincos)
+            degridder_plain_tiles<2, kSincosOcml><<<blocks, kThreads, 0, stream>>>(a, static_cast<int>(per));
+        else
+            degridder_plain_tiles<2, kSincosHw><<<blocks, kThreads, 0, stream>>>(a, static_cast<int>(per));
+        return hipGetLastError();
+    }
     if ((pairs + kThreads - 1) / kThreads * a.p.nr_subgrids < kDegridFill)
         return launch_degrid_plain_chunks<1>(a, accurate_sincos, stream);
     if (plain_degrid_channels_for(a.channels != nullptr, a.p.nr_channels) == 4)

@@ -54,3 +54,28 @@ def test_batch_equals_oneshot_and_the_cpu_restatement(S, n, T, C):
     b.degrid()
     eb = rel_l2(b.visibilities_out(), oracle_degrid(w, sub))
     assert same and eb <= PARITY and np.array_equal(b.visibilities_out() == 0, vis == 0)
+
+
+@pytest.mark.parametrize("S,n,T,C", [(128, 1, 3, 1), (10, 2, 7, 2), (24, 2, 5, 64), (34, 2, 130, 4), (32, 64, 9, 3),
+                                     (32, 65, 9, 3), (16, 2, 300, 6)])
+def test_matrix_tiles_of_the_smallest_plans_give_the_bits_of_the_vector_form(S, n, T, C):
+    """One-shot plans of at most a wave of 64 pixels per SIMD (two of 64 visibilities) run on the matrix cores, batches on
+    the vector units: the same sums in the same order, also where channels, pixels or visibilities do not fill a step of
+    four or a tile of 16.  Identity A-terms (Jones terms are fused differently in the degridders)."""
+    w = make(S, n, T, C, 7 * S + n)
+    w["aterms"] = observation.identity_aterms(1, 3, S)
+    rng = np.random.default_rng(2)
+    sub = (rng.standard_normal((n, 4, S, S)) + 1j * rng.standard_normal((n, 4, S, S))).astype(np.complex64)
+    d = DeviceWorkload(w)
+    plan = d.plan()
+    d.grid(plan)
+    got = d.subgrids()
+    d.degrid(plan, d_subgrids=upload(sub))
+    vis = d.visibilities_out()
+    b = DeviceBatch([w], precision="fp32")
+    b.grid()
+    assert np.array_equal(b.subgrids(), got)
+    b.classes[0]["d_subgrids"].copy_(upload(sub))
+    b.degrid()
+    assert np.array_equal(b.visibilities_out(), vis)
+    assert per_subgrid_rel_l2(got, oracle_grid(w)).max() <= PARITY and rel_l2(vis, oracle_degrid(w, sub)) <= PARITY
