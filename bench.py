@@ -159,6 +159,28 @@ def kernel_key(precision, path, direction, shape=None, plain_shape=None):
     return f"{direction}_mfma_queue<{dt}, {split}, {tiles}, {batch}, {'true' if pm else 'false'}>"
 
 
+def pass_kernel(precision, path, direction, shape, S, nr_subgrids, plain_shape=None):
+    """The kernel that does a pass's work: the separable kernels where a 3-product form's subgrids are at most 64^2 (the
+    per-pair kernels keep the subgrids whose w spreads too far), else kernel_key's.  Several subgrid sizes, each with its
+    kernel: joined."""
+    if isinstance(S, list):
+        keys = [pass_kernel(precision, path, direction, shape[k] if isinstance(shape, list) else shape, S[k],
+                            nr_subgrids[k], plain_shape) for k in range(len(S))]
+        return None if None in keys else " + ".join(dict.fromkeys(keys))
+    if not precision.endswith("x3") or S > 64:
+        return kernel_key(precision, path, direction, shape, plain_shape)
+    dt = 0 if precision.startswith("bf16") else 1
+    if direction == "gridder":
+        tiles = "1, 2, 1" if S <= 16 else "2, 3, 1" if S <= 24 else "2, 4, 1" if S <= 32 else "3, 3, 2" if S <= 48 \
+            else "4, 2, 4"
+        if nr_subgrids <= 256:
+            tiles = f"{1 if S <= 16 else 2 if S <= 32 else 3 if S <= 48 else 4}, 1, 1"
+        waves = 8 if S <= 32 and nr_subgrids * -(-S // 8) <= 256 else 4
+        return f"grid_separable<{dt}, {tiles}, {waves}>"
+    steps = "2, 1, 4" if S <= 16 else "3, 1, 4" if S <= 24 else "4, 1, 4" if S <= 32 else "3, 2, 4" if S <= 48 else "4, 2, 8"
+    return f"degrid_separable<{dt}, {steps}>"
+
+
 def pipe_profile(config, key):
     """VALU and matrix-core utilisation of kernel `key` from the committed rocprofv3 --pmc summary for this workload
     (profiles/pipe_utilisation_<config>.json), or None when it was not profiled."""
@@ -174,11 +196,13 @@ MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense FP16 / BF16 matrix peak, published
 
 
 def roofline_record(config, precision, key, dominant, flops, sincos, t_dom):
-    """The roofline of the dominant kernel.  The gridder and degridder are bound by VALU issue (phases, sin/cos and,
-    for the mixed forms, the hi/lo split), far from HBM and from the matrix-core peak, so `frac` is the
-    FP32-equivalent algorithmic rate against the FP32 peak, with the committed counters beside it: VALU busy and
-    VALU instructions per (pixel, visibility) pair, the matrix cores' utilisation (counter and algorithmic MFMA
-    rate against the FP16/BF16 peak) and the sin/cos rate against the half-rate v_sin / v_cos peak."""
+    """The roofline of the dominant kernel.  The separable kernels are bound by the matrix cores at the power limit:
+    `frac` is their MFMA rate (128 flops per (pixel, visibility) pair) against the published FP16/BF16 peak.  The per-pair
+    and plain FP32 kernels are bound by VALU issue (phases, sin/cos and, for the mixed forms, the hi/lo split), far
+    from HBM and from the matrix-core peak, so there it is the FP32-equivalent algorithmic rate against the FP32 peak,
+    with the committed counters beside it: VALU busy and VALU instructions per pair, the matrix cores' utilisation
+    (counter and algorithmic MFMA rate) and the sin/cos rate against the half-rate v_sin / v_cos peak."""
+    separable = key is not None and "separable" in key
     achieved = flops / t_dom / 1e12
     traffic = measured_traffic(config, key)
     pipes = pipe_profile(config, key)
@@ -190,23 +214,29 @@ def roofline_record(config, precision, key, dominant, flops, sincos, t_dom):
                 "mfma_util_pct": pipes.get("MfmaUtil"), "source": pipes["source"],
                 "note": "counters of the committed profile of this kernel on this workload (mean per launch); "
                         "insts_per_pair = SQ_INSTS_VALU x 64 lanes / (pixel, visibility) pairs of the pass"}
+    peak = FP32_PEAK_TFLOPS
+    if separable:
+        achieved, peak = mfma_flops / t_dom / 1e12, MFMA_PEAK_TFLOPS
     return {
-        "bound": "valu",
+        "bound": "mfma" if separable else "valu",
         "kernel": key,
         "pass": dominant,
         "achieved": achieved,
-        "peak": FP32_PEAK_TFLOPS,
+        "peak": peak,
         "unit": "TFLOP/s",
-        "frac": achieved / FP32_PEAK_TFLOPS,
+        "frac": achieved / peak,
         "traffic": None if traffic is None else traffic["bytes"],
         "traffic_detail": traffic,
-        "flop_model": "P*(5*T + 34*V) + 134*P per subgrid (FP32-equivalent algorithmic flops), sincos separate",
+        "flop_model": "128 per (pixel, visibility) pair: 4 MFMA products of 32 (3 of the hi/lo split, 1 of the w-term's "
+                      "remainder)" if separable else
+                      "P*(5*T + 34*V) + 134*P per subgrid (FP32-equivalent algorithmic flops), sincos separate",
         "valu": valu,
         "mfma": None if not mfma_flops else {
             "achieved_tflops": mfma_flops / t_dom / 1e12, "peak_tflops": MFMA_PEAK_TFLOPS,
             "frac": mfma_flops / t_dom / 1e12 / MFMA_PEAK_TFLOPS,
-            "note": "algorithmic MFMA flops: 128 per pair for the 3-product split (2 instructions), 64 single"},
-        "transcendental": trans_rate(sincos, t_dom),
+            "note": "algorithmic MFMA flops: 128 per pair for the 3-product split, 64 single"},
+        # The separable kernels form phasors per row and per column, not per pair.
+        "transcendental": None if separable else trans_rate(sincos, t_dom),
     }
 
 
@@ -656,13 +686,15 @@ def run_batched_config(args):
     plain = forms[-1] if len(forms) > 1 and forms[-1]["precision"] == "fp32" else None
     tg, td = head["gridder_ms"] / 1e3, head["degridder_ms"] / 1e3
     dominant, t_dom = ("degridder", td) if td > tg else ("gridder", tg)
-    dom_key = kernel_key(head["precision"], "batched", dominant, runner.shapes[dominant])
+    dom_key = pass_kernel(head["precision"], "batched", dominant, runner.shapes[dominant],
+                          [int(c["subgrid_size"]) for c in bo["classes"]], [int(c["nr_subgrids"]) for c in bo["classes"]])
     roofline = roofline_record(args.config, head["precision"], dom_key, dominant, flops, sincos, t_dom)
     if dom_key is None:  # one launch per class with different shapes
         roofline["kernel"] = " + ".join(kernel_key(head["precision"], "batched", dominant, sh)
                                         for sh in runner.shapes[dominant])
-    roofline["flop_model"] = ("P*(5*T + 34*V) + 134*P per subgrid, V = selected visibilities (FP32-equivalent "
-                              "algorithmic flops), sincos separate")
+    if roofline["bound"] == "valu":
+        roofline["flop_model"] = ("P*(5*T + 34*V) + 134*P per subgrid, V = selected visibilities (FP32-equivalent "
+                                  "algorithmic flops), sincos separate")
 
     cpu = None
     if not args.no_cpu:
@@ -838,8 +870,8 @@ def main():
     head_runner = runners[-1]
     from idgx import plain_kernel_shape
 
-    dom_key = kernel_key(head["precision"], head["path"], dominant, head_runner.shapes[dominant],
-                         plain_shape=plain_kernel_shape(dw.plan(), ch is not None))
+    dom_key = pass_kernel(head["precision"], head["path"], dominant, head_runner.shapes[dominant], S,
+                          int(w["nr_subgrids"]), plain_shape=plain_kernel_shape(dw.plan(), ch is not None))
     roofline = roofline_record(args.config, head["precision"], dom_key, dominant, flops, sincos, t_dom)
     roofline.update(algorithmic_bytes=bytes_dom, hbm_gbs_algorithmic=bytes_dom / t_dom / 1e9)
 

@@ -81,7 +81,8 @@ typedef enum
      * v_sin_f32/v_cos_f32. */
     IDGX_FLAG_ACCURATE_SINCOS = 1,
     /* Mixed forms: evaluate the per-pair phase qu x' + qv y' + dw n as an FP32 MFMA (v_mfma_f32_16x16x4_f32)
-     * instead of three VALU fused multiply-adds.  Same accuracy; a tuning choice. */
+     * instead of three VALU fused multiply-adds.  Same accuracy; a tuning choice.  One-shot plans with it run the
+     * per-pair kernels. */
     IDGX_FLAG_PHASE_MFMA = 2
 } idgx_flags;
 
@@ -381,6 +382,8 @@ int idgx_plan_segments(const idgx_planner *planner, const float *d_uvw, const do
  * vis_offset[s+1]), each entry (t << 16) | c relative to the subgrid's first row and channel window.  Creation
  * allocates the queue memory; the execution entry points allocate nothing, and idgx_batch_capture records them into
  * a hipGraph (no memset nodes) for idgx_batch_launch.
+ * The 3-product forms first take one launch per class of the separable kernels (subgrids up to 64^2, fields up to about
+ * 0.17 rad); the persistent launch then has only the subgrids whose w spreads too far over their visibilities.
  * Every precision batches: the mixed forms run their persistent MFMA kernels (shapes idgx_batch_shape_info), plain
  * FP32 the persistent forms of the plain kernels (shapes idgx_batch_plain_shape_info), which skip unselected
  * (flagged) samples instead of multiplying them by zero and otherwise round like idgx_grid / idgx_degrid.  They

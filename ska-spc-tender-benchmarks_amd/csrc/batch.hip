@@ -19,6 +19,10 @@
 // workgroups of an XCD take their own queue first and the others' when it is empty, so a subgrid's prepared pixels
 // (degridder) or visibilities (gridder), which every item of the subgrid stages again, are fetched into one L2.
 //
+// Separable forms: a class of a 3-product form whose plan allows it first takes a launch of the separable kernels, a
+// workgroup per subgrid, heaviest first; each marks the subgrids whose w spreads too far, and the persistent launch
+// that follows takes only their items (and ends at once where a class has none).
+//
 // Degridder pixels: before the persistent degridder, one workgroup per subgrid applies taper and A-terms and
 // splits the pixels into the packed words the degridder stages (32 B per pixel slot), so the work items copy
 // them instead of recomputing them for every chunk of visibilities.

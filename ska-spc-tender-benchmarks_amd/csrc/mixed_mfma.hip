@@ -1,5 +1,7 @@
-// Mixed-precision gridder and degridder for gfx950: FP64 phase-argument reduction, FP32 phasors, and the
-// phasor x data contraction on v_mfma_f32_16x16x32_{bf16,f16} with FP32 accumulation.
+// Mixed-precision gridder and degridder for gfx950, a phasor per (pixel, visibility) pair: FP64 phase-argument reduction,
+// FP32 phasors, and the phasor x data contraction on v_mfma_f32_16x16x32_{bf16,f16} with FP32 accumulation.  The
+// 3-product forms run the separable kernels (separable.hip) for subgrids up to 64^2 and fields up to about 0.17 rad, and
+// these for the subgrids whose w spreads too far; larger subgrids, wider fields and the single-product forms run these.
 //
 // Phase reduction.  With l = (x' + 1/2) delta, x' = x - S/2 (an integer), delta = image_size / S, and
 //     du = k_c u_t / 2pi - u_off,  dv = ...,  dw = k_c w_t / 2pi - w_off      (wavelengths, formed in FP64,

@@ -18,10 +18,11 @@ import json
 import os
 import sys
 
-KERNELS = ["gridder_plain_queue_tiles", "gridder_plain_queue", "degridder_plain_queue", "gridder_plain",
+KERNELS = ["grid_separable", "degrid_separable", "gridder_plain_tiles", "degridder_plain_tiles",
+           "gridder_plain_queue_tiles", "gridder_plain_queue", "degridder_plain_queue", "gridder_plain",
            "degridder_plain", "gridder_mfma_queue_tiles", "gridder_mfma_queue", "degridder_mfma_queue",
            "degrid_prepare_kernel", "gridder_mfma", "degridder_mfma", "subgrid_fft_kernel", "adder_kernel",
-           "splitter_kernel", "fft_col_kernel", "fft_row_kernel", "wstack_row_kernel", "copy_box_kernel",
+           "splitter_kernel", "fft_col_kernel", "fft_row_kernel", "wstack_row_kernel",
            "clear_band_kernel",
            "checkerboard_kernel", "wstack_to_image_kernel", "wstack_from_image_kernel", "reset_counters_kernel"]
 
@@ -31,7 +32,7 @@ def short_name(name):
     instantiation (precision, tile shape) keeps its own row; "copy" for the calibration copy."""
     for k in KERNELS:
         i = name.find(k)
-        if i < 0 or (k.startswith("gridder") and name[i - 2:i] == "de"):
+        if i < 0 or (k.startswith("grid") and name[i - 2:i] == "de"):
             continue
         if name[i + len(k):i + len(k) + 1] not in ("<", "(", ""):
             continue
