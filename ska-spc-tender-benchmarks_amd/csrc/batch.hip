@@ -72,12 +72,15 @@ struct idgx_batch
     int qbegin[2][idgx::kMaxClasses][idgx::kQueues + 1] = {};
     int single_qbegin[2][idgx::kQueues + 1] = {};
     int *d_counters = nullptr;
-    // Classes that take the separable kernels: their tables, most visibilities of one subgrid, and in device memory the
-    // subgrids heaviest first, then per direction the marks of those left to the per-pair kernels.
+    // Classes that take the separable kernels: their tables, most visibilities of one subgrid, and in one device array
+    // each class's subgrids heaviest first (from order_offset), then per direction the marks of all classes' subgrids
+    // left to the per-pair kernels (order_total each).
     bool separable[idgx::kMaxClasses] = {};
     idgx::SeparableTables tables[idgx::kMaxClasses] = {};
     long long most_vis[idgx::kMaxClasses] = {};
-    int *d_order[idgx::kMaxClasses] = {};
+    int *d_order = nullptr;
+    size_t order_offset[idgx::kMaxClasses] = {};
+    size_t order_total = 0;
     // Degridder pixels prepared once per subgrid and pass (per class): split words, FP16 scales, slot n table.
     uint4 *d_prepared[idgx::kMaxClasses] = {};
     int *d_prepared_scale[idgx::kMaxClasses] = {};
@@ -439,8 +442,8 @@ hipError_t run_separable(idgx_batch *b, QueueArgs &q, int k, bool gridder, hipSt
         return hipSuccess;
     idgx::SeparableArgs sp{};
     sp.tables = b->tables[k];
-    sp.order = b->d_order[k];
-    sp.leftover = b->d_order[k] + (1 + dir) * static_cast<size_t>(a.p.nr_subgrids);
+    sp.order = b->d_order + b->order_offset[k];
+    sp.leftover = b->d_order + (1 + dir) * b->order_total + b->order_offset[k];
     sp.leftover_any = b->d_counters + dir * kDirCounters + idgx::kMaxClasses * idgx::kQueues + k;
     sp.per = idgx::separable_chunk(b->most_vis[k], a.p.nr_subgrids);
     const hipError_t e = gridder ? idgx::launch_grid_separable(a, sp, b->precision, st)
@@ -580,6 +583,7 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
     }
     if (e == hipSuccess)
         e = hipMalloc(&b->d_counters, 2 * kDirCounters * sizeof(int));
+    std::vector<int> order;
     for (int k = 0; k < nr_classes && e == hipSuccess; ++k)
     {
         const idgx_plan &p = b->plans[k];
@@ -589,12 +593,18 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
         b->separable[k] = p.nr_subgrids > 0 && idgx::separable_tables(geometry, b->precision, b->tables[k]);
         if (!b->separable[k])
             continue;
-        const std::vector<int> order = heaviest_first(b->vis_count[k]);
-        b->most_vis[k] = b->vis_count[k][order[0]];
-        // The order, then each direction's leftover marks.
-        e = hipMalloc(&b->d_order[k], 3 * order.size() * sizeof(int));
+        const std::vector<int> heaviest = heaviest_first(b->vis_count[k]);
+        b->most_vis[k] = b->vis_count[k][heaviest[0]];
+        b->order_offset[k] = order.size();
+        order.insert(order.end(), heaviest.begin(), heaviest.end());
+    }
+    if (!order.empty() && e == hipSuccess)
+    {
+        // One array and one copy for all classes.
+        b->order_total = order.size();
+        e = hipMalloc(&b->d_order, 3 * order.size() * sizeof(int));
         if (e == hipSuccess)
-            e = hipMemcpy(b->d_order[k], order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice);
+            e = hipMemcpy(b->d_order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice);
     }
     for (int k = 0; k < nr_classes && e == hipSuccess && !plain(b); ++k)
     {
@@ -955,10 +965,10 @@ extern "C" void idgx_batch_destroy(idgx_batch *b)
             (void)hipFree(b->d_items[dir]);
     if (b->d_counters)
         (void)hipFree(b->d_counters);
+    if (b->d_order)
+        (void)hipFree(b->d_order);
     for (int k = 0; k < idgx::kMaxClasses; ++k)
     {
-        if (b->d_order[k])
-            (void)hipFree(b->d_order[k]);
         if (b->d_prepared[k])
             (void)hipFree(b->d_prepared[k]);
         if (b->d_prepared_scale[k])
