@@ -71,10 +71,12 @@ struct idgx_batch
     // [qbegin[j] + k]; counters [direction][class][queue] (the merged queue uses class 0's).
     int qbegin[2][idgx::kMaxClasses][idgx::kQueues + 1] = {};
     int single_qbegin[2][idgx::kQueues + 1] = {};
+    // One device array holds the counters, the launch order and the classes' prepared scales and slot tables (below).
+    char *d_fixed = nullptr;
     int *d_counters = nullptr;
-    // Classes that take the separable kernels: their tables, most visibilities of one subgrid, and in one device array
-    // each class's subgrids heaviest first (from order_offset), then per direction the marks of all classes' subgrids
-    // left to the per-pair kernels (order_total each).
+    // Classes that take the separable kernels: their tables, most visibilities of one subgrid, and in device memory each
+    // class's subgrids heaviest first (from order_offset), then per direction the marks of all classes' subgrids left to
+    // the per-pair kernels (order_total each).
     bool separable[idgx::kMaxClasses] = {};
     idgx::SeparableTables tables[idgx::kMaxClasses] = {};
     long long most_vis[idgx::kMaxClasses] = {};
@@ -581,8 +583,6 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
         b->single_offset[dir] = total;
         e = hipMalloc(&b->d_items[dir], std::max<size_t>(1, 2 * total) * sizeof(uint2));
     }
-    if (e == hipSuccess)
-        e = hipMalloc(&b->d_counters, 2 * kDirCounters * sizeof(int));
     std::vector<int> order;
     for (int k = 0; k < nr_classes && e == hipSuccess; ++k)
     {
@@ -598,23 +598,35 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
         b->order_offset[k] = order.size();
         order.insert(order.end(), heaviest.begin(), heaviest.end());
     }
-    if (!order.empty() && e == hipSuccess)
-    {
-        // One array and one copy for all classes.
-        b->order_total = order.size();
-        e = hipMalloc(&b->d_order, 3 * order.size() * sizeof(int));
-        if (e == hipSuccess)
-            e = hipMemcpy(b->d_order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice);
-    }
+    b->order_total = order.size();
+    size_t bytes = 0, scale_at[idgx::kMaxClasses] = {}, coord_at[idgx::kMaxClasses] = {};
+    const auto take = [&bytes](size_t n) {
+        const size_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
+    };
+    const size_t counters_at = take(2 * kDirCounters * sizeof(int)), order_at = take(3 * order.size() * sizeof(int));
     for (int k = 0; k < nr_classes && e == hipSuccess && !plain(b); ++k)
     {
         const int S = b->plans[k].subgrid_size;
         const long long n = std::max(1, b->plans[k].nr_subgrids);
         e = hipMalloc(&b->d_prepared[k], idgx::degrid_prepared_bytes(S, n));
-        if (e == hipSuccess)
-            e = hipMalloc(&b->d_prepared_scale[k], n * sizeof(int));
-        if (e == hipSuccess)
-            e = hipMalloc(&b->d_slot_coord[k], static_cast<size_t>(S) * idgx::degrid_row_stride(S) * sizeof(float4));
+        scale_at[k] = take(n * sizeof(int));
+        coord_at[k] = take(static_cast<size_t>(S) * idgx::degrid_row_stride(S) * sizeof(float4));
+    }
+    if (e == hipSuccess)
+        e = hipMalloc(&b->d_fixed, bytes);
+    if (e == hipSuccess)
+    {
+        b->d_counters = reinterpret_cast<int *>(b->d_fixed + counters_at);
+        b->d_order = reinterpret_cast<int *>(b->d_fixed + order_at);
+        for (int k = 0; k < nr_classes && !plain(b); ++k)
+        {
+            b->d_prepared_scale[k] = reinterpret_cast<int *>(b->d_fixed + scale_at[k]);
+            b->d_slot_coord[k] = reinterpret_cast<float4 *>(b->d_fixed + coord_at[k]);
+        }
+        if (!order.empty())
+            e = hipMemcpy(b->d_order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice);
     }
     int rc = to_status(e);
     for (int k = 0; k < nr_classes && rc == IDGX_OK; ++k)
@@ -963,18 +975,10 @@ extern "C" void idgx_batch_destroy(idgx_batch *b)
     for (int dir = 0; dir < 2; ++dir)
         if (b->d_items[dir])
             (void)hipFree(b->d_items[dir]);
-    if (b->d_counters)
-        (void)hipFree(b->d_counters);
-    if (b->d_order)
-        (void)hipFree(b->d_order);
+    if (b->d_fixed)
+        (void)hipFree(b->d_fixed);
     for (int k = 0; k < idgx::kMaxClasses; ++k)
-    {
         if (b->d_prepared[k])
             (void)hipFree(b->d_prepared[k]);
-        if (b->d_prepared_scale[k])
-            (void)hipFree(b->d_prepared_scale[k]);
-        if (b->d_slot_coord[k])
-            (void)hipFree(b->d_slot_coord[k]);
-    }
     delete b;
 }
