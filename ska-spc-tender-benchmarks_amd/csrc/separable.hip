@@ -204,14 +204,30 @@ __device__ __forceinline__ double pixel_n_series(double l, double m)
     return p * r2;
 }
 
-// e^{2 pi i w n} of pixel (x, y).
+// e^{2 pi i w n} of pixel (x, y), to about an FP32 rounding: every visibility of the subgrid shares its error, so the
+// quarter turns come off in FP64 and what is left, within an eighth of a turn, takes the Taylor series (cut off below
+// 2e-9) in place of v_sin / v_cos.  Distance of a gridded subgrid from 64 bits, per-pair kernels / v_sin and v_cos / the
+// series: 8 visibilities 1.30e-7 / 1.87e-7 / 1.62e-7, 72 visibilities 1.72e-7 / 1.95e-7 / 1.71e-7, 512 visibilities
+// 3.4e-7 / 2.5e-7 / 2.3e-7.  The series costs 1.5 % of the gridder on 24^2 subgrids of 129 visibilities.
 __device__ __forceinline__ cfloat pixel_rotation(int x, int y, int S, double delta, double w)
 {
     const double n = pixel_n_series((x + 0.5 - 0.5 * S) * delta, (y + 0.5 - 0.5 * S) * delta);
-    double t = w * n;
-    t -= __builtin_rint(t);
-    const float f = static_cast<float>(t);
-    return {__builtin_amdgcn_cosf(f), __builtin_amdgcn_sinf(f)};
+    const double t = __builtin_amdgcn_fract(w * n);
+    const float quarters = __builtin_rintf(4.F * static_cast<float>(t)); // 0 to 4
+    const int q = static_cast<int>(quarters);
+    const float f = static_cast<float>(__builtin_fma(-0.25, static_cast<double>(quarters), t)), f2 = f * f;
+    // In turns: powers of 2 pi over the factorials, and 2 pi itself in two parts.
+    float ps = __builtin_fmaf(f2, 42.0586939F, -76.7058598F), pc = __builtin_fmaf(f2, -26.4262568F, 60.2446414F);
+    ps = __builtin_fmaf(ps, f2, 81.6052493F);
+    pc = __builtin_fmaf(pc, f2, -85.4568172F);
+    ps = __builtin_fmaf(ps, f2, -41.3417022F);
+    pc = __builtin_fmaf(pc, f2, 64.9393940F);
+    ps = __builtin_fmaf(ps, f2, -1.74845553e-7F);
+    pc = __builtin_fmaf(pc, f2, -19.7392088F);
+    const float sn = __builtin_fmaf(f, 6.28318548F, f * ps), cs = __builtin_fmaf(pc, f2, 1.F);
+    const float re = q & 1 ? sn : cs, im = q & 1 ? cs : sn;
+    // Quarter turns 0, 1, 2, 3: (c, s), (-s, c), (-c, -s), (s, -c).
+    return {(q + 1) & 2 ? -re : re, q & 2 ? -im : im};
 }
 
 // (vr + i vi) (cs + i sn) with the phasor of lane J of the quad: four FMA-class instructions that read the phasor
