@@ -41,7 +41,9 @@ namespace idgx
 {
 namespace
 {
-constexpr float kEpsNone = 3e-7F; // below the FP32 rounding of the phases
+// Below this the term is worth 0.27 of it at most in the root mean square, 2.7e-8 (at 3e-7 it was 8e-8, seen in subgrids
+// of 8 visibilities: 1.44e-7 from 64 bits against 1.60e-7; no case got slower by more than its runs differ).
+constexpr float kEpsNone = 1e-7F;
 constexpr float kEpsMost = 1e-3F; // eps^2 / 2 <= 5e-7 at one corner pixel for the visibility farthest in w
 constexpr float kTurnsMost = 4.F; // |d a|: keeps the phases' FP32 rounding at the level of qu xh
 constexpr float kTermScale = 1024.F; // moves the product term's factors into FP16's normal range
@@ -207,7 +209,7 @@ __device__ __forceinline__ double pixel_n_series(double l, double m)
 // e^{2 pi i w n} of pixel (x, y), to about an FP32 rounding: every visibility of the subgrid shares its error, so the
 // quarter turns come off in FP64 and what is left, within an eighth of a turn, takes the Taylor series (cut off below
 // 2e-9) in place of v_sin / v_cos.  Distance of a gridded subgrid from 64 bits, per-pair kernels / v_sin and v_cos / the
-// series: 8 visibilities 1.30e-7 / 1.87e-7 / 1.62e-7, 72 visibilities 1.72e-7 / 1.95e-7 / 1.71e-7, 512 visibilities
+// series: 8 visibilities 1.30e-7 / 1.87e-7 / 1.60e-7, 72 visibilities 1.72e-7 / 1.95e-7 / 1.71e-7, 512 visibilities
 // 3.4e-7 / 2.5e-7 / 2.3e-7.  The series costs 1.5 % of the gridder on 24^2 subgrids of 129 visibilities.
 __device__ __forceinline__ cfloat pixel_rotation(int x, int y, int S, double delta, double w)
 {
