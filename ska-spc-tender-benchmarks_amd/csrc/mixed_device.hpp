@@ -91,13 +91,14 @@ template <int DT> __device__ __forceinline__ void split2(float x0, float x1, uin
 // rescaled exactly when a later batch needs a larger scale, and the final result is multiplied back.
 constexpr int kF16TargetExp = 14;
 
+// Never below -126, whose inverse is still finite: fainter values (below 2^-112) stay that much smaller instead.
 __device__ __forceinline__ int scale_exponent(float maxabs)
 {
     if (!(maxabs > 0.F))
         return -126;
     int e;
     (void)frexpf(maxabs, &e); // maxabs in [2^(e-1), 2^e)
-    return e - kF16TargetExp;
+    return max(e - kF16TargetExp, -126);
 }
 
 // Phases of a 16 x 16 tile: D[i][j] = sum_k A[i][k] B[k][j], K = 4 (fourth component zero).
