@@ -322,11 +322,13 @@ int idgx_wstack_from_image(const idgx_plan *plan, const void *d_image, int z_min
  * image row is transformed for every layer while n(l, m) stays in registers, so neither the layers' image-domain
  * planes nor a separate w-screen pass touch HBM.  The screens there take v_sin / v_cos of the FP64-reduced fraction
  * of a turn (about 1e-7 absolute), not FP64 sincospi.  One layer at w_step 0 has no screen to apply and takes the
- * passes of idgx_grid_fft_box, reading from one array and writing to the other.  idgx_grid_to_image otherwise keeps a scratch of
- * nr_layers x G x (box width rounded out to 64-column tiles) cells per device, allocated on first use and grown
+ * passes of idgx_grid_fft_box, reading from one array and writing to the other.
+ * Scratch: idgx_image_to_grid uses that of idgx_grid_fft.  idgx_grid_to_image keeps one of its own per device, which no
+ * other call uses: nr_layers x G x (box width rounded out to 64-column tiles) cells, allocated on first use and grown
  * (after a device synchronisation, which also makes a growing call unsuitable for hipGraph capture) when a call
- * needs more; calls that overlap on one device share it, so issue them from one host thread on one stream.  Other
- * sizes run the two calls one after the other.
+ * needs more; for one layer at w_step 0 (64 MB of planes, or one plane when larger) per size, allocated on first use.
+ * Calls that overlap on one device and use the same scratch race, so issue them from one host thread on one stream.
+ * Other sizes run the two calls one after the other.
  * No counterpart in the reference (its benchmark stops at the subgrids).  d_image must not alias d_grid. */
 int idgx_grid_to_image(const idgx_plan *plan, void *d_grid, int z_min, int nr_layers, const int32_t box[4],
                        void *d_image, void *stream);

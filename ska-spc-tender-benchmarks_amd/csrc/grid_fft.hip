@@ -1062,12 +1062,20 @@ bool stockham_size(int G)
 }
 
 // Scratch per (device, user, size), created on first use and kept for the life of the process.  The user tells
-// apart buffers that are live at the same time: the three-pass transform's (user 0) and the radix-3 decimation's
-// sub-planes (user 1), which the three-pass transform of those sub-planes must not share.
+// apart buffers that may be live at the same time: the three-pass transform's, the radix-3 decimation's sub-planes (which
+// the three-pass transform of those sub-planes must not share), the four-step columns' of fft_plane_scratch, and the
+// transform inside grid_to_image, which may run on another stream beside a transform of the same size.
+enum ScratchUser
+{
+    kThreePassScratch = 0,
+    kRadix3Scratch = 1,
+    // 2: the four-step columns (fft_plane_scratch)
+    kToImageScratch = 3,
+};
 std::mutex g_scratch_mutex;
 std::map<std::tuple<int, int, long long>, float2 *> g_scratch;
 
-hipError_t fft_scratch(long long elements, float2 *&out, int user = 0)
+hipError_t fft_scratch(long long elements, float2 *&out, int user)
 {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -1185,7 +1193,8 @@ FftArgs fft_args(int gx, int gy, bool centred)
 // allocated on first use.
 template <int SG>
 hipError_t stockham_fft2d(const float2 *src, float2 *dst, int gx, int gy, long long planes, bool centred,
-                          hipStream_t st, const FftBox &box = FftBox(), bool no_alloc = false)
+                          hipStream_t st, const FftBox &box = FftBox(), bool no_alloc = false,
+                          ScratchUser user = kThreePassScratch)
 {
     FftArgs A = fft_args(gx, gy, centred);
     const long long plane = static_cast<long long>(gx) * gy;
@@ -1199,7 +1208,7 @@ hipError_t stockham_fft2d(const float2 *src, float2 *dst, int gx, int gy, long l
         e = static_scratch(A.scratch);
     }
     else
-        e = fft_scratch(group * plane, A.scratch);
+        e = fft_scratch(group * plane, A.scratch, user);
     if (e != hipSuccess)
         return e;
     if (box.mode == kSparseInput)
@@ -1477,7 +1486,7 @@ hipError_t radix3_fft2d(const float2 *src, float2 *dst, int N, long long planes,
     const int M = N / 3;
     const long long plane = static_cast<long long>(N) * N;
     FftArgs A;
-    hipError_t e = fft_scratch(plane, A.scratch, 1);
+    hipError_t e = fft_scratch(plane, A.scratch, kRadix3Scratch);
     if (e != hipSuccess)
         return e;
     A.gx = N;
@@ -1678,7 +1687,7 @@ hipError_t launch_grid_wstack(void *grid, void *image, int G, int z_min, int nr_
         b.y0 = box[2];
         b.y1 = box[3];
         float2 *g = static_cast<float2 *>(grid), *img = static_cast<float2 *>(image);
-        return to_image ? stockham_fft2d<-1>(g, img, G, G, planes, true, st, b)
+        return to_image ? stockham_fft2d<-1>(g, img, G, G, planes, true, st, b, false, kToImageScratch)
                         : stockham_fft2d<1>(img, g, G, G, planes, true, st, b);
     }
     WsArgs W{};
