@@ -74,12 +74,13 @@ struct idgx_batch
     // One device array holds the counters, the launch order and the classes' prepared scales and slot tables (below).
     char *d_fixed = nullptr;
     int *d_counters = nullptr;
-    // Classes that take the separable kernels: their tables, most visibilities of one subgrid, and in device memory each
+    // Classes that take the separable kernels: their tables, visibility counts, and in device memory each
     // class's subgrids heaviest first (from order_offset), then per direction the marks of all classes' subgrids left to
     // the per-pair kernels (order_total each).
     bool separable[idgx::kMaxClasses] = {};
     idgx::SeparableTables tables[idgx::kMaxClasses] = {};
     long long most_vis[idgx::kMaxClasses] = {};
+    int few_vis[idgx::kMaxClasses] = {}; // subgrids of at most separable_few_visibilities(): the order's last
     int *d_order = nullptr;
     size_t order_offset[idgx::kMaxClasses] = {};
     size_t order_total = 0;
@@ -448,7 +449,7 @@ hipError_t run_separable(idgx_batch *b, QueueArgs &q, int k, bool gridder, hipSt
     sp.leftover = b->d_order + (1 + dir) * b->order_total + b->order_offset[k];
     sp.leftover_any = b->d_counters + dir * kDirCounters + idgx::kMaxClasses * idgx::kQueues + k;
     sp.per = idgx::separable_chunk(b->most_vis[k], a.p.nr_subgrids);
-    const hipError_t e = gridder ? idgx::launch_grid_separable(a, sp, b->precision, st)
+    const hipError_t e = gridder ? idgx::launch_grid_separable(a, sp, b->precision, {b->most_vis[k], b->few_vis[k]}, st)
                                  : idgx::launch_degrid_separable(a, sp, b->precision, b->most_vis[k], st);
     a.leftover = sp.leftover;
     a.leftover_any = sp.leftover_any;
@@ -595,6 +596,9 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
             continue;
         const std::vector<int> heaviest = heaviest_first(b->vis_count[k]);
         b->most_vis[k] = b->vis_count[k][heaviest[0]];
+        b->few_vis[k] = static_cast<int>(std::count_if(b->vis_count[k].begin(), b->vis_count[k].end(), [](int64_t v) {
+            return v <= idgx::separable_few_visibilities();
+        }));
         b->order_offset[k] = order.size();
         order.insert(order.end(), heaviest.begin(), heaviest.end());
     }

@@ -161,16 +161,26 @@ struct SeparableTables
 struct SeparableArgs
 {
     SeparableTables tables;
-    const int *order;  // workgroup -> subgrid (null: plan order)
+    const int *order;  // workgroup -> subgrid, most visibilities first (null: plan order)
+    int count;         // gridder: subgrids of the launch
     int *leftover;     // per subgrid: 1 where the per-pair kernels have to run (null: they run inside the launch)
     int *leftover_any; // set to 1 with the first of them
     long long per;     // degridder: visibilities per workgroup, a multiple of 256
 };
+// Visibilities of a gridder call's subgrids: the most that one has, and with an order how many have at most
+// separable_few_visibilities().
+struct GridCounts
+{
+    long long most_vis;
+    int few;
+};
+long long separable_few_visibilities();
 // Whether the plan's subgrids take the separable kernels, and their tables.
 bool separable_tables(const PlanDev &p, int precision, SeparableTables &t);
 // Degridder visibilities per workgroup (SeparableArgs::per) for n subgrids of at most max_vis visibilities.
 long long separable_chunk(long long max_vis, int n);
-hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, hipStream_t st);
+hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, const GridCounts &n,
+                                 hipStream_t st);
 hipError_t launch_degrid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, long long max_vis,
                                    hipStream_t st);
 

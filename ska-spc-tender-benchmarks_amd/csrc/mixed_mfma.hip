@@ -451,7 +451,8 @@ hipError_t launch_grid_mixed(const KernelArgs &a, int precision, bool pm, hipStr
 {
     SeparableArgs sp{};
     if (!pm && separable_tables(a.p, precision, sp.tables))
-        return launch_grid_separable(a, sp, precision, st);
+        return launch_grid_separable(a, sp, precision,
+                                     {static_cast<long long>(a.p.max_nr_timesteps) * a.p.nr_channels, 0}, st);
     switch (precision)
     {
     case IDGX_MIXED_BF16X3:

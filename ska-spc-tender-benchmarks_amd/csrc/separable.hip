@@ -36,6 +36,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstddef>
+#include <type_traits>
 
 namespace idgx
 {
@@ -51,6 +52,11 @@ constexpr float kTermScale = 1024.F; // moves the product term's factors into FP
 // stays within four times kEpsMost: fields up to about 0.17 rad at S = 32, 0.13 at S = 64.  In wider ones the per-pair
 // items would often run inside these kernels, at fewer waves per SIMD than in their own.
 constexpr double kSeparableField = 4e-3;
+// FP16 gridding of a subgrid of so few visibilities forms its phasors by their series and always takes the product term:
+// over few visibilities the errors of v_sin and v_cos, here of two phasors a pair instead of one, do not average out.
+// Distance from 64 bits over that of the per-pair kernels, worst of S = 16 .. 48, with v_sin and v_cos / by the series:
+// 8 visibilities 1.08 / 0.94, 16 1.09 / 0.94, 32 1.03 / 0.92, 48 0.99.
+constexpr int kFewVisibilities = 72;
 constexpr int kFewSubgrids = 256;  // the CUs: a workgroup per subgrid would leave some of them idle
 constexpr int kChunk = 64;        // visibilities a wave stages at a time, one per lane
 constexpr int kValStride = 80;    // staged values of one correlation (64, padded: fewer LDS bank conflicts)
@@ -206,18 +212,10 @@ __device__ __forceinline__ double pixel_n_series(double l, double m)
     return p * r2;
 }
 
-// e^{2 pi i w n} of pixel (x, y), to about an FP32 rounding: every visibility of the subgrid shares its error, so the
-// quarter turns come off in FP64 and what is left, within an eighth of a turn, takes the Taylor series (cut off below
-// 2e-9) in place of v_sin / v_cos.  Distance of a gridded subgrid from 64 bits, per-pair kernels / v_sin and v_cos / the
-// series: 8 visibilities 1.30e-7 / 1.87e-7 / 1.60e-7, 72 visibilities 1.72e-7 / 1.95e-7 / 1.71e-7, 512 visibilities
-// 3.4e-7 / 2.5e-7 / 2.3e-7.  The series costs 1.5 % of the gridder on 24^2 subgrids of 129 visibilities.
-__device__ __forceinline__ cfloat pixel_rotation(int x, int y, int S, double delta, double w)
+// e^{2 pi i (f + q / 4)} for |f| <= 1/8 of a turn, to about an FP32 rounding: the Taylor series, cut off below 2e-9.
+__device__ __forceinline__ cfloat phasor_series(float f, int q)
 {
-    const double n = pixel_n_series((x + 0.5 - 0.5 * S) * delta, (y + 0.5 - 0.5 * S) * delta);
-    const double t = __builtin_amdgcn_fract(w * n);
-    const float quarters = __builtin_rintf(4.F * static_cast<float>(t)); // 0 to 4
-    const int q = static_cast<int>(quarters);
-    const float f = static_cast<float>(__builtin_fma(-0.25, static_cast<double>(quarters), t)), f2 = f * f;
+    const float f2 = f * f;
     // In turns: powers of 2 pi over the factorials, and 2 pi itself in two parts.
     float ps = __builtin_fmaf(f2, 42.0586939F, -76.7058598F), pc = __builtin_fmaf(f2, -26.4262568F, 60.2446414F);
     ps = __builtin_fmaf(ps, f2, 81.6052493F);
@@ -230,6 +228,34 @@ __device__ __forceinline__ cfloat pixel_rotation(int x, int y, int S, double del
     const float re = q & 1 ? sn : cs, im = q & 1 ? cs : sn;
     // Quarter turns 0, 1, 2, 3: (c, s), (-s, c), (-c, -s), (s, -c).
     return {(q + 1) & 2 ? -re : re, q & 2 ? -im : im};
+}
+
+// e^{2 pi i ph}: v_sin and v_cos, or (SERIES) the series, about three times their instructions.
+template <bool SERIES> __device__ __forceinline__ void phasor(float ph, float &sn, float &cs)
+{
+    if constexpr (SERIES)
+    {
+        const float quarters = __builtin_rintf(4.F * ph);
+        const cfloat r = phasor_series(__builtin_fmaf(-0.25F, quarters, ph), static_cast<int>(quarters));
+        cs = r.re;
+        sn = r.im;
+    }
+    else
+    {
+        sn = __builtin_amdgcn_sinf(ph);
+        cs = __builtin_amdgcn_cosf(ph);
+    }
+}
+
+// e^{2 pi i w n} of pixel (x, y): every visibility of the subgrid shares its error, so the quarter turns come off in FP64
+// and what is left takes the series.  It costs 1.5 % of the gridder on 24^2 subgrids of 129 visibilities.
+__device__ __forceinline__ cfloat pixel_rotation(int x, int y, int S, double delta, double w)
+{
+    const double n = pixel_n_series((x + 0.5 - 0.5 * S) * delta, (y + 0.5 - 0.5 * S) * delta);
+    const double t = __builtin_amdgcn_fract(w * n);
+    const float quarters = __builtin_rintf(4.F * static_cast<float>(t)); // 0 to 4
+    return phasor_series(static_cast<float>(__builtin_fma(-0.25, static_cast<double>(quarters), t)),
+                         static_cast<int>(quarters));
 }
 
 // (vr + i vi) (cs + i sn) with the phasor of lane J of the quad: four FMA-class instructions that read the phasor
@@ -303,13 +329,13 @@ __device__ __forceinline__ void split_rows(float c, float s, uint32_t &re_hi, ui
     im_lo = pack2<DT>(rs, rc);
 }
 
-// The rows of i f (c + i s) in single halves, from the split rows (FP16) or the phasor (BF16): re = -f (s, c),
-// im = f (c, -s).
-template <int DT>
+// The rows of i f (c + i s) in single halves: re = -f (s, c), im = f (c, -s).  FP16: from the split rows, with three
+// roundings to halves; BF16, and FP16 with ONCE: from the phasor, with one.
+template <int DT, bool ONCE = false>
 __device__ __forceinline__ void term_rows(float c, float s, float f, uint32_t re_hi, uint32_t im_hi, uint32_t &re,
                                           uint32_t &im)
 {
-    if constexpr (DT == kFP16)
+    if constexpr (DT == kFP16 && !ONCE)
     {
         const f16x2 ff = __builtin_bit_cast(f16x2, pack2<DT>(f, f));
         re = __builtin_bit_cast(uint32_t, -ff * __builtin_bit_cast(f16x2, im_hi));
@@ -365,7 +391,7 @@ template <int YT> struct RowCoords
 };
 
 // 8 staged visibilities onto the wave's pixels: all rows, NT tiles of 8 columns x 4 correlations.
-template <int DT, int YT, int NT, bool TERM>
+template <int DT, int YT, int NT, bool TERM, bool SERIES>
 __device__ __forceinline__ void grid_step(const GridStage &st, const float2 *tab, int base, int x0, float half_s,
                                           const RowCoords<YT> &rc, f32x16 (&acc)[NT][YT])
 {
@@ -382,10 +408,11 @@ __device__ __forceinline__ void grid_step(const GridStage &st, const float2 *tab
             for (int j = 0; j < 4; ++j)
             {
                 const float ph = __builtin_fmaf(qv[j], rc.yh[t], de[j] * rc.ya[t]);
-                const float sn = __builtin_amdgcn_sinf(ph), cs = __builtin_amdgcn_cosf(ph);
+                float sn, cs;
+                phasor<SERIES>(ph, sn, cs);
                 split_rows<DT>(cs, sn, ah[2 * t][j], al[2 * t][j], ah[2 * t + 1][j], al[2 * t + 1][j]);
                 if constexpr (TERM)
-                    term_rows<DT>(cs, sn, de[j] * rc.yg[t], ah[2 * t][j], ah[2 * t + 1][j], at[2 * t][j],
+                    term_rows<DT, SERIES>(cs, sn, de[j] * rc.yg[t], ah[2 * t][j], ah[2 * t + 1][j], at[2 * t][j],
                                   at[2 * t + 1][j]);
             }
     }
@@ -402,11 +429,12 @@ __device__ __forceinline__ void grid_step(const GridStage &st, const float2 *tab
         {
             const float d = j ? de.y : de.x;
             const float ph = __builtin_fmaf(j ? qv.y : qv.x, rc.yh[k], d * rc.ya[k]);
-            const float sn = __builtin_amdgcn_sinf(ph), cs = __builtin_amdgcn_cosf(ph);
+            float sn, cs;
+            phasor<SERIES>(ph, sn, cs);
             split_rows<DT>(cs, sn, ah[t][j], al[t][j], ah[t][j + 2], al[t][j + 2]);
             if constexpr (TERM)
             {
-                term_rows<DT>(cs, sn, d * rc.yg[k], ah[t][j], ah[t][j + 2], at[t][j], at[t][j + 2]);
+                term_rows<DT, SERIES>(cs, sn, d * rc.yg[k], ah[t][j], ah[t][j + 2], at[t][j], at[t][j + 2]);
                 swap_rows16(at[t][j], at[t][j + 2]);
             }
             swap_rows16(ah[t][j], ah[t][j + 2]);
@@ -423,7 +451,8 @@ __device__ __forceinline__ void grid_step(const GridStage &st, const float2 *tab
         const int x = x0 + 8 * nt + ((lane & 31) >> 2);
         const float2 tb = tab[x];
         const float ph = __builtin_fmaf(qux, static_cast<float>(x) - half_s, dex * tb.x);
-        const float sn = __builtin_amdgcn_sinf(ph), cs = __builtin_amdgcn_cosf(ph);
+        float sn, cs;
+        phasor<SERIES>(ph, sn, cs);
         const cfloat vx[4] = {quad_product<0>(cs, sn, v01[0], v01[1]), quad_product<1>(cs, sn, v01[2], v01[3]),
                               quad_product<2>(cs, sn, v23[0], v23[1]), quad_product<3>(cs, sn, v23[2], v23[3])};
         uint32_t bh[4], bl[4], bt[4];
@@ -433,7 +462,7 @@ __device__ __forceinline__ void grid_step(const GridStage &st, const float2 *tab
         {
             split2<DT>(vx[j].re, vx[j].im, bh[j], bl[j]);
             if constexpr (TERM)
-                bt[j] = DT == kFP16 ? mul_f16x2(bh[j], gg) : pack2<DT>(vx[j].re * tb.y, vx[j].im * tb.y);
+                bt[j] = DT == kFP16 && !SERIES ? mul_f16x2(bh[j], gg) : pack2<DT>(vx[j].re * tb.y, vx[j].im * tb.y);
         }
 #pragma unroll
         for (int t = 0; t < YT; ++t)
@@ -495,7 +524,7 @@ __device__ __forceinline__ RawVisibility load_visibility(const KernelArgs &a, co
 
 // One wave's chunks of V visibilities: chunk `first` (whose visibilities are in raw), then every step-th.  n
 // visibilities per chunk, a multiple of 8, at most kChunk.
-template <int DT, int YT, int NT, bool TERM>
+template <int DT, int YT, int NT, bool TERM, bool SERIES>
 __device__ __forceinline__ int grid_sum(const KernelArgs &a, const SeparableArgs &sp, const Selection &sel, int V, int T,
                                         int nc, long long row0, int c0, const CentreOffsets &off, double wc,
                                         int first, int step, int n, RawVisibility raw, int x0, GridStage &st,
@@ -555,7 +584,7 @@ __device__ __forceinline__ int grid_sum(const KernelArgs &a, const SeparableArgs
         raw = load_visibility(a, sel, lane < n ? v0 + step * n + lane : V, V, T, nc, row0, c0);
         const int nsteps = min(n, V - v0 + 7) >> 3;
         for (int k = 0; k < nsteps; ++k)
-            grid_step<DT, YT, NT, TERM>(st, tab, 8 * k, x0, half_s, rc, acc);
+            grid_step<DT, YT, NT, TERM, SERIES>(st, tab, 8 * k, x0, half_s, rc, acc);
     }
     return scale_exp;
 }
@@ -578,16 +607,25 @@ template <int YT, int NT> constexpr int grid_waves()
     return YT * NT <= 2 ? 4 : YT * NT <= 3 || (YT == 2 && NT == 3) ? 3 : 2;
 }
 
+// Which subgrids of a launch a kernel grids, by their visibilities (kFewVisibilities).  Kernels with wide column tiles
+// have one form for each: a kernel with both would spill in its main loop (24^2 subgrids of 129 visibilities: 7 % slower).
+enum GridSubgrids
+{
+    kEvery,
+    kMany,
+    kFew
+};
+
 // Workgroup (part, subgrid) grids columns [part, part + 1) x 8 NT NX of a subgrid: its waves take NX column ranges and
 // WAVES / NX interleaved chunks of visibilities; the partial sums meet in LDS 16 or 32 rows at a time, in a fixed order.
-template <int DT, int YT, int NT, int NX, int WAVES>
+template <int DT, int YT, int NT, int NX, int WAVES, GridSubgrids WHICH>
 __global__ __launch_bounds__(64 * WAVES, (grid_waves<YT, NT>())) void grid_separable(KernelArgs a, SeparableArgs sp)
 {
     constexpr int kCols = NX * NT * 8, kSplits = WAVES / NX, kCount = 64 * WAVES;
     constexpr int kPass = NT == 1 ? 32 : 16; // rows of the subgrid whose sums meet at a time
     __shared__ GridLds<kCols, kSplits, kPass, WAVES> sm;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int part = blockIdx.x / a.p.nr_subgrids, b = blockIdx.x - part * a.p.nr_subgrids;
+    const int part = blockIdx.x / sp.count, b = blockIdx.x - part * sp.count;
     const int s = sp.order ? sp.order[b] : b;
     const int S = a.p.S, P = S * S;
     const idgx_metadata m = a.metadata[s];
@@ -597,6 +635,9 @@ __global__ __launch_bounds__(64 * WAVES, (grid_waves<YT, NT>())) void grid_separ
     const bool ok = subgrid_in_bounds(a.p, m, row0, c0, nc);
     Selection sel;
     const int T = m.nr_timesteps, V = ok ? selection_of(a, s, T, nc, sel) : 0;
+    // Without an order, which the host has split at the count, both launches go over all subgrids.
+    if (WHICH != kEvery && !sp.order && (V <= kFewVisibilities) != (WHICH == kFew))
+        return; // uniform
     // Chunks short enough for every split to have one.
     const int split = wave / NX, n = min(kChunk, ((V + kSplits - 1) / kSplits + 7) & ~7);
     RawVisibility raw = load_visibility(a, sel, lane < n ? split * n + lane : V, V, T, nc, row0, c0);
@@ -637,13 +678,19 @@ __global__ __launch_bounds__(64 * WAVES, (grid_waves<YT, NT>())) void grid_separ
             for (int i = 0; i < 16; ++i)
                 acc[nt][t][i] = 0.F;
     const int xb = part * kCols, x0 = xb + (wave % NX) * NT * 8;
+    const auto sum = [&](auto term, auto series) {
+        return grid_sum<DT, YT, NT, term.value, series.value>(a, sp, sel, V, T, nc, row0, c0, off, wr.centre, split,
+                                                              kSplits, n, raw, x0, sm.stage[wave], sm.tab, acc);
+    };
     int scale_exp;
-    if (eps <= kEpsNone)
-        scale_exp = grid_sum<DT, YT, NT, false>(a, sp, sel, V, T, nc, row0, c0, off, wr.centre, split, kSplits, n, raw,
-                                                x0, sm.stage[wave], sm.tab, acc);
+    if constexpr (DT == kFP16 && WHICH == kFew)
+        scale_exp = sum(std::true_type{}, std::true_type{});
+    else if (DT == kFP16 && WHICH == kEvery && V <= kFewVisibilities)
+        scale_exp = sum(std::true_type{}, std::bool_constant<DT == kFP16 && WHICH == kEvery>{});
+    else if (eps <= kEpsNone)
+        scale_exp = sum(std::false_type{}, std::false_type{});
     else
-        scale_exp = grid_sum<DT, YT, NT, true>(a, sp, sel, V, T, nc, row0, c0, off, wr.centre, split, kSplits, n, raw,
-                                               x0, sm.stage[wave], sm.tab, acc);
+        scale_exp = sum(std::true_type{}, std::false_type{});
     const float unscale = DT == kFP16 ? ldexpf(1.F, scale_exp) : 1.F;
     float2 *out = reinterpret_cast<float2 *>(a.subgrids_out) + static_cast<size_t>(s) * kCorr * P;
     const float4 *aterms = reinterpret_cast<const float4 *>(a.aterms);
@@ -1049,14 +1096,40 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
 
 // ---- launchers --------------------------------------------------------------------------------------------------
 
-template <int DT, int YT, int NT, int NX, int WAVES = kWaves>
+template <int DT, int YT, int NT, int NX, int WAVES, GridSubgrids WHICH>
 hipError_t launch_grid(const KernelArgs &a, const SeparableArgs &sp, hipStream_t st)
 {
-    const long long parts = (a.p.S + 8 * NT * NX - 1) / (8 * NT * NX), blocks = parts * a.p.nr_subgrids;
+    const long long parts = (a.p.S + 8 * NT * NX - 1) / (8 * NT * NX), blocks = parts * sp.count;
     if (blocks > 0x7fffffffLL)
         return hipErrorInvalidConfiguration;
-    grid_separable<DT, YT, NT, NX, WAVES><<<static_cast<unsigned>(blocks), 64 * WAVES, 0, st>>>(a, sp);
+    if (blocks > 0)
+        grid_separable<DT, YT, NT, NX, WAVES, WHICH><<<static_cast<unsigned>(blocks), 64 * WAVES, 0, st>>>(a, sp);
     return hipGetLastError();
+}
+
+// Subgrids of many visibilities, then those of few (the last `few` of an order; without one, any may be).
+template <int DT, int YT, int NT, int NX>
+hipError_t launch_grid_wide(const KernelArgs &a, SeparableArgs sp, const GridCounts &n, hipStream_t st)
+{
+    if constexpr (DT != kFP16)
+    {
+        return launch_grid<DT, YT, NT, NX, kWaves, kEvery>(a, sp, st);
+    }
+    else
+    {
+        hipError_t e = hipSuccess;
+        sp.count = sp.order ? a.p.nr_subgrids - n.few : a.p.nr_subgrids;
+        if (n.most_vis > kFewVisibilities)
+            e = launch_grid<DT, YT, NT, NX, kWaves, kMany>(a, sp, st);
+        if (e != hipSuccess)
+            return e;
+        if (sp.order)
+        {
+            sp.order += sp.count;
+            sp.count = n.few;
+        }
+        return launch_grid<DT, YT, NT, NX, kWaves, kFew>(a, sp, st);
+    }
 }
 
 // Row tiles and column tiles per wave and column ranges for subgrid size S.  One wave holds all columns up to S = 32
@@ -1064,26 +1137,27 @@ hipError_t launch_grid(const KernelArgs &a, const SeparableArgs &sp, hipStream_t
 // takes a workgroup per 8 columns, which forms the row phasors once per 8 columns; where even those leave CUs idle, one
 // of 8 waves (45 subgrids of 32^2 with 2048 visibilities: 30.4 -> 25.8 us; of 16^2: 24.2 -> 19.5), which would cost
 // larger plans up to a quarter (231 subgrids of 32^2 with 256: 16.9 -> 20.9) and subgrids above 32^2 a tenth.
-template <int DT> hipError_t grid_size(const KernelArgs &a, const SeparableArgs &sp, hipStream_t st)
+template <int DT>
+hipError_t grid_size(const KernelArgs &a, const SeparableArgs &sp, const GridCounts &n, hipStream_t st)
 {
     const int S = a.p.S;
     const bool few = a.p.nr_subgrids <= kFewSubgrids;
     const bool fewer = static_cast<long long>(a.p.nr_subgrids) * ((S + 7) / 8) <= kFewSubgrids;
     if (S <= 16)
-        return fewer ? launch_grid<DT, 1, 1, 1, 8>(a, sp, st)
-               : few ? launch_grid<DT, 1, 1, 1>(a, sp, st)
-                     : launch_grid<DT, 1, 2, 1>(a, sp, st);
+        return fewer ? launch_grid<DT, 1, 1, 1, 8, kEvery>(a, sp, st)
+               : few ? launch_grid<DT, 1, 1, 1, kWaves, kEvery>(a, sp, st)
+                     : launch_grid_wide<DT, 1, 2, 1>(a, sp, n, st);
     if (S <= 32 && fewer)
-        return launch_grid<DT, 2, 1, 1, 8>(a, sp, st);
+        return launch_grid<DT, 2, 1, 1, 8, kEvery>(a, sp, st);
     if (S <= 32 && few)
-        return launch_grid<DT, 2, 1, 1>(a, sp, st);
+        return launch_grid<DT, 2, 1, 1, kWaves, kEvery>(a, sp, st);
     if (S <= 24)
-        return launch_grid<DT, 2, 3, 1>(a, sp, st);
+        return launch_grid_wide<DT, 2, 3, 1>(a, sp, n, st);
     if (S <= 32)
-        return launch_grid<DT, 2, 4, 1>(a, sp, st);
+        return launch_grid_wide<DT, 2, 4, 1>(a, sp, n, st);
     if (S <= 48)
-        return few ? launch_grid<DT, 3, 1, 1>(a, sp, st) : launch_grid<DT, 3, 3, 2>(a, sp, st);
-    return few ? launch_grid<DT, 4, 1, 1>(a, sp, st) : launch_grid<DT, 4, 2, 4>(a, sp, st);
+        return few ? launch_grid<DT, 3, 1, 1, kWaves, kEvery>(a, sp, st) : launch_grid_wide<DT, 3, 3, 2>(a, sp, n, st);
+    return few ? launch_grid<DT, 4, 1, 1, kWaves, kEvery>(a, sp, st) : launch_grid_wide<DT, 4, 2, 4>(a, sp, n, st);
 }
 
 template <int DT, int KS, int YB, int WAVES>
@@ -1158,9 +1232,17 @@ long long separable_chunk(long long max_vis, int n)
     return (most + chunks - 1) / chunks * kStep;
 }
 
-hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, hipStream_t st)
+long long separable_few_visibilities()
 {
-    return precision == IDGX_MIXED_FP16X3 ? grid_size<kFP16>(a, sp, st) : grid_size<kBF16>(a, sp, st);
+    return kFewVisibilities;
+}
+
+hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &args, int precision, const GridCounts &n,
+                                 hipStream_t st)
+{
+    SeparableArgs sp = args;
+    sp.count = a.p.nr_subgrids;
+    return precision == IDGX_MIXED_FP16X3 ? grid_size<kFP16>(a, sp, n, st) : grid_size<kBF16>(a, sp, n, st);
 }
 
 hipError_t launch_degrid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, long long max_vis,
