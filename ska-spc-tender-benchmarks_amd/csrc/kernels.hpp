@@ -157,6 +157,7 @@ struct SeparableTables
 {
     float a[kSeparableMax / 2], g[kSeparableMax / 2];
     float eps, a_max;
+    float eps_grid, eps_degrid; // limits: subgrids beyond them are the per-pair kernels'
 };
 struct SeparableArgs
 {

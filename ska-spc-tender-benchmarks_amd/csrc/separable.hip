@@ -12,7 +12,7 @@
 // / 8 + ..., so the remainder is (l^2 - l0^2)(m^2 - l0^2) / 4 to first order: 3.5e-7 at a field of 0.1 rad).  So
 //     e^{2 pi i phase} = X(x) Y(y) (1 + i eps g(x) g(y)),   eps = 2 pi c d,
 //     X = e^{2 pi i (qu xh + d a(x))},  Y = e^{2 pi i (qv yh + d a(y))}
-// up to eps^2 / 2.  Subgrids with |eps| <= kEpsNone run without the product term; up to kEpsMost with it; the others
+// up to eps^2 / 2.  Subgrids with |eps| <= kEpsNone run without the product term; up to a limit (separable_tables) with it; the others
 // (fields far wider than 0.1 rad, or w far from constant over a subgrid) take the per-pair items.
 //
 // Contraction, on v_mfma_f32_32x32x16.  Gridder: pixel[y][x, corr] = sum_v Y[y][v] (V[v][corr] X[v][x]), one real GEMM
@@ -20,7 +20,7 @@
 // the product V X, which a lane forms in FP32 for one (x, corr) and four visibilities and splits into hi/lo halves: per
 // (pixel, visibility) pair 1/S of that work.  Three MFMAs per tile (hi hi, lo hi, hi lo; BF16 also lo lo) and one for the
 // product term, whose factor i eps g(y) goes into a second set of rows and g(x) into the columns, as single halves (eps
-// <= 1e-3 scales their rounding).  A wave owns all rows of NT column tiles (8 columns x 4 correlations each) and its own
+// scales their rounding).  A wave owns all rows of NT column tiles (8 columns x 4 correlations each) and its own
 // chunks of visibilities; no operand passes through LDS, and the waves only meet when their sums are added.
 // Degridder: H[x, corr][v] = sum_y P[y][x, corr] Y[y][v], the pixels split once per workgroup and read from LDS in the A
 // operand's order, then vis[v][corr] = sum_x X[x][v] H[x, corr][v] on the VALU: 16 FMAs per (column, visibility).
@@ -45,11 +45,19 @@ namespace
 // Below this the term is worth 0.27 of it at most in the root mean square, 2.7e-8 (at 3e-7 it was 8e-8, seen in subgrids
 // of 8 visibilities: 1.44e-7 from 64 bits against 1.60e-7; no case got slower by more than its runs differ).
 constexpr float kEpsNone = 1e-7F;
-constexpr float kEpsMost = 1e-3F; // eps^2 / 2 <= 5e-7 at one corner pixel for the visibility farthest in w
+// Largest eps, per pixel of the subgrid's side.  The term's operands are single halves, in the gridder an error of 4e-4 eps
+// for FP16 (2.8e-4 for kFewVisibilities), beside eps^2 / 2; the error of the per-pair kernels grows with the side, the
+// degridder's most (it rounds 24 bits of phase per pixel).  Distance from 64 bits over theirs at these limits, 48
+// subgrids with random uv: gridder 0.85 to 1.00, degridder 0.75 to 1.00; gridder on the subgrids with the largest eps of
+// 76,865 of 32^2 (1.8e-4) 0.70, of 20,780 of 48^2 (3.9e-4) 0.77, of 13,747 of 64^2 (2e-4) 0.83.  At 1e-3 for every size
+// it was 2.7 (16^2) to 1.1 (64^2).  BF16, whose 16 bits of each factor are 3.2e-6 off for every size, has one limit, where
+// the term's 8 bits add 1 % to that (at 1e-3 20 %).
+constexpr double kEpsGrid = 1e-5, kEpsDegrid = 2.5e-5;
+constexpr double kEpsMost = 1e-3, kEpsBF16 = 4e-4;
 constexpr float kTurnsMost = 4.F; // |d a|: keeps the phases' FP32 rounding at the level of qu xh
 constexpr float kTermScale = 1024.F; // moves the product term's factors into FP16's normal range
 // Plans take these kernels where a spread of w of S / image_size wavelengths (the subgrid's own extent in u and v)
-// stays within four times kEpsMost: fields up to about 0.17 rad at S = 32, 0.13 at S = 64.  In wider ones the per-pair
+// stays within 4e-3: fields up to about 0.17 rad at S = 32, 0.13 at S = 64.  In wider ones the per-pair
 // items would often run inside these kernels, at fewer waves per SIMD than in their own.
 constexpr double kSeparableField = 4e-3;
 // FP16 gridding of a subgrid of so few visibilities forms its phasors by their series and always takes the product term:
@@ -647,7 +655,7 @@ __global__ __launch_bounds__(64 * WAVES, (grid_waves<YT, NT>())) void grid_separ
     if (V > 0) // (without visibilities nothing reads the table)
         wr = w_range<WAVES, false>(a, row0, T, c0, nc, sm.slots, none);
     const float eps = wr.half * sp.tables.eps;
-    const bool fits = eps <= kEpsMost && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
+    const bool fits = eps <= sp.tables.eps_grid && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
     if (sp.leftover && tid == 0 && part == 0)
     {
         sp.leftover[s] = fits ? 0 : 1;
@@ -1032,7 +1040,7 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
     if constexpr (DT == kFP16)
         wr = w_range<WAVES, true>(a, row0, T, c0, nc, sm.slots, vmax);
     const float eps = wr.half * sp.tables.eps;
-    const bool fits = eps <= kEpsMost && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
+    const bool fits = eps <= sp.tables.eps_degrid && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
     if (sp.leftover && tid == 0 && chunk == 0)
     {
         sp.leftover[s] = fits ? 0 : 1;
@@ -1219,6 +1227,9 @@ bool separable_tables(const PlanDev &p, int precision, SeparableTables &t)
     }
     t.a_max = static_cast<float>(a_max);
     t.eps = static_cast<float>(2.0 * M_PI * c);
+    const bool fp16 = precision == IDGX_MIXED_FP16X3;
+    t.eps_grid = static_cast<float>(fp16 ? std::min(S * kEpsGrid, kEpsMost) : kEpsBF16);
+    t.eps_degrid = static_cast<float>(fp16 ? std::min(S * kEpsDegrid, kEpsMost) : kEpsBF16);
     return t.eps * (S / image) <= kSeparableField;
 }
 
