@@ -445,6 +445,7 @@ hipError_t run_separable(idgx_batch *b, QueueArgs &q, int k, bool gridder, hipSt
         return hipSuccess;
     idgx::SeparableArgs sp{};
     sp.tables = b->tables[k];
+    sp.limits = idgx::separable_limits(sp.tables, gridder);
     sp.order = b->d_order + b->order_offset[k];
     sp.leftover = b->d_order + (1 + dir) * b->order_total + b->order_offset[k];
     sp.leftover_any = b->d_counters + dir * kDirCounters + idgx::kMaxClasses * idgx::kQueues + k;

@@ -9,6 +9,13 @@
 namespace idgx
 {
 // Arguments shared by the gridder and degridder kernels, passed by value.
+// What decides whether the separable kernels take a subgrid: the largest eps (half the spread of w times eps), and the
+// largest a.  eps_most 0: no separable launch.
+struct SeparableLimits
+{
+    float eps, eps_most, a_max;
+};
+
 struct KernelArgs
 {
     PlanDev p;
@@ -38,6 +45,8 @@ struct KernelArgs
     // kernels, and whether they left any (null: every subgrid is the per-pair kernels').
     const int *leftover;
     const int *leftover_any;
+    // One-shot per-pair launches behind a separable one, which has done the subgrids within these limits.
+    SeparableLimits limits;
 };
 
 // Persistent-kernel work over up to kMaxClasses subgrid classes (one subgrid size each): the items are
@@ -164,7 +173,9 @@ struct SeparableArgs
     SeparableTables tables;
     const int *order;  // workgroup -> subgrid, most visibilities first (null: plan order)
     int count;         // gridder: subgrids of the launch
-    int *leftover;     // per subgrid: 1 where the per-pair kernels have to run (null: they run inside the launch)
+    SeparableLimits limits;
+    int *leftover;     // per subgrid: 1 where the per-pair kernels have to run (null: no marks)
+    bool leave;        // no marks: those subgrids are left to a launch that follows (false: they run inside this one)
     int *leftover_any; // set to 1 with the first of them
     long long per;     // degridder: visibilities per workgroup, a multiple of 256
 };
@@ -178,6 +189,9 @@ struct GridCounts
 long long separable_few_visibilities();
 // Whether the plan's subgrids take the separable kernels, and their tables.
 bool separable_tables(const PlanDev &p, int precision, SeparableTables &t);
+// The limits of one direction, and whether a one-shot call should expect subgrids beyond them.
+SeparableLimits separable_limits(const SeparableTables &t, bool gridder);
+bool separable_may_leave(const PlanDev &p, const SeparableLimits &l);
 // Degridder visibilities per workgroup (SeparableArgs::per) for n subgrids of at most max_vis visibilities.
 long long separable_chunk(long long max_vis, int n);
 hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, const GridCounts &n,

@@ -26,6 +26,7 @@ enum DType
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
+constexpr float kTurnsMost = 4.F; // separable kernels, |d a|: keeps the phases' FP32 rounding at the level of qu xh
 // Default tile shape: gridder 8 tiles of 16 pixels per wave with 256 visibilities per LDS batch, degridder 4 tiles
 // of 16 visibilities per wave with 256 pixels per LDS batch.
 constexpr int kDefaultPT = 8, kDefaultVB = 256, kDefaultVT = 4, kDefaultPB = 256;
@@ -323,6 +324,84 @@ __device__ __forceinline__ void degrid_pixel(const KernelArgs &a, const idgx_met
         apply_a1h_p_a2(px, a1, a2);
     else
         apply_a1_p_a2h(px, a1, a2);
+}
+
+struct WRange
+{
+    double centre; // middle of k w / 2 pi over the subgrid's rows and channels
+    float half;    // half its width
+};
+
+// Range of w (wavelengths) over a subgrid's rows and channel window, and the largest vmax: every thread of the workgroup
+// gets the same.  One LDS-only barrier, which also covers what the caller has written (loads stay in flight across it).
+template <int WAVES, bool MAX>
+__device__ __forceinline__ WRange w_range(const KernelArgs &a, long long row0, int T, int c0, int nc,
+                                          float (&slots)[WAVES][5], float &vmax)
+{
+    float wlo = __builtin_inff(), whi = -__builtin_inff(), klo = __builtin_inff(), khi = -__builtin_inff();
+    for (int t = threadIdx.x; t < T; t += 64 * WAVES)
+    {
+        const float w = a.uvw[3 * (row0 + t) + 2];
+        wlo = fminf(wlo, w);
+        whi = fmaxf(whi, w);
+    }
+    for (int c = threadIdx.x; c < nc; c += 64 * WAVES)
+    {
+        const float k = a.wavenumbers[c0 + c];
+        klo = fminf(klo, k);
+        khi = fmaxf(khi, k);
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1)
+    {
+        wlo = fminf(wlo, __shfl_xor(wlo, d));
+        whi = fmaxf(whi, __shfl_xor(whi, d));
+        klo = fminf(klo, __shfl_xor(klo, d));
+        khi = fmaxf(khi, __shfl_xor(khi, d));
+        if constexpr (MAX)
+            vmax = fmaxf(vmax, __shfl_xor(vmax, d));
+    }
+    if ((threadIdx.x & 63) == 0)
+    {
+        float *s = slots[threadIdx.x >> 6];
+        s[0] = wlo, s[1] = whi, s[2] = klo, s[3] = khi, s[4] = vmax;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+    {
+        wlo = fminf(wlo, slots[w][0]);
+        whi = fmaxf(whi, slots[w][1]);
+        klo = fminf(klo, slots[w][2]);
+        khi = fmaxf(khi, slots[w][3]);
+        if constexpr (MAX)
+            vmax = fmaxf(vmax, slots[w][4]);
+    }
+    const double p0 = static_cast<double>(wlo) * klo, p1 = static_cast<double>(wlo) * khi;
+    const double p2 = static_cast<double>(whi) * klo, p3 = static_cast<double>(whi) * khi;
+    const double lo = fmin(fmin(p0, p1), fmin(p2, p3)) * kInv2Pi, hi = fmax(fmax(p0, p1), fmax(p2, p3)) * kInv2Pi;
+    return {0.5 * (lo + hi), static_cast<float>(0.5 * (hi - lo))};
+}
+
+// Whether the separable kernels take a subgrid whose w spreads by `half` to both sides (false for NaN).
+__device__ __forceinline__ bool separable_fits(const SeparableLimits &l, float half)
+{
+    return half * l.eps <= l.eps_most && half * l.a_max <= kTurnsMost;
+}
+
+// Whether a one-shot workgroup has nothing to do: a separable launch before this one has done subgrid s, by the range of w
+// that it decides by, or the subgrid has no visibility `first`.  Uniform.
+__device__ __forceinline__ bool separable_done(const KernelArgs &a, int s, long long first, float (&slots)[kWaves][5])
+{
+    const idgx_metadata m = a.metadata[s];
+    int c0, nc;
+    channel_window(a, s, c0, nc);
+    const long long row0 = first_row(a.metadata, m);
+    Selection sel;
+    if (!subgrid_in_bounds(a.p, m, row0, c0, nc) || selection_of(a, s, m.nr_timesteps, nc, sel) <= first)
+        return true;
+    float none = 0.F;
+    return separable_fits(a.limits, w_range<kWaves, false>(a, row0, m.nr_timesteps, c0, nc, slots, none).half);
 }
 
 template <int PT, int VB> struct GridderShared

@@ -1,6 +1,6 @@
 // Mixed-precision gridder and degridder for gfx950, a phasor per (pixel, visibility) pair: FP64 phase-argument reduction,
 // FP32 phasors, and the phasor x data contraction on v_mfma_f32_16x16x32_{bf16,f16} with FP32 accumulation.  The
-// 3-product forms run the separable kernels (separable.hip) for subgrids up to 64^2 and fields up to about 0.17 rad, and
+// 3-product forms run the separable kernels (separable.hip) for subgrids up to 64^2 and fields up to 0.13 to 0.16 rad, and
 // these for the subgrids whose w spreads too far; larger subgrids, wider fields and the single-product forms run these.
 //
 // Phase reduction.  With l = (x' + 1/2) delta, x' = x - S/2 (an integer), delta = image_size / S, and
@@ -76,12 +76,41 @@ __global__ __launch_bounds__(kThreads, (gridder_min_blocks<PT, VB>())) void grid
     gridder_item<DT, SPLIT, PT, VB, PM>(a, blockIdx.x - pblk * a.p.nr_subgrids, pblk, sm);
 }
 
+// Behind a separable launch: the items of the subgrids that it left, over their workgroups.  (A kernel of its own: the
+// check costs the one above, a workgroup per item of which many have nothing to do, up to 1.7 times its time.)
+template <int DT, int PT, int VB>
+__global__ __launch_bounds__(kThreads, (gridder_min_blocks<PT, VB>())) void gridder_left(KernelArgs a, int items)
+{
+    __shared__ GridderShared<PT, VB> sm;
+    __shared__ float slots[kWaves][5];
+    const int part = blockIdx.x / a.p.nr_subgrids, s = blockIdx.x - part * a.p.nr_subgrids;
+    if (separable_done(a, s, 0, slots))
+        return; // uniform
+    for (int i = part; i < items; i += gridDim.x / a.p.nr_subgrids)
+    {
+        gridder_item<DT, true, PT, VB, false>(a, s, i, sm);
+        __syncthreads();
+    }
+}
+
 template <int DT, bool SPLIT, int VT, int PB, bool PM>
 __global__ __launch_bounds__(kThreads, (degridder_min_blocks<VT, PB>())) void degridder_mfma(KernelArgs a)
 {
     __shared__ DegridderShared<VT, PB> sm;
     const int vblk = blockIdx.x / a.p.nr_subgrids;
     degridder_item<DT, SPLIT, VT, PB, PM, false>(a, blockIdx.x - vblk * a.p.nr_subgrids, vblk, sm);
+}
+
+template <int DT, int VT, int PB>
+__global__ __launch_bounds__(kThreads, (degridder_min_blocks<VT, PB>())) void degridder_left(KernelArgs a, int items)
+{
+    __shared__ DegridderShared<VT, PB> sm;
+    __shared__ float slots[kWaves][5];
+    const int part = blockIdx.x / a.p.nr_subgrids, s = blockIdx.x - part * a.p.nr_subgrids;
+    if (separable_done(a, s, static_cast<long long>(part) * kWaves * VT * 16, slots))
+        return; // uniform
+    for (int i = part; i < items; i += gridDim.x / a.p.nr_subgrids)
+        degridder_item<DT, true, VT, PB, false, false>(a, s, i, sm);
 }
 
 template <int DT, bool SPLIT, int PT, int VB, bool PM>
@@ -310,13 +339,38 @@ int grid_tiles_for(int S)
     return best;
 }
 
+// Whether a one-shot launch runs behind a separable one.
+bool behind_separable(const KernelArgs &a)
+{
+    return a.limits.eps_most != 0.F;
+}
+
+// Workgroups per subgrid of a one-shot launch: one per item, but behind a separable launch, where most of them only find
+// that the subgrid is done, no more than fill the chip four times (8166 subgrids of 40^2, none left, both directions:
+// 80 us with one per item).
+long long oneshot_parts(const KernelArgs &a, long long items)
+{
+    constexpr long long kWorkgroups = 4096;
+    return behind_separable(a) ? std::min(items, std::max(1LL, kWorkgroups / a.p.nr_subgrids)) : items;
+}
+
 template <int DT, bool SPLIT, int PT, bool PM> hipError_t grid_mfma_tiles(const KernelArgs &a, hipStream_t st)
 {
     const GridUnits gu = grid_units(a.p.S, PT);
-    const long long blocks = static_cast<long long>(a.p.nr_subgrids) * ((gu.units + kWaves - 1) / kWaves);
+    const int items = (gu.units + kWaves - 1) / kWaves;
+    const long long blocks = a.p.nr_subgrids * oneshot_parts(a, items);
     if (blocks > 0x7fffffffLL)
         return hipErrorInvalidConfiguration;
-    gridder_mfma<DT, SPLIT, PT, kDefaultVB, PM><<<static_cast<unsigned>(blocks), kThreads, 0, st>>>(a);
+    const unsigned n = static_cast<unsigned>(blocks);
+    if constexpr (SPLIT && !PM)
+    {
+        if (behind_separable(a))
+        {
+            gridder_left<DT, PT, kDefaultVB><<<n, kThreads, 0, st>>>(a, items);
+            return hipGetLastError();
+        }
+    }
+    gridder_mfma<DT, SPLIT, PT, kDefaultVB, PM><<<n, kThreads, 0, st>>>(a);
     return hipGetLastError();
 }
 
@@ -344,13 +398,22 @@ template <int DT, bool SPLIT> hipError_t degrid_mfma(const KernelArgs &a, bool p
     constexpr int chunk = kWaves * kDefaultVT * 16;
     const long long vmax = static_cast<long long>(a.p.max_nr_timesteps) * a.p.nr_channels;
     const long long per = vmax > 0 ? (vmax + chunk - 1) / chunk : 1;
-    const long long blocks = static_cast<long long>(a.p.nr_subgrids) * per;
+    const long long blocks = a.p.nr_subgrids * oneshot_parts(a, per);
     if (blocks > 0x7fffffffLL)
         return hipErrorInvalidConfiguration;
+    const unsigned n = static_cast<unsigned>(blocks);
+    if constexpr (SPLIT)
+    {
+        if (behind_separable(a))
+        {
+            degridder_left<DT, kDefaultVT, kDefaultPB><<<n, kThreads, 0, st>>>(a, static_cast<int>(per));
+            return hipGetLastError();
+        }
+    }
     if (pm)
-        degridder_mfma<DT, SPLIT, kDefaultVT, kDefaultPB, true><<<static_cast<unsigned>(blocks), kThreads, 0, st>>>(a);
+        degridder_mfma<DT, SPLIT, kDefaultVT, kDefaultPB, true><<<n, kThreads, 0, st>>>(a);
     else
-        degridder_mfma<DT, SPLIT, kDefaultVT, kDefaultPB, false><<<static_cast<unsigned>(blocks), kThreads, 0, st>>>(a);
+        degridder_mfma<DT, SPLIT, kDefaultVT, kDefaultPB, false><<<n, kThreads, 0, st>>>(a);
     return hipGetLastError();
 }
 
@@ -447,12 +510,24 @@ hipError_t launch_queue(const QueueArgs &q, int precision, bool gridder, int sha
 }
 } // namespace
 
-hipError_t launch_grid_mixed(const KernelArgs &a, int precision, bool pm, hipStream_t st)
+// One-shot plans of the separable kernels: where the plan lets expect subgrids that they leave, a launch of the per-pair
+// kernels behind them, whose workgroups end at once for the others.  All subgrids of 256 visibilities left, per-pair
+// kernels alone / with their items inside the separable launch / behind it: gridder 40 of 64^2 33 / 151 / 39 us, 6000 of
+// 32^2 577 / 658 / 627 us; degridder 6000 of 64^2 2164 / 3786 / 2443 us.
+hipError_t launch_grid_mixed(const KernelArgs &args, int precision, bool pm, hipStream_t st)
 {
+    KernelArgs a = args;
     SeparableArgs sp{};
     if (!pm && separable_tables(a.p, precision, sp.tables))
-        return launch_grid_separable(a, sp, precision,
-                                     {static_cast<long long>(a.p.max_nr_timesteps) * a.p.nr_channels, 0}, st);
+    {
+        sp.limits = separable_limits(sp.tables, true);
+        sp.leave = separable_may_leave(a.p, sp.limits);
+        const hipError_t e = launch_grid_separable(
+            a, sp, precision, {static_cast<long long>(a.p.max_nr_timesteps) * a.p.nr_channels, 0}, st);
+        if (e != hipSuccess || !sp.leave)
+            return e;
+        a.limits = sp.limits;
+    }
     switch (precision)
     {
     case IDGX_MIXED_BF16X3:
@@ -468,14 +543,20 @@ hipError_t launch_grid_mixed(const KernelArgs &a, int precision, bool pm, hipStr
     }
 }
 
-hipError_t launch_degrid_mixed(const KernelArgs &a, int precision, bool pm, hipStream_t st)
+hipError_t launch_degrid_mixed(const KernelArgs &args, int precision, bool pm, hipStream_t st)
 {
+    KernelArgs a = args;
     SeparableArgs sp{};
     if (!pm && separable_tables(a.p, precision, sp.tables))
     {
         const long long vmax = static_cast<long long>(a.p.max_nr_timesteps) * a.p.nr_channels;
+        sp.limits = separable_limits(sp.tables, false);
+        sp.leave = separable_may_leave(a.p, sp.limits);
         sp.per = separable_chunk(vmax, a.p.nr_subgrids);
-        return launch_degrid_separable(a, sp, precision, vmax, st);
+        const hipError_t e = launch_degrid_separable(a, sp, precision, vmax, st);
+        if (e != hipSuccess || !sp.leave)
+            return e;
+        a.limits = sp.limits;
     }
     switch (precision)
     {

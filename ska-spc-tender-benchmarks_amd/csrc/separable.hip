@@ -54,12 +54,15 @@ constexpr float kEpsNone = 1e-7F;
 // the term's 8 bits add 1 % to that (at 1e-3 20 %).
 constexpr double kEpsGrid = 1e-5, kEpsDegrid = 2.5e-5;
 constexpr double kEpsMost = 1e-3, kEpsBF16 = 4e-4;
-constexpr float kTurnsMost = 4.F; // |d a|: keeps the phases' FP32 rounding at the level of qu xh
 constexpr float kTermScale = 1024.F; // moves the product term's factors into FP16's normal range
-// Plans take these kernels where a spread of w of S / image_size wavelengths (the subgrid's own extent in u and v)
-// stays within 4e-3: fields up to about 0.17 rad at S = 32, 0.13 at S = 64.  In wider ones the per-pair
-// items would often run inside these kernels, at fewer waves per SIMD than in their own.
-constexpr double kSeparableField = 4e-3;
+// Plans take these kernels where a half spread of w of S / image_size wavelengths (the subgrid's own extent in u and v)
+// is worth at most so many times S kEpsGrid: fields up to 0.166 and 0.131 rad.  Observations spread w by 0.1 to 0.4 of that.
+// Times over those of the per-pair kernels, gridder and degridder (2016 baselines, 32^2 and 64^2 subgrids; 780, 16^2), with
+// the share of subgrids left to them: 32^2 at 0.13 rad 0.47 (5 %) and 0.37, at 0.16 0.68 (59 %) and 0.42; 64^2 at 0.16 0.48
+// (19 %) and 0.39 (4 %); 24^2 at 0.16 0.81 (70 %) and 0.53 (5 %); 16^2 at 0.13 0.74 (48 %) and 0.40, but in batches at
+// 0.14 0.89 (68 %) and 1.07 (3 %: the queue's walk over all items outweighs the small subgrids).
+constexpr double kFieldMost = 10.0, kFieldMostSmall = 5.0;
+constexpr int kFieldSmall = 24; // the latter below this subgrid size
 // FP16 gridding of a subgrid of so few visibilities forms its phasors by their series and always takes the product term:
 // over few visibilities the errors of v_sin and v_cos, here of two phasors a pair instead of one, do not average out.
 // Distance from 64 bits over that of the per-pair kernels, worst of S = 16 .. 48, with v_sin and v_cos / by the series:
@@ -108,63 +111,6 @@ template <int WAVES> size_t degrid_lds_bytes(int S, int rows)
     const size_t cols = static_cast<size_t>((S + 7) / 8) * 8;
     return std::max(offsetof(DegridLds<WAVES>, pixels) + rows * cols * 4 * 2 * sizeof(uint32_t),
                     sizeof(DegridderShared<kDefaultVT, kDefaultPB>));
-}
-
-struct WRange
-{
-    double centre; // middle of k w / 2 pi over the subgrid's rows and channels
-    float half;    // half its width
-};
-
-// Range of w (wavelengths) over a subgrid's rows and channel window, and the largest vmax: every thread of the workgroup
-// gets the same.  One LDS-only barrier, which also covers what the caller has written (loads stay in flight across it).
-template <int WAVES, bool MAX>
-__device__ __forceinline__ WRange w_range(const KernelArgs &a, long long row0, int T, int c0, int nc,
-                                          float (&slots)[WAVES][5], float &vmax)
-{
-    float wlo = __builtin_inff(), whi = -__builtin_inff(), klo = __builtin_inff(), khi = -__builtin_inff();
-    for (int t = threadIdx.x; t < T; t += 64 * WAVES)
-    {
-        const float w = a.uvw[3 * (row0 + t) + 2];
-        wlo = fminf(wlo, w);
-        whi = fmaxf(whi, w);
-    }
-    for (int c = threadIdx.x; c < nc; c += 64 * WAVES)
-    {
-        const float k = a.wavenumbers[c0 + c];
-        klo = fminf(klo, k);
-        khi = fmaxf(khi, k);
-    }
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1)
-    {
-        wlo = fminf(wlo, __shfl_xor(wlo, d));
-        whi = fmaxf(whi, __shfl_xor(whi, d));
-        klo = fminf(klo, __shfl_xor(klo, d));
-        khi = fmaxf(khi, __shfl_xor(khi, d));
-        if constexpr (MAX)
-            vmax = fmaxf(vmax, __shfl_xor(vmax, d));
-    }
-    if ((threadIdx.x & 63) == 0)
-    {
-        float *s = slots[threadIdx.x >> 6];
-        s[0] = wlo, s[1] = whi, s[2] = klo, s[3] = khi, s[4] = vmax;
-    }
-    lds_barrier();
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w)
-    {
-        wlo = fminf(wlo, slots[w][0]);
-        whi = fmaxf(whi, slots[w][1]);
-        klo = fminf(klo, slots[w][2]);
-        khi = fmaxf(khi, slots[w][3]);
-        if constexpr (MAX)
-            vmax = fmaxf(vmax, slots[w][4]);
-    }
-    const double p0 = static_cast<double>(wlo) * klo, p1 = static_cast<double>(wlo) * khi;
-    const double p2 = static_cast<double>(whi) * klo, p3 = static_cast<double>(whi) * khi;
-    const double lo = fmin(fmin(p0, p1), fmin(p2, p3)) * kInv2Pi, hi = fmax(fmax(p0, p1), fmax(p2, p3)) * kInv2Pi;
-    return {0.5 * (lo + hi), static_cast<float>(0.5 * (hi - lo))};
 }
 
 // q / cols for q < 4096 and cols <= 64 (q (cols - 1) < 2^20): two instructions instead of a division.
@@ -655,7 +601,7 @@ __global__ __launch_bounds__(64 * WAVES, (grid_waves<YT, NT>())) void grid_separ
     if (V > 0) // (without visibilities nothing reads the table)
         wr = w_range<WAVES, false>(a, row0, T, c0, nc, sm.slots, none);
     const float eps = wr.half * sp.tables.eps;
-    const bool fits = eps <= sp.tables.eps_grid && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
+    const bool fits = separable_fits(sp.limits, wr.half);
     if (sp.leftover && tid == 0 && part == 0)
     {
         sp.leftover[s] = fits ? 0 : 1;
@@ -664,10 +610,11 @@ __global__ __launch_bounds__(64 * WAVES, (grid_waves<YT, NT>())) void grid_separ
     }
     if (!fits)
     {
-        if (!sp.leftover && part == 0 && tid < kThreads) // waves that have ended do not take part in the others' barriers
+        if (!sp.leftover && !sp.leave && tid < kThreads) // waves that have ended are not waited for at barriers
         {
+            // The subgrid's per-pair items over its workgroups.
             const int items = (grid_units(S, kDefaultPT).units + kWaves - 1) / kWaves;
-            for (int i = 0; i < items; ++i)
+            for (int i = part; i < items; i += gridDim.x / sp.count)
             {
                 gridder_item<DT, true, kDefaultPT, kDefaultVB, false>(a, s, i, sm.direct);
                 __syncthreads();
@@ -1040,7 +987,7 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
     if constexpr (DT == kFP16)
         wr = w_range<WAVES, true>(a, row0, T, c0, nc, sm.slots, vmax);
     const float eps = wr.half * sp.tables.eps;
-    const bool fits = eps <= sp.tables.eps_degrid && wr.half * sp.tables.a_max <= kTurnsMost; // false for NaN
+    const bool fits = separable_fits(sp.limits, wr.half);
     if (sp.leftover && tid == 0 && chunk == 0)
     {
         sp.leftover[s] = fits ? 0 : 1;
@@ -1049,7 +996,7 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
     }
     if (!fits)
     {
-        if (sp.leftover || tid >= kThreads) // waves that have ended do not take part in the others' barriers
+        if (sp.leftover || sp.leave || tid >= kThreads) // waves that have ended are not waited for at barriers
             return;
         constexpr int per = kWaves * kDefaultVT * 16;
         auto &direct = *reinterpret_cast<DegridderShared<kDefaultVT, kDefaultPB> *>(lds);
@@ -1230,7 +1177,7 @@ bool separable_tables(const PlanDev &p, int precision, SeparableTables &t)
     const bool fp16 = precision == IDGX_MIXED_FP16X3;
     t.eps_grid = static_cast<float>(fp16 ? std::min(S * kEpsGrid, kEpsMost) : kEpsBF16);
     t.eps_degrid = static_cast<float>(fp16 ? std::min(S * kEpsDegrid, kEpsMost) : kEpsBF16);
-    return t.eps * (S / image) <= kSeparableField;
+    return t.eps * (S / image) <= (S < kFieldSmall ? kFieldMostSmall : kFieldMost) * (S * kEpsGrid);
 }
 
 // A whole subgrid per workgroup (its pixels are prepared once) unless that leaves CUs without work: then as many
@@ -1241,6 +1188,18 @@ long long separable_chunk(long long max_vis, int n)
     const long long most = std::max(1LL, (max_vis + kStep - 1) / kStep);
     const long long chunks = std::min(most, std::max(1LL, kWorkgroups / std::max(1, n)));
     return (most + chunks - 1) / chunks * kStep;
+}
+
+SeparableLimits separable_limits(const SeparableTables &t, bool gridder)
+{
+    return {t.eps, gridder ? t.eps_grid : t.eps_degrid, t.a_max};
+}
+
+// Where a half spread of S / image_size wavelengths lies beyond the limit.  Below that the call has one launch, and a
+// subgrid that is left all the same runs its items there, several times slower where it has the chip to itself.
+bool separable_may_leave(const PlanDev &p, const SeparableLimits &l)
+{
+    return l.eps * p.S / p.image_size > l.eps_most;
 }
 
 long long separable_few_visibilities()

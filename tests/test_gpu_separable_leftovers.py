@@ -1,0 +1,114 @@
+"""Subgrids that the separable kernels leave to the per-pair ones, because their w spreads too far, on every route of the
+latter: inside a one-shot launch, behind it, in a batch's launch per class and in its merged launch, with every compiled
+tile shape, with each class's own tiles, and in a captured graph.
+
+Every workload holds subgrids of both kinds; that is asserted on the host from w and the product term's limits.
+
+Bars: an FP32 phase of up to 16 turns per axis is off by at most 2 x 4.8e-7 turns and the sine and cosine by 1.1e-7, 7e-6
+rad together; the FP16 halves add 2^-21, so 1e-5 for fp16x3.  The BF16 halves hold 16 bits of each factor: 2^-16 each on
+top, so 4e-5."""
+import numpy as np
+import pytest
+
+from helpers import oracle_degrid, oracle_grid, rel_l2
+from idgx import CHANNELS_DTYPE, METADATA_DTYPE, observation
+from idgx.device import DeviceWorkload, upload
+from test_gpu_separable import corner_remainder
+
+pytestmark = pytest.mark.gpu
+
+BAR = {"fp16x3": 1e-5, "bf16x3": 4e-5}
+PAST = 4e-3  # eps of the subgrids to be left: past every limit (1e-5 S, 2.5e-5 S, 1e-3, 4e-4)
+WITHIN = 5e-5
+
+
+def make(S, counts, left, image, C=9, seed=0, K=4, first_row=0):
+    """Subgrids of counts[i] timesteps x a channel window each; w of those in `left` spreads to an eps of PAST, of the
+    others to one of WITHIN."""
+    rng = np.random.default_rng(seed)
+    n, G = len(counts), 2048
+    md, ch = np.zeros(n, METADATA_DTYPE), np.zeros(n, CHANNELS_DTYPE)
+    k = np.linspace(3.39, 3.4, C).astype(np.float32)
+    rows = int(sum(counts))
+    uvw = np.zeros((rows, 3), np.float32)
+    r = 0
+    for i, T in enumerate(counts):
+        md[i] = (0, first_row + r, T, 0, i % K, (i + 1) % K, *rng.integers(0, G - S, 2), 0)
+        c0 = int(rng.integers(0, C - 1))
+        ch[i] = (c0, int(rng.integers(1, C - c0 + 1)))
+        centre = (np.array([md["x"][i], md["y"][i]]) + S / 2 - G / 2) / image
+        half = max(1, S // 2 - 4) / image
+        kc = float(k[c0]) / (2 * np.pi)
+        uvw[r:r + T, :2] = (centre + rng.uniform(-half, half, (T, 2))) / kc
+        spread = (PAST if i in left else WITHIN) / (2 * np.pi * corner_remainder(S, image))
+        w = rng.uniform(-spread, spread, T)
+        w[0], w[-1] = -spread, spread
+        uvw[r:r + T, 2] = w / kc
+        r += T
+    return dict(uvw=uvw, wavenumbers=k, metadata=md, channels=ch, nr_subgrids=n, subgrid_size=S, grid_size=G,
+                spheroidal=observation.prolate_spheroidal_taper(S), aterms=observation.jones_aterms(rng, 1, K, S),
+                nr_stations=K, nr_aterm_slots=1, nr_rows=rows, image_size=np.float32(image), w_step=0.0,
+                max_nr_timesteps=int(max(counts)), visibilities=observation.random_visibilities(rows, C, seed))
+
+
+def largest_eps(w, first_row=0):
+    """eps of every subgrid: the product term's phase at the corner for half its spread of w."""
+    md, ch, k = w["metadata"], w["channels"], w["wavenumbers"].astype(np.float64) / (2 * np.pi)
+    c = corner_remainder(w["subgrid_size"], float(w["image_size"]))
+    out = []
+    for s in range(md.size):
+        r, c0 = int(md["time_offset"][s]) - first_row, int(ch["channel_begin"][s])
+        x = w["uvw"][r:r + int(md["nr_timesteps"][s]), 2].astype(np.float64)
+        p = np.outer([x.min(), x.max()], [k[c0], k[c0 + int(ch["nr_channels"][s]) - 1]])
+        out.append(np.pi * (p.max() - p.min()) * c)
+    return np.array(out)
+
+
+def assert_both_kinds(w, left, first_row=0):
+    eps = largest_eps(w, first_row)
+    rest = [s for s in range(w["nr_subgrids"]) if s not in left]
+    # Limits of a size: the gridder's 1e-5 S and 4e-4, the degridder's 1e-3 at most.
+    assert left and (eps[list(left)] > 1e-3).all() and rest and (eps[rest] < 8e-5).all()
+
+
+def model(w, seed=5):
+    rng = np.random.default_rng(seed)
+    S, n = w["subgrid_size"], w["nr_subgrids"]
+    return (rng.standard_normal((n, 4, S, S)) + 1j * rng.standard_normal((n, 4, S, S))).astype(np.complex64)
+
+
+def check(w, form, sub, grids, vis, first_row=0):
+    """Every subgrid and its visibilities against FP64 (vis: the rows from first_row on)."""
+    w = dict(w, metadata=w["metadata"].copy())
+    w["metadata"]["time_offset"] -= first_row
+    g64, v64 = oracle_grid(w, fp64=True), oracle_degrid(w, sub, fp64=True)
+    md, ch = w["metadata"], w["channels"]
+    worst = [0.0, 0.0]
+    for s in range(md.size):
+        r, c = int(md["time_offset"][s]), int(ch["channel_begin"][s])
+        at = slice(r, r + int(md["nr_timesteps"][s])), slice(c, c + int(ch["nr_channels"][s]))
+        worst[0] = max(worst[0], rel_l2(grids[s], g64[s]))
+        worst[1] = max(worst[1], rel_l2(vis[at], v64[at]))
+    print(f"S={w['subgrid_size']} {form}: gridder worst {worst[0]:.2e}, degridder worst {worst[1]:.2e}")
+    assert worst[0] <= BAR[form] and worst[1] <= BAR[form]
+
+
+@pytest.mark.parametrize("form", ["fp16x3", "bf16x3"])
+@pytest.mark.parametrize("S, image", [(16, 0.05), (16, 0.12), (24, 0.1), (32, 0.06), (32, 0.16), (40, 0.1), (64, 0.06),
+                                      (64, 0.12)])
+@pytest.mark.parametrize("n", [6, 262])
+def test_one_shot(S, image, n, form):
+    """Fields whose one-shot calls take one launch (0.05, 0.06) and two; workgroups of 8 columns and of whole subgrids;
+    subgrids of few and many visibilities of both kinds."""
+    rng = np.random.default_rng(S + n)
+    counts = [int(t) for t in rng.integers(2, 40, n)]
+    left = set(range(1, n, 3))
+    w = make(S, counts, left, image, seed=S)
+    assert_both_kinds(w, left)
+    sub = model(w)
+    d = DeviceWorkload(w)
+    plan = d.plan(precision=form)
+    d.grid(plan)
+    got = d.subgrids()
+    d.degrid(plan, d_subgrids=upload(sub))
+    check(w, form, sub, got, d.visibilities_out())
