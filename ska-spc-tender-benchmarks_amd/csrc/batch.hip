@@ -816,16 +816,39 @@ extern "C" int idgx_batch_autotune(idgx_batch *b, const idgx_batch_data *data, i
         ms /= repeats;
         return e;
     };
+    // Which classes have work for the persistent launch (the shapes are its tiles): a class of the separable kernels only
+    // where they leave subgrids.
+    const auto find_busy = [&](int dir, bool(&busy)[idgx::kMaxClasses]) {
+        int any[idgx::kMaxClasses] = {};
+        int e = run(b, data, dir == 0, st);
+        if (e == IDGX_OK && (hipStreamSynchronize(st) != hipSuccess ||
+                             hipMemcpy(any, b->d_counters + dir * kDirCounters + idgx::kMaxClasses * idgx::kQueues,
+                                       sizeof(any), hipMemcpyDeviceToHost) != hipSuccess))
+            e = IDGX_ERR_DEVICE;
+        for (int k = 0; k < b->nr_classes; ++k)
+            busy[k] = b->nr_items[dir][k] > 0 && (!b->separable[k] || any[k] != 0);
+        return e;
+    };
     float total[2] = {0.F, 0.F};
     // Each class is tuned on its own launch: the launches of a direction run one after another.
     for (int dir = 0; dir < 2 && rc == IDGX_OK; ++dir)
     {
         const bool gridder = dir == 0;
+        bool busy[idgx::kMaxClasses] = {};
+        rc = find_busy(dir, busy);
+        const bool any_busy = std::find(busy, busy + b->nr_classes, true) != busy + b->nr_classes;
         const bool offer_single = single_mode(b, dir);
         for (int k = 0; k < b->nr_classes && rc == IDGX_OK; ++k)
         {
             float best = -1.F;
             int best_shape = b->shape[dir][k];
+            if (!busy[k]) // its shape stays
+            {
+                float ms = 0.F;
+                rc = timed(gridder, k, ms);
+                total[dir] += ms;
+                continue;
+            }
             for (int sh = 0; sh < shape_count(b) && rc == IDGX_OK; ++sh)
             {
                 // One roctx range per trial, for rocprofv3 --marker-trace.
@@ -855,6 +878,11 @@ extern "C" int idgx_batch_autotune(idgx_batch *b, const idgx_batch_data *data, i
         // fastest of them is kept, which may leave the direction in per-class mode.
         float best = -1.F;
         int best_shape = -1;
+        if (!any_busy)
+        {
+            rc = timed(gridder, -1, total[dir]);
+            continue;
+        }
         static_assert(idgx::kShapeTilesPerClass == -2, "the trials below run -2 (tiles per class), -1, 0, 1, ...");
         for (int sh = gridder ? idgx::kShapeTilesPerClass : -1; sh < shape_count(b) && rc == IDGX_OK; ++sh)
         {

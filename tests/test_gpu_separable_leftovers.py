@@ -112,3 +112,80 @@ def test_one_shot(S, image, n, form):
     got = d.subgrids()
     d.degrid(plan, d_subgrids=upload(sub))
     check(w, form, sub, got, d.visibilities_out())
+
+
+# ---- batches of three classes over one set of rows -----------------------------------------------------------------
+
+SIZES = (24, 32, 48)
+
+
+def make_classes(lefts, seed=0):
+    """Classes of SIZES, lefts[k] the subgrids to be left in class k; every class carries the shared rows."""
+    classes, first = [], 0
+    rng = np.random.default_rng(seed)
+    for k, S in enumerate(SIZES):
+        w = make(S, [int(t) for t in rng.integers(2, 60, 12)], lefts[k], 0.1, seed=seed + k, first_row=first)
+        if lefts[k]:
+            assert_both_kinds(w, lefts[k], first)
+        else:
+            assert (largest_eps(w, first) < 8e-5).all()
+        classes.append(dict(w, first_row=first, own_rows=w["nr_rows"]))
+        first += w["nr_rows"]
+    uvw = np.concatenate([w["uvw"] for w in classes])
+    vis = np.concatenate([w["visibilities"] for w in classes])
+    for w in classes:
+        w["own_uvw"], w["own_vis"] = w["uvw"], w["visibilities"]
+        w.update(uvw=uvw, visibilities=vis, nr_rows=first)
+    return classes
+
+
+def own(w):
+    """A class with its own rows only, for the oracle."""
+    return dict(w, uvw=w["own_uvw"], visibilities=w["own_vis"], nr_rows=w["own_rows"])
+
+
+def three_classes(form, lefts=({1, 4, 7}, {0, 2, 9, 11}, {3, 5})):
+    from idgx import Batch
+    from idgx.device import DeviceBatch
+
+    classes = make_classes(lefts)
+    d = DeviceBatch(classes, precision=form)
+    models = [model(w, seed=k) for k, w in enumerate(classes)]
+    # The model subgrids are buffers of their own: the gridder writes the classes'.
+    d.models = [upload(m) for m in models]
+    d.predict = Batch.data(d.d_uvw, d.d_wavenumbers, d.d_visibilities, d.d_vis_out,
+                           [dict(c, d_subgrids=m) for c, m in zip(d.classes, d.models)])
+    return d, classes, models
+
+
+def run(d):
+    for c in d.classes:
+        c["d_subgrids"].zero_()
+    d.d_vis_out.zero_()
+    d.grid()
+    d.batch.degrid(d.predict)
+    return [d.subgrids(k) for k in range(len(d.classes))], d.visibilities_out()
+
+
+def check_classes(classes, models, form, grids, vis):
+    for k, w in enumerate(classes):
+        rows = slice(w["first_row"], w["first_row"] + w["own_rows"])
+        check(own(w), form, models[k], grids[k], vis[rows], w["first_row"])
+
+
+def test_autotuner_leaves_the_shapes_of_classes_without_leftovers():
+    """Their persistent launch finds no work, so its time says nothing about a shape."""
+    for lefts, kept in ((({1, 4}, set(), {3}), (1,)), ((set(), set(), set()), (0, 1, 2))):
+        d, classes, models = three_classes("fp16x3", lefts)
+        shape = len(d.batch.shapes()) - 3
+        d.batch.set_single_launch(-1, -1)
+        d.batch.set_shape(shape, shape)
+        tg, td = d.batch.autotune(d.data, repeats=1)
+        assert tg > 0 and td > 0 and d.batch.single_launch() == (-1, -1)
+        for k in kept:
+            assert d.batch.class_shape(k) == (shape, shape)
+        if len(kept) == 3:
+            d.batch.set_single_launch(shape, shape)
+            tg, td = d.batch.autotune(d.data, repeats=1)
+            assert tg > 0 and td > 0 and d.batch.single_launch() == (shape, shape)
+        check_classes(classes, models, "fp16x3", *run(d))
