@@ -189,3 +189,93 @@ def test_autotuner_leaves_the_shapes_of_classes_without_leftovers():
             tg, td = d.batch.autotune(d.data, repeats=1)
             assert tg > 0 and td > 0 and d.batch.single_launch() == (shape, shape)
         check_classes(classes, models, "fp16x3", *run(d))
+
+
+def assert_same_bits(a, b):
+    assert all(x.tobytes() == y.tobytes() for x, y in zip(a[0], b[0])) and a[1].tobytes() == b[1].tobytes()
+
+
+@pytest.mark.parametrize("form", ["fp16x3", "bf16x3"])
+def test_every_tile_shape_per_class_and_merged(form):
+    """Each compiled shape as a launch per class and as the merged launch, whose items write the same bits."""
+    d, classes, models = three_classes(form)
+    for shape in range(len(d.batch.shapes())):
+        d.batch.set_single_launch(-1, -1)
+        d.batch.set_shape(shape, shape)
+        per_class = run(d)
+        assert d.batch.last_launches() == (3, 3)
+        check_classes(classes, models, form, *per_class)
+        d.batch.set_single_launch(shape, shape)
+        merged = run(d)
+        assert d.batch.last_launches() == (1, 1)
+        assert_same_bits(per_class, merged)
+
+
+@pytest.mark.parametrize("form", ["fp16x3", "bf16x3"])
+def test_tiles_per_class(form):
+    """Every compiled count of tiles per wave for each class in turn, merged with each class's own against launches per
+    class."""
+    from idgx import SHAPE_TILES_PER_CLASS
+
+    d, classes, models = three_classes(form)
+    shapes = d.batch.shapes()
+    tiles = [shapes.index((t, 256, 0)) for t in (2, 3, 4, 6, 8)]
+    degrid = shapes.index((4, 256, 0))
+    for i in range(len(tiles)):
+        for k in range(3):
+            d.batch.set_class_shape(k, tiles[(i + k) % len(tiles)], degrid)
+        d.batch.set_single_launch(-1, -1)
+        per_class = run(d)
+        d.batch.set_single_launch(SHAPE_TILES_PER_CLASS, degrid)
+        merged = run(d)
+        assert_same_bits(per_class, merged)
+        check_classes(classes, models, form, *merged)
+
+
+@pytest.mark.parametrize("merged", [False, True])
+@pytest.mark.parametrize("lefts", [({1, 4, 7}, {0, 2, 9, 11}, {3, 5}), (set(), {0, 2, 9, 11}, set())])
+def test_graph_replays(lefts, merged):
+    """Capture with leftovers in every class and in one; replays on fresh outputs, with eager work between them."""
+    import torch
+
+    from idgx import SHAPE_TILES_PER_CLASS, STAGE_DEGRID, STAGE_GRID
+
+    d, classes, models = three_classes("fp16x3", lefts)
+    if merged:
+        d.batch.set_single_launch(SHAPE_TILES_PER_CLASS, d.batch.shapes().index((4, 256, 0)))
+    else:
+        d.batch.set_single_launch(-1, -1)
+    eager = run(d)
+    check_classes(classes, models, "fp16x3", *eager)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    for stage, data, read in ((STAGE_GRID, d.data, lambda: [d.subgrids(k) for k in range(3)]),
+                              (STAGE_DEGRID, d.predict, d.visibilities_out)):
+        d.batch.capture(data, stage, stream)
+        for r in range(3):
+            for c in d.classes:
+                c["d_subgrids"].zero_()
+            d.d_vis_out.zero_()
+            torch.cuda.synchronize()
+            d.batch.launch(stream)
+            stream.synchronize()
+            got = read()
+            if stage == STAGE_GRID:
+                assert all(x.tobytes() == y.tobytes() for x, y in zip(got, eager[0])), f"replay {r}"
+            else:
+                assert got.tobytes() == eager[1].tobytes(), f"replay {r}"
+            assert float(torch.ones(1000, device="cuda").sum()) == 1000.0
+
+
+def test_leftovers_come_and_go_with_the_data():
+    """The same batch on data with other leftovers: nothing of the previous pass's marks remains."""
+    d, classes, models = three_classes("fp16x3")
+    first = run(d)
+    calm = [dict(c) for c in make_classes((set(), {2}, set()), seed=0)]
+    # Same counts, windows and rows: only uvw changes.
+    assert all((a["metadata"] == b["metadata"]).all() for a, b in zip(calm, classes))
+    keep = d.d_uvw.clone()
+    d.d_uvw.copy_(upload(calm[0]["uvw"]))
+    check_classes([dict(c, own_vis=w["own_vis"]) for c, w in zip(calm, classes)], models, "fp16x3", *run(d))
+    d.d_uvw.copy_(keep)
+    assert_same_bits(first, run(d))
