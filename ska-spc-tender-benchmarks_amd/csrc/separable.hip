@@ -996,7 +996,10 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
     }
     if (!fits)
     {
-        if (sp.leftover || sp.leave || tid >= kThreads) // waves that have ended are not waited for at barriers
+        if (sp.leftover || sp.leave)
+            return;
+        __syncthreads(); // the item's staging overlies the table and the slots, which other waves may still read
+        if (tid >= kThreads) // waves that have ended are not waited for at barriers
             return;
         constexpr int per = kWaves * kDefaultVT * 16;
         auto &direct = *reinterpret_cast<DegridderShared<kDefaultVT, kDefaultPB> *>(lds);
