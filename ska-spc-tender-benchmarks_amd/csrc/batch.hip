@@ -170,27 +170,36 @@ int class_tiles(const idgx_batch *b, int shape)
     return plain(b) ? plain_work(b, true, shape) : idgx::mixed_shape(shape).tiles;
 }
 
-// What a plain launch of `shape` (or of every class's own) asks the kernels for.
-int plain_launch(const idgx_batch *b, bool gridder, int shape)
+// The kernel of a plain launch of `shape` (or of every class's own) over class `cls`, or all of them (-1).
+idgx::PlainKernel plain_kernel(const idgx_batch *b, bool gridder, int shape, int cls)
 {
-    return shape == idgx::kShapeTilesPerClass ? shape : plain_work(b, gridder, shape);
+    idgx::PlainKernel p{accurate_sincos(b), gridder, true,
+                        shape == idgx::kShapeTilesPerClass ? shape : plain_work(b, gridder, shape)};
+    for (int k = 0; k < b->nr_classes && p.work > 0; ++k)
+        if (cls < 0 || k == cls)
+        {
+            const int S = b->plans[k].subgrid_size;
+            const int last = idgx::plain_grid_items_per_subgrid(p.work, S) - 1;
+            p.whole = p.whole && idgx::plain_grid_item_pixels(p.work, S, last) ==
+                                     idgx::plain_grid_item_pixels(p.work, 2 * S, 0);
+        }
+    return p;
 }
 
-int workgroups_for(const idgx_batch *b, bool gridder, int shape)
+int workgroups_for(const idgx_batch *b, bool gridder, int shape, int cls)
 {
-    return plain(b) ? idgx::plain_queue_workgroups(accurate_sincos(b), gridder, plain_launch(b, gridder, shape))
+    return plain(b) ? idgx::plain_queue_workgroups(plain_kernel(b, gridder, shape, cls))
                     : idgx::queue_workgroups(b->precision, gridder, shape);
 }
 
-hipError_t launch_queue(const idgx_batch *b, const QueueArgs &q, bool gridder, int shape, int workgroups,
-                        hipStream_t st)
+// A persistent launch over `items` of class `cls` (-1: of all): no more workgroups than items (each asks all queues for work before it ends, one atomic
+// after the other on the same counters).
+hipError_t launch_queue(const idgx_batch *b, const QueueArgs &q, bool gridder, int shape, int cls, int resident,
+                        int items, hipStream_t st)
 {
+    const int workgroups = std::min(resident, items);
     if (plain(b))
-    {
-        const int work = plain_launch(b, gridder, shape);
-        return gridder ? idgx::launch_grid_plain_queue(q, accurate_sincos(b), work, workgroups, st)
-                       : idgx::launch_degrid_plain_queue(q, accurate_sincos(b), work, workgroups, st);
-    }
+        return idgx::launch_plain_queue(q, plain_kernel(b, gridder, shape, cls), workgroups, st);
     return gridder ? idgx::launch_grid_mixed_queue(q, b->precision, shape, workgroups, st)
                    : idgx::launch_degrid_mixed_queue(q, b->precision, shape, workgroups, st);
 }
@@ -343,7 +352,7 @@ int upload_queue(idgx_batch *b, bool gridder, int k, int shape)
     }
     b->nr_items[dir][k] = static_cast<int>(flat.size());
     b->shape[dir][k] = shape;
-    b->workgroups[dir][k] = workgroups_for(b, gridder, shape);
+    b->workgroups[dir][k] = workgroups_for(b, gridder, shape, k);
     return b->workgroups[dir][k] > 0 ? IDGX_OK : IDGX_ERR_DEVICE;
 }
 
@@ -383,7 +392,7 @@ int upload_single_queue(idgx_batch *b, bool gridder, int shape)
     }
     b->single_items[dir] = static_cast<int>(flat.size());
     b->single_shape[dir] = shape;
-    b->single_workgroups[dir] = workgroups_for(b, gridder, shape);
+    b->single_workgroups[dir] = workgroups_for(b, gridder, shape, -1);
     return b->single_workgroups[dir] > 0 ? IDGX_OK : IDGX_ERR_DEVICE;
 }
 
@@ -486,7 +495,8 @@ int run(idgx_batch *b, const idgx_batch_data *d, bool gridder, hipStream_t st, i
         q.counter = b->d_counters + dir * kDirCounters;
         for (int k = 0; k < idgx::kMaxClasses; ++k)
             q.tiles[k] = b->single_tiles[k];
-        e = launch_queue(b, q, gridder, b->single_shape[dir], b->single_workgroups[dir], st);
+        e = launch_queue(b, q, gridder, b->single_shape[dir], -1, b->single_workgroups[dir],
+                         b->single_items[dir], st);
         b->last_launches[dir] += e == hipSuccess;
         return to_status(e);
     }
@@ -508,7 +518,7 @@ int run(idgx_batch *b, const idgx_batch_data *d, bool gridder, hipStream_t st, i
         std::memcpy(qk.queue_begin, b->qbegin[dir][k], sizeof(qk.queue_begin));
         qk.nr_queues = idgx::kQueues;
         qk.counter = b->d_counters + dir * kDirCounters + k * idgx::kQueues;
-        e = launch_queue(b, qk, gridder, b->shape[dir][k], b->workgroups[dir][k], st);
+        e = launch_queue(b, qk, gridder, b->shape[dir][k], k, b->workgroups[dir][k], b->nr_items[dir][k], st);
         b->last_launches[dir] += e == hipSuccess;
     }
     return to_status(e);
@@ -565,11 +575,23 @@ extern "C" int idgx_batch_create(const idgx_batch_class *classes, int nr_classes
     }
     for (int dir = 0; dir < 2 && plain(b); ++dir)
     {
-        long long items = 0;
+        idgx::PlainWork work{};
         for (int k = 0; k < nr_classes; ++k)
-            items += static_cast<long long>(
-                item_count(b, dir == 0, k, default_shape(b, dir == 0, b->plans[k].subgrid_size)));
-        b->fine[dir] = idgx::plain_fine_items(dir == 0, items);
+        {
+            const int S = b->plans[k].subgrid_size;
+            work.items += static_cast<long long>(item_count(b, dir == 0, k, default_shape(b, dir == 0, S)));
+            work.subgrids += b->plans[k].nr_subgrids;
+            work.fine_grid_items +=
+                static_cast<long long>(b->plans[k].nr_subgrids) * idgx::plain_grid_items_per_subgrid(1, S);
+            const long long per = idgx::plain_degrid_visibilities_per_item(1);
+            for (const int64_t v : b->vis_count[k])
+            {
+                work.fine_degrid_items += (v + per - 1) / per;
+                work.visibilities += v;
+                work.pairs += v * S * S;
+            }
+        }
+        b->fine[dir] = idgx::plain_fine_items(dir == 0, work);
     }
     hipError_t e = hipSuccess;
     for (int dir = 0; dir < 2 && e == hipSuccess; ++dir)

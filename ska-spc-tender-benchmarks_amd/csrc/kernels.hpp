@@ -215,15 +215,27 @@ struct PlainShape
 int plain_shape_count();
 PlainShape plain_shape(int i);
 int plain_default_shape(bool gridder, int S);
-// Plans whose items of the default shape would not fill the chip take one pixel or visibility per thread in any shape.
-bool plain_fine_items(bool gridder, long long items);
+// A batch's work: items of the direction's default shapes, gridder and degridder items of one pixel or visibility per
+// thread, subgrids, visibilities, pairs of a pixel and a visibility.
+struct PlainWork
+{
+    long long items, fine_grid_items, fine_degrid_items, subgrids, visibilities, pairs;
+};
+// Plans whose items of the default shape would not fill the chip take one pixel or visibility per thread in any shape,
+// where their items are worth it.
+bool plain_fine_items(bool gridder, const PlainWork &w);
 int plain_grid_items_per_subgrid(int pixels, int S);
 long long plain_grid_item_pixels(int pixels, int S, int item);
 int plain_degrid_visibilities_per_item(int entries);
-// `work`: gridder pixels per thread (kShapeTilesPerClass: each class's own), degridder visibilities per thread.
-hipError_t launch_grid_plain_queue(const QueueArgs &q, bool accurate_sincos, int work, int workgroups, hipStream_t st);
-hipError_t launch_degrid_plain_queue(const QueueArgs &q, bool accurate_sincos, int work, int workgroups, hipStream_t st);
-int plain_queue_workgroups(bool accurate_sincos, bool gridder, int work);
+// `work`: gridder pixels per thread (kShapeTilesPerClass: each class's own), degridder visibilities per thread.  `whole`:
+// the gridder items have all their pixels (256 x work divides the subgrids').
+struct PlainKernel
+{
+    bool accurate_sincos, gridder, whole;
+    int work;
+};
+hipError_t launch_plain_queue(const QueueArgs &q, const PlainKernel &k, int workgroups, hipStream_t st);
+int plain_queue_workgroups(const PlainKernel &k);
 hipError_t launch_grid_mixed(const KernelArgs &a, int precision, bool phase_mfma, hipStream_t stream);
 hipError_t launch_degrid_mixed(const KernelArgs &a, int precision, bool phase_mfma, hipStream_t stream);
 

@@ -53,12 +53,32 @@ __device__ __forceinline__ void cmac4(float *acc, float4 va, float4 vb, float cs
     acc[7] = __builtin_fmaf(vb.z, sn, acc[7]);
 }
 
-// The same sums of one value on N pixels (visibilities) side by side, acc(i) the i-th one's.  Runs of instructions that
-// read the same component first are faster than N calls of cmac4: 24.25 VALU instructions per pair either way, but the
-// gridder's items of 1024 pixels took 5600 us against 5360 (6409 subgrids of 32^2; with (sin, cos) terms 6340).
+// The same sums, each one's two terms next to each other: faster where several pixels of a thread take turns (3000
+// subgrids of 48^2 with 1024 visibilities, three pixels per thread: cmac4_group 3656 us, this 3534; four, 32^2, 256
+// visibilities, 12,000 subgrids: 1726 and 1676).
+__device__ __forceinline__ void cmac4_pairs(float *acc, float4 va, float4 vb, float cs, float sn)
+{
+    const float x[4] = {va.x, va.z, vb.x, vb.z}, y[4] = {va.y, va.w, vb.y, vb.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        acc[2 * j] = __builtin_fmaf(x[j], cs, acc[2 * j]);
+        acc[2 * j] = __builtin_fmaf(-y[j], sn, acc[2 * j]);
+        acc[2 * j + 1] = __builtin_fmaf(y[j], cs, acc[2 * j + 1]);
+        acc[2 * j + 1] = __builtin_fmaf(x[j], sn, acc[2 * j + 1]);
+    }
+}
+
+// The same sums of one value on N pixels (visibilities) side by side, acc(i) the i-th one's: the degridder's two or four
+// visibilities per thread (3000 subgrids of 48^2 with 1024 visibilities: N calls of cmac4 3960 us, this 3835).
 template <int N, class Acc>
 __device__ __forceinline__ void cmac4_group(Acc acc, float4 va, float4 vb, const float (&cs)[N], const float (&sn)[N])
 {
+    if constexpr (N == 1)
+    {
+        cmac4(acc(0), va, vb, cs[0], sn[0]);
+        return;
+    }
     const float x[4] = {va.x, va.z, vb.x, vb.z}, y[4] = {va.y, va.w, vb.y, vb.w};
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -194,8 +214,9 @@ constexpr int kGridUnroll = 4;
 // or 3 (S = 24, 48) pixels per thread side by side at five waves per SIMD, 780 baselines x 256 timesteps x 64 channels:
 // S = 32 7956 -> 7278 us, S = 48 16333 -> 15777 us, S = 24 (where a third of the lanes' third pixels were idle) 5541 ->
 // 4300 us; 45 subgrids of 32^2 with 2048 visibilities each, which leave CUs idle either way, 478 -> 143 us.
-template <int SC>
-__global__ __launch_bounds__(kThreads, SC == kSincosHw ? 8 : 1) void gridder_plain(KernelArgs a)
+// NPIX 3 and 4: large plans whose blocks of 768 or 1024 pixels are whole, where they are faster (launch_grid_plain).
+template <int NPIX, int SC>
+__global__ __launch_bounds__(kThreads, SC == kSincosHw ? (NPIX == 1 ? 8 : 5) : 1) void gridder_plain(KernelArgs a)
 {
     __shared__ float4 s_vis[2 * kGridBatchVis];
     __shared__ float4 s_uvw[kGridBatchVis];
@@ -212,9 +233,12 @@ __global__ __launch_bounds__(kThreads, SC == kSincosHw ? 8 : 1) void gridder_pla
     const long long C = a.p.nr_channels;
     const Offsets off = gridder_offsets(m, a.p.S, a.p.G, a.p.image_size, a.p.w_step);
     const float4 *vis = reinterpret_cast<const float4 *>(a.visibilities);
-    const int pbase = blockIdx.y * kThreads, p = pbase + tid;
+    const int pbase = blockIdx.y * (kThreads * NPIX), p = pbase + tid;
     const bool wave_live = pbase + (tid & ~63) < P; // wave-uniform
-    PlainPixel px = plain_pixel(a, off, min(p, P - 1));
+    PlainPixel px[NPIX];
+#pragma unroll
+    for (int i = 0; i < NPIX; ++i)
+        px[i] = plain_pixel(a, off, min(p + i * kThreads, P - 1));
     for (int cb = 0; ok && cb < nc; cb += kGridChunk)
     {
         const int cc = min(kGridChunk, nc - cb);
@@ -240,20 +264,42 @@ __global__ __launch_bounds__(kThreads, SC == kSincosHw ? 8 : 1) void gridder_pla
             for (int t = 0; wave_live && t < tb; ++t)
             {
                 const float4 uv = s_uvw[t];
-                const float pidx = (uv.x * px.l + uv.y * px.m) + uv.z * px.n;
-#pragma unroll kGridUnroll
-                for (int c = 0; c < cc; ++c)
+                float pidx[NPIX];
+#pragma unroll
+                for (int i = 0; i < NPIX; ++i)
+                    pidx[i] = (uv.x * px[i].l + uv.y * px[i].m) + uv.z * px[i].n;
+                if constexpr (NPIX == 1)
                 {
-                    const float phase = px.offset - pidx * s_wn[c];
-                    float sn, cs;
-                    sincos_rad<SC>(phase, sn, cs);
-                    cmac4(px.acc, s_vis[2 * (t * cc + c)], s_vis[2 * (t * cc + c) + 1], cs, sn);
+#pragma unroll kGridUnroll
+                    for (int c = 0; c < cc; ++c)
+                    {
+                        const float phase = px[0].offset - pidx[0] * s_wn[c];
+                        float sn, cs;
+                        sincos_rad<SC>(phase, sn, cs);
+                        cmac4(px[0].acc, s_vis[2 * (t * cc + c)], s_vis[2 * (t * cc + c) + 1], cs, sn);
+                    }
+                }
+                else
+                {
+                    for (int c = 0; c < cc; ++c)
+                    {
+                        const float4 va = s_vis[2 * (t * cc + c)], vb = s_vis[2 * (t * cc + c) + 1];
+#pragma unroll
+                        for (int i = 0; i < NPIX; ++i)
+                        {
+                            float sn, cs;
+                            sincos_rad<SC>(px[i].offset - pidx[i] * s_wn[c], sn, cs);
+                            cmac4_pairs(px[i].acc, va, vb, cs, sn);
+                        }
+                    }
                 }
             }
         }
     }
-    if (p < P)
-        store_plain_pixel(a, m, s, p, ok, px.acc);
+#pragma unroll
+    for (int i = 0; i < NPIX; ++i)
+        if (p + i * kThreads < P)
+            store_plain_pixel(a, m, s, p + i * kThreads, ok, px[i].acc);
 }
 
 // Plans that leave SIMDs without a wave of 64 pixels: a wave per 16 pixels, on the matrix cores (a workgroup 64 pixels).
@@ -706,11 +752,16 @@ __device__ __forceinline__ void grid_runs(const PlainGridShared &sm, int nruns, 
             const float4 va = sm.ent[3 * e];
             const float4 vb = sm.ent[3 * e + 1];
             const float k = sm.ent[3 * e + 2].x;
-            float sn[N], cs[N];
 #pragma unroll
             for (int i = 0; i < N; ++i)
-                sincos_rad<SC>(px[i].offset - pidx[i] * k, sn[i], cs[i]);
-            cmac4_group<N>([&](int i) { return px[i].acc; }, va, vb, cs, sn);
+            {
+                float sn, cs;
+                sincos_rad<SC>(px[i].offset - pidx[i] * k, sn, cs);
+                if constexpr (N == 1)
+                    cmac4(px[i].acc, va, vb, cs, sn);
+                else
+                    cmac4_pairs(px[i].acc, va, vb, cs, sn);
+            }
         };
         if constexpr (UNROLL > 1)
         {
@@ -732,7 +783,9 @@ __device__ __forceinline__ void grid_runs(const PlainGridShared &sm, int nruns, 
 // Entries are staged 256 at a time; the entries of a stage that share a timestep form a run (a workgroup scan over
 // "timestep differs from the previous entry"), and each run forms the per-pixel index term (u l + v m) + w n once, as
 // the dense kernel does per timestep.
-template <int NPIX, int SC>
+// WHOLE: every item of the launch has all its pixels (the plan's sizes decide), which leaves the kernel without the other
+// loop and its registers (three pixels per thread: 94 -> 75 VGPRs, six workgroups per CU for five).
+template <int NPIX, int SC, bool WHOLE>
 __device__ __forceinline__ void gridder_plain_item(const KernelArgs &a, int s, int pblk, PlainGridShared &sm)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -814,7 +867,7 @@ __device__ __forceinline__ void gridder_plain_item(const KernelArgs &a, int s, i
             sm.run_start[nruns] = nb;
         __syncthreads();
         nruns = __builtin_amdgcn_readfirstlane(nruns);
-        if (live == NPIX)
+        if (WHOLE || live == NPIX)
         {
             grid_runs<NPIX, NPIX == 1 ? kGridUnroll : 1, SC>(sm, nruns, px);
         }
@@ -983,18 +1036,18 @@ __device__ __forceinline__ void degridder_plain_item(const KernelArgs &a, int s,
     }
 }
 
-template <int NPIX, int SC>
-__global__ __launch_bounds__(kThreads, SC == kSincosHw ? (NPIX == 1 ? 8 : 5) : 1) void gridder_plain_queue(QueueArgs q)
+template <int NPIX, int SC, bool WHOLE>
+__global__ __launch_bounds__(kThreads, SC == kSincosHw ? (NPIX == 1 ? 8 : 5) : 4) void gridder_plain_queue(QueueArgs q)
 {
     __shared__ PlainGridShared sm;
     int cls, s, blk;
     while (next_queue_item(q, cls, s, blk))
-        gridder_plain_item<NPIX, SC>(q.cls[cls], s, blk, sm);
+        gridder_plain_item<NPIX, SC, WHOLE>(q.cls[cls], s, blk, sm);
 }
 
 // One launch over items of several subgrid classes, each with its class's pixels per thread (q.tiles[class]).
 template <int SC>
-__global__ __launch_bounds__(kThreads, SC == kSincosHw ? 5 : 1) void gridder_plain_queue_tiles(QueueArgs q)
+__global__ __launch_bounds__(kThreads, SC == kSincosHw ? 5 : 4) void gridder_plain_queue_tiles(QueueArgs q)
 {
     __shared__ PlainGridShared sm;
     int cls, s, blk;
@@ -1003,16 +1056,16 @@ __global__ __launch_bounds__(kThreads, SC == kSincosHw ? 5 : 1) void gridder_pla
         switch (q.tiles[cls]) // workgroup-uniform
         {
         case 1:
-            gridder_plain_item<1, SC>(q.cls[cls], s, blk, sm);
+            gridder_plain_item<1, SC, false>(q.cls[cls], s, blk, sm);
             break;
         case 2:
-            gridder_plain_item<2, SC>(q.cls[cls], s, blk, sm);
+            gridder_plain_item<2, SC, false>(q.cls[cls], s, blk, sm);
             break;
         case 3:
-            gridder_plain_item<3, SC>(q.cls[cls], s, blk, sm);
+            gridder_plain_item<3, SC, false>(q.cls[cls], s, blk, sm);
             break;
         default:
-            gridder_plain_item<4, SC>(q.cls[cls], s, blk, sm);
+            gridder_plain_item<4, SC, false>(q.cls[cls], s, blk, sm);
             break;
         }
     }
@@ -1040,20 +1093,26 @@ __global__ __launch_bounds__(kThreads, (degrid_plain_queue_min_blocks<NCH, SC>()
 constexpr PlainShape kPlainShapes[] = {{4, 2}, {3, 4}, {2, 1}};
 constexpr int kNumPlainShapes = sizeof(kPlainShapes) / sizeof(kPlainShapes[0]);
 
-template <int SC> void *plain_grid_queue_fn(int pixels)
+template <int PIXELS, int SC> void *plain_grid_queue_fn(bool whole)
+{
+    return whole ? reinterpret_cast<void *>(&gridder_plain_queue<PIXELS, SC, true>)
+                 : reinterpret_cast<void *>(&gridder_plain_queue<PIXELS, SC, false>);
+}
+
+template <int SC> void *plain_grid_queue_fn(int pixels, bool whole)
 {
     switch (pixels)
     {
     case kShapeTilesPerClass:
         return reinterpret_cast<void *>(&gridder_plain_queue_tiles<SC>);
     case 1:
-        return reinterpret_cast<void *>(&gridder_plain_queue<1, SC>);
+        return reinterpret_cast<void *>(&gridder_plain_queue<1, SC, false>);
     case 2:
-        return reinterpret_cast<void *>(&gridder_plain_queue<2, SC>);
+        return plain_grid_queue_fn<2, SC>(whole);
     case 3:
-        return reinterpret_cast<void *>(&gridder_plain_queue<3, SC>);
+        return plain_grid_queue_fn<3, SC>(whole);
     case 4:
-        return reinterpret_cast<void *>(&gridder_plain_queue<4, SC>);
+        return plain_grid_queue_fn<4, SC>(whole);
     default:
         return nullptr;
     }
@@ -1074,31 +1133,54 @@ template <int SC> void *plain_degrid_queue_fn(int entries)
     }
 }
 
-// `work`: gridder pixels per thread (or kShapeTilesPerClass), degridder visibilities per thread.
-void *plain_queue_fn(bool accurate_sincos, bool gridder, int work)
+void *plain_queue_fn(const PlainKernel &k)
 {
-    if (gridder)
-        return accurate_sincos ? plain_grid_queue_fn<kSincosOcml>(work) : plain_grid_queue_fn<kSincosHw>(work);
-    return accurate_sincos ? plain_degrid_queue_fn<kSincosOcml>(work) : plain_degrid_queue_fn<kSincosHw>(work);
+    if (k.gridder)
+        return k.accurate_sincos ? plain_grid_queue_fn<kSincosOcml>(k.work, k.whole)
+                                 : plain_grid_queue_fn<kSincosHw>(k.work, k.whole);
+    return k.accurate_sincos ? plain_degrid_queue_fn<kSincosOcml>(k.work) : plain_degrid_queue_fn<kSincosHw>(k.work);
 }
+} // namespace
 
-hipError_t launch_plain_queue(const QueueArgs &q, bool accurate_sincos, bool gridder, int work, int workgroups,
-                              hipStream_t st)
+hipError_t launch_plain_queue(const QueueArgs &q, const PlainKernel &k, int workgroups, hipStream_t st)
 {
-    void *fn = plain_queue_fn(accurate_sincos, gridder, work);
+    void *fn = plain_queue_fn(k);
     if (!fn || workgroups <= 0)
         return hipErrorInvalidValue;
     QueueArgs arg = q;
     void *args[] = {&arg};
     return hipLaunchKernel(fn, dim3(workgroups), dim3(kThreads), args, 0, st);
 }
-} // namespace
 
 // Waves of 64 pixels (visibilities) up to which a one-shot plan takes the tile forms: one per SIMD for the gridder, whose
 // time does not fall below one wave's (45 subgrids of 32^2, 720 waves: 156 -> 105 us; 66, 1056 waves: 185 -> 159; 91, 1456
 // waves: 189 -> 187; 120 of 24^2, 1080 waves: 67 -> 69), two for the degridder (1440 waves: 143 -> 94 us; 120 subgrids of
 // 48^2, 1920 waves: 306 -> 268; 91 of 32^2, 2912 waves: 168 -> 179).
 constexpr long long kTileGridWaves = 1024, kTileDegridWaves = 2048;
+
+template <int NPIX> hipError_t launch_grid_plain_pixels(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
+{
+    const dim3 grid(a.p.nr_subgrids, (a.p.S * a.p.S + kThreads * NPIX - 1) / (kThreads * NPIX));
+    if (accurate_sincos)
+        gridder_plain<NPIX, kSincosOcml><<<grid, kThreads, 0, stream>>>(a);
+    else
+        gridder_plain<NPIX, kSincosHw><<<grid, kThreads, 0, stream>>>(a);
+    return hipGetLastError();
+}
+
+// Pixels per thread of the one-shot gridder: one, but four (or three, plain_grid_pixels_for) in large plans whose blocks
+// of that many are nearly whole, for large subgrids and with the accurate sine and cosine.  2100 subgrids, one pixel / four
+// or three: 96^2 with 16 and 128 visibilities 318 / 315 and 1413 / 1389 us, 128^2 with 16 555 / 553, but 64^2 with 1024 4353 / 4331; accurate, 64^2
+// with 16 and 128 211 / 196 and 1000 / 973, 128^2 with 128 3895 / 3560.
+int oneshot_pixels(const KernelArgs &a, bool accurate_sincos)
+{
+    constexpr long long kBlocks = 2048;
+    const long long P = static_cast<long long>(a.p.S) * a.p.S;
+    const int n = plain_grid_pixels_for(a.p.S);
+    const long long blocks = (P + kThreads * n - 1) / (kThreads * n);
+    const bool whole = 100 * P >= 88 * blocks * kThreads * n;
+    return whole && blocks * a.p.nr_subgrids >= kBlocks && a.p.S >= (accurate_sincos ? 32 : 72) ? n : 1;
+}
 
 hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
@@ -1112,12 +1194,10 @@ hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStrea
             gridder_plain_tiles<kSincosHw><<<grid, kThreads, 0, stream>>>(a);
         return hipGetLastError();
     }
-    const dim3 grid(a.p.nr_subgrids, (a.p.S * a.p.S + kThreads - 1) / kThreads);
-    if (accurate_sincos)
-        gridder_plain<kSincosOcml><<<grid, kThreads, 0, stream>>>(a);
-    else
-        gridder_plain<kSincosHw><<<grid, kThreads, 0, stream>>>(a);
-    return hipGetLastError();
+    const int pixels = oneshot_pixels(a, accurate_sincos);
+    return pixels == 4   ? launch_grid_plain_pixels<4>(a, accurate_sincos, stream)
+           : pixels == 3 ? launch_grid_plain_pixels<3>(a, accurate_sincos, stream)
+                         : launch_grid_plain_pixels<1>(a, accurate_sincos, stream);
 }
 
 // Items of the default shapes, or one-shot degridder workgroups, that fill the chip.  Smaller plans run one pixel or
@@ -1125,6 +1205,7 @@ hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStrea
 // 291 -> 246 us; 276 of them 753 -> 577 us, where the degridder gains at S = 32 and 48 (436 -> 411 us) and loses at S = 24
 // (262 -> 286 us), so its line lies below (1104 items).
 constexpr long long kGridFill = 2048, kDegridItems = 1024, kDegridFill = 1280;
+constexpr long long kGridFewItems = 1024, kFineVisibilities = 512, kFinePairs = 110000; // plain_fine_items
 
 template <int NCH> hipError_t launch_degrid_plain_chunks(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
@@ -1204,9 +1285,22 @@ int plain_default_shape(bool gridder, int S)
     return 0;
 }
 
-bool plain_fine_items(bool gridder, long long items)
+// One pixel per thread makes three to nine items of one: each costs the queue 0.1 us, and of 256 pixels saves 0.15 us per
+// visibility of the subgrid as long as the chip is not full.  Gridder time over that of the default shapes, by
+// visibilities a subgrid: 512 of 32^2 (2048 items for 512) 16 1.68, 256 1.27, 512 0.85; 1000 of them 256 1.35, 512 0.97, 1024
+// 0.86; 2000 512 1.11, 1024 0.99; 276 of 24^2 (828 for 276) 0.6 to 0.7 at any count.
+// Degridder: subgrids of up to 256 visibilities leave half the waves of an item of 512 without any (3000 of 48^2 with 128
+// 0.73, 256 0.95); beyond, small plans where an item of 256 has kFinePairs pixels x visibilities (1000 of 24^2 with 288
+// 1.09, of 32^2 0.97).
+bool plain_fine_items(bool gridder, const PlainWork &w)
 {
-    return items < (gridder ? kGridFill : kDegridItems);
+    if (!gridder)
+        return w.visibilities <= w.subgrids * kThreads ||
+               (w.items < kDegridItems &&
+                (w.fine_degrid_items <= kDegridFill || w.pairs >= w.fine_degrid_items * kFinePairs));
+    return w.fine_grid_items <= kGridFewItems ||
+           (w.items < kGridFill && w.visibilities >= w.subgrids * kFineVisibilities &&
+            (w.items < kGridFill / 2 || w.visibilities >= w.subgrids * 2 * kFineVisibilities));
 }
 
 int plain_grid_items_per_subgrid(int pixels, int S)
@@ -1227,21 +1321,9 @@ int plain_degrid_visibilities_per_item(int entries)
     return kThreads * entries;
 }
 
-hipError_t launch_grid_plain_queue(const QueueArgs &q, bool accurate_sincos, int work, int workgroups,
-                                   hipStream_t st)
+int plain_queue_workgroups(const PlainKernel &k)
 {
-    return launch_plain_queue(q, accurate_sincos, true, work, workgroups, st);
-}
-
-hipError_t launch_degrid_plain_queue(const QueueArgs &q, bool accurate_sincos, int work, int workgroups,
-                                     hipStream_t st)
-{
-    return launch_plain_queue(q, accurate_sincos, false, work, workgroups, st);
-}
-
-int plain_queue_workgroups(bool accurate_sincos, bool gridder, int work)
-{
-    void *fn = plain_queue_fn(accurate_sincos, gridder, work);
+    void *fn = plain_queue_fn(k);
     if (!fn)
         return 0;
     int dev = 0, cus = 0, per_cu = 0;
