@@ -132,23 +132,27 @@ def trans_rate(sincos_pairs, seconds):
 
 
 def kernel_key(precision, path, direction, shape=None, plain_shape=None):
-    """Name of the kernel instantiation that runs a pass, as rocprofv3 reports it (the rows of the PMC summaries).
-    plain_shape: (gridder pixels, degridder channels) per thread of the plain one-shot kernels, from the library's
-    own rule (idgx_plain_kernel_shape)."""
+    """Name of the plain or per-pair kernel instantiation that runs a pass, as rocprofv3 reports it (the rows of the PMC
+    summaries).  plain_shape: (gridder pixels, degridder channels) per thread of the plain one-shot kernels, 0 for the
+    tile kernels (idgx_oneshot_plain_shape).  shape: the batch's; plain gridders with a third item, whether the blocks
+    are whole (idgx_batch_plain_work)."""
+    gridder = direction == "gridder"
     if precision == "fp32":
         if path == "one-shot":
-            return f"{direction}_plain<{plain_shape[0] if direction == 'gridder' else plain_shape[1]}, 1>"
+            n = plain_shape[0 if gridder else 1]
+            return f"{direction}_plain<{n}, 1>" if n else f"{direction}_plain_tiles<{'' if gridder else '2, '}1>"
         if shape == "tiles per class":
             return "gridder_plain_queue_tiles<1>"
         if isinstance(shape, list):
             if len(set(shape)) != 1:
                 return None
             shape = shape[0]
-        return f"{direction}_plain_queue<{shape[0] if direction == 'gridder' else shape[1]}, 1>"
+        whole = f", {'true' if shape[2] else 'false'}" if gridder and len(shape) > 2 else ""
+        return f"{direction}_plain_queue<{shape[0] if gridder else shape[1]}, 1{whole}>"
     dt = 0 if precision.startswith("bf16") else 1
     split = "true" if precision.endswith("x3") else "false"
     if path == "one-shot":
-        return f"{direction}_mfma<{dt}, {split}, {8 if direction == 'gridder' else 4}, 256, false>"
+        return f"{direction}_mfma<{dt}, {split}, {8 if gridder else 4}, 256, false>"
     if shape == "tiles per class":  # one launch, every item with its class's tiles per wave
         return f"gridder_mfma_queue_tiles<{dt}, {split}>"
     if isinstance(shape, list):  # one shape per class: one kernel only when they agree
@@ -159,37 +163,41 @@ def kernel_key(precision, path, direction, shape=None, plain_shape=None):
     return f"{direction}_mfma_queue<{dt}, {split}, {tiles}, {batch}, {'true' if pm else 'false'}>"
 
 
-def pass_kernel(precision, path, direction, shape, S, nr_subgrids, plain_shape=None):
-    """The kernel that does a pass's work: the separable kernels where a 3-product form's subgrids are at most 64^2 (the
-    per-pair kernels keep the subgrids whose w spreads too far), else kernel_key's.  Several subgrid sizes, each with its
-    kernel: joined."""
-    if isinstance(S, list):
-        keys = [pass_kernel(precision, path, direction, shape[k] if isinstance(shape, list) else shape, S[k],
-                            nr_subgrids[k], plain_shape) for k in range(len(S))]
-        return None if None in keys else " + ".join(dict.fromkeys(keys))
-    if not precision.endswith("x3") or S > 64:
-        return kernel_key(precision, path, direction, shape, plain_shape)
-    dt = 0 if precision.startswith("bf16") else 1
-    if direction == "gridder":
-        tiles = "1, 2, 1" if S <= 16 else "2, 3, 1" if S <= 24 else "2, 4, 1" if S <= 32 else "3, 3, 2" if S <= 48 \
-            else "4, 2, 4"
-        if nr_subgrids <= 256:
-            tiles = f"{1 if S <= 16 else 2 if S <= 32 else 3 if S <= 48 else 4}, 1, 1"
-        waves = 8 if S <= 32 and nr_subgrids * -(-S // 8) <= 256 else 4
-        return f"grid_separable<{dt}, {tiles}, {waves}>"
-    steps = "2, 1, 4" if S <= 16 else "3, 1, 4" if S <= 24 else "4, 1, 4" if S <= 32 else "3, 2, 4" if S <= 48 else "4, 2, 8"
-    return f"degrid_separable<{dt}, {steps}>"
+def pass_kernel(precision, path, direction, shape, plans, most_vis, plain_shape=None):
+    """The kernel that does most of a pass's work, for plans of one or more subgrid sizes (joined by " + "): where the
+    library takes their subgrids to the separable kernels (idgx_separable_shape), that kernel, else kernel_key's.  Chunks
+    whose w spreads too far are the per-pair kernels' all the same."""
+    from idgx import separable_shape
+
+    keys = []
+    for k, (plan, most) in enumerate(zip(plans, most_vis)):
+        args = separable_shape(plan, direction == "gridder", most)
+        if args:
+            keys.append(f"{'grid' if direction == 'gridder' else 'degrid'}_separable<{', '.join(map(str, args))}>")
+        else:
+            keys.append(kernel_key(precision, path, direction, shape[k] if isinstance(shape, list) else shape,
+                                   plain_shape))
+    return None if None in keys else " + ".join(dict.fromkeys(keys))
 
 
 def pipe_profile(config, key):
     """VALU and matrix-core utilisation of kernel `key` from the committed rocprofv3 --pmc summary for this workload
-    (profiles/pipe_utilisation_<config>.json), or None when it was not profiled."""
+    (profiles/pipe_utilisation_<config>.json), or None when it was not profiled.  Several kernels (joined by " + "): counts
+    summed, percentages weighted by their busy cycles."""
     path = os.path.join(ROOT, "profiles", f"pipe_utilisation_{config}.json")
     if key is None or not os.path.exists(path):
         return None
     with open(path) as f:
-        k = json.load(f).get(key)
-    return None if k is None else dict(k, source=os.path.relpath(path, ROOT))
+        rows = json.load(f)
+    rows = [rows.get(k) for k in key.split(" + ")]
+    if None in rows:
+        return None
+    cycles = [r["GRBM_GUI_ACTIVE"] for r in rows]
+    out = {c: sum(r[c] for r in rows) for c in rows[0] if all(c in r for r in rows)}
+    for c in ("VALUBusy", "MfmaUtil"):
+        if c in out:
+            out[c] = sum(r[c] * n for r, n in zip(rows, cycles)) / sum(cycles)
+    return dict(out, source=os.path.relpath(path, ROOT))
 
 
 MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense FP16 / BF16 matrix peak, published
@@ -197,11 +205,12 @@ MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense FP16 / BF16 matrix peak, published
 
 def roofline_record(config, precision, key, dominant, flops, sincos, t_dom):
     """The roofline of the dominant kernel.  The separable kernels are bound by the matrix cores at the power limit:
-    `frac` is their MFMA rate (128 flops per (pixel, visibility) pair) against the published FP16/BF16 peak.  The per-pair
-    and plain FP32 kernels are bound by VALU issue (phases, sin/cos and, for the mixed forms, the hi/lo split), far
-    from HBM and from the matrix-core peak, so there it is the FP32-equivalent algorithmic rate against the FP32 peak,
-    with the committed counters beside it: VALU busy and VALU instructions per pair, the matrix cores' utilisation
-    (counter and algorithmic MFMA rate) and the sin/cos rate against the half-rate v_sin / v_cos peak."""
+    `frac` is a nominal MFMA rate (128 flops per (pixel, visibility) pair of the pass, whatever a subgrid issues) against
+    the published FP16/BF16 peak.  The per-pair and plain FP32 kernels are bound by VALU issue (phases, sin/cos and, for
+    the mixed forms, the hi/lo split), far from HBM and from the matrix-core peak, so there it is the FP32-equivalent
+    algorithmic rate against the FP32 peak, with the committed counters beside it: VALU busy and VALU instructions per
+    pair, the matrix cores' utilisation (counter and nominal MFMA rate) and the sin/cos rate against the half-rate
+    v_sin / v_cos peak."""
     separable = key is not None and "separable" in key
     achieved = flops / t_dom / 1e12
     traffic = measured_traffic(config, key)
@@ -227,21 +236,25 @@ def roofline_record(config, precision, key, dominant, flops, sincos, t_dom):
         "frac": achieved / peak,
         "traffic": None if traffic is None else traffic["bytes"],
         "traffic_detail": traffic,
-        "flop_model": "128 per (pixel, visibility) pair: 4 MFMA products of 32 (3 of the hi/lo split, 1 of the w-term's "
-                      "remainder)" if separable else
+        "flop_model": "nominal: 128 per (pixel, visibility) pair, 4 MFMA products of 32.  Issued: FP16 96, or 128 with "
+                      "the product term of the w-term's remainder; BF16 128 or 160; padding, and chunks left to the "
+                      "per-pair kernels, apart (mfma.issued_tflops)" if separable else
                       "P*(5*T + 34*V) + 134*P per subgrid (FP32-equivalent algorithmic flops), sincos separate",
         "valu": valu,
         "mfma": None if not mfma_flops else {
             "achieved_tflops": mfma_flops / t_dom / 1e12, "peak_tflops": MFMA_PEAK_TFLOPS,
             "frac": mfma_flops / t_dom / 1e12 / MFMA_PEAK_TFLOPS,
-            "note": "algorithmic MFMA flops: 128 per pair for the 3-product split, 64 single"},
+            "issued_tflops": None if not separable or pipes is None or not pipes.get("SQ_INSTS_MFMA") else
+                             pipes["SQ_INSTS_MFMA"] * 2 * 32 * 32 * 16 / t_dom / 1e12,
+            "note": "nominal MFMA flops: 128 per pair for the 3-product split, 64 single; issued: SQ_INSTS_MFMA of the "
+                    "committed profile of this kernel, 32x32x16 products"},
         # The separable kernels form phasors per row and per column, not per pair.
         "transcendental": None if separable else trans_rate(sincos, t_dom),
     }
 
 
 def form_rates(precision, tg, td, flops, sincos, bytes_by_direction=None):
-    """Per-direction rates of one form: FP32-equivalent rate against the FP32 peak, algorithmic MFMA rate against
+    """Per-direction rates of one form: FP32-equivalent rate against the FP32 peak, nominal MFMA rate against
     the FP16/BF16 matrix peak (128 flops per pair with the 3-product split, 64 single) and, when the algorithmic
     bytes are known, HBM GB/s at those bytes."""
     split = 1.0 if precision.endswith("x3") else 0.5
@@ -258,15 +271,19 @@ def form_rates(precision, tg, td, flops, sincos, bytes_by_direction=None):
 
 def measured_traffic(config, key):
     """HBM bytes per launch of kernel `key` from the committed rocprofv3 --pmc summary (FETCH_SIZE + WRITE_SIZE,
-    scaled by the copy-kernel calibration) for this workload, or None when it was not profiled."""
+    scaled by the copy-kernel calibration) for this workload, or None when it was not profiled.  Several kernels (joined
+    by " + "): their sum."""
     path = os.path.join(ROOT, "profiles", f"hbm_traffic_{config}.json")
     if key is None or not os.path.exists(path):
         return None
     with open(path) as f:
-        k = json.load(f).get("kernels", {}).get(key)
-    return None if k is None else {"bytes": k["traffic_bytes"], "read_bytes": k["read_bytes"],
-                                   "write_bytes": k["write_bytes"], "kernel": key,
-                                   "source": os.path.relpath(path, ROOT)}
+        kernels = json.load(f).get("kernels", {})
+    rows = [kernels.get(k) for k in key.split(" + ")]
+    if None in rows:
+        return None
+    total = {c: sum(r[c] for r in rows) for c in ("traffic_bytes", "read_bytes", "write_bytes")}
+    return {"bytes": total["traffic_bytes"], "read_bytes": total["read_bytes"], "write_bytes": total["write_bytes"],
+            "kernel": key, "source": os.path.relpath(path, ROOT)}
 
 
 class OneShot:
@@ -310,7 +327,10 @@ class Batched:
 
     def describe(self, tg, td):
         """Shapes, launch mode and queue sizes of the batch as it now runs."""
+        from idgx import separable_shape
+
         classes = [c["w"] for c in self.db.classes]
+        self.plans = [c["plan"] for c in self.db.classes]
         table = self.db.batch.shape_table()
         plain = self.precision == "fp32"
         per_class = [self.db.batch.class_shape(k) for k in range(len(classes))]
@@ -323,23 +343,32 @@ class Batched:
                 self.shapes[direction] = "tiles per class"
             else:
                 self.shapes[direction] = table[single[i]]
+            if plain and self.shapes[direction] != "tiles per class":  # as launched: (pixels, visibilities, whole)
+                work = [self.db.batch.plain_work(k) for k in range(len(classes))]
+                self.shapes[direction] = [(px, nv, whole) for px, whole, nv in work]
 
-        def shape_fields(g, d):
+        def shape_fields(k, g, d):
             if plain:
-                return {"gridder": {"pixels_per_thread": table[g][0]},
-                        "degridder": {"visibilities_per_thread": table[d][1]}}
+                px, _, nv = self.db.batch.plain_work(k)
+                return {"gridder": {"pixels_per_thread": px or table[g][0]},
+                        "degridder": {"visibilities_per_thread": nv}}
             return {"gridder": {"tiles_per_wave": table[g][0], "lds_visibilities": table[g][1],
                                 "phase_mfma": table[g][2]},
                     "degridder": {"tiles_per_wave": table[d][0], "lds_pixels": table[d][1],
                                   "phase_mfma": table[d][2]}}
 
         items = self.db.batch.items()
-        self.info = {"launches": {d: ("one per class" if single[i] == -1 else "one over all classes")
+        separable = [bool(separable_shape(p, True, 0)) for p in self.plans]
+        self.info = {"separable": separable,
+                     "launches_of": "the persistent kernels" + (
+                         ", behind the separable kernels' launch per class, for the chunks those leave; items, workgroups "
+                         "and shapes are theirs" if any(separable) else ""),
+                     "launches": {d: ("one per class" if single[i] == -1 else "one over all classes")
                                   for i, d in enumerate(("gridder", "degridder"))},
                      "single_launch_shapes": {d: (self.shapes[d] if single[i] != -1 else None)
                                               for i, d in enumerate(("gridder", "degridder"))},
-                     "shapes_per_class": [dict({"subgrid_size": int(c["subgrid_size"])}, **shape_fields(g, d))
-                                          for c, (g, d) in zip(classes, per_class)],
+                     "shapes_per_class": [dict({"subgrid_size": int(c["subgrid_size"])}, **shape_fields(k, g, d))
+                                          for k, (c, (g, d)) in enumerate(zip(classes, per_class))],
                      "queue_items": {"gridder": items[0], "degridder": items[1]},
                      "persistent_workgroups": {"gridder": items[2], "degridder": items[3]},
                      "autotune_ms": {"gridder": tg, "degridder": td}}
@@ -687,11 +716,8 @@ def run_batched_config(args):
     tg, td = head["gridder_ms"] / 1e3, head["degridder_ms"] / 1e3
     dominant, t_dom = ("degridder", td) if td > tg else ("gridder", tg)
     dom_key = pass_kernel(head["precision"], "batched", dominant, runner.shapes[dominant],
-                          [int(c["subgrid_size"]) for c in bo["classes"]], [int(c["nr_subgrids"]) for c in bo["classes"]])
+                          runner.plans, [int(np.diff(c["vis_offset"]).max()) for c in bo["classes"]])
     roofline = roofline_record(args.config, head["precision"], dom_key, dominant, flops, sincos, t_dom)
-    if dom_key is None:  # one launch per class with different shapes
-        roofline["kernel"] = " + ".join(kernel_key(head["precision"], "batched", dominant, sh)
-                                        for sh in runner.shapes[dominant])
     if roofline["bound"] == "valu":
         roofline["flop_model"] = ("P*(5*T + 34*V) + 134*P per subgrid, V = selected visibilities (FP32-equivalent "
                                   "algorithmic flops), sincos separate")
@@ -868,10 +894,13 @@ def main():
     dominant, t_dom = ("degridder", td) if td > tg else ("gridder", tg)
     bytes_dom = bytes_by_direction[dominant]
     head_runner = runners[-1]
-    from idgx import plain_kernel_shape
+    from idgx import oneshot_plain_shape
 
-    dom_key = pass_kernel(head["precision"], head["path"], dominant, head_runner.shapes[dominant], S,
-                          int(w["nr_subgrids"]), plain_shape=plain_kernel_shape(dw.plan(), ch is not None))
+    head_plan = dw.plan(precision=head["precision"])
+    widths = C if ch is None else ch["nr_channels"].astype(np.int64)
+    dom_key = pass_kernel(head["precision"], head["path"], dominant, head_runner.shapes[dominant], [head_plan],
+                          [int((md["nr_timesteps"].astype(np.int64) * widths).max())],
+                          plain_shape=oneshot_plain_shape(head_plan, ch is not None))
     roofline = roofline_record(args.config, head["precision"], dom_key, dominant, flops, sincos, t_dom)
     roofline.update(algorithmic_bytes=bytes_dom, hbm_gbs_algorithmic=bytes_dom / t_dom / 1e9)
 

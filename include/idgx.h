@@ -492,12 +492,31 @@ int idgx_batch_items(const idgx_batch *batch, int *gridder_items, int *degridder
                      int *degridder_workgroups);
 
 /* Work per thread of the plain FP32 forms for a plan that fills the chip: pixels per thread of a batch's gridder items
- * (4, or 3 where that fits the subgrid better: S = 24, 48; the one-shot gridder takes one) and channels per thread of
- * the one-shot degridder (4 without channel windows when the channel count is a multiple of 4, else 2), which name the
- * kernel instantiation a profile reports (degridder_plain<channels, 1>).  Smaller plans run one pixel, channel or
- * visibility per thread in every form.  No GPU needed. */
+ * (4, or 3 where that fits the subgrid better: S = 24, 48) and channels per thread of the one-shot degridder (4 without
+ * channel windows when the channel count is a multiple of 4, else 2).  Smaller plans run one pixel, channel or visibility
+ * per thread in every form.  No GPU needed. */
 int idgx_plain_kernel_shape(const idgx_plan *plan, int has_channel_windows, int *gridder_pixels_per_thread,
                             int *degridder_channels_per_thread);
+
+/* What the following three tell is which kernel a call runs, as a profile names it.  No GPU needed.
+ *
+ * The plain FP32 one-shot kernels of this plan: gridder_plain<pixels, s> and degridder_plain<channels, s>, s = 1 or, with
+ * IDGX_FLAG_ACCURATE_SINCOS, 0; where 0 pixels or channels come back, gridder_plain_tiles<s> or
+ * degridder_plain_tiles<2, s>. */
+int idgx_oneshot_plain_shape(const idgx_plan *plan, int has_channel_windows, int *gridder_pixels_per_thread,
+                             int *degridder_channels_per_thread);
+
+/* The separable kernel that takes the plan's subgrids, in one-shot calls and batches alike: grid_separable<arguments> or
+ * degrid_separable<arguments>, whose number is 6 or 4, or 0 where the per-pair kernels do all the work.  Gridder plans with
+ * subgrids of more and of fewer visibilities can have a launch for each; this is the one of subgrids with
+ * most_visibilities. */
+int idgx_separable_shape(const idgx_plan *plan, int gridder, int64_t most_visibilities, int *nr_arguments,
+                         int arguments[6]);
+
+/* The plain FP32 kernels of class cls as the batch now launches it: gridder_plain_queue<pixels, s, whole> (0 pixels: one
+ * launch in which every class has its own, gridder_plain_queue_tiles<s>) and degridder_plain_queue<visibilities, s>. */
+int idgx_batch_plain_work(const idgx_batch *batch, int cls, int *gridder_pixels, int *gridder_whole,
+                          int *degridder_visibilities);
 
 /* Name of a status code. */
 const char *idgx_strerror(int status);

@@ -520,6 +520,34 @@ extern "C" int idgx_plain_kernel_shape(const idgx_plan *plan, int has_channel_wi
     return IDGX_OK;
 }
 
+extern "C" int idgx_oneshot_plain_shape(const idgx_plan *plan, int has_channel_windows, int *gridder_pixels_per_thread,
+                                        int *degridder_channels_per_thread)
+{
+    const int rc = check_plan_struct(plan);
+    if (rc != IDGX_OK)
+        return rc;
+    if (gridder_pixels_per_thread)
+        *gridder_pixels_per_thread = idgx::oneshot_grid_pixels(to_dev(plan), accurate_sincos(plan));
+    if (degridder_channels_per_thread)
+        *degridder_channels_per_thread = idgx::oneshot_degrid_channels(to_dev(plan), has_channel_windows != 0);
+    return IDGX_OK;
+}
+
+extern "C" int idgx_separable_shape(const idgx_plan *plan, int gridder, int64_t most_visibilities, int *nr_arguments,
+                                    int arguments[6])
+{
+    const int rc = check_plan_struct(plan);
+    if (rc != IDGX_OK)
+        return rc;
+    if (!nr_arguments || !arguments)
+        return IDGX_ERR_INVALID_ARGUMENT;
+    *nr_arguments = 0;
+    if (plan->nr_subgrids > 0 && !(plan->flags & IDGX_FLAG_PHASE_MFMA))
+        *nr_arguments = idgx::separable_kernel_shape(to_dev(plan), plan->precision, gridder != 0, most_visibilities,
+                                                     arguments);
+    return IDGX_OK;
+}
+
 extern "C" const char *idgx_strerror(int status)
 {
     switch (status)

@@ -1011,6 +1011,26 @@ extern "C" int idgx_batch_items(const idgx_batch *b, int *gridder_items, int *de
     return IDGX_OK;
 }
 
+extern "C" int idgx_batch_plain_work(const idgx_batch *b, int cls, int *gridder_pixels, int *gridder_whole,
+                                     int *degridder_visibilities)
+{
+    if (!b || cls < 0 || cls >= b->nr_classes || !plain(b))
+        return IDGX_ERR_INVALID_ARGUMENT;
+    const auto kernel = [&](bool gridder) {
+        const int dir = gridder ? 0 : 1;
+        return single_mode(b, dir) ? plain_kernel(b, gridder, b->single_shape[dir], -1)
+                                   : plain_kernel(b, gridder, b->shape[dir][cls], cls);
+    };
+    const idgx::PlainKernel g = kernel(true), d = kernel(false);
+    if (gridder_pixels)
+        *gridder_pixels = g.work > 0 ? g.work : 0;
+    if (gridder_whole)
+        *gridder_whole = g.work > 1 && g.whole;
+    if (degridder_visibilities)
+        *degridder_visibilities = d.work;
+    return IDGX_OK;
+}
+
 extern "C" int idgx_batch_last_launches(const idgx_batch *b, int *gridder_launches, int *degridder_launches)
 {
     if (!b)

@@ -198,11 +198,17 @@ hipError_t launch_grid_separable(const KernelArgs &a, const SeparableArgs &sp, i
                                  hipStream_t st);
 hipError_t launch_degrid_separable(const KernelArgs &a, const SeparableArgs &sp, int precision, long long max_vis,
                                    hipStream_t st);
+// Template arguments of the kernel that takes the plan's subgrids (the gridder's for those of most_vis visibilities), and
+// their number: 0 where the per-pair kernels run.
+int separable_kernel_shape(const PlanDev &p, int precision, bool gridder, long long most_vis, int shape[6]);
 
 hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream);
 hipError_t launch_degrid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream);
-int plain_grid_pixels_for(int S);                                  // pixels per thread of launch_grid_plain
-int plain_degrid_channels_for(bool channel_windows, int nr_channels); // channels per thread of launch_degrid_plain
+// Pixels and channels per thread of the one-shot kernels (0: the tile kernels).
+int oneshot_grid_pixels(const PlanDev &p, bool accurate_sincos);
+int oneshot_degrid_channels(const PlanDev &p, bool channel_windows);
+int plain_grid_pixels_for(int S);                                     // pixels per thread of a batch's gridder items
+int plain_degrid_channels_for(bool channel_windows, int nr_channels); // oneshot_degrid_channels of plans that fill the chip
 
 // Persistent work-queue forms of the plain FP32 kernels (batches).  Shape i: gridder pixels per thread and
 // degridder visibilities per thread; kShapeTilesPerClass (gridder) gives every item its class's pixels per thread

@@ -1168,36 +1168,42 @@ template <int NPIX> hipError_t launch_grid_plain_pixels(const KernelArgs &a, boo
     return hipGetLastError();
 }
 
-// Pixels per thread of the one-shot gridder: one, but four (or three, plain_grid_pixels_for) in large plans whose blocks
-// of that many are nearly whole, for large subgrids and with the accurate sine and cosine.  2100 subgrids, one pixel / four
-// or three: 96^2 with 16 and 128 visibilities 318 / 315 and 1413 / 1389 us, 128^2 with 16 555 / 553, but 64^2 with 1024 4353 / 4331; accurate, 64^2
-// with 16 and 128 211 / 196 and 1000 / 973, 128^2 with 128 3895 / 3560.
-int oneshot_pixels(const KernelArgs &a, bool accurate_sincos)
+// Pixels per thread of the one-shot gridder: the tile kernel's for the smallest plans, else one, but four (or three,
+// plain_grid_pixels_for) in large plans whose blocks of that many are nearly whole, for large subgrids and with the
+// accurate sine and cosine.  2100 subgrids, one pixel / four or three: 96^2 with 16 and 128 visibilities 318 / 315 and
+// 1413 / 1389 us, 128^2 with 16 555 / 553, but 64^2 with 1024 4353 / 4331; accurate, 64^2 with 16 and 128 211 / 196 and
+// 1000 / 973, 128^2 with 128 3895 / 3560.
+int oneshot_grid_pixels(const PlanDev &p, bool accurate_sincos)
 {
     constexpr long long kBlocks = 2048;
-    const long long P = static_cast<long long>(a.p.S) * a.p.S;
-    const int n = plain_grid_pixels_for(a.p.S);
+    const long long P = static_cast<long long>(p.S) * p.S;
+    if (p.nr_subgrids * ((P + 63) / 64) <= kTileGridWaves)
+        return 0;
+    const int n = plain_grid_pixels_for(p.S);
     const long long blocks = (P + kThreads * n - 1) / (kThreads * n);
     const bool whole = 100 * P >= 88 * blocks * kThreads * n;
-    return whole && blocks * a.p.nr_subgrids >= kBlocks && a.p.S >= (accurate_sincos ? 32 : 72) ? n : 1;
+    return whole && blocks * p.nr_subgrids >= kBlocks && p.S >= (accurate_sincos ? 32 : 72) ? n : 1;
 }
 
 hipError_t launch_grid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
-    const long long S = a.p.S, waves = a.p.nr_subgrids * ((S * S + 63) / 64);
-    if (waves <= kTileGridWaves)
+    switch (oneshot_grid_pixels(a.p, accurate_sincos))
     {
-        const dim3 grid(a.p.nr_subgrids, static_cast<unsigned>((S * S + 63) / 64));
-        if (accurate_sincos)
-            gridder_plain_tiles<kSincosOcml><<<grid, kThreads, 0, stream>>>(a);
-        else
-            gridder_plain_tiles<kSincosHw><<<grid, kThreads, 0, stream>>>(a);
-        return hipGetLastError();
+    case 4:
+        return launch_grid_plain_pixels<4>(a, accurate_sincos, stream);
+    case 3:
+        return launch_grid_plain_pixels<3>(a, accurate_sincos, stream);
+    case 1:
+        return launch_grid_plain_pixels<1>(a, accurate_sincos, stream);
+    default:
+        break;
     }
-    const int pixels = oneshot_pixels(a, accurate_sincos);
-    return pixels == 4   ? launch_grid_plain_pixels<4>(a, accurate_sincos, stream)
-           : pixels == 3 ? launch_grid_plain_pixels<3>(a, accurate_sincos, stream)
-                         : launch_grid_plain_pixels<1>(a, accurate_sincos, stream);
+    const dim3 grid(a.p.nr_subgrids, static_cast<unsigned>((static_cast<long long>(a.p.S) * a.p.S + 63) / 64));
+    if (accurate_sincos)
+        gridder_plain_tiles<kSincosOcml><<<grid, kThreads, 0, stream>>>(a);
+    else
+        gridder_plain_tiles<kSincosHw><<<grid, kThreads, 0, stream>>>(a);
+    return hipGetLastError();
 }
 
 // Items of the default shapes, or one-shot degridder workgroups, that fill the chip.  Smaller plans run one pixel or
@@ -1229,24 +1235,37 @@ template <int NCH> hipError_t launch_degrid_plain_chunks(const KernelArgs &a, bo
 // (windows of 13.5 channels on average: 90 % of the lanes busy with four, 96.7 % with two) 82.3 and 79.6 ms.
 // Plans too small to fill the chip take one: 45 subgrids of 32^2 with 2048 visibilities each 202 -> 143 us, 276 of them
 // 428 -> 385 us (496: 628 -> 640 us).
+int oneshot_degrid_channels(const PlanDev &p, bool channel_windows)
+{
+    const long long pairs = static_cast<long long>(p.max_nr_timesteps) * ((p.nr_channels + 1) / 2);
+    if ((2 * pairs + 63) / 64 * p.nr_subgrids <= kTileDegridWaves)
+        return 0;
+    if ((pairs + kThreads - 1) / kThreads * p.nr_subgrids < kDegridFill)
+        return 1;
+    return plain_degrid_channels_for(channel_windows, p.nr_channels);
+}
+
 hipError_t launch_degrid_plain(const KernelArgs &a, bool accurate_sincos, hipStream_t stream)
 {
-    const long long pairs = static_cast<long long>(a.p.max_nr_timesteps) * ((a.p.nr_channels + 1) / 2);
-    if ((2 * pairs + 63) / 64 * a.p.nr_subgrids <= kTileDegridWaves)
+    switch (oneshot_degrid_channels(a.p, a.channels != nullptr))
     {
-        const long long per = std::max(1LL, (pairs + kThreads / 4 - 1) / (kThreads / 4));
-        const unsigned blocks = static_cast<unsigned>(per * a.p.nr_subgrids);
-        if (accurate_sincos)
-            degridder_plain_tiles<2, kSincosOcml><<<blocks, kThreads, 0, stream>>>(a, static_cast<int>(per));
-        else
-            degridder_plain_tiles<2, kSincosHw><<<blocks, kThreads, 0, stream>>>(a, static_cast<int>(per));
-        return hipGetLastError();
-    }
-    if ((pairs + kThreads - 1) / kThreads * a.p.nr_subgrids < kDegridFill)
-        return launch_degrid_plain_chunks<1>(a, accurate_sincos, stream);
-    if (plain_degrid_channels_for(a.channels != nullptr, a.p.nr_channels) == 4)
+    case 4:
         return launch_degrid_plain_chunks<4>(a, accurate_sincos, stream);
-    return launch_degrid_plain_chunks<2>(a, accurate_sincos, stream);
+    case 2:
+        return launch_degrid_plain_chunks<2>(a, accurate_sincos, stream);
+    case 1:
+        return launch_degrid_plain_chunks<1>(a, accurate_sincos, stream);
+    default:
+        break;
+    }
+    const long long pairs = static_cast<long long>(a.p.max_nr_timesteps) * ((a.p.nr_channels + 1) / 2);
+    const long long per = std::max(1LL, (pairs + kThreads / 4 - 1) / (kThreads / 4));
+    const unsigned blocks = static_cast<unsigned>(per * a.p.nr_subgrids);
+    if (accurate_sincos)
+        degridder_plain_tiles<2, kSincosOcml><<<blocks, kThreads, 0, stream>>>(a, static_cast<int>(per));
+    else
+        degridder_plain_tiles<2, kSincosHw><<<blocks, kThreads, 0, stream>>>(a, static_cast<int>(per));
+    return hipGetLastError();
 }
 
 // Pixels per thread of a batch's gridder items for subgrid size S: 4 (1024 per item) unless 3 (768) fits the subgrid

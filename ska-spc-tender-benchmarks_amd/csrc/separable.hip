@@ -563,7 +563,7 @@ template <int YT, int NT> constexpr int grid_waves()
 
 // Which subgrids of a launch a kernel grids, by their visibilities (kFewVisibilities).  Kernels with wide column tiles
 // have one form for each: a kernel with both would spill in its main loop (24^2 subgrids of 129 visibilities: 7 % slower).
-enum GridSubgrids
+enum GridSubgrids : int
 {
     kEvery,
     kMany,
@@ -572,7 +572,7 @@ enum GridSubgrids
 
 // Workgroup (part, subgrid) grids columns [part, part + 1) x 8 NT NX of a subgrid: its waves take NX column ranges and
 // WAVES / NX interleaved chunks of visibilities; the partial sums meet in LDS 16 or 32 rows at a time, in a fixed order.
-template <int DT, int YT, int NT, int NX, int WAVES, GridSubgrids WHICH>
+template <int DT, int YT, int NT, int NX, int WAVES, int WHICH>
 __global__ __launch_bounds__(64 * WAVES, (grid_waves<YT, NT>())) void grid_separable(KernelArgs a, SeparableArgs sp)
 {
     constexpr int kCols = NX * NT * 8, kSplits = WAVES / NX, kCount = 64 * WAVES;
@@ -1054,7 +1054,7 @@ __global__ __launch_bounds__(64 * WAVES, KS <= 3 && YB == 1 ? 3 : 2) void degrid
 
 // ---- launchers --------------------------------------------------------------------------------------------------
 
-template <int DT, int YT, int NT, int NX, int WAVES, GridSubgrids WHICH>
+template <int DT, int YT, int NT, int NX, int WAVES, int WHICH>
 hipError_t launch_grid(const KernelArgs &a, const SeparableArgs &sp, hipStream_t st)
 {
     const long long parts = (a.p.S + 8 * NT * NX - 1) / (8 * NT * NX), blocks = parts * sp.count;
@@ -1090,32 +1090,47 @@ hipError_t launch_grid_wide(const KernelArgs &a, SeparableArgs sp, const GridCou
     }
 }
 
-// Row tiles and column tiles per wave and column ranges for subgrid size S.  One wave holds all columns up to S = 32
-// (128 accumulators); larger subgrids spread them over two or four waves.  A plan that would leave CUs without work
-// takes a workgroup per 8 columns, which forms the row phasors once per 8 columns; where even those leave CUs idle, one
-// of 8 waves (45 subgrids of 32^2 with 2048 visibilities: 30.4 -> 25.8 us; of 16^2: 24.2 -> 19.5), which would cost
-// larger plans up to a quarter (231 subgrids of 32^2 with 256: 16.9 -> 20.9) and subgrids above 32^2 a tenth.
+// A gridder kernel's row tiles and column tiles per wave, column ranges and waves; `wide`: one form per kind of subgrid.
+template <int YT, int NT, int NX, int WAVES = kWaves, bool WIDE = (WAVES == kWaves && NT > 1)> struct GridShape
+{
+    static constexpr int yt = YT, nt = NT, nx = NX, waves = WAVES;
+    static constexpr bool wide = WIDE;
+};
+
+// f(the shape) for n subgrids of size S.  One wave holds all columns up to S = 32 (128 accumulators); larger subgrids
+// spread them over two or four waves.  A plan that would leave CUs without work takes a workgroup per 8 columns, which
+// forms the row phasors once per 8 columns; where even those leave CUs idle, one of 8 waves (45 subgrids of 32^2 with
+// 2048 visibilities: 30.4 -> 25.8 us; of 16^2: 24.2 -> 19.5), which would cost larger plans up to a quarter (231 subgrids
+// of 32^2 with 256: 16.9 -> 20.9) and subgrids above 32^2 a tenth.
+template <typename F> auto grid_shape(int S, int n, const F &f)
+{
+    const bool few = n <= kFewSubgrids;
+    const bool fewer = static_cast<long long>(n) * ((S + 7) / 8) <= kFewSubgrids;
+    if (S <= 16)
+        return fewer ? f(GridShape<1, 1, 1, 8>{}) : few ? f(GridShape<1, 1, 1>{}) : f(GridShape<1, 2, 1>{});
+    if (S <= 32 && fewer)
+        return f(GridShape<2, 1, 1, 8>{});
+    if (S <= 32 && few)
+        return f(GridShape<2, 1, 1>{});
+    if (S <= 24)
+        return f(GridShape<2, 3, 1>{});
+    if (S <= 32)
+        return f(GridShape<2, 4, 1>{});
+    if (S <= 48)
+        return few ? f(GridShape<3, 1, 1>{}) : f(GridShape<3, 3, 2>{});
+    return few ? f(GridShape<4, 1, 1>{}) : f(GridShape<4, 2, 4>{});
+}
+
 template <int DT>
 hipError_t grid_size(const KernelArgs &a, const SeparableArgs &sp, const GridCounts &n, hipStream_t st)
 {
-    const int S = a.p.S;
-    const bool few = a.p.nr_subgrids <= kFewSubgrids;
-    const bool fewer = static_cast<long long>(a.p.nr_subgrids) * ((S + 7) / 8) <= kFewSubgrids;
-    if (S <= 16)
-        return fewer ? launch_grid<DT, 1, 1, 1, 8, kEvery>(a, sp, st)
-               : few ? launch_grid<DT, 1, 1, 1, kWaves, kEvery>(a, sp, st)
-                     : launch_grid_wide<DT, 1, 2, 1>(a, sp, n, st);
-    if (S <= 32 && fewer)
-        return launch_grid<DT, 2, 1, 1, 8, kEvery>(a, sp, st);
-    if (S <= 32 && few)
-        return launch_grid<DT, 2, 1, 1, kWaves, kEvery>(a, sp, st);
-    if (S <= 24)
-        return launch_grid_wide<DT, 2, 3, 1>(a, sp, n, st);
-    if (S <= 32)
-        return launch_grid_wide<DT, 2, 4, 1>(a, sp, n, st);
-    if (S <= 48)
-        return few ? launch_grid<DT, 3, 1, 1, kWaves, kEvery>(a, sp, st) : launch_grid_wide<DT, 3, 3, 2>(a, sp, n, st);
-    return few ? launch_grid<DT, 4, 1, 1, kWaves, kEvery>(a, sp, st) : launch_grid_wide<DT, 4, 2, 4>(a, sp, n, st);
+    return grid_shape(a.p.S, a.p.nr_subgrids, [&](auto k) {
+        using K = decltype(k);
+        if constexpr (K::wide)
+            return launch_grid_wide<DT, K::yt, K::nt, K::nx>(a, sp, n, st);
+        else
+            return launch_grid<DT, K::yt, K::nt, K::nx, K::waves, kEvery>(a, sp, st);
+    });
 }
 
 template <int DT, int KS, int YB, int WAVES>
@@ -1133,19 +1148,31 @@ hipError_t launch_degrid(const KernelArgs &a, const SeparableArgs &sp, long long
     return hipGetLastError();
 }
 
-// 8-row steps held at once, and passes, for subgrid size S.
+// A degridder kernel's 8-row steps held at once, passes and waves.
+template <int KS, int YB, int WAVES> struct DegridShape
+{
+    static constexpr int ks = KS, yb = YB, waves = WAVES;
+};
+
+template <typename F> auto degrid_shape(int S, const F &f)
+{
+    if (S <= 16)
+        return f(DegridShape<2, 1, 4>{});
+    if (S <= 24)
+        return f(DegridShape<3, 1, 4>{});
+    if (S <= 32)
+        return f(DegridShape<4, 1, 4>{});
+    if (S <= 48)
+        return f(DegridShape<3, 2, 4>{});
+    return f(DegridShape<4, 2, 8>{});
+}
+
 template <int DT> hipError_t degrid_size(const KernelArgs &a, const SeparableArgs &sp, long long blocks, hipStream_t st)
 {
-    const int S = a.p.S;
-    if (S <= 16)
-        return launch_degrid<DT, 2, 1, 4>(a, sp, blocks, st);
-    if (S <= 24)
-        return launch_degrid<DT, 3, 1, 4>(a, sp, blocks, st);
-    if (S <= 32)
-        return launch_degrid<DT, 4, 1, 4>(a, sp, blocks, st);
-    if (S <= 48)
-        return launch_degrid<DT, 3, 2, 4>(a, sp, blocks, st);
-    return launch_degrid<DT, 4, 2, 8>(a, sp, blocks, st);
+    return degrid_shape(a.p.S, [&](auto k) {
+        using K = decltype(k);
+        return launch_degrid<DT, K::ks, K::yb, K::waves>(a, sp, blocks, st);
+    });
 }
 
 double host_n(double l, double m)
@@ -1228,5 +1255,25 @@ hipError_t launch_degrid_separable(const KernelArgs &a, const SeparableArgs &sp,
         return hipErrorInvalidConfiguration;
     return precision == IDGX_MIXED_FP16X3 ? degrid_size<kFP16>(a, sp, blocks, st)
                                           : degrid_size<kBF16>(a, sp, blocks, st);
+}
+
+int separable_kernel_shape(const PlanDev &p, int precision, bool gridder, long long most_vis, int shape[6])
+{
+    SeparableTables t;
+    if (!separable_tables(p, precision, t))
+        return 0;
+    shape[0] = precision == IDGX_MIXED_FP16X3 ? kFP16 : kBF16;
+    if (!gridder)
+        return degrid_shape(p.S, [&](auto k) {
+            using K = decltype(k);
+            shape[1] = K::ks, shape[2] = K::yb, shape[3] = K::waves;
+            return 4;
+        });
+    return grid_shape(p.S, p.nr_subgrids, [&](auto k) {
+        using K = decltype(k);
+        shape[1] = K::yt, shape[2] = K::nt, shape[3] = K::nx, shape[4] = K::waves;
+        shape[5] = !K::wide || shape[0] != kFP16 ? kEvery : most_vis > kFewVisibilities ? kMany : kFew;
+        return 6;
+    });
 }
 } // namespace idgx

@@ -189,6 +189,10 @@ def lib():
         L.idgx_batch_shape_info.argtypes = [ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 3
         L.idgx_batch_plain_shape_info.argtypes = [ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 2
         L.idgx_plain_kernel_shape.argtypes = [ctypes.POINTER(Plan), ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 2
+        L.idgx_oneshot_plain_shape.argtypes = L.idgx_plain_kernel_shape.argtypes
+        L.idgx_separable_shape.argtypes = [ctypes.POINTER(Plan), ctypes.c_int, ctypes.c_int64,
+                                           ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]
+        L.idgx_batch_plain_work.argtypes = [vp, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 3
         L.idgx_batch_autotune.argtypes = [vp, ctypes.POINTER(BatchData), ctypes.c_int, vp,
                                           ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_float)]
         L.idgx_batch_grid.argtypes = [vp, ctypes.POINTER(BatchData), vp]
@@ -488,6 +492,24 @@ def plain_kernel_shape(plan, has_channel_windows):
     return px.value, nch.value
 
 
+def oneshot_plain_shape(plan, has_channel_windows):
+    """(pixels per thread of the gridder, channels per thread of the degridder) of the plain FP32 one-shot kernels that
+    this plan runs; 0: the tile kernels."""
+    px, nch = ctypes.c_int(), ctypes.c_int()
+    _check(lib().idgx_oneshot_plain_shape(ctypes.byref(plan), int(bool(has_channel_windows)), ctypes.byref(px),
+                                          ctypes.byref(nch)), "idgx_oneshot_plain_shape")
+    return px.value, nch.value
+
+
+def separable_shape(plan, gridder, most_visibilities):
+    """Template arguments of the separable kernel that takes the plan's subgrids of most_visibilities visibilities; ()
+    where the per-pair kernels run."""
+    n, args = ctypes.c_int(), (ctypes.c_int * 6)()
+    _check(lib().idgx_separable_shape(ctypes.byref(plan), int(bool(gridder)), int(most_visibilities), ctypes.byref(n),
+                                      args), "idgx_separable_shape")
+    return tuple(args[:n.value])
+
+
 def _check(rc, what):
     if rc != OK:
         raise IdgxError(rc, what)
@@ -553,6 +575,14 @@ class Batch:
         g, d = ctypes.c_int(), ctypes.c_int()
         _check(lib().idgx_batch_get_shape(self.handle, ctypes.byref(g), ctypes.byref(d)), "idgx_batch_get_shape")
         return g.value, d.value
+
+    def plain_work(self, cls):
+        """(gridder pixels per thread, whether its blocks are whole, degridder visibilities per thread) of class cls as a
+        plain FP32 batch now launches it; 0 pixels: one launch, every class with its own."""
+        px, whole, nv = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+        _check(lib().idgx_batch_plain_work(self.handle, int(cls), ctypes.byref(px), ctypes.byref(whole),
+                                           ctypes.byref(nv)), "idgx_batch_plain_work")
+        return px.value, bool(whole.value), nv.value
 
     def set_class_shape(self, cls, gridder_shape, degridder_shape):
         _check(lib().idgx_batch_set_class_shape(self.handle, cls, gridder_shape, degridder_shape),
