@@ -72,21 +72,12 @@ __device__ __forceinline__ double image_n(int X, int Y, int G, double image_size
     return r2 >= 1.0 ? 1.0 : r2 / (1.0 + sqrt(1.0 - r2));
 }
 
-// image_n by its series, within 1e-11 of itself for r^2 <= 0.02 (fields up to 0.2 rad): 10 FP64 operations instead of a
-// square root and a division.
+// image_n by its series, for fields up to 0.2 rad.
 constexpr double kSeriesField = 0.2;
 __device__ __forceinline__ double image_n_series(int X, int Y, int G, double image_size)
 {
     const double l = (X - 0.5 * G) * (image_size / G), m = (Y - 0.5 * G) * (image_size / G);
-    const double r2 = __builtin_fma(l, l, m * m);
-    double p = 33.0 / 2048.0;
-    p = __builtin_fma(p, r2, 21.0 / 1024.0);
-    p = __builtin_fma(p, r2, 7.0 / 256.0);
-    p = __builtin_fma(p, r2, 5.0 / 128.0);
-    p = __builtin_fma(p, r2, 1.0 / 16.0);
-    p = __builtin_fma(p, r2, 1.0 / 8.0);
-    p = __builtin_fma(p, r2, 1.0 / 2.0);
-    return p * r2;
+    return n_series(l, m);
 }
 
 // exp(sign 2 pi i w n) with w = (z + 0.5) w_step, reduced to a fraction of a turn in FP64.
@@ -221,29 +212,6 @@ template <int R, int SG> __device__ __forceinline__ void dft(float2 *v)
             v[k + R / 2] = f2sub(e[k], t);
         }
     }
-}
-
-// A point loaded or stored past the caches (nontemporal) or through them.
-template <bool ONCE> __device__ __forceinline__ float2 load_point(const float2 *p)
-{
-    if constexpr (ONCE)
-    {
-        typedef float pair __attribute__((ext_vector_type(2)));
-        const pair r = __builtin_nontemporal_load(reinterpret_cast<const pair *>(p));
-        return make_float2(r[0], r[1]);
-    }
-    else
-        return *p;
-}
-template <bool ONCE> __device__ __forceinline__ void store_point(float2 *p, float2 v)
-{
-    if constexpr (ONCE)
-    {
-        typedef float pair __attribute__((ext_vector_type(2)));
-        __builtin_nontemporal_store(pair{v.x, v.y}, reinterpret_cast<pair *>(p));
-    }
-    else
-        *p = v;
 }
 
 enum FftPass

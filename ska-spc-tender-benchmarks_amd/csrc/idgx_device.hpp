@@ -190,6 +190,49 @@ __device__ __forceinline__ void load_jones(const float4 *aterms, size_t pixel_in
     a[3] = {hi.z, hi.w};
 }
 
+// n(l, m) = 1 - sqrt(1 - r^2) by its series: within 1e-11 of itself for r^2 <= 0.02 (fields up to 0.2 rad), in 10 FP64
+// operations instead of a square root and a division.
+__device__ __forceinline__ double n_series(double l, double m)
+{
+    const double r2 = __builtin_fma(l, l, m * m);
+    double p = 33.0 / 2048.0;
+    p = __builtin_fma(p, r2, 21.0 / 1024.0);
+    p = __builtin_fma(p, r2, 7.0 / 256.0);
+    p = __builtin_fma(p, r2, 5.0 / 128.0);
+    p = __builtin_fma(p, r2, 1.0 / 16.0);
+    p = __builtin_fma(p, r2, 1.0 / 8.0);
+    p = __builtin_fma(p, r2, 1.0 / 2.0);
+    return p * r2;
+}
+
+// ---- memory ---------------------------------------------------------------------------------------------------
+
+// A point loaded or stored past the caches (nontemporal) or through them.
+template <bool ONCE, class V> __device__ __forceinline__ V load_point(const V *p)
+{
+    if constexpr (ONCE)
+    {
+        typedef decltype(V::x) pair __attribute__((ext_vector_type(2)));
+        const pair r = __builtin_nontemporal_load(reinterpret_cast<const pair *>(p));
+        V v;
+        v.x = r[0];
+        v.y = r[1];
+        return v;
+    }
+    else
+        return *p;
+}
+template <bool ONCE, class V> __device__ __forceinline__ void store_point(V *p, V v)
+{
+    if constexpr (ONCE)
+    {
+        typedef decltype(V::x) pair __attribute__((ext_vector_type(2)));
+        __builtin_nontemporal_store(pair{v.x, v.y}, reinterpret_cast<pair *>(p));
+    }
+    else
+        *p = v;
+}
+
 // ---- plan checks done on the device ----------------------------------------------------------------------------
 
 struct PlanDev

@@ -152,20 +152,6 @@ __device__ __forceinline__ Slopes reduce_slopes(float u, float v, float w, float
     return s;
 }
 
-// n(l, m) = 1 - sqrt(1 - r^2) by its series: within 1e-11 of itself for r^2 <= 0.02 (fields up to 0.2 rad).
-__device__ __forceinline__ double pixel_n_series(double l, double m)
-{
-    const double r2 = __builtin_fma(l, l, m * m);
-    double p = 33.0 / 2048.0;
-    p = __builtin_fma(p, r2, 21.0 / 1024.0);
-    p = __builtin_fma(p, r2, 7.0 / 256.0);
-    p = __builtin_fma(p, r2, 5.0 / 128.0);
-    p = __builtin_fma(p, r2, 1.0 / 16.0);
-    p = __builtin_fma(p, r2, 1.0 / 8.0);
-    p = __builtin_fma(p, r2, 1.0 / 2.0);
-    return p * r2;
-}
-
 // e^{2 pi i (f + q / 4)} for |f| <= 1/8 of a turn, to about an FP32 rounding: the Taylor series, cut off below 2e-9.
 __device__ __forceinline__ cfloat phasor_series(float f, int q)
 {
@@ -205,7 +191,7 @@ template <bool SERIES> __device__ __forceinline__ void phasor(float ph, float &s
 // and what is left takes the series.  It costs 1.5 % of the gridder on 24^2 subgrids of 129 visibilities.
 __device__ __forceinline__ cfloat pixel_rotation(int x, int y, int S, double delta, double w)
 {
-    const double n = pixel_n_series((x + 0.5 - 0.5 * S) * delta, (y + 0.5 - 0.5 * S) * delta);
+    const double n = n_series((x + 0.5 - 0.5 * S) * delta, (y + 0.5 - 0.5 * S) * delta);
     const double t = __builtin_amdgcn_fract(w * n);
     const float quarters = __builtin_rintf(4.F * static_cast<float>(t)); // 0 to 4
     return phasor_series(static_cast<float>(__builtin_fma(-0.25, static_cast<double>(quarters), t)),

@@ -51,32 +51,6 @@ template <> struct Vec<double>
     using type = double2;
 };
 
-// A point loaded or stored past the caches (nontemporal) or through them.
-template <bool ONCE, class V> __device__ __forceinline__ V load_point(const V *p)
-{
-    if constexpr (ONCE)
-    {
-        typedef decltype(V::x) pair __attribute__((ext_vector_type(2)));
-        const pair r = __builtin_nontemporal_load(reinterpret_cast<const pair *>(p));
-        V v;
-        v.x = r[0];
-        v.y = r[1];
-        return v;
-    }
-    else
-        return *p;
-}
-template <bool ONCE, class V> __device__ __forceinline__ void store_point(V *p, V v)
-{
-    if constexpr (ONCE)
-    {
-        typedef decltype(V::x) pair __attribute__((ext_vector_type(2)));
-        __builtin_nontemporal_store(pair{v.x, v.y}, reinterpret_cast<pair *>(p));
-    }
-    else
-        *p = v;
-}
-
 // body(std::bool_constant<once>): one of two copies of a tile's loads or stores, by a launch-wide flag.
 template <class Body> __device__ __forceinline__ void with_policy(bool once, Body &&body)
 {
