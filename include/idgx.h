@@ -384,8 +384,9 @@ int idgx_plan_segments(const idgx_planner *planner, const float *d_uvw, const do
  * vis_offset[s+1]), each entry (t << 16) | c relative to the subgrid's first row and channel window.  Creation
  * allocates the queue memory; the execution entry points allocate nothing, and idgx_batch_capture records them into
  * a hipGraph (no memset nodes) for idgx_batch_launch.
- * The 3-product forms first take one launch per class of the separable kernels (subgrids up to 64^2, fields up to 0.13 rad, from 24^2
- * 0.16); the persistent launch then has only the subgrids whose w spreads too far over their visibilities.
+ * The 3-product forms first take one launch per class of the separable kernels (two where FP16 gridders have subgrids of
+ * many and of few visibilities; subgrids up to 64^2, fields up to 0.13 rad, from 24^2 0.16); the persistent launch then
+ * has only the subgrids whose w spreads too far over their visibilities.
  * Every precision batches: the mixed forms run their persistent MFMA kernels (shapes idgx_batch_shape_info), plain
  * FP32 the persistent forms of the plain kernels (shapes idgx_batch_plain_shape_info), which skip unselected
  * (flagged) samples instead of multiplying them by zero and otherwise round like idgx_grid / idgx_degrid.  They

@@ -192,8 +192,8 @@ int workgroups_for(const idgx_batch *b, bool gridder, int shape, int cls)
                     : idgx::queue_workgroups(b->precision, gridder, shape);
 }
 
-// A persistent launch over `items` of class `cls` (-1: of all): no more workgroups than items (each asks all queues for work before it ends, one atomic
-// after the other on the same counters).
+// A persistent launch over `items` of class `cls` (-1: of all): no more workgroups than items (each asks all queues for
+// work before it ends, one atomic after the other on the same counters).
 hipError_t launch_queue(const idgx_batch *b, const QueueArgs &q, bool gridder, int shape, int cls, int resident,
                         int items, hipStream_t st)
 {

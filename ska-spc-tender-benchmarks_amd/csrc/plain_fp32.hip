@@ -1306,8 +1306,8 @@ int plain_default_shape(bool gridder, int S)
 
 // One pixel per thread makes three to nine items of one: each costs the queue 0.1 us, and of 256 pixels saves 0.15 us per
 // visibility of the subgrid as long as the chip is not full.  Gridder time over that of the default shapes, by
-// visibilities a subgrid: 512 of 32^2 (2048 items for 512) 16 1.68, 256 1.27, 512 0.85; 1000 of them 256 1.35, 512 0.97, 1024
-// 0.86; 2000 512 1.11, 1024 0.99; 276 of 24^2 (828 for 276) 0.6 to 0.7 at any count.
+// visibilities a subgrid: 512 of 32^2 (2048 items for 512) 16 1.68, 256 1.27, 512 0.85; 1000 of them 256 1.35, 512 0.97,
+// 1024 0.86; 2000 512 1.11, 1024 0.99; 276 of 24^2 (828 for 276) 0.6 to 0.7 at any count.
 // Degridder: subgrids of up to 256 visibilities leave half the waves of an item of 512 without any (3000 of 48^2 with 128
 // 0.73, 256 0.95); beyond, small plans where an item of 256 has kFinePairs pixels x visibilities (1000 of 24^2 with 288
 // 1.09, of 32^2 0.97).

@@ -6,14 +6,17 @@
 //     qu xh + qv yh + dw n(l, m),    qu = du delta, qv = dv delta  (du, dv, dw relative to the subgrid's centre).
 // The w-term is taken apart in two steps.  Per subgrid, w0 = the middle of the range of w over its visibilities:
 // e^{2 pi i w0 n} is one exact rotation per pixel, applied to the gridder's result and to the degridder's pixels.
-// For the rest, d = dw - w0, n splits into an additive part and a remainder that is a product to about 1e-6 of itself:
+// For the rest, d = dw - w0, n splits into an additive part and a remainder that is a product but for 2e-6 of its corner
+// value at a field of 0.1 rad (2e-5 at 0.17):
 //     n(l, m) = a(l) + a(m) + c g(l) g(m),   a(l) = n(l, l0) - n(l0, l0) / 2,  l0 = l_max / sqrt(2),
 // where c = n's remainder at the corner and g, |g| <= 1, its profile along the edge (n = (l^2 + m^2) / 2 + (l^2 + m^2)^2
 // / 8 + ..., so the remainder is (l^2 - l0^2)(m^2 - l0^2) / 4 to first order: 3.5e-7 at a field of 0.1 rad).  So
 //     e^{2 pi i phase} = X(x) Y(y) (1 + i eps g(x) g(y)),   eps = 2 pi c d,
 //     X = e^{2 pi i (qu xh + d a(x))},  Y = e^{2 pi i (qv yh + d a(y))}
-// up to eps^2 / 2.  Subgrids with |eps| <= kEpsNone run without the product term; up to a limit (separable_tables) with it; the others
-// (fields far wider than 0.1 rad, or w far from constant over a subgrid) take the per-pair items.
+// up to eps^2 / 2.  Subgrids with |eps| <= kEpsNone run without the product term (FP16 gridders of few visibilities always
+// with it), up to a limit (kEpsGrid, kEpsDegrid) with it; the others (fields wider than 0.1 rad, or w far from constant over
+// a subgrid) are left to the per-pair kernels: a launch of theirs behind this one, or where a one-shot plan lets expect
+// none, their items inside it.
 //
 // Contraction, on v_mfma_f32_32x32x16.  Gridder: pixel[y][x, corr] = sum_v Y[y][v] (V[v][corr] X[v][x]), one real GEMM
 // with the rows (y, re/im), the columns (x, corr) and k = (v, re/im): the rows hold Y's two real embeddings, the B operand
@@ -27,10 +30,10 @@
 //
 // What bounds it: the matrix cores, at the power limit.  A pair costs 128 flop there (4 products of 32).  On 128 stations,
 // 64 channels, 76,865 subgrids of 32^2 (136.3 G pairs) a pass is 17.4 PFLOP, 14.7 ms at the rate a large FP16 product
-// reaches on the card (1186 TFLOP/s, clocks at 1.7 to 2.0 GHz).  Measured: gridder 41.2 -> 15.8 ms, degridder 41.3 ->
-// 15.2 ms; the per-pair kernels, 8.25 VALU instructions per pair (two of them transcendental), were VALU-issue bound at
-// 97 %; these issue 2.2 and 1.7.  The interleaving of MFMA and VALU instructions (scheduling groups, wave priorities)
-// and the tile (16 x 16 x 32: more cycles at a higher clock) moved the time by less than 3 %.
+// reaches on the card (1186 TFLOP/s, clocks at 1.7 to 2.0 GHz).  Measured: gridder 41.2 -> 16.1 ms, degridder 41.3 ->
+// 15.2 ms (cards differ by 3 %); the per-pair kernels, 8.25 VALU instructions per pair (two of them transcendental), were
+// VALU-issue bound at 97 %; these issue 2.2 and 1.7.  The interleaving of MFMA and VALU instructions (scheduling groups,
+// wave priorities) and the tile (16 x 16 x 32: more cycles at a higher clock) moved the time by less than 3 %.
 #include "mixed_device.hpp"
 
 #include <algorithm>
